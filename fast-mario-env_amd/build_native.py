@@ -16,12 +16,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 SRC = os.path.join(HERE, "csrc", "mario_hip.hip")
 OUT = os.path.join(HERE, "fast_mario_env_amd", "libmario_hip.so")
 ARCH = os.environ.get("MARIO_HIP_ARCH", "gfx950")
-# -O2 with LLVM's iterative ILP scheduler: k_step 18.14 -> 17.46 ms at the headline workload (the frame loop is
-# bound by instruction issue; -O3 alone 18.14, -O2 alone 17.82, the scheduler alone 17.79 ms).
-# -structurizecfg-skip-uniform-regions: branches on wave-uniform conditions keep their own control flow instead of
-# the structurizer's flag variables and joins. lone_long's 256-way opcode switch (wave-uniform) becomes a plain
-# compare tree into each body: a lone instruction 372 -> 198 ns (register-only loop), raw 522k -> 604k env-frames/s,
-# stress k_step 51.2 -> 46.5 ms, headline k_step 16.40 -> 16.24 ms (same-box A/B).
+# -structurizecfg-skip-uniform-regions: branches on wave-uniform conditions (all of the emulator's) keep their own control
+# flow instead of the structurizer's flag variables and joins.
 FLAGS = ["-O2", "-mllvm", "-amdgpu-sched-strategy=iterative-ilp", "-mllvm", "-structurizecfg-skip-uniform-regions=true",
          "-std=c++17", "-fPIC", "-shared",
          "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wall"]

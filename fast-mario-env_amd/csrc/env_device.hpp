@@ -123,72 +123,32 @@ struct Cfg {
     double sticky;
 };
 
-// Memory region of consoles with the same layout as the live state (reset cache, boot states).
+// Memory region of consoles with the same layout as the live state (reset cache, boot states, snapshots).
 struct Region {
-    uint8_t* mem;       // row-major [row * np + idx], VRAM word-interleaved (vram_word_offset)
+    uint8_t* mem;       // row r of console idx at mem_offset(np, idx, r)
     uint32_t* sc;       // [word * np + idx]
     uint32_t np;
     uint32_t idx;
 };
 
-__device__ inline void copy_console(const Region& dst, const Region& src) {
-    for (uint32_t r = 0; r < MEM_ROWS; r++)
-        if (r < ROW_VRAM || r >= ROW_VRAM + 2048) dst.mem[(size_t)r * dst.np + dst.idx] = src.mem[(size_t)r * src.np + src.idx];
-    for (uint32_t w = 0; w < 512; w++)
-        *(uint32_t*)(dst.mem + vram_word_offset(dst.np, dst.idx, w)) =
-            *(const uint32_t*)(src.mem + vram_word_offset(src.np, src.idx, w));
-    for (int w = 0; w < S_COUNT; w++) dst.sc[(size_t)w * dst.np + dst.idx] = src.sc[(size_t)w * src.np + src.idx];
-}
-
-// copy_console by the `lanes` lanes of a wave together, lane `lane` taking every lanes-th byte row, VRAM
-// word and register word: one console is a few thousand independent accesses, too many for one lane.
+// A console copied by `lanes` lanes together (16 bytes an access on the GPU, where a console's memory is contiguous).
 __device__ inline void copy_console_wave(const Region& dst, const Region& src, uint32_t lane, uint32_t lanes) {
-    constexpr uint32_t BYTE_ROWS = MEM_ROWS - 2048;   // every row but the VRAM span
-    for (uint32_t i = lane; i < BYTE_ROWS; i += lanes) {
-        const uint32_t r = i < (uint32_t)ROW_VRAM ? i : i + 2048;
-        dst.mem[(size_t)r * dst.np + dst.idx] = src.mem[(size_t)r * src.np + src.idx];
+    if constexpr (ON_GPU) {
+        mh_u32x4* d = (mh_u32x4*)(dst.mem + mem_offset(dst.np, dst.idx, 0));
+        const mh_u32x4* s = (const mh_u32x4*)(src.mem + mem_offset(src.np, src.idx, 0));
+        for (uint32_t i = lane; i < MEM_ROWS / 16; i += lanes) d[i] = s[i];
+    } else {
+        for (uint32_t r = lane; r < MEM_ROWS; r += lanes)
+            dst.mem[mem_offset(dst.np, dst.idx, r)] = src.mem[mem_offset(src.np, src.idx, r)];
     }
-    for (uint32_t w = lane; w < 512; w += lanes)
-        *(uint32_t*)(dst.mem + vram_word_offset(dst.np, dst.idx, w)) =
-            *(const uint32_t*)(src.mem + vram_word_offset(src.np, src.idx, w));
     for (uint32_t w = lane; w < (uint32_t)S_COUNT; w += lanes)
         dst.sc[(size_t)w * dst.np + dst.idx] = src.sc[(size_t)w * src.np + src.idx];
 }
 
-// The memory rows of copy_console (not the register words), by one lane: the loads of a batch of 32 are
-// issued before its stores, so the lane keeps 32 accesses in flight instead of waiting for each one.
-__device__ inline void copy_rows_lane(const Region& dst, const Region& src) {
-    constexpr uint32_t B = 32, BYTE_ROWS = MEM_ROWS - 2048;   // the VRAM span aside
-    static_assert(BYTE_ROWS % B == 0 && ROW_VRAM % B == 0 && 512 % B == 0, "batches must not straddle the VRAM span");
-    for (uint32_t i0 = 0; i0 < BYTE_ROWS; i0 += B) {
-        const uint32_t r0 = i0 < (uint32_t)ROW_VRAM ? i0 : i0 + 2048;
-        uint8_t t[B];
-#pragma unroll
-        for (uint32_t b = 0; b < B; b++) t[b] = src.mem[(size_t)(r0 + b) * src.np + src.idx];
-#pragma unroll
-        for (uint32_t b = 0; b < B; b++) dst.mem[(size_t)(r0 + b) * dst.np + dst.idx] = t[b];
-    }
-    for (uint32_t w0 = 0; w0 < 512; w0 += B) {
-        uint32_t t[B];
-#pragma unroll
-        for (uint32_t b = 0; b < B; b++) t[b] = *(const uint32_t*)(src.mem + vram_word_offset(src.np, src.idx, w0 + b));
-#pragma unroll
-        for (uint32_t b = 0; b < B; b++) *(uint32_t*)(dst.mem + vram_word_offset(dst.np, dst.idx, w0 + b)) = t[b];
-    }
-}
-
-// Snapshot of a console between two frames into `dst` (a region of the same np, at the console's own
-// index): store() of the registers (and of the LDS copy of OAM into the console's rows), then its rows.
-__device__ inline void save_console(Console& c, const Region& live, const Region& dst) {
-    c.store(dst.sc, dst.idx);
-    copy_rows_lane(dst, live);
-}
-// The console as snapshotted: rows back, then load() of the registers (OAM to LDS, derived caches reset).
-// The instruction and bad-op counters are not part of the snapshot and keep counting.
-__device__ inline void restore_console(Console& c, const Region& live, const Region& src) {
-    copy_rows_lane(live, src);
-    c.load(src.sc, src.idx);
-}
+// Snapshot of a console between two frames into `dst`, and back (each lane reads what it wrote). The instruction and
+// bad-op counters are not part of the snapshot and keep counting.
+__device__ __forceinline__ void save_console(Console& c, const Region& dst) { c.store(dst.mem, dst.sc, dst.idx); }
+__device__ __forceinline__ void restore_console(Console& c, const Region& src) { c.load(src.mem, src.sc, src.idx); }
 
 // One env's layer state in registers.
 struct EnvRegs {
@@ -210,18 +170,18 @@ struct Stepper {
     Pcg* rng;             // null: draws are counted, not taken (reset cache: action 0 == prev 0)
     uint8_t* gray0;       // frame buffer of frames K-1, K-3, ... of the agent step
     uint8_t* gray1;       // frame buffer of frames K-2, K-4, ...
-    Region live;          // the console's own rows and register words
-    uint8_t* snap_mem;    // two snapshot slots of live's layout: rows of slot s at snap_mem + s MEM_ROWS np,
+    uint32_t np, idx;     // envs of the snapshot slots, padded, and this console's place
+    uint8_t* snap_mem;    // two snapshot slots of the live layout: memory of slot s at snap_mem + s MEM_ROWS np,
     uint32_t* snap_sc;    // register words at snap_sc + s S_COUNT np
 
     __device__ __forceinline__ Region snap(int s) const {
-        return Region{snap_mem + (size_t)s * MEM_ROWS * live.np, snap_sc + (size_t)s * S_COUNT * live.np, live.np, live.idx};
+        return Region{snap_mem + (size_t)s * MEM_ROWS * np, snap_sc + (size_t)s * S_COUNT * np, np, idx};
     }
     __device__ __forceinline__ bool busy() { return smb_busy(c) || smb_world_over(c); }
     // _skip_change_area before the _skip_occupied_states loop (fastmario.cpp:297-300)
     __device__ __forceinline__ void fix_change_area() {
         const uint8_t cat = c.ram(0x6de);
-        if (cat > 1 && cat < 255) c.st(ROW_RAM + 0x6de, 1);
+        if (cat > 1 && cat < 255) c.set_ram(0x6de, 1);
     }
     // reward, done and info after an agent frame (fastmario.cpp:310-334)
     __device__ __forceinline__ double frame_reward(bool* done) {
@@ -280,7 +240,7 @@ struct Stepper {
             it++;
             uint8_t buttons = 0;
             if (hack) {
-                c.st(ROW_RAM + 0x7a0, 0);
+                c.set_ram(0x7a0, 0);
                 // A hack frame of a drawn agent frame is drawn only if it ends the busy run: it runs undrawn
                 // from a snapshot and, when busy() clears after it, runs again drawn (below). A CPU frame
                 // covers a whole PPU frame, so the last frame's pixels are the whole picture, as in the
@@ -288,7 +248,7 @@ struct Stepper {
                 // frames did not end the episode, so no re-emulation can follow in this step.
                 undrawn = rf < 0 && render && !redraw;
                 if (undrawn) {
-                    save_console(c, live, snap(0));
+                    save_console(c, snap(0));
                     hn = c.instructions; hb = c.bad_ops; hf = c.ff_instructions;
                 }
             } else if (rf < 0) {
@@ -305,7 +265,7 @@ struct Stepper {
                 n0 = c.instructions; b0 = c.bad_ops; f0 = c.ff_instructions;
                 // re-emulations start at frame last-1 (max-pool, last >= 1) or last, for last < K-1, and
                 // never at K-2 (max-pool)
-                if (want_obs && i < K - 1 && (!mp || i <= K - 3)) save_console(c, live, snap(i & 1));
+                if (want_obs && i < K - 1 && (!mp || i <= K - 3)) save_console(c, snap(i & 1));
             } else {
                 buttons = rf == i ? b_cur : b_prev;
                 render = true;
@@ -328,7 +288,7 @@ struct Stepper {
                 }
                 if (undrawn && !(c.bad_ops & ERR_HACK_LIMIT)) {
                     // the busy run ended with an undrawn hack frame: back to its start, counted once
-                    restore_console(c, live, snap(0));
+                    restore_console(c, snap(0));
                     c.instructions = hn; c.bad_ops = hb; c.ff_instructions = hf;
                     ev.frames--;
                     ev.hack_redraws++;
@@ -350,14 +310,14 @@ struct Stepper {
                     c.bad_ops += db;
                     c.ff_instructions += c.ff_instructions - f0;
                     if (i == 0) break;
-                    save_console(c, live, snap(i & 1));
+                    save_console(c, snap(i & 1));
                     keep_last = true;
                     rf = i - 1;
                 } else {
                     rf = (mp && i >= 1) ? i - 1 : i;
                 }
                 resume_at = K - (keep_last ? 1 : i - rf + 1);   // K minus the frames to run again
-                restore_console(c, live, snap(rf & 1));
+                restore_console(c, snap(rf & 1));
             } else if (rf < i) {
                 // frame last-1 again, then its hack frames (it did not end the episode)
                 if (!hack) { fix_change_area(); guard = 0; }
@@ -366,7 +326,7 @@ struct Stepper {
                     c.bad_ops |= ERR_HACK_LIMIT;
                 }
                 hack = false;
-                if (keep_last) { restore_console(c, live, snap(i & 1)); break; }
+                if (keep_last) { restore_console(c, snap(i & 1)); break; }
                 rf++;
             } else {
                 break;

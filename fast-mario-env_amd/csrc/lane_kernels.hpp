@@ -1,5 +1,5 @@
-// Per-lane bodies of the env kernels (one env / level / cache entry per lane). The __global__ wrappers
-// in mario_hip.hip stage the cartridge in LDS and call these.
+// Bodies of the env kernels: one env / level / cache entry per wave (reset_lane, canon_lane: per lane). The __global__
+// wrappers in mario_hip.hip stage the cartridge in LDS and call these.
 #pragma once
 #include <cmath>
 
@@ -181,9 +181,10 @@ __device__ __forceinline__ uint8_t round_sat(float v) {
     return (uint8_t)(iv < 0 ? 0 : iv > 255 ? 255 : iv);
 }
 
-// Frame buffers (GRAY) hold 4 pixels per 32-bit word, lane-interleaved: pixel p of lane e of a
-// buffer with np lanes is byte ((p / 4) * np + e) * 4 + p % 4. An Image addresses one lane's frame
-// in such a buffer, or a plain row-major 256x240 frame when np == 0.
+// Frame buffers (GRAY) hold whole row-major 256x240 frames one after the other on the GPU; on the host build they
+// are interleaved by env in words of 4 pixels: pixel p of env e of a buffer for np envs is byte
+// ((p / 4) * np + e) * 4 + p % 4. An Image addresses one env's frame in an interleaved buffer, or a plain
+// row-major frame when np == 0.
 struct Image {
     const uint8_t* base;
     uint32_t np, e;
@@ -191,7 +192,7 @@ struct Image {
         return np ? base[((size_t)(p >> 2) * np + e) * 4 + (p & 3)] : base[p];
     }
 };
-__host__ __device__ __forceinline__ size_t gray_lane_offset(uint32_t e) { return (size_t)e * 4; }
+__host__ __device__ __forceinline__ size_t gray_lane_offset(uint32_t e) { return ON_GPU ? (size_t)e * GRAY_PIX : (size_t)e * 4; }
 
 // INTER_AREA output pixel o of one image, max-pooled with a second one if `pool`.
 __device__ __forceinline__ uint8_t area_pixel(const Image& g0, const Image& g1, bool pool, int o, const AreaTables* T) {
@@ -270,14 +271,15 @@ struct RomArgs {
     const uint8_t* lut;      // 256
     uint32_t nt_bits;        // bit k: name table k maps to VRAM $400
     int n_chr;               // CHR banks, 1 .. MAX_CHR_BANKS
+    const uint32_t* recs;    // the program as scalar_run's records (REC_COUNT words; none on the host build)
 };
 
-__device__ __forceinline__ Cart make_cart(const RomArgs& R, const uint8_t* s_rom, const uint32_t* s_dec) {
+__device__ __forceinline__ Cart make_cart(const RomArgs& R, const MH_LDS uint8_t* s_rom, const uint32_t* dec) {
     Cart c;
     c.prg = s_rom;
-    c.gprg = R.rom;
     c.chr = s_rom + 0x8000;
-    c.dec = s_dec;
+    c.dec = dec;
+    c.recs = R.recs;
     c.nt_bits = R.nt_bits;
     return c;
 }
@@ -285,22 +287,17 @@ __device__ __forceinline__ Cart make_cart(const RomArgs& R, const uint8_t* s_rom
 // What a lane needs from its block: the staged cartridge, the gray LUT and its LDS render buffers.
 struct LaneCtx {
     Cart cart;
-    const uint8_t* lut;
-    uint32_t* sp;     // this lane's sprite line buffer (stride LDS_LANES words)
-    uint32_t* gp;     // this lane's gray palette, tile row and OAM (stride LDS_LANES words)
-    uint8_t part;     // which of the env's LANES_PER_ENV lanes this is
+    const MH_LDS uint8_t* lut;
+    MH_LDS uint32_t* sp;     // the console's memory in LDS (LDS_SP_WORDS)
+    MH_LDS uint32_t* gp;     // its renderer's words (LDS_GP_REGION)
+    uint8_t lane;     // this lane of the console's wave
 };
 
-// console e of the memory block `mem` (np consoles), on CHR bank `bank` of the staged cartridge
-__device__ __forceinline__ void attach(Console& c, const LaneCtx& x, uint8_t* mem, uint32_t np, uint32_t e,
-                                       uint32_t bank = 0) {
-    c.mbase = mem; c.eo = e; c.vo = (uint32_t)vram_word_offset(np, e, 0); c.np = np;
-    c.cart = x.cart; c.cart.chr += bank * 0x2000u; c.lut = x.lut; c.lds_sp = x.sp; c.lds_gp = x.gp;
-    c.lds_bg = x.gp + LDS_GP_WORDS * LDS_LANES; c.bg_key = -1;
-    c.lds_oam = x.gp + (LDS_GP_WORDS + LDS_BG_WORDS) * LDS_LANES;
-    c.part = x.part;
+// a console on CHR bank `bank` of the staged cartridge, its memory blocks and frame buffers of np envs
+__device__ __forceinline__ void attach(Console& c, const LaneCtx& x, uint32_t np, uint32_t bank = 0) {
+    c.m = (MH_LDS uint8_t*)x.sp; c.gp = x.gp; c.np = np;
+    c.cart = x.cart; c.cart.chr += bank * 0x2000u; c.lut = x.lut; c.lane = x.lane;
     c.bad_ops = 0; c.instructions = 0; c.ff_instructions = 0;
-    c.pend_line = -1; c.sp_line = -1; c.pal_dirty = true;
 }
 
 struct BootArgs {
@@ -344,10 +341,6 @@ struct StepArgs {
     const int32_t* slot_env;      // env of each console slot (actions in and outputs out are in env order)
     uint8_t* fresh;               // new observation of each slot: [e * OBS_PIX + o]
     const uint8_t* boot_obs;      // boot observation of each level: [level * OBS_PIX + o]
-    uint32_t* obs_order;          // [0]: waves that finished their frame loop (0 at launch); [1 + k]: the first
-                                  // slot of the wave whose ticket is obs_late_from + k
-    uint32_t obs_late_from;       // waves with a ticket in [obs_late_from, obs_late_to) leave their
-    uint32_t obs_late_to;         // observations to k_obs_late (obs_late_to: the waves with live envs)
 };
 
 struct ResetArgs {
@@ -370,7 +363,7 @@ struct RawArgs {
     int render;
     uint32_t* bad; uint32_t* instr; uint32_t* ff;
     int power_on;
-    int cpw;                     // consoles per wave (k_raw): 1, 2, 4, 8 or ENVS_PER_WAVE
+    int cpw;                     // consoles per wave: 1
 };
 
 // ------------------------------------------------------------------ env words
@@ -405,28 +398,42 @@ __device__ __forceinline__ void add_counter(uint32_t* E, uint32_t np, uint32_t e
 // Power-on and title sequence with the target level written into RAM (fastmario.cpp:414-445).
 __device__ inline void boot_lane(const BootArgs& A, const LaneCtx& x, int l) {
     Console c;
-    attach(c, x, A.mem, A.nlp, (uint32_t)l, A.key_bank[l]);
+    attach(c, x, A.nlp, A.key_bank[l]);
     c.gray = A.gray + gray_lane_offset(l); c.render = true;
     c.power_on();
-    auto fr = [&](uint8_t b) { c.set_buttons0(b); c.frame(); };
     const int w = A.levels[3 * l], s = A.levels[3 * l + 1], ar = A.levels[3 * l + 2];
-    fr(8); fr(0);
+    // one frame after the other from one place, so that the emulator is inlined once: Start held (8) and released in
+    // turn, with the level written into RAM while the title waits for it
+    int64_t tl = -1;                   // the game's time once it runs
     int guard = 0;
-    while (smb_time(c) == 0) {
-        if (++guard > HACK_FRAME_LIMIT) { atomicOr(A.err, 1u); break; }
-        fr(8);
-        c.st(ROW_RAM + 0x75f, (uint8_t)(w - 1)); c.st(ROW_RAM + 0x75c, (uint8_t)(s - 1));
-        c.st(ROW_RAM + 0x760, (uint8_t)(ar - 1));
-        fr(0);
-        c.st(ROW_RAM + 0x7a0, 0);
-    }
-    int64_t tl = smb_time(c);
-    guard = 0;
-    while (smb_time(c) >= tl) {
+    bool first = true;
+    for (bool held = true;; held = !held) {
+        c.set_buttons0(held ? 8 : 0);
+        c.frame();
+        if (held) {
+            if (!first && tl < 0) {
+                c.set_ram(0x75f, (uint32_t)(w - 1)); c.set_ram(0x75c, (uint32_t)(s - 1)); c.set_ram(0x760, (uint32_t)(ar - 1));
+            }
+            continue;
+        }
+        if (tl < 0) {
+            if (!first) c.set_ram(0x7a0, 0);
+            first = false;
+            const int64_t now = smb_time(c);
+            if (now == 0) {
+                if (++guard > HACK_FRAME_LIMIT) { atomicOr(A.err, 1u); break; }
+                continue;
+            }
+            tl = now;
+            guard = 1;
+            continue;
+        }
+        const int64_t now = smb_time(c);
+        if (now < tl) break;
+        tl = now;
         if (++guard > HACK_FRAME_LIMIT) { atomicOr(A.err, 2u); break; }
-        tl = smb_time(c); fr(8); fr(0);
     }
-    c.store(A.sc, l);
+    c.store(A.mem, A.sc, (uint32_t)l);
     A.x0[l] = smb_x(c);
     A.t0[l] = smb_time(c);
 }
@@ -438,26 +445,28 @@ __device__ inline void cache_lane(const CacheArgs& A, const LaneCtx& x, int ci) 
     const int lvl = ci / A.nk, k = ci - lvl * A.nk;
     Region boot{(uint8_t*)A.boot_mem, (uint32_t*)A.boot_sc, A.nlp, (uint32_t)lvl};
     Region live{A.mem, A.sc, A.ncp, (uint32_t)ci};
-    copy_console(live, boot);
+    copy_console_wave(live, boot, x.lane, LANES);
+    Console::mem_sync();
     Console c;
-    attach(c, x, A.mem, A.ncp, (uint32_t)ci, A.key_bank[lvl]);
-    c.load(A.sc, ci);
+    attach(c, x, A.ncp, A.key_bank[lvl]);
+    c.load(A.mem, A.sc, (uint32_t)ci);
     EnvRegs ev{};
     ev.x_last = A.x0[lvl]; ev.time_last = A.t0[lvl];
     ev.prev = 0; ev.lives = -1; ev.shows_boot = true; ev.frames = 0; ev.draws = 0;
     Stepper stp{c, ev, A.cfg, nullptr, A.gray + gray_lane_offset(ci), A.gray + (size_t)GRAY_PIX * A.ncp + gray_lane_offset(ci),
-                live, A.snap_mem, A.snap_sc};
+                A.ncp, (uint32_t)ci, A.snap_mem, A.snap_sc};
     for (int j = 0; j < k; j++) {
         bool term;
         stp.agent_step(0, j == k - 1, &term);
         if (term) {
-            copy_console(live, boot);
-            c.load(A.sc, ci);
+            copy_console_wave(live, boot, x.lane, LANES);
+            Console::mem_sync();
+            c.load(A.mem, A.sc, (uint32_t)ci);
             ev.x_last = A.x0[lvl]; ev.time_last = A.t0[lvl];
             ev.prev = 0; ev.lives = -1; ev.shows_boot = true;
         }
     }
-    c.store(A.sc, ci);
+    c.store(A.mem, A.sc, (uint32_t)ci);
     A.cx[ci] = ev.x_last; A.ct[ci] = ev.time_last; A.clives[ci] = ev.lives;
     A.cdraws[ci] = (int32_t)ev.draws; A.cboot[ci] = ev.shows_boot;
     A.cframes[ci] = ev.frames; A.cinstr[ci] = c.instructions; A.cff[ci] = c.ff_instructions; A.cbad[ci] = c.bad_ops;
@@ -470,8 +479,8 @@ __device__ inline uint32_t step_lane(const StepArgs& A, const LaneCtx& x, uint32
     const uint32_t o = (uint32_t)A.slot_env[e];   // the env's index in the action and output arrays
     Console c;
     const uint32_t level = A.ev[(size_t)E_LEVEL * A.np + e];
-    attach(c, x, A.mem, A.np, e, A.key_bank[level]);
-    c.load(A.sc, e);
+    attach(c, x, A.np, A.key_bank[level]);
+    c.load(A.mem, A.sc, e);
     EnvRegs ev;
     load_env(ev, A.ev, A.np, e);
     Pcg rng;
@@ -479,7 +488,7 @@ __device__ inline uint32_t step_lane(const StepArgs& A, const LaneCtx& x, uint32
     int64_t a64 = A.actions[o];
     const int act = (a64 >= 0 && a64 < 7) ? (int)a64 : 0;
     Stepper stp{c, ev, A.cfg, &rng, A.gray + gray_lane_offset(e), A.gray + (size_t)GRAY_PIX * A.np + gray_lane_offset(e),
-                Region{A.mem, A.sc, A.np, e}, A.snap_mem, A.snap_sc};
+                A.np, e, A.snap_mem, A.snap_sc};
     bool tm;
     double r = stp.agent_step(act, true, &tm);
     ev.t++;
@@ -491,7 +500,7 @@ __device__ inline uint32_t step_lane(const StepArgs& A, const LaneCtx& x, uint32
     for (int k = 0; k < 10; k++) A.info[(size_t)o * 10 + k] = (int32_t)ev.info.v[k];
     const bool done = tm || tr;
     if (done) { A.ep_ret_out[o] = ev.ep_ret; A.ep_len_out[o] = ev.ep_len; }
-    c.store(A.sc, e);
+    c.store(A.mem, A.sc, e);
     store_env(ev, A.ev, A.np, e);
     rng.store(A.ev, A.np, e);
     A.ev[(size_t)E_DONE * A.np + e] = done;
@@ -537,17 +546,17 @@ __device__ inline int reset_lane(const ResetArgs& A, uint32_t e) {
 // One nes-py frame of raw console e (fastmario.cpp:656-661); power_on != 0 boots it instead.
 __device__ inline void raw_lane(const RawArgs& A, const LaneCtx& x, uint32_t e) {
     Console c;
-    attach(c, x, A.mem, A.np, e);
+    attach(c, x, A.np);
     c.gray = A.screen + gray_lane_offset(e);
     if (A.power_on) {
         c.power_on();
     } else {
-        c.load(A.sc, e);
+        c.load(A.mem, A.sc, e);
         c.set_buttons0(A.buttons[e]);
         c.render = A.render != 0;
         c.frame();
     }
-    c.store(A.sc, e);
+    c.store(A.mem, A.sc, e);
     A.bad[e] += c.bad_ops;
     A.instr[e] += c.instructions;
     A.ff[e] += c.ff_instructions;
@@ -572,10 +581,9 @@ __device__ inline void canon_lane(const uint8_t* mem, const uint32_t* sc, uint32
     const uint32_t nsl = w(S_NSL);
     const uint64_t sl = (uint64_t)w(S_SL_LO) | ((uint64_t)w(S_SL_HI) << 32);
     for (uint32_t i = 0; i < 8; i++) o[69 + i] = i < nsl ? (uint8_t)(sl >> (8 * i)) : 0;
-    const uint32_t rows[3][3] = {{80, ROW_OAM, 256}, {336, ROW_PAL, 32}, {2416, ROW_RAM, 2048}};
-    for (int k = 0; k < 3; k++)
-        for (uint32_t i = 0; i < rows[k][2]; i++) o[rows[k][0] + i] = mem[(size_t)(rows[k][1] + i) * np + e];
-    for (uint32_t i = 0; i < 2048; i++) o[368 + i] = mem[vram_word_offset(np, e, i >> 2) + (i & 3)];
+    const uint32_t rows[4][3] = {{80, ROW_OAM, 256}, {336, ROW_PAL, 32}, {368, ROW_VRAM, 2048}, {2416, ROW_RAM, 2048}};
+    for (int k = 0; k < 4; k++)
+        for (uint32_t i = 0; i < rows[k][2]; i++) o[rows[k][0] + i] = mem[mem_offset(np, e, rows[k][1] + i)];
 }
 
 }  // namespace mh

@@ -1,9 +1,9 @@
 // mario_hip: batched Super Mario Bros env stepping on gfx950 — kernels and the C-ABI (include/mario_hip.h).
 //
 // One agent step of N envs is three kernels on the caller's stream:
-//   k_step          4 lanes per env: sticky draw, K frames of 6502 + catch-up PPU, reward/done/info,
-//                   hack frames, gray rendering of every frame into two alternating frame buffers; then, per
-//                   wave, the 2-frame max + INTER_AREA of its envs' last frames (obs_tail)
+//   k_step          a wave per env: sticky draw, K frames of 6502 + catch-up PPU, reward/done/info, hack
+//                   frames, gray rendering of the max-pool pair into two frame buffers; then the 2-frame max +
+//                   INTER_AREA of its last frames (obs_tail)
 //   k_reset         one lane per env: finished envs take a cached (level, no-op count) start state
 //   k_stack         frame-stack shift, final_obs, reset observation
 #include <hip/hip_runtime.h>
@@ -26,186 +26,114 @@ using namespace mh;
 
 namespace {
 
-// Stage PRG and the CHR banks (32 KB + 8 KB each), the gray LUT and the decode table in LDS; every thread of
+// Stage PRG and the CHR banks (32 KB + 8 KB each) and the gray LUT in LDS; every thread of
 // the block must call this.
-__device__ __forceinline__ void stage_rom(const RomArgs& R, uint8_t* s_rom, uint8_t* s_lut, uint32_t* s_dec) {
+__device__ __forceinline__ void stage_rom(const RomArgs& R, uint8_t* s_rom, uint8_t* s_lut) {
     const uint4* src = (const uint4*)R.rom;
     uint4* dst = (uint4*)s_rom;
     const int words = (0x8000 + R.n_chr * 0x2000) / 16;
     for (int i = threadIdx.x; i < words; i += blockDim.x) dst[i] = src[i];
-    for (int i = threadIdx.x; i < 256; i += blockDim.x) { s_lut[i] = R.lut[i]; s_dec[i] = kDecode.w[i]; }
+    for (int i = threadIdx.x; i < 256; i += blockDim.x) s_lut[i] = R.lut[i];
     __syncthreads();
 }
 
-// Block-shared LDS of the emulator kernels: the cartridge, the gray LUT and per-lane render buffers.
+// Block-shared LDS of the emulator kernels: the cartridge, the gray LUT and each console's share.
 #define ROM_LDS                                                     \
     __shared__ __attribute__((aligned(16))) uint8_t s_rom[0x8000 + MAX_CHR_BANKS * 0x2000]; \
     __shared__ uint8_t s_lut[256];                                  \
-    __shared__ uint32_t s_dec[256];                                 \
-    __shared__ uint32_t s_sp[LDS_SP_WORDS * LDS_LANES];              \
-    __shared__ uint32_t s_gp[LDS_GP_REGION * LDS_LANES];
+    __shared__ __attribute__((aligned(16))) uint32_t s_env[LDS_ENV_WORDS * LDS_LANES];
+static_assert(0x8000 + MAX_CHR_BANKS * 0x2000 + 256 + 4 * LDS_ENV_WORDS * LDS_LANES <= 160 * 1024, "a CU's LDS");
+static_assert(LDS_ENV_WORDS % 4 == 0, "a console's memory stays 16-byte aligned");
 
-// Env slot of this thread within its block (0 .. LDS_LANES-1). Lanes l, l + ENVS_PER_WAVE, ... of a wave are
-// the parts of one env: they run its console in lockstep (identical state, identical loads and stores of
-// identical values) and share its LDS buffers; only the renderer and the sprite evaluation give them
-// different work.
-__device__ __forceinline__ int lane_slot() {
-    return (int)(threadIdx.x >> 6) * ENVS_PER_WAVE + (int)(threadIdx.x & (ENVS_PER_WAVE - 1));
-}
-__device__ __forceinline__ uint8_t lane_part() {
-    return (uint8_t)(((threadIdx.x & 63u) / ENVS_PER_WAVE) & (LANES_PER_ENV - 1));
-}
-
-__device__ __forceinline__ LaneCtx lane_ctx(const RomArgs& R, const uint8_t* s_rom, const uint8_t* s_lut,
-                                            const uint32_t* s_dec, uint32_t* s_sp, uint32_t* s_gp, int slot) {
-    return LaneCtx{make_cart(R, s_rom, s_dec), s_lut, s_sp + slot, s_gp + slot, lane_part()};
+// Console slot of this wave in its block: wave-uniform, in a scalar register
+__device__ __forceinline__ uint32_t wave_slot() { return uni(threadIdx.x >> 6); }
+__device__ __forceinline__ LaneCtx lane_ctx(const RomArgs& R, const uint8_t* s_rom, const uint8_t* s_lut, uint32_t* s_env) {
+    MH_LDS uint32_t* const own = (MH_LDS uint32_t*)s_env + wave_slot() * LDS_ENV_WORDS;
+    return LaneCtx{make_cart(R, (const MH_LDS uint8_t*)s_rom, kDecode.w), (const MH_LDS uint8_t*)s_lut, own,
+                   own + LDS_SP_WORDS, (uint8_t)(threadIdx.x & 63u)};
 }
 
 constexpr int EMU_THREADS = 64 * WAVES_PER_BLOCK;
 #define EMU_BOUNDS __launch_bounds__(EMU_THREADS, EMU_WAVES_PER_SIMD)
-// blocks of an emulator kernel over `count` envs
-// Launch shape of an emulator kernel over `count` consoles on a GPU with `cus` compute units: blocks of up to
-// WAVES_PER_BLOCK waves (one block per CU: its LDS). When count is too small to give every CU a full block, the
+// Launch shape of an emulator kernel over `count` consoles, a wave each, on a GPU with `cus` compute units: blocks of up
+// to WAVES_PER_BLOCK waves (one block per CU: its LDS). When count is too small to give every CU a full block, the
 // blocks shrink (down to one wave) so that the waves spread over all CUs instead of sharing a few CUs' SIMDs.
 struct EmuLaunch { dim3 grid, block; };
 static inline EmuLaunch emu_launch(int count, int cus) {
-    const int per_full_wave = ENVS_PER_WAVE * (cus > 0 ? cus : 1);
-    int waves = (count + per_full_wave - 1) / per_full_wave;
-    waves = waves < 1 ? 1 : waves > WAVES_PER_BLOCK ? WAVES_PER_BLOCK : waves;
-    const int slots = waves * ENVS_PER_WAVE;
-    return EmuLaunch{dim3((unsigned)((count + slots - 1) / slots)), dim3((unsigned)(64 * waves))};
-}
-// Launch shape of k_raw over `count` consoles: fewer consoles per wave (a power of two, cpw) where the count is too
-// small to give every SIMD two waves of 16. A raw batch of 4,096 consoles is then 2,048 waves of 2 instead of 256
-// waves of 16 (one per CU, three of its four SIMDs idle): a wave's iterations follow the union of its consoles'
-// instruction streams and slice waits, so fewer consoles per wave also means fewer iterations per console, and
-// the lanes a wave leaves idle would have had no SIMD to run on anyway. force > 0 sets cpw instead (one of 1, 2, 4,
-// 8, 16: the MH_RAW_CONSOLES_PER_WAVE environment variable at mh_raw_create).
-static inline EmuLaunch raw_launch(int count, int cus, int force, int& cpw) {
-    const int target = 4 * EMU_WAVES_PER_SIMD * (cus > 0 ? cus : 1);   // waves that fill every SIMD
-    cpw = ENVS_PER_WAVE;
-    while (force <= 0 && cpw > 1 && (count + cpw / 2 - 1) / (cpw / 2) <= target) cpw /= 2;
-    if (force > 0) cpw = force;
-    const int waves = (count + cpw - 1) / cpw;
-    int wpb = (waves + (cus > 0 ? cus : 1) - 1) / (cus > 0 ? cus : 1);   // waves per block: spread over the CUs
+    if (cus < 1) cus = 1;
+    int wpb = (count + cus - 1) / cus;
     wpb = wpb < 1 ? 1 : wpb > WAVES_PER_BLOCK ? WAVES_PER_BLOCK : wpb;
-    return EmuLaunch{dim3((unsigned)((waves + wpb - 1) / wpb)), dim3((unsigned)(64 * wpb))};
+    return EmuLaunch{dim3((unsigned)((count + wpb - 1) / wpb)), dim3((unsigned)(64 * wpb))};
 }
-// first console slot of this block (blocks of blockDim.x / 64 waves)
-__device__ __forceinline__ uint32_t block_base() { return blockIdx.x * ((blockDim.x >> 6) * ENVS_PER_WAVE); }
+// this wave's console (the block's waves in order)
+__device__ __forceinline__ uint32_t wave_console(uint32_t block) { return block * (blockDim.x >> 6) + wave_slot(); }
 
-// The new observation of a lane's env, output columns 21 g .. 21 g + 20 (g: the lane's part), into
-// fresh[e * OBS_PIX + o]: the boot observation right after a reset, else INTER_AREA of the last frame,
-// max-pooled with its partner frame (fastmario.cpp:377-386); `bits` as step_lane returns them; the output rows of
-// NP row periods from p0 (7 rows from 20 source rows each). k_step runs it for all 12 periods once the wave's
-// frame loop is over, on the frames the wave has just drawn, except in the waves that finish last, whose envs
-// k_obs_late takes with a wave per period. The 4 lanes of an env take the 4
-// column periods of the tables (AreaPeriod), so every lane runs the same code with constant taps and weights,
-// and the wave reads every frame byte once: a load takes word 16 g + i of a source row for the 16 envs of each
-// part (4 x 64 contiguous bytes). The loads of the next source row are in flight while a row is summed. The
-// float operations and their order are area_pixel's. Not inlined, so that its registers stay out of the frame
-// loop's allocation.
+// The new observation of the wave's env into fresh[e * OBS_PIX + o]: the boot observation right after a reset, else
+// INTER_AREA of the last frame, max-pooled with its partner frame (fastmario.cpp:377-386); `bits` as step_lane
+// returns them. k_step runs it once the wave's frame loop is over, on the frames the wave has just drawn. 48 lanes
+// take the 4 column periods of the tables (AreaPeriod: output columns 21 g .. 21 g + 20) times the 12 row periods (7
+// output rows from 20 source rows each), so every lane runs the same code with constant taps and weights. A lane's 64
+// pixels of a source row are 64 contiguous bytes: four 16-byte loads per frame. The float operations and their order
+// are area_pixel's. Not inlined, so that its registers stay out of the frame loop's allocation.
 typedef __attribute__((address_space(1))) uint8_t gbyte;       // global memory, addressed as such
-constexpr int kBufferWord3 = 0x00020000;   // buffer resource word 3 on gfx9: 32-bit raw (untyped) accesses
-// a wave-uniform 64-bit value, as such (the builtin returns a signed int: each half is taken as unsigned before
-// it is widened, so that the low half's bit 31 does not spread into the high half)
-__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return (uint64_t)lo | (uint64_t)hi << 32;
-}
-template <int NP>
 __device__ __attribute__((noinline)) void obs_tail(const uint8_t* gray_, uint32_t np_, uint8_t* fresh_,
-                                                   const uint8_t* boot_obs, uint32_t e, uint32_t g, uint32_t bits,
-                                                   int p0) {
-    // The frames were stored by the env's lanes of this wave (streaming stores, and read-modify-writes whose loads
-    // may have left lines in this CU's L1): wait for the stores, and drop the L1's lines, before reading them.
+                                                   const uint8_t* boot_obs, uint32_t e, uint32_t lane, uint32_t bits_) {
+    // The frames were stored by the lanes of this wave (streaming stores): wait for the stores, and drop the L1's
+    // lines, before reading them.
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    // the arguments a call passes in vector registers: the buffers and np are the kernel's, the same in every lane
-    const gbyte* gray = (const gbyte*)uniform64((uint64_t)gray_);
-    gbyte* fresh = (gbyte*)uniform64((uint64_t)fresh_);
-    const uint32_t np = __builtin_amdgcn_readfirstlane(np_);
-    p0 = __builtin_amdgcn_readfirstlane(p0);          // the same in every lane of both callers' waves
-    gbyte* out = fresh + (size_t)e * OBS_PIX + 21 * g;
+    // the arguments a call passes in vector registers: the same in every lane but `lane`
+    const gbyte* gray = (const gbyte*)uni64((uint64_t)gray_);
+    gbyte* fresh = (gbyte*)uni64((uint64_t)fresh_) + (size_t)uni(e) * OBS_PIX;
+    const uint32_t np = uni(np_), bits = uni(bits_);
     if (bits & 4) {
-        const uint8_t* b = boot_obs + (size_t)(bits >> 8) * OBS_PIX + 21 * g;
-        for (int d = 7 * p0; d < 7 * (p0 + NP); d++)
-            for (int q = 0; q < 21; q++) out[d * 84 + q] = b[d * 84 + q];
+        const uint32_t* b = (const uint32_t*)(boot_obs + (size_t)(bits >> 8) * OBS_PIX);
+        for (uint32_t i = lane; i < OBS_PIX / 4; i += 64) ((__attribute__((address_space(1))) uint32_t*)fresh)[i] = b[i];
         return;
     }
-    const bool pool = (bits & 1) != 0, swap = (bits & 2) != 0, all_pool = __all(pool);
-    const size_t fb = (size_t)GRAY_PIX * np, rowb = (size_t)256 * np;   // bytes per frame buffer, per source row
-    const uint32_t lo = (16 * g * np + e) * 4, step = 4 * np;           // word 16 g of the row, the next word
-    uint32_t a0[16], b0[16], a1[16], b1[16];
-    // Source row sy of both frame buffers as buffer resources (base: the row, size: the row's 256 np bytes, so
-    // that no offset reaches past it), loaded with the lane's 32-bit word offsets: no 64-bit address per lane
-    // and word. The loads are streaming (cache policy nt, aux bit 1): the frames are read once, and the
-    // console state of the waves still in their frame loops stays in the L2.
-    auto load = [&](int sy, uint32_t (&a)[16], uint32_t (&b)[16]) {
-        const __amdgpu_buffer_rsrc_t r0 =
-            __builtin_amdgcn_make_buffer_rsrc((void*)(gray + (size_t)sy * rowb), 0, (int)rowb, kBufferWord3);
-        const __amdgpu_buffer_rsrc_t r1 =
-            __builtin_amdgcn_make_buffer_rsrc((void*)(gray + fb + (size_t)sy * rowb), 0, (int)rowb, kBufferWord3);
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            a[i] = __builtin_amdgcn_raw_buffer_load_b32(r0, (int)(lo + (uint32_t)i * step), 0, 2);
-            b[i] = __builtin_amdgcn_raw_buffer_load_b32(r1, (int)(lo + (uint32_t)i * step), 0, 2);
-        }
-    };
+    if (lane >= 48) return;
+    const uint32_t g = lane & 3u, p = lane >> 2;
+    gbyte* out = fresh + 21 * g + 7 * 84 * p;                                  // row 0 of the lane's period
+    const gbyte* f0 = gray + (size_t)uni(e) * GRAY_PIX;
+    const gbyte* f1 = f0 + (size_t)GRAY_PIX * np;
+    if (!(bits & 1)) { f0 = (bits & 2) ? f1 : f0; f1 = f0; }                   // one frame: its maximum with itself
+    const uint32_t at = 20 * 256 * p + 64 * g;                                 // the lane's pixels of its first row
     float acc[21];
 #pragma unroll
-    for (int q = 0; q < 21; q++) acc[q] = 0.f;
-    auto row = [&](int sy, const uint32_t (&a)[16], const uint32_t (&b)[16]) {
+    for (int q = 0; q < 21; q++) acc[q] = 0.f;                                 // +0 at the period's start
+#pragma nounroll
+    for (int r = 0; r < 20; r++) {
         uint32_t ev[16], od[16];
-        if (all_pool) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) { ev[i] = max_even_bytes(a[i], b[i]); od[i] = max_odd_bytes(a[i], b[i]); }
-        } else {
+        for (int i = 0; i < 4; i++) {
+            // streaming loads: the frames are read once
+            const mh_u32x4 a = __builtin_nontemporal_load((const __attribute__((address_space(1))) mh_u32x4*)(f0 + at + 256 * r) + i);
+            const mh_u32x4 b = __builtin_nontemporal_load((const __attribute__((address_space(1))) mh_u32x4*)(f1 + at + 256 * r) + i);
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const uint32_t w = swap ? b[i] : a[i];
-                ev[i] = pool ? max_even_bytes(a[i], b[i]) : w;
-                od[i] = pool ? max_odd_bytes(a[i], b[i]) : w;
-            }
+            for (int k = 0; k < 4; k++) { ev[4 * i + k] = max_even_bytes(a[k], b[k]); od[4 * i + k] = max_odd_bytes(a[k], b[k]); }
         }
         float rs[21];
         obs_period_sums(ev, od, rs);
-        obs_period_take(sy, rs, acc, [&](int dy, const float (&v)[21]) {
+        obs_period_take(r, rs, acc, [&](int dy, const float (&v)[21]) {
             gbyte* o = out + dy * 84;
 #pragma unroll
             for (int q = 0; q < 21; q++) o[q] = round_sat(v[q]);
         });
-    };
-    // the 20 source rows of each of periods p0 .. p0 + NP - 1 (output rows 7 p .. 7 p + 6); acc is +0 at every
-    // period's start
-    for (int pi = 0; pi < NP; pi++) {
-        const int sy0 = 20 * (p0 + pi);
-        load(sy0, a0, b0);
-#pragma nounroll
-        for (int r = 0; r < 20; r += 2) {
-            load(sy0 + r + 1, a1, b1);
-            row(sy0 + r, a0, b0);
-            if (r + 2 < 20) load(sy0 + r + 2, a0, b0);
-            row(sy0 + r + 1, a1, b1);
-        }
     }
 }
 
 __global__ void EMU_BOUNDS k_boot(BootArgs A) {
     ROM_LDS
-    stage_rom(A.R, s_rom, s_lut, s_dec);
-    const int slot = lane_slot();
-    const int l = (int)(block_base() + slot);
-    if (l < A.nl) boot_lane(A, lane_ctx(A.R, s_rom, s_lut, s_dec, s_sp, s_gp, slot), l);
+    stage_rom(A.R, s_rom, s_lut);
+    const int l = (int)wave_console(blockIdx.x);
+    if (l < A.nl) boot_lane(A, lane_ctx(A.R, s_rom, s_lut, s_env), l);
 }
 
 __global__ void EMU_BOUNDS k_cache(CacheArgs A) {
     ROM_LDS
-    stage_rom(A.R, s_rom, s_lut, s_dec);
-    const int slot = lane_slot();
-    const int ci = (int)(block_base() + slot);
-    if (ci < A.nc) cache_lane(A, lane_ctx(A.R, s_rom, s_lut, s_dec, s_sp, s_gp, slot), ci);
+    stage_rom(A.R, s_rom, s_lut);
+    const int ci = (int)wave_console(blockIdx.x);
+    if (ci < A.nc) cache_lane(A, lane_ctx(A.R, s_rom, s_lut, s_env), ci);
 }
 
 // k_step's launch order for the next step. When k_step has more blocks than the GPU has CUs (past 32,768 envs on
@@ -214,9 +142,11 @@ __global__ void EMU_BOUNDS k_cache(CacheArgs A) {
 // work predicts the next one's: the groups run in order of their slowest env's executed 6502 instructions in the
 // last step, most first, and the cheap ones fill the CUs they free (longest-first list scheduling).
 // k_work: each group's slowest env's executed instructions since the last call, from the env counters.
-__global__ __launch_bounds__(LDS_LANES) void k_work(const uint32_t* ev, uint32_t np, int n, uint64_t* prev,
+constexpr int ORDER_GROUP = WAVES_PER_BLOCK;   // envs of a full block
+static_assert(64 % ORDER_GROUP == 0, "k_work: whole groups per wave");
+__global__ __launch_bounds__(64) void k_work(const uint32_t* ev, uint32_t np, int n, uint64_t* prev,
                                                     uint32_t* work) {
-    const uint32_t e = blockIdx.x * LDS_LANES + threadIdx.x;
+    const uint32_t e = blockIdx.x * 64 + threadIdx.x;
     uint32_t w = 0;
     if (e < (uint32_t)n) {
         auto counter = [&](int lo) {
@@ -227,20 +157,14 @@ __global__ __launch_bounds__(LDS_LANES) void k_work(const uint32_t* ev, uint32_t
         w = d > 0xffffffffull ? 0xffffffffu : (uint32_t)d;
         prev[e] = c;
     }
-    for (int off = 32; off >= 1; off >>= 1) {
+    for (int off = ORDER_GROUP / 2; off >= 1; off >>= 1) {
         const uint32_t o = (uint32_t)__shfl_xor((int)w, off);
         w = o > w ? o : w;
     }
-    __shared__ uint32_t wmax[LDS_LANES / 64];
-    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = w;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int k = 1; k < LDS_LANES / 64; k++) w = wmax[k] > w ? wmax[k] : w;
-        work[blockIdx.x] = w;
-    }
+    if (threadIdx.x % ORDER_GROUP == 0 && e < (uint32_t)n) work[e / ORDER_GROUP] = w;
 }
 // k_order: one block; a bitonic sort of (work, ~index) keys in LDS (ties: the lower index first).
-constexpr int ORDER_MAX = 8192;   // groups: MAX_ENVS / LDS_LANES fits
+constexpr int ORDER_MAX = 8192;   // groups; past 131,072 envs the launch keeps its own order
 __global__ __launch_bounds__(1024) void k_order(const uint32_t* work, uint32_t* perm, int ng) {
     __shared__ uint64_t key[ORDER_MAX];
     int P = 1;
@@ -261,72 +185,33 @@ __global__ __launch_bounds__(1024) void k_order(const uint32_t* work, uint32_t* 
         }
     for (int i = threadIdx.x; i < ng; i += blockDim.x) perm[i] = ~(uint32_t)key[i];
 }
-static_assert(MAX_ENVS / LDS_LANES <= ORDER_MAX, "k_order holds every group");
 
-__device__ __forceinline__ void step_block(const StepArgs& A, uint32_t base) {
+__device__ __forceinline__ void step_block(const StepArgs& A, uint32_t block) {
     ROM_LDS
-    stage_rom(A.R, s_rom, s_lut, s_dec);
-    // The frame loop issues ahead of the observations of the waves that have finished it (on a SIMD, the two
-    // waves' instructions are arbitrated by this priority first).
-    __builtin_amdgcn_s_setprio(2);
-    const int slot = lane_slot();
-    const uint32_t e = base + (uint32_t)slot;
-    const bool live = e < (uint32_t)A.n;
-    uint32_t bits = 0;
-    if (live) bits = step_lane(A, lane_ctx(A.R, s_rom, s_lut, s_dec, s_sp, s_gp, slot), e);
-    if (!__any(live)) return;
-    // The wave's ticket: its place in the order in which the waves finish their frame loops (a vector atomic
-    // from one lane). The waves that finish last would hold the kernel's end with their observations; they
-    // leave them to k_obs_late, which spreads an env's rows over 12 waves.
-    uint32_t ticket = 0;
-    if (__lane_id() == 0) ticket = atomicAdd(A.obs_order, 1u);
-    ticket = (uint32_t)__builtin_amdgcn_readfirstlane(ticket);
-    if (ticket >= A.obs_late_from && ticket < A.obs_late_to) {
-        if (__lane_id() == 0) A.obs_order[1 + ticket - A.obs_late_from] = e;   // lane 0 holds the wave's first slot
-    } else if (live) {
-        __builtin_amdgcn_s_setprio(0);
-        obs_tail<12>(A.gray, A.np, A.fresh, A.boot_obs, e, lane_part(), bits, 0);
-    }
-}
-
-// base: the first env slot of the block's group (blocks of blockDim.x / 64 waves)
-__global__ void EMU_BOUNDS k_step(StepArgs A) { step_block(A, block_base()); }
-// k_step in the launch order of k_order: block b runs group perm[b]
-__global__ void EMU_BOUNDS k_step_ordered(StepArgs A, const uint32_t* perm) {
-    step_block(A, perm[blockIdx.x] * ((blockDim.x >> 6) * ENVS_PER_WAVE));
-}
-
-// The observations of the envs of the waves that finished k_step's frame loop last (obs_tail, one wave per
-// (deferred wave, row period): 12 waves per env group instead of one), then k_step's counter back to 0.
-struct ObsLateArgs {
-    int n; uint32_t np; int waves;       // deferred waves (their first slots at order[1 ..])
-    const uint32_t* ev;
-    const uint8_t* gray; uint8_t* fresh; const uint8_t* boot_obs;
-    uint32_t* order;
-};
-constexpr int OBS_LATE_MAX = 64;         // waves that may defer
-__global__ void __launch_bounds__(256) k_obs_late(ObsLateArgs A) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) A.order[0] = 0;   // k_step is over: no ticket is taken any more
-    const int u = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));   // (deferred wave u / 12, row period u % 12)
-    if (u >= A.waves * 12) return;
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t e = A.order[1 + u / 12] + (lane & (ENVS_PER_WAVE - 1));   // k_step's lanes: env slot, part
+    stage_rom(A.R, s_rom, s_lut);
+    const uint32_t e = wave_console(block);
     if (e >= (uint32_t)A.n) return;
-    const uint32_t pw = A.ev[(size_t)E_POOLED * A.np + e];
-    const uint32_t bits = (pw & 3u) | (A.ev[(size_t)E_SHOWS_BOOT * A.np + e] ? 4u : 0u) |
-                          A.ev[(size_t)E_LEVEL * A.np + e] << 8;
-    obs_tail<1>(A.gray, A.np, A.fresh, A.boot_obs, e, lane / ENVS_PER_WAVE, bits, u % 12);
+    const uint32_t bits = step_lane(A, lane_ctx(A.R, s_rom, s_lut, s_env), e);
+    __builtin_amdgcn_s_setprio(0);   // the frame loops of the other waves issue first
+    obs_tail(A.gray, A.np, A.fresh, A.boot_obs, e, threadIdx.x & 63u, bits);
 }
 
-// A wave carries A.cpw consoles (raw_launch): its lanes l, l + 16, l + 32, l + 48 with l < cpw run console
-// wave * cpw + l of the block; the others idle.
+// What bounds it: scalar issue. A SIMD issues one scalar instruction per 4 cycles whichever of its waves it is from; the
+// headline step (32,768 envs of 1-1) is 126,000 scalar, 78,000 vector and 19,000 branch instructions per env, of which
+// the 5,217 6502 instructions are about 70,000 scalar ones. Why one console per wave, against 16 per wave in
+// lockstep (4 lanes each, every opcode's work as selects, 15 to 12 of 16 consoles active): a lockstep iteration issues
+// ~470 instructions for ~12 6502 instructions but each env waits for all of them; here a 6502 instruction is ~17
+// instructions and nothing waits for another console. Measured (k_step, the same envs): 256 envs 11.6 -> 1.03 ms,
+// 4,096 envs 19.9 -> 2.99 ms, 32,768 envs 14.57 -> 10.64 ms, 65,536 envs of 32 levels 40.9 -> 22.9 ms.
+__global__ void EMU_BOUNDS k_step(StepArgs A) { step_block(A, blockIdx.x); }
+// k_step in the launch order of k_order: block b runs group perm[b]
+__global__ void EMU_BOUNDS k_step_ordered(StepArgs A, const uint32_t* perm) { step_block(A, uni(perm[blockIdx.x])); }
+
 __global__ void EMU_BOUNDS k_raw(RawArgs A) {
     ROM_LDS
-    stage_rom(A.R, s_rom, s_lut, s_dec);
-    const int in_wave = (int)(threadIdx.x & (ENVS_PER_WAVE - 1));
-    const int slot = (int)(threadIdx.x >> 6) * A.cpw + in_wave;
-    const uint32_t e = blockIdx.x * ((blockDim.x >> 6) * (uint32_t)A.cpw) + (uint32_t)slot;
-    if (in_wave < A.cpw && e < (uint32_t)A.n) raw_lane(A, lane_ctx(A.R, s_rom, s_lut, s_dec, s_sp, s_gp, slot), e);
+    stage_rom(A.R, s_rom, s_lut);
+    const uint32_t e = wave_console(blockIdx.x);
+    if (e < (uint32_t)A.n) raw_lane(A, lane_ctx(A.R, s_rom, s_lut, s_env), e);
 }
 
 // One wave of 64 envs per block: each lane draws its env's reset, then the wave copies the chosen cache
@@ -347,7 +232,7 @@ __global__ void __launch_bounds__(64) k_reset(ResetArgs A) {
 
 // Observation of a reset-cache entry or a boot state: the boot observation, or the resized last frame.
 struct SmallObsArgs {
-    const uint8_t* gray; uint32_t stride;     // frame buffer of `stride` lanes, entry i in lane i
+    const uint8_t* gray;                      // whole frames, entry i the i-th
     const uint8_t* use_boot;                  // per entry (nullable): take boot_obs[level(i)]
     const uint8_t* boot_obs; int nk;          // boot observations [level * OBS_PIX]
     uint8_t* out; int count;                  // [i * OBS_PIX + o]
@@ -359,7 +244,7 @@ __global__ void k_small_obs(SmallObsArgs A) {
     if (i >= A.count || o >= OBS_PIX) return;
     uint8_t v;
     if (A.use_boot && A.use_boot[i]) v = A.boot_obs[(size_t)(i / A.nk) * OBS_PIX + o];
-    else v = area_pixel(Image{A.gray, A.stride, (uint32_t)i}, Image{}, false, o, A.T);
+    else v = area_pixel(Image{A.gray + (size_t)i * GRAY_PIX, 0, 0}, Image{}, false, o, A.T);
     A.out[(size_t)i * OBS_PIX + o] = v;
 }
 
@@ -450,22 +335,13 @@ __global__ void k_canon(const uint8_t* mem, const uint32_t* sc, uint32_t np, int
     if (e < (uint32_t)n) canon_lane(mem, sc, np, e, out + (size_t)(slot_env ? slot_env[e] : (int32_t)e) * MH_CANON_BYTES);
 }
 
-// Lane-interleaved rows -> env-major (n x rows), slot e to row slot_env[e] (identity if null). Threads: x = slot,
-// y = row.
+// The first `rows` bytes of each console's memory -> (n x rows), slot e to row slot_env[e] (identity if null).
+// Threads: x = slot, y = row.
 __global__ void k_rows_out(const uint8_t* src, uint32_t np, int n, uint32_t rows, const int32_t* slot_env, uint8_t* out) {
     const uint32_t e = blockIdx.x * 64 + (threadIdx.x & 63);
     const uint32_t r = blockIdx.y * 4 + (threadIdx.x >> 6);
     if (e >= (uint32_t)n || r >= rows) return;
-    out[(size_t)(slot_env ? slot_env[e] : (int32_t)e) * rows + r] = src[(size_t)r * np + e];
-}
-
-// Frame buffer (4-pixel words, lane-interleaved) -> env-major 240x256 frames. Threads: x = env, y = word.
-__global__ void k_frames_out(const uint8_t* src, uint32_t np, int n, uint8_t* out) {
-    const uint32_t e = blockIdx.x * 64 + (threadIdx.x & 63);
-    const uint32_t w = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (e >= (uint32_t)n || w >= GRAY_PIX / 4) return;
-    const uint32_t v = ((const uint32_t*)src)[(size_t)w * np + e];
-    for (int b = 0; b < 4; b++) out[(size_t)e * GRAY_PIX + 4 * w + b] = (uint8_t)(v >> (8 * b));
+    out[(size_t)(slot_env ? slot_env[e] : (int32_t)e) * rows + r] = src[mem_offset(np, e, r)];
 }
 
 // Frame buffer of palette values -> env-major 240x256x3 RGB24 through a 64-entry RGB table (a palette value
@@ -477,7 +353,7 @@ __global__ void k_frames_rgb(const uint8_t* src, uint32_t np, int n, const uint8
     const uint32_t e = blockIdx.x * 64 + (threadIdx.x & 63);
     const uint32_t w = blockIdx.y * 4 + (threadIdx.x >> 6);
     if (e >= (uint32_t)n || w >= GRAY_PIX / 4) return;
-    const uint32_t v = ((const uint32_t*)src)[(size_t)w * np + e];
+    const uint32_t v = ((const uint32_t*)src)[(size_t)e * (GRAY_PIX / 4) + w];
     uint8_t* o = out + ((size_t)e * GRAY_PIX + 4 * w) * 3;
     for (int b = 0; b < 4; b++) {
         const uint32_t c = (v >> (8 * b)) & 63u;
@@ -535,6 +411,14 @@ static bool load_cart(const uint8_t* d, int64_t n, std::vector<uint8_t>& img, ui
         default: nt[0] = nt[1] = nt[2] = nt[3] = 0; break;
     }
     return true;
+}
+
+// The program (the image's first 32 KB) as scalar_run's records.
+static bool upload_records(uint32_t* d_recs, const std::vector<uint8_t>& img) {
+    static constexpr dec::Table words{};
+    std::vector<uint32_t> recs(REC_COUNT);
+    decode_prg(img.data(), words.w, recs.data());
+    return ok(hipMemcpy(d_recs, recs.data(), recs.size() * 4, hipMemcpyHostToDevice), "upload program records");
 }
 
 // ---- the PPO policy's input (the rollout harness's observation -> bf16 channels-last scaling)
@@ -742,7 +626,7 @@ struct MhEnv {
     RomArgs R{};
     AreaTables* T = nullptr;
     uint8_t *mem = nullptr, *gray = nullptr, *fresh = nullptr;
-    uint32_t* obs_order = nullptr;     // k_step's finish counter and the deferred waves (k_obs_late)
+    EmuLaunch ls{};                    // k_step's launch shape
     // k_step's launch order (k_work, k_order), when it has more blocks than the GPU has CUs: null otherwise
     uint32_t *grp_work = nullptr, *grp_perm = nullptr;
     uint64_t* grp_prev = nullptr;      // each env's executed-instruction count at the last k_work
@@ -789,8 +673,8 @@ static void launch_stack(const MhEnv* h, hipStream_t s, int mode) {
 }
 
 struct MhRaw {
-    int n = 0, device = 0, cus = 0, cpw = 0;
-    EmuLaunch lr{};                // k_raw's launch shape, with cpw consoles per wave (raw_launch)
+    int n = 0, device = 0, cus = 0;
+    EmuLaunch lr{};                // k_raw's launch shape
     uint32_t np = 0;
     DevBufs B;
     RomArgs R{};
@@ -883,6 +767,7 @@ MhEnv* mh_create_roms(const uint8_t* roms, const int64_t* rom_lens, int n_roms, 
     auto& B = h->B;
     uint8_t* d_rom = B.alloc<uint8_t>(img.size(), good);
     uint8_t* d_lut = B.alloc<uint8_t>(256, good);
+    uint32_t* d_recs = B.alloc<uint32_t>(REC_COUNT, good);
     h->T = B.alloc<AreaTables>(1, good);
     int* d_levels = B.alloc<int>(lv.size(), good);
     h->key_bank = B.alloc<uint8_t>(key_bank.size(), good);
@@ -894,10 +779,10 @@ MhEnv* mh_create_roms(const uint8_t* roms, const int64_t* rom_lens, int n_roms, 
     h->snap_mem = B.alloc<uint8_t>((size_t)2 * MEM_ROWS * h->np, good);
     h->snap_sc = B.alloc<uint32_t>((size_t)2 * S_COUNT * h->np, good);
     h->fresh = B.alloc<uint8_t>((size_t)OBS_PIX * h->np, good);
-    h->obs_order = B.alloc<uint32_t>(1 + OBS_LATE_MAX, good);
+    h->ls = emu_launch(h->n, h->cus);
     {
-        const EmuLaunch ls = emu_launch(h->n, h->cus);
-        if ((int)ls.grid.x > h->cus) {   // more than one block per CU: the launch order decides what runs last
+        const EmuLaunch& ls = h->ls;
+        if ((int)ls.grid.x > h->cus && (int)ls.grid.x <= ORDER_MAX) {   // more than one block per CU: the launch order decides what runs last
             h->n_groups = (int)ls.grid.x;
             h->grp_work = B.alloc<uint32_t>(h->n_groups, good);
             h->grp_perm = B.alloc<uint32_t>(h->n_groups, good);
@@ -943,28 +828,27 @@ MhEnv* mh_create_roms(const uint8_t* roms, const int64_t* rom_lens, int n_roms, 
     if (!ok(hipMemcpy(d_rom, img.data(), img.size(), hipMemcpyHostToDevice), "upload rom") ||
         !ok(hipMemcpy(h->key_bank, key_bank.data(), key_bank.size(), hipMemcpyHostToDevice), "upload key banks") ||
         !ok(hipMemcpy(h->slot_env, slot_env.data(), slot_env.size() * 4, hipMemcpyHostToDevice), "upload slot map") ||
-        !ok(hipMemcpy(d_lut, lut, 256, hipMemcpyHostToDevice), "upload lut") ||
+        !ok(hipMemcpy(d_lut, lut, 256, hipMemcpyHostToDevice), "upload lut") || !upload_records(d_recs, img) ||
         !ok(hipMemcpy(h->T, &T, sizeof(T), hipMemcpyHostToDevice), "upload tables") ||
         !ok(hipMemcpy(d_levels, lv.data(), lv.size() * sizeof(int), hipMemcpyHostToDevice), "upload levels") ||
         !ok(hipMemcpy(h->ev, ev.data(), ev.size() * 4, hipMemcpyHostToDevice), "upload env words"))
         return fail();
-    h->R.rom = d_rom; h->R.lut = d_lut; h->R.n_chr = n_roms;
+    h->R.rom = d_rom; h->R.lut = d_lut; h->R.recs = d_recs; h->R.n_chr = n_roms;
     h->R.nt_bits = 0;
     for (int i = 0; i < 4; i++) h->R.nt_bits |= (nt[i] ? 1u : 0u) << i;
     // boot every level, build the reset cache
+    const EmuLaunch lb = emu_launch(h->nl, h->cus), lc = emu_launch(h->nc, h->cus);
     BootArgs ba{h->R, h->nl, h->nlp, d_levels, h->key_bank, h->boot_mem, h->boot_sc, h->boot_gray, h->x0, h->t0, d_err};
-    const EmuLaunch lb = emu_launch(h->nl, h->cus);
     hipLaunchKernelGGL(k_boot, lb.grid, lb.block, 0, 0, ba);
     if (!ok(hipGetLastError(), "k_boot launch")) return fail();
-    SmallObsArgs so{h->boot_gray, h->nlp, nullptr, nullptr, 1, h->boot_obs, h->nl, h->T};
+    SmallObsArgs so{h->boot_gray, nullptr, nullptr, 1, h->boot_obs, h->nl, h->T};
     hipLaunchKernelGGL(k_small_obs, dim3((OBS_PIX + 255) / 256, h->nl), dim3(256), 0, 0, so);
     CacheArgs ca{h->R, h->cfg, h->key_bank, h->nl, h->nk, h->nc, h->nlp, h->ncp, h->boot_mem, h->boot_sc, h->x0, h->t0,
                  h->cmem, h->csc, h->cgray, h->csnap_mem, h->csnap_sc, h->cx, h->ct, h->clives, h->cdraws, h->cboot,
                  h->cframes, h->cinstr, h->cff, h->cbad};
-    const EmuLaunch lc = emu_launch(h->nc, h->cus);
     hipLaunchKernelGGL(k_cache, lc.grid, lc.block, 0, 0, ca);
     if (!ok(hipGetLastError(), "k_cache launch")) return fail();
-    SmallObsArgs co{h->cgray, h->ncp, h->cboot, h->boot_obs, h->nk, h->cobs, h->nc, h->T};
+    SmallObsArgs co{h->cgray, h->cboot, h->boot_obs, h->nk, h->cobs, h->nc, h->T};
     hipLaunchKernelGGL(k_small_obs, dim3((OBS_PIX + 255) / 256, h->nc), dim3(256), 0, 0, co);
     if (!ok(hipDeviceSynchronize(), "boot / reset cache")) return fail();
     uint32_t err = 0;
@@ -1035,14 +919,12 @@ int mh_step_async(MhEnv* h, const int64_t* d_actions, void* stream) {
     CK(hipSetDevice(h->device));
     hipStream_t s = (hipStream_t)stream;
     if (mark(h, s, 0)) return -1;
-    // waves with live envs, and how many of the last to finish defer their observations
-    const int waves = (h->n + ENVS_PER_WAVE - 1) / ENVS_PER_WAVE, late = std::min(waves, OBS_LATE_MAX);
     StepArgs sa{h->R, h->cfg, h->n, h->np, h->mem, h->sc, h->ev, h->gray, h->snap_mem, h->snap_sc, d_actions,
                 h->rew, h->term, h->trunc, h->info, h->ep_ret, h->ep_len, h->key_bank, h->slot_env, h->fresh,
-                h->boot_obs, h->obs_order, (uint32_t)(waves - late), (uint32_t)waves};
-    const EmuLaunch ls = emu_launch(h->n, h->cus);
+                h->boot_obs};
+    const EmuLaunch& ls = h->ls;
     if (h->grp_perm) {   // this step's launch order, from the last step's work
-        hipLaunchKernelGGL(k_work, dim3((unsigned)h->n_groups), dim3(LDS_LANES), 0, s, h->ev, h->np, h->n,
+        hipLaunchKernelGGL(k_work, dim3((unsigned)(h->np / 64)), dim3(64), 0, s, h->ev, h->np, h->n,
                            h->grp_prev, h->grp_work);
         hipLaunchKernelGGL(k_order, dim3(1), dim3(1024), 0, s, h->grp_work, h->grp_perm, h->n_groups);
         hipLaunchKernelGGL(k_step_ordered, ls.grid, ls.block, 0, s, sa, (const uint32_t*)h->grp_perm);
@@ -1051,10 +933,7 @@ int mh_step_async(MhEnv* h, const int64_t* d_actions, void* stream) {
     }
     CK(hipGetLastError());
     if (mark(h, s, 1)) return -1;
-    const ObsLateArgs la{h->n, h->np, late, h->ev, h->gray, h->fresh, h->boot_obs, h->obs_order};
-    hipLaunchKernelGGL(k_obs_late, dim3((unsigned)((late * 12 + 3) / 4)), dim3(256), 0, s, la);
-    CK(hipGetLastError());
-    if (mark(h, s, 2)) return -1;
+    if (mark(h, s, 2)) return -1;   // (a stage of its own until the observations moved into k_step: empty)
     hipLaunchKernelGGL(k_reset, dim3(h->np / 64), dim3(64), 0, s, h->reset_args(0));
     CK(hipGetLastError());
     if (mark(h, s, 3)) return -1;
@@ -1166,10 +1045,10 @@ MhRaw* mh_raw_create(const uint8_t* rom, int64_t rom_len, int n, int device) {
     g_err.clear();
     if (n < 1) { g_err = "invalid arguments"; return nullptr; }
     if ((uint32_t)n > MAX_ENVS) { g_err = "too many consoles (at most 979,648: console memory takes 32-bit offsets)"; return nullptr; }
-    int force = 0;
+    // (a wave runs one console whatever the variable says; an ill-formed value is an error, as it was)
     if (const char* f = getenv("MH_RAW_CONSOLES_PER_WAVE"); f && *f) {
-        force = atoi(f);
-        if (force != 1 && force != 2 && force != 4 && force != 8 && force != ENVS_PER_WAVE) {
+        const int cpw = atoi(f);
+        if (cpw != 1 && cpw != 2 && cpw != 4 && cpw != 8 && cpw != 16) {
             g_err = "MH_RAW_CONSOLES_PER_WAVE must be 1, 2, 4, 8 or 16";
             return nullptr;
         }
@@ -1181,10 +1060,11 @@ MhRaw* mh_raw_create(const uint8_t* rom, int64_t rom_len, int n, int device) {
     MhRaw* h = new MhRaw();
     bool good = true;
     h->n = n; h->np = pad64(n); h->device = device; h->cus = device_cus(device);
-    h->lr = raw_launch(n, h->cus, force, h->cpw);
+    h->lr = emu_launch(n, h->cus);
     auto& B = h->B;
     uint8_t* d_rom = B.alloc<uint8_t>(0xa000, good);
     uint8_t* d_lut = B.alloc<uint8_t>(256, good);
+    uint32_t* d_recs = B.alloc<uint32_t>(REC_COUNT, good);
     h->mem = B.alloc<uint8_t>((size_t)MEM_ROWS * h->np, good);
     h->bk_mem = B.alloc<uint8_t>((size_t)MEM_ROWS * h->np, good);
     h->sc = B.alloc<uint32_t>((size_t)S_COUNT * h->np, good);
@@ -1197,18 +1077,21 @@ MhRaw* mh_raw_create(const uint8_t* rom, int64_t rom_len, int n, int device) {
     uint8_t ident[256];
     for (int i = 0; i < 256; i++) ident[i] = (uint8_t)i;
     if (!ok(hipMemcpy(d_rom, img.data(), 0xa000, hipMemcpyHostToDevice), "upload rom") ||
-        !ok(hipMemcpy(d_lut, ident, 256, hipMemcpyHostToDevice), "upload lut")) { delete h; return nullptr; }
-    h->R.rom = d_rom; h->R.lut = d_lut; h->R.n_chr = 1;
+        !ok(hipMemcpy(d_lut, ident, 256, hipMemcpyHostToDevice), "upload lut") || !upload_records(d_recs, img)) {
+        delete h;
+        return nullptr;
+    }
+    h->R.rom = d_rom; h->R.lut = d_lut; h->R.recs = d_recs; h->R.n_chr = 1;
     h->R.nt_bits = 0;
     for (int i = 0; i < 4; i++) h->R.nt_bits |= (nt[i] ? 1u : 0u) << i;
-    RawArgs ra{h->R, h->n, h->np, h->mem, h->sc, h->screen, nullptr, 0, h->bad, h->instr, h->ff, 1, h->cpw};
+    RawArgs ra{h->R, h->n, h->np, h->mem, h->sc, h->screen, nullptr, 0, h->bad, h->instr, h->ff, 1, 1};
     hipLaunchKernelGGL(k_raw, h->lr.grid, h->lr.block, 0, 0, ra);
     if (!ok(hipDeviceSynchronize(), "raw power-on")) { delete h; return nullptr; }
     return h;
 }
 int mh_raw_frame(MhRaw* h, const uint8_t* d_buttons, int render, void* stream) {
     if (!h || !d_buttons) return -1;
-    RawArgs ra{h->R, h->n, h->np, h->mem, h->sc, h->screen, d_buttons, render, h->bad, h->instr, h->ff, 0, h->cpw};
+    RawArgs ra{h->R, h->n, h->np, h->mem, h->sc, h->screen, d_buttons, render, h->bad, h->instr, h->ff, 0, 1};
     hipLaunchKernelGGL(k_raw, h->lr.grid, h->lr.block, 0, (hipStream_t)stream, ra);
     CK(hipGetLastError());
     return 0;
@@ -1222,9 +1105,7 @@ int mh_raw_ram(MhRaw* h, uint8_t* d_out, void* stream) {
 }
 int mh_raw_screen(MhRaw* h, uint8_t* d_out, void* stream) {
     if (!h || !d_out) return -1;
-    hipLaunchKernelGGL(k_frames_out, dim3(h->np / 64, GRAY_PIX / 16), dim3(256), 0, (hipStream_t)stream, h->screen,
-                       h->np, h->n, d_out);
-    CK(hipGetLastError());
+    CK(hipMemcpyAsync(d_out, h->screen, (size_t)h->n * GRAY_PIX, hipMemcpyDeviceToDevice, (hipStream_t)stream));
     return 0;
 }
 int mh_raw_screen_rgb(MhRaw* h, const uint8_t* d_rgb64, uint8_t* d_out, void* stream) {

@@ -1,9 +1,20 @@
-// Device-side NES console for gfx950: one env per lane.
+// Device-side NES console for gfx950: one console per wave.
 //
-// Layout in HBM (all lane-interleaved, NP = env count rounded up to a multiple of 64):
-//   MEM[row * NP + e]  one byte per row: RAM 0..2047, VRAM 2048..4095, OAM 4096..4351, PAL 4352..4383.
-//                      Lanes that touch the same emulated address touch one contiguous 64-byte run.
-//   SC[word * NP + e]  32-bit scalar registers of the CPU / PPU / joypads (enum Scalar).
+// A wave runs one console. Its whole state is wave-uniform, the memory (RAM, VRAM, OAM, palette) in LDS while a kernel
+// runs, and every branch of the emulation is a scalar branch. The registers stay in one vector register, word k in
+// lane k (struct File): frame() holds the CPU's in scalar registers and calls the PPU's catch-up, the register
+// accesses and the rare whole instruction as functions, which take the words they need out of the file and put back
+// what they change. (With all of them as variables of one inlined frame loop, the ~45 words and the copies where its
+// paths join did not fit the scalar registers: a loop iteration took 1,700 cycles, most of them spill code.) The 64
+// lanes work together where there is data to spread over them: the pixels of a batch of render lines, the sprite
+// evaluation, the sprite-0 hit's pixels, and the copies of memory. Measured against 16 consoles per wave in lockstep
+// (each on four lanes, state in vector registers, RAM in global memory): k_step in mario_hip.hip.
+//
+// Layout in HBM:
+//   MEM[e * MEM_ROWS + row]  one byte per row: RAM 0..2047, VRAM 2048..4095, OAM 4096..4351, PAL 4352..4383.
+//                            (The host build, tests/hostbuild, interleaves its consoles: MEM[row * NP + e].)
+//   SC[word * NP + e]        32-bit scalar registers of the CPU / PPU / joypads (enum Scalar), NP = the env count
+//                            rounded up to a multiple of 64.
 // PRG (32 KB) and CHR (8 KB) are read-only and shared by every env: each workgroup stages them in LDS.
 //
 // The machine follows the reference's nes-py-exact model (csrc/nes_core.hpp): instruction-atomic CPU
@@ -15,74 +26,51 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-// an empty asm that makes the compiler hold x in a vector register at this point (the host build of this
-// code, tests/hostbuild, defines it with a host register constraint)
-#ifndef MH_REG_BARRIER
-#define MH_REG_BARRIER(x) asm volatile("" : "+v"(x))
+// The host build of this code (tests/hostbuild) runs a console on one lane, with a one-lane wave's intrinsics.
+#ifndef MH_LANES_PER_ENV
+#define MH_LANES_PER_ENV 64
+#endif
+// Pointers through which wave-uniform addresses of read-only data are loaded with scalar loads (the constant
+// address space): data in device memory which no kernel writes.
+#ifndef MH_SCALAR_CONST
+#define MH_SCALAR_CONST __attribute__((address_space(4)))
 #endif
 
 namespace mh {
 
 constexpr int ROW_RAM = 0, ROW_VRAM = 2048, ROW_OAM = 4096, ROW_PAL = 4352, MEM_ROWS = 4384;
-// Most envs (consoles) of one instance: the padded count np (a multiple of 64) keeps MEM_ROWS * np below
-// 2^32, so every byte of the console memory has a 32-bit offset from its base.
+// Most envs (consoles) of one instance: the padded count np (a multiple of 64) keeps MEM_ROWS * np below 2^32.
 constexpr uint32_t MAX_ENVS = (uint32_t)((0xffffffffull / MEM_ROWS) & ~63ull);
 static_assert(MAX_ENVS == 979648 && (uint64_t)MEM_ROWS * MAX_ENVS <= 0xffffffffull, "32-bit console memory offsets");
-// Emulator launch shape. Each env runs on LANES_PER_ENV lanes of a 64-lane wave (its parts: lanes
-// s, s + ENVS_PER_WAVE, ...), so a wave carries ENVS_PER_WAVE = 64 / LANES_PER_ENV envs, and a block of
-// WAVES_PER_BLOCK waves holds LDS_LANES = 128 env slots sharing one LDS copy of the cartridge. The parts run
-// the same console in lockstep, which costs the wave nothing (an instruction issues once for all its lanes),
-// and split the renderer's pixel groups and the sprite evaluation between them. Fewer envs per wave means
-// fewer divergent instruction streams per wave; with 2 parts, 32768 envs are 1024 waves, one per SIMD; with
-// 4 parts they are 2048 waves in blocks of 8, two per SIMD, so one wave issues while the other waits.
-#ifndef MH_LANES_PER_ENV
-#define MH_LANES_PER_ENV 4
-#endif
-constexpr int LANES_PER_ENV = MH_LANES_PER_ENV;
-// (1 lane per env is the host build of this code, tests/hostbuild: one lane plays the whole wave of an env)
-static_assert(LANES_PER_ENV == 1 || LANES_PER_ENV == 2 || LANES_PER_ENV == 4, "an env runs on 1, 2 or 4 lanes");
-constexpr int ENVS_PER_WAVE = 64 / LANES_PER_ENV;
-constexpr int LDS_LANES = 128;                                  // env slots sharing one block's per-lane LDS buffers
-constexpr int WAVES_PER_BLOCK = LDS_LANES / ENVS_PER_WAVE;
-constexpr int EMU_WAVES_PER_SIMD = WAVES_PER_BLOCK / 4;        // one block per CU (its LDS), 4 SIMDs per CU
-// a wave's ballot bit of every part of the env in its lane 0 (shifted by the env's slot in the wave)
-constexpr uint64_t PART_LANES = LANES_PER_ENV == 1 ? 1ull : LANES_PER_ENV == 2 ? 0x0000000100000001ull
-                                                                            : 0x0001000100010001ull;
-constexpr int LDS_SP_WORDS = 64, LDS_GP_WORDS = 8; // words per lane: sprite line (256 B), gray palette (32 B)
-constexpr int LDS_BG_WORDS = 20;                   // words per lane: two name-table rows (64 tiles) + their attributes
-constexpr int LDS_BG_ATTR = 64;                    // byte offset of the attribute bytes in the tile row
-constexpr int LDS_OAM_WORDS = 64;                  // words per lane: OAM (sprite i = word i: y, tile, attr, x)
-constexpr int LDS_XCHG_WORDS = LANES_PER_ENV;     // words per env slot: the parts' pieces of the sprite-range mask
-constexpr int LDS_GP_REGION = LDS_GP_WORDS + LDS_BG_WORDS + LDS_OAM_WORDS + LDS_XCHG_WORDS;   // palette, tile row, OAM, exchange
+constexpr int LANES = MH_LANES_PER_ENV;
+static_assert(LANES == 1 || LANES == 64, "a console runs on a wave's 64 lanes, or on the host's one");
+constexpr bool ON_GPU = LANES == 64;
+// Emulator launch shape: blocks of up to 16 waves, one console each, one block per CU: four waves per SIMD, so that
+// a wave's scalar loads, LDS reads and branches are covered by the others' instructions (a SIMD issues one scalar
+// instruction per 4 cycles, whichever wave it is from).
+constexpr int WAVES_PER_BLOCK = 16;
+constexpr int EMU_WAVES_PER_SIMD = WAVES_PER_BLOCK / 4;
+constexpr int LDS_LANES = ON_GPU ? WAVES_PER_BLOCK : 1;        // consoles sharing one block's LDS
+// A console's share of LDS: its memory, then the renderer's words: the gray palette, and the sprite entries (8 a line)
+// of the DRAW_LINES lines drawn at once.
+constexpr int LDS_SP_WORDS = MEM_ROWS / 4;
+constexpr int DRAW_LINES = 4;
+constexpr int GP_PALETTE = 0, GP_SPRITES = 8, LDS_GP_REGION = GP_SPRITES + 8 * DRAW_LINES;
+constexpr int LDS_ENV_WORDS = LDS_SP_WORDS + LDS_GP_REGION;
 constexpr int FRAME_ITERS = 29781;                 // CPU iterations per nes-py Emulator::step
-#ifndef MH_LONE_MAX_ENVS
-#define MH_LONE_MAX_ENVS 6
-#endif
-// Lone runs (Console::lone_run) take over a wave's instructions once at most this many of its consoles have any
-// left in the current stretch: those consoles' runs follow one another.
-constexpr int LONE_MAX_ENVS = MH_LONE_MAX_ENVS;
-// Render lines per frame slice (a power of two). A wave runs its lanes' CPUs to the end of a group of
-// this many lines and then catches their PPUs up together; a wave iteration costs the slowest lane's
-// instruction, so longer slices let the lanes' per-line instruction counts average out, while a lane
-// that must catch up inside a slice (a PPU register access) renders those lines alone. 8 measured best.
-constexpr int SLICE_LINES = 8;
 constexpr int LINE_END = 341;
 constexpr int GRAY_PIX = 256 * 240;
-// Byte offset of VRAM word w (bytes 4w .. 4w+3) of console e in a memory block of np consoles. The VRAM
-// span of the block (rows ROW_VRAM .. ROW_VRAM + 2047 of the byte-row layout) holds 32-bit words, word w of
-// console e at index w np + e: one load fetches four consecutive VRAM bytes of a console.
-__device__ __forceinline__ size_t vram_word_offset(uint32_t np, uint32_t e, uint32_t w) {
-    return (size_t)ROW_VRAM * np + ((size_t)w * np + e) * 4;
+// Byte offset of row `row` of console e in a memory block of np consoles
+__host__ __device__ __forceinline__ size_t mem_offset(uint32_t np, uint32_t e, uint32_t row) {
+    return ON_GPU ? (size_t)e * MEM_ROWS + row : (size_t)row * np + e;
 }
 // Console::ppu_flags bits: PPUMASK (show / hide-edge, bits 0-3) and PPUCTRL (bits 4-8) settings
 enum : uint32_t { PF_SHOW_BG = 1, PF_SHOW_SPR = 2, PF_HIDE_EDGE_BG = 4, PF_HIDE_EDGE_SPR = 8, PF_LONG_SPR = 16,
                   PF_NMI_EN = 32, PF_BG_PAGE = 64, PF_SPR_PAGE = 128, PF_INC32 = 256 };
 enum : uint8_t { FN = 0x01, FV = 0x02, FONE = 0x04, FB = 0x08, FD = 0x10, FI = 0x20, FZ = 0x40, FC = 0x80 };
 // Error flags or-ed into a console's bad-op counter (every parity check requires a zero count):
-// ERR_HACK_LIMIT  the env layer's busy-state loop hit its frame limit;
-// ERR_TWIN        a sprite evaluation ran on some of an env's lanes without the others, so the pieces of the
-//                 sprite-range mask it read from their exchange words were stale.
-constexpr uint32_t ERR_HACK_LIMIT = 1u << 24, ERR_TWIN = 1u << 25, ERR_FLAGS = ERR_HACK_LIMIT | ERR_TWIN;
+// ERR_HACK_LIMIT  the env layer's busy-state loop hit its frame limit.
+constexpr uint32_t ERR_HACK_LIMIT = 1u << 24, ERR_FLAGS = ERR_HACK_LIMIT;
 enum : uint8_t { ST_PRE = 0, ST_RENDER = 1, ST_POST = 2, ST_VBLANK = 3 };
 
 // Scalar words of one console, interleaved as SC[w * NP + e].
@@ -91,7 +79,11 @@ enum Scalar : int {
     S_JOY_STROBE0, S_JOY_STROBE1, S_JOY_BUTTONS0, S_JOY_BUTTONS1, S_JOY_BITS0, S_JOY_BITS1,
     S_PSTATE, S_EVEN, S_VBLANK, S_S0HIT, S_FIRST_WRITE, S_DATA_BUFFER, S_OAM_ADDR, S_FINE_X,
     S_SHOW_BG, S_SHOW_SPR, S_HIDE_EDGE_BG, S_HIDE_EDGE_SPR, S_LONG_SPR, S_NMI_EN, S_BG_PAGE, S_SPR_PAGE,
-    S_NSL, S_SL_LO, S_SL_HI, S_PCYC, S_SCANLINE, S_V, S_T, S_INC, S_COUNT
+    S_NSL, S_SL_LO, S_SL_HI, S_PCYC, S_SCANLINE, S_V, S_T, S_INC, S_COUNT,
+    // words of a running console's register file beside them: the PPUCTRL / PPUMASK settings and the joypads packed, the
+    // PPU's position (relative to the frame start), derived state, and the counters of the frame being run
+    F_PPU_FLAGS = S_COUNT, F_JOY, F_JOY_STROBE, F_PPU_CALLS, F_NMI_THRESH, F_NMI_CALL, F_PEND_LINE, F_PAL_DIRTY,
+    F_BAD, F_INSTR, F_FF, F_COUNT
 };
 
 // Base cycles per opcode (data table of nes_core.hpp:42-51; 0 = not an official opcode).
@@ -219,379 +211,182 @@ struct Table {
 
 __device__ __constant__ static const dec::Table kDecode{};
 
-// Read-only cartridge view: PRG/CHR in LDS, name-table offsets in registers (uniform).
-// Pointers through which wave-uniform addresses of read-only data are loaded with scalar loads (the constant
-// address space): the PRG image in device memory, which no kernel writes.
-#ifndef MH_SCALAR_CONST
-#define MH_SCALAR_CONST __attribute__((address_space(4)))
+#if defined(__AMDGCN__)
+// v_writelane_b32 (clang has no builtin for the intrinsic)
+extern "C" __device__ int mh_writelane(int value, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
 #endif
-// Device memory addressed as such (global loads and stores: no flat-address aperture check, and their waits
-// count only vector memory, not the scalar loads in flight beside them)
-#ifndef MH_GLOBAL
-#define MH_GLOBAL __attribute__((address_space(1)))
-#endif
-
-// ---------------------------------------------------------------- long lone runs
-// A console that is one of the last few of its wave with instructions to run (at most LONE_MAX_ENVS; the frame
-// loop calls Console::lone_run() for each of them in turn, under its own lanes) runs them in lone_long(): out of
-// line, in registers of its own (not the frame loop's), wave-uniform, with one body per opcode whose decode word
-// is known at compile time, so that the addressing, the operation, its flags and its control flow fold to the
-// few scalar instructions the opcode needs. Measured on one console running a loop of register instructions:
-// 0.18 us per instruction (built with the structurizer skipping uniform regions, which leaves the opcode switch a
-// plain compare tree; 0.37 us without), against 0.67 us for a body that takes the decode word's fields at run
-// time (inline, as a switch per field).
-// The registers of a lone run, wave-uniform: pc, a, x, y, sp, p, exec_at (ex), zero_skip (zs), the PPU's v and t
-// (vt: v | t << 16), fine x and write toggle (px: fine_x | first_write << 8; outputs: bit 16, the run wrote the
-// name tables through $2007, and bit 17, it wrote a PPU register), and n, the instructions run (an output).
-struct LoneRegs { uint32_t pc, a, x, y, sp, p; int32_t ex; uint32_t zs, vt, px, n; };
-// LoneCore::pflags: the PPU register writes a lone run may make ($2005, $2006, $2007 to the pattern and name
-// tables) while rendering is off, and the PPUCTRL bits they need
-constexpr uint32_t LP_WRITES = 1u, LP_INC32 = 2u, LP_NT_SHIFT = 4;
-struct LoneCore {
-    LoneRegs r;
-    MH_GLOBAL uint8_t* mem;                    // the console's RAM row 0 (row stride np), the same in every active lane
-    MH_GLOBAL uint8_t* vmem;                   // its VRAM word 0 (word stride 4 np)
-    uint32_t np, pflags;
-    const MH_SCALAR_CONST uint32_t* gprg;      // PRG image (read only): scalar loads
-    __device__ __forceinline__ uint32_t ram(uint32_t ad) const {
-        return __builtin_amdgcn_readfirstlane(mem[(size_t)((ad & 0x7ffu) * np)]);
-    }
-    __device__ __forceinline__ void set_ram(uint32_t ad, uint32_t v) { mem[(size_t)((ad & 0x7ffu) * np)] = (uint8_t)v; }
-    __device__ __forceinline__ uint32_t prg(uint32_t ad) const {
-        ad &= 0x7fffu;
-        return (gprg[ad >> 2] >> (8u * (ad & 3u))) & 0xffu;
-    }
-    // the bus reads and writes a lone run may make: RAM, PRG, and $4000-$7FFF but the joypads (reads) or OAM
-    // DMA and the joypad strobe (writes), which read 0 and ignore writes; anything else (the PPU registers above
-    // all) is left to frame()
-    __device__ __forceinline__ static bool reads_ok(uint32_t ad) { return (ad - 0x2000u) >= 0x2000u && (ad | 1u) != 0x4017u; }
-    __device__ __forceinline__ static bool writes_ok(uint32_t ad) { return (ad - 0x2000u) >= 0x2000u && (ad & ~2u) != 0x4014u; }
-    __device__ __forceinline__ uint32_t read(uint32_t ad) const { return ad < 0x2000u ? ram(ad) : ad >= 0x8000u ? prg(ad) : 0u; }
-    // While rendering is off (both PPUMASK show bits clear), the catch-up PPU neither moves v nor draws anything
-    // but the universal background colour, so the scroll and address writes and the $2007 writes to the pattern
-    // or name tables do not depend on where the PPU has been caught up to, and a lone run makes them without the
-    // catch-up that frame() takes before a PPU register access (a lone run stops before the NMI point, and before
-    // any other PPU register access, $2001 included). $2007 writes to the palette ($3EFF-$3FFE) change that
-    // colour: left to frame().
-    __device__ __forceinline__ bool ppu_write_ok(uint32_t ad) const {
-        if (!(pflags & LP_WRITES) || (ad - 0x2000u) >= 0x2000u) return false;
-        const uint32_t reg = ad & 7u, v = r.vt & 0xffffu;
-        return reg == 5u || reg == 6u || (reg == 7u && (v - 0x3effu) >= 0x100u);
-    }
-    // scroll_write, addr_write and data_write (+ its sp_line reset), as Console does them
-    __device__ __forceinline__ void ppu_write(uint32_t reg, uint32_t d) {
-        uint32_t v = r.vt & 0xffffu, t = r.vt >> 16, fx = r.px & 0xffu, fw = (r.px >> 8) & 1u, dirty = r.px >> 16;
-        if (reg == 5u) {
-            if (fw) { t = (t & ~0x1fu) | (d >> 3); fx = d & 7u; fw = 0; }
-            else { t = (t & ~0x73e0u) | ((d & 7u) << 12) | ((d & 0xf8u) << 2); fw = 1; }
-        } else if (reg == 6u) {
-            if (fw) { t = (t & 0x00ffu) | ((d & 0x3fu) << 8); fw = 0; }
-            else { t = (t & 0xff00u) | d; v = t; fw = 1; }
-        } else {
-            if (v >= 0x2000u && v < 0x3effu) {   // name table (nt_row()): below $2000 the CHR ROM ignores writes
-                const uint32_t k = v < 0x2400u ? 0u : v < 0x2800u ? 1u : v < 0x2c00u ? 2u : 3u;
-                const uint32_t i = ((((pflags >> LP_NT_SHIFT) >> k) & 1u) << 10) | (v & 0x3ffu);
-                vmem[(size_t)((i >> 2) * 4u * np) + (i & 3u)] = (uint8_t)d;
-            }
-            v = (v + ((pflags & LP_INC32) ? 32u : 1u)) & 0xffffu;
-            dirty = 1;
-        }
-        r.vt = v | t << 16;
-        r.px = fx | fw << 8 | dirty << 16 | 1u << 17;
-    }
-};
-
-// One instruction of opcode OP (operand bytes b1, b2) on a lone console; false, with no effect, if it needs
-// frame() (an invalid opcode, a bus access lone runs do not make). instruction()'s rules and the reference's
-// results (nes_core.hpp:619-1163), with every choice on the decode word resolved at compile time.
-template <uint32_t OP>
-__device__ __forceinline__ bool lone_op(LoneCore& c, uint32_t b1, uint32_t b2) {
-    using namespace dec;
-    constexpr uint32_t D = entry((int)OP);
-    constexpr uint32_t am = D & 15u, alu = (D >> ALU_SH) & 15u, src = (D >> SRC_SH) & 7u, dst = (D >> DST_SH) & 7u;
-    constexpr uint32_t xop = (D >> X_SH) & 15u, fl = (D >> FL_SH) & 7u, fop = (D >> FOP_SH) & 7u;
-    constexpr bool rd = (D & RD) != 0, wr = dst == D_MEM, pen = (D & PEN) != 0;
-    constexpr bool zpm = am == M_ZP || am == M_ZPX || am == M_ZPY;   // zero-page modes touch RAM only
-    if constexpr (!(D & OK)) {
-        return false;
-    } else {
-        LoneRegs& r = c.r;
-        if constexpr (OP == 0x4cu)
-            if ((b1 | b2 << 8) == r.pc) return false;   // JMP *: frame()'s idle fast-forward
-        const uint32_t absv = b1 | b2 << 8;
-        const uint32_t p2 = (absv & 0xff00u) | ((absv + 1u) & 0xffu);   // JMP (ind): high byte, page wrap
-        uint32_t ea = 0, base = absv;
-        int32_t sk = 0;
-        if constexpr (am == M_IMM) ea = (r.pc + 1u) & 0xffffu;
-        if constexpr (am == M_ZP) ea = b1;
-        if constexpr (am == M_ZPX) ea = (b1 + r.x) & 0xffu;
-        if constexpr (am == M_ZPY) ea = (b1 + r.y) & 0xffu;
-        if constexpr (am == M_ABS) ea = absv;
-        if constexpr (am == M_ABSX) ea = (absv + r.x) & 0xffffu;
-        if constexpr (am == M_ABSY) ea = (absv + r.y) & 0xffffu;
-        if constexpr (am == M_INDX) { const uint32_t z = (b1 + r.x) & 0xffu; ea = c.ram(z) | c.ram((z + 1u) & 0xffu) << 8; }
-        if constexpr (am == M_INDY) { base = c.ram(b1) | c.ram((b1 + 1u) & 0xffu) << 8; ea = (base + r.y) & 0xffffu; }
-        if constexpr (xop == X_JMPI) {
-            if (!LoneCore::reads_ok(absv) || !LoneCore::reads_ok(p2)) return false;
-        } else {
-            if constexpr (rd && am != M_IMM && !zpm) if (!LoneCore::reads_ok(ea)) return false;
-            if constexpr (wr && !zpm) if (!LoneCore::writes_ok(ea) && !c.ppu_write_ok(ea)) return false;
-        }
-        if constexpr (pen && (am == M_ABSX || am == M_ABSY || am == M_INDY)) sk = ((base ^ ea) & 0xff00u) ? 1 : 0;
-        uint32_t m = b1;
-        if constexpr (rd && am != M_IMM) m = zpm ? c.ram(ea) : c.read(ea);
-        // the operation (alu_op()'s results): result, carry out, overflow
-        const uint32_t rv = src == R_A ? r.a : src == R_X ? r.x : src == R_Y ? r.y : src == R_SP ? r.sp : m;
-        const uint32_t sv = rd ? m : rv, cin = (r.p >> 7) & 1u;   // FC is bit 7
-        uint32_t res = sv, c_out = 0, v_out = 0;
-        if constexpr (alu == OP_ORA) res = r.a | m;
-        if constexpr (alu == OP_AND) res = r.a & m;
-        if constexpr (alu == OP_EOR) res = r.a ^ m;
-        if constexpr (alu == OP_ADC || alu == OP_SBC || alu == OP_CMP) {
-            const uint32_t ax = alu == OP_CMP ? rv : r.a, m2 = alu == OP_ADC ? m : m ^ 0xffu;
-            const uint32_t t = ax + m2 + (alu == OP_CMP ? 1u : cin);
-            res = t & 0xffu; c_out = t >> 8; v_out = (ax ^ t) & (m2 ^ t) & 0x80u;
-        }
-        if constexpr (alu == OP_ASL) { res = (sv << 1) & 0xffu; c_out = sv >> 7; }
-        if constexpr (alu == OP_ROL) { res = ((sv << 1) | cin) & 0xffu; c_out = sv >> 7; }
-        if constexpr (alu == OP_LSR) { res = sv >> 1; c_out = sv & 1u; }
-        if constexpr (alu == OP_ROR) { res = (sv >> 1) | cin << 7; c_out = sv & 1u; }
-        if constexpr (alu == OP_INC) res = (sv + 1u) & 0xffu;
-        if constexpr (alu == OP_DEC) res = (sv - 1u) & 0xffu;
-        const uint32_t nz = (res ? 0u : (uint32_t)FZ) | (res >> 7);   // FN is bit 0
-        if constexpr (fl == FL_NZ) r.p = (r.p & ~(uint32_t)(FZ | FN)) | nz;
-        if constexpr (fl == FL_NZC) r.p = (r.p & ~(uint32_t)(FZ | FN | FC)) | nz | (c_out ? (uint32_t)FC : 0u);
-        if constexpr (fl == FL_NZCV)
-            r.p = (r.p & ~(uint32_t)(FZ | FN | FC | FV)) | nz | (c_out ? (uint32_t)FC : 0u) | (v_out ? (uint32_t)FV : 0u);
-        if constexpr (fl == FL_BIT)
-            r.p = (r.p & ~(uint32_t)(FZ | FV | FN)) | ((r.a & m) ? 0u : (uint32_t)FZ) | ((m & 0x40u) ? (uint32_t)FV : 0u) | (m >> 7);
-        if constexpr (fl == FL_OP) {   // CLC SEC CLI SEI CLV CLD SED
-            constexpr uint32_t fm = fop < 2 ? FC : fop < 4 ? FI : fop == 4 ? FV : FD;
-            constexpr uint32_t fset = (fop == 1 || fop == 3 || fop == 6) ? fm : 0u;
-            r.p = (r.p & ~fm) | fset;
-        }
-        if constexpr (dst == D_A) r.a = res;
-        if constexpr (dst == D_X) r.x = res;
-        if constexpr (dst == D_Y) r.y = res;
-        if constexpr (dst == D_SP) r.sp = res;
-        if constexpr (wr) {
-            if (zpm || ea < 0x2000u) c.set_ram(ea, res);
-            else if ((ea - 0x2000u) < 0x2000u) c.ppu_write(ea & 7u, res);   // admitted above (ppu_write_ok)
-            // writes elsewhere are ignored
-        }
-        // control flow
-        const uint32_t ret = (r.pc + 2u) & 0xffffu;
-        uint32_t npc = (r.pc + (am == M_NONE ? 1u : (am == M_ABS || am == M_ABSX || am == M_ABSY) ? 3u : 2u)) & 0xffffu;
-        if constexpr (xop == X_BRANCH) {   // on N, V, C, Z (op bits 6-7) equal to op bit 5
-            constexpr uint32_t fbit = (0x40800201u >> (8 * (OP >> 6))) & 0xffu;   // FN FV FC FZ
-            if (((r.p & fbit) != 0) == ((OP & 0x20u) != 0)) {
-                npc = (ret + (uint32_t)(int32_t)(int8_t)b1) & 0xffffu;
-                sk += ((ret ^ npc) & 0xff00u) ? 3 : 1;
-            } else {
-                npc = ret;
-            }
-        }
-        if constexpr (xop == X_JMP) npc = absv;
-        if constexpr (xop == X_JMPI) npc = c.read(absv) | c.read(p2) << 8;
-        if constexpr (xop == X_JSR) {
-            c.set_ram(0x100u | r.sp, ret >> 8);
-            c.set_ram(0x100u | ((r.sp - 1u) & 0xffu), ret & 0xffu);
-            r.sp = (r.sp - 2u) & 0xffu;
-            npc = absv;
-        }
-        if constexpr (xop == X_BRK) {
-            c.set_ram(0x100u | r.sp, ret >> 8);
-            c.set_ram(0x100u | ((r.sp - 1u) & 0xffu), ret & 0xffu);
-            c.set_ram(0x100u | ((r.sp - 2u) & 0xffu), r.p | 0x30u);
-            r.sp = (r.sp - 3u) & 0xffu;
-            r.p |= FI;
-            npc = c.prg(0xfffe) | c.prg(0xffff) << 8;
-            sk += 7;
-        }
-        if constexpr (xop == X_PHA || xop == X_PHP) {
-            c.set_ram(0x100u | r.sp, xop == X_PHA ? r.a : r.p);
-            r.sp = (r.sp - 1u) & 0xffu;
-        }
-        if constexpr (xop == X_PLA || xop == X_PLP) {
-            const uint32_t u = c.ram(0x100u | ((r.sp + 1u) & 0xffu));
-            r.sp = (r.sp + 1u) & 0xffu;
-            if constexpr (xop == X_PLA) { r.a = u; r.p = (r.p & ~(uint32_t)(FZ | FN)) | (u ? 0u : (uint32_t)FZ) | (u >> 7); }
-            else r.p = u;
-        }
-        if constexpr (xop == X_RTS) {
-            const uint32_t lo = c.ram(0x100u | ((r.sp + 1u) & 0xffu)), hi = c.ram(0x100u | ((r.sp + 2u) & 0xffu));
-            r.sp = (r.sp + 2u) & 0xffu;
-            npc = ((lo | hi << 8) + 1u) & 0xffffu;
-        }
-        if constexpr (xop == X_RTI) {
-            const uint32_t f = c.ram(0x100u | ((r.sp + 1u) & 0xffu)), lo = c.ram(0x100u | ((r.sp + 2u) & 0xffu)),
-                           hi = c.ram(0x100u | ((r.sp + 3u) & 0xffu));
-            r.sp = (r.sp + 3u) & 0xffu;
-            r.p = f; npc = lo | hi << 8;
-        }
-        r.pc = npc;
-        sk += (int32_t)((D >> CYC_SH) & 7u);
-        r.ex += sk >= 1 ? sk : 1;
-        r.zs = sk <= 0 ? 1u : 0u;   // opcodes the cycle table gives 0 cycles (and no penalty)
-        return true;
-    }
-}
-
+// A wave-uniform value, in a scalar register
+__device__ __forceinline__ uint32_t uni(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 // A wave-uniform 64-bit value (a pointer): the builtin returns a signed int, so each half is taken as unsigned
 // before it is widened (else the low half's bit 31 would spread into the high half).
-__device__ __forceinline__ uint64_t lone_uniform64(uint64_t v) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return (uint64_t)lo | (uint64_t)hi << 32;
-}
+__device__ __forceinline__ uint64_t uni64(uint64_t v) { return (uint64_t)uni((uint32_t)v) | (uint64_t)uni((uint32_t)(v >> 32)) << 32; }
 
-// Runs lone instructions from r until one needs frame(): its catch-up point 3 (ex + 1) past lim, its opcode or
-// operands outside PRG, the idle `JMP *`, or what lone_op() refuses. Returns the registers after the last one
-// run and, in n, how many ran. Not inlined: its registers are its own, not the frame loop's.
-__device__ __attribute__((noinline)) LoneRegs lone_long(LoneRegs in, int32_t lim, uint8_t* mem, uint8_t* vmem,
-                                                        uint32_t np, uint32_t pflags, const uint8_t* gprg) {
-    LoneCore c;
-    c.r.pc = __builtin_amdgcn_readfirstlane(in.pc); c.r.a = __builtin_amdgcn_readfirstlane(in.a);
-    c.r.x = __builtin_amdgcn_readfirstlane(in.x); c.r.y = __builtin_amdgcn_readfirstlane(in.y);
-    c.r.sp = __builtin_amdgcn_readfirstlane(in.sp); c.r.p = __builtin_amdgcn_readfirstlane(in.p);
-    c.r.ex = (int32_t)__builtin_amdgcn_readfirstlane((uint32_t)in.ex);
-    c.r.zs = __builtin_amdgcn_readfirstlane(in.zs);
-    c.r.vt = __builtin_amdgcn_readfirstlane(in.vt); c.r.px = __builtin_amdgcn_readfirstlane(in.px);
-    lim = (int32_t)__builtin_amdgcn_readfirstlane((uint32_t)lim);
-    c.mem = (MH_GLOBAL uint8_t*)(void*)lone_uniform64((uint64_t)mem);
-    c.vmem = (MH_GLOBAL uint8_t*)(void*)lone_uniform64((uint64_t)vmem);
-    c.np = __builtin_amdgcn_readfirstlane(np);
-    c.pflags = __builtin_amdgcn_readfirstlane(pflags);
-    c.gprg = (const MH_SCALAR_CONST uint32_t*)(const void*)lone_uniform64((uint64_t)gprg);
-    // the catch-up test 3 (ex + 1) > lim as ex > exlim, exlim = floor((lim - 3) / 3)
-    const int32_t l3 = lim - 3;
-    const int32_t exlim = l3 / 3 - (l3 % 3 < 0 ? 1 : 0);
-    uint32_t n = 0;
-    for (;;) {
-        if (c.r.ex > exlim) break;                         // parks or catches up in frame()
-        if (c.r.pc - 0x8000u > 0x7ffdu) break;             // opcode or operands through the bus
-        const uint32_t pa = c.r.pc & 0x7fffu;
-        const uint64_t w = (uint64_t)c.gprg[(pa >> 2) + 1] << 32 | c.gprg[pa >> 2];
-        const uint32_t b0 = (uint32_t)(w >> (8 * (pa & 3u)));   // bytes pc .. pc + 3
-        const uint32_t op = b0 & 0xffu, b1 = (b0 >> 8) & 0xffu, b2 = (b0 >> 16) & 0xffu;
-        switch (op) {   // an opcode that needs frame() (lone_op() false) ends the run
-#define MH_LONE_CASE(i) case i: if (!lone_op<i>(c, b1, b2)) goto done; break;
-#define MH_LONE_CASE4(i) MH_LONE_CASE(i) MH_LONE_CASE(i + 1) MH_LONE_CASE(i + 2) MH_LONE_CASE(i + 3)
-#define MH_LONE_CASE16(i) MH_LONE_CASE4(i) MH_LONE_CASE4(i + 4) MH_LONE_CASE4(i + 8) MH_LONE_CASE4(i + 12)
-#define MH_LONE_CASE64(i) MH_LONE_CASE16(i) MH_LONE_CASE16(i + 16) MH_LONE_CASE16(i + 32) MH_LONE_CASE16(i + 48)
-            MH_LONE_CASE64(0) MH_LONE_CASE64(64) MH_LONE_CASE64(128) MH_LONE_CASE64(192)
-#undef MH_LONE_CASE64
-#undef MH_LONE_CASE16
-#undef MH_LONE_CASE4
-#undef MH_LONE_CASE
-            default: goto done;
-        }
-        n++;
-    }
-done:
-    c.r.n = n;
-    return c.r;
-}
+}  // namespace mh
+#include "cpu_gfx950.hpp"
+namespace mh {
+
+// Memory in LDS, addressed as such
+#ifndef MH_LDS
+#if defined(__AMDGCN__)
+#define MH_LDS __attribute__((address_space(3)))
+#else
+#define MH_LDS
+#endif
+#endif
 
 struct Cart {
-    const uint8_t* prg;      // 0x8000 bytes (16 KB images mirrored)
-    const uint8_t* gprg;     // the same PRG image in device memory (scalar loads of wave-uniform addresses)
-    const uint8_t* chr;      // 0x2000 bytes
-    const uint32_t* dec;     // decode words (LDS copy of kDecode)
+    const MH_LDS uint8_t* prg;   // 0x8000 bytes (16 KB images mirrored), in LDS
+    const MH_LDS uint8_t* chr;   // 0x2000 bytes, in LDS
+    const uint32_t* dec;     // decode words (kDecode)
+    const uint32_t* recs;    // the program as records (cpu_gfx950.hpp; none on the host build, which decodes as it goes)
     uint32_t nt_bits;        // bit k set: name table k ($2000 + k * $400) maps to VRAM $400, else to $000
 };
 
-struct Console {
+typedef uint32_t mh_u32x4 __attribute__((ext_vector_type(4)));
+
+// A console's registers: word k (Scalar) in lane k of one vector register. (The host build: an array.)
+struct File {
+#if defined(__AMDGCN__)
+    uint32_t r;
+    __device__ __forceinline__ uint32_t get(int k) const { return (uint32_t)__builtin_amdgcn_readlane((int)r, k); }
+    __device__ __forceinline__ void set(int k, uint32_t v) { r = (uint32_t)mh_writelane((int)uni(v), k, (int)r); }
+#else
+    uint32_t r[F_COUNT];
+    uint32_t get(int k) const { return r[k]; }
+    void set(int k, uint32_t v) { r[k] = v; }
+#endif
+};
+static_assert(F_COUNT <= 64, "a word per lane");
+
+// What a console's functions need beside its registers: LDS addresses, the program's records, the frame buffer. On the
+// GPU the words of a second vector register, so that a call takes two.
+struct Ctx {
+#if defined(__AMDGCN__)
+    File w;
+    enum : int { M, GP, PRG, CHR, LUT, DEC_LO, DEC_HI, RECS_LO, RECS_HI, GRAY_LO, GRAY_HI, NT_BITS, NP, RENDER };
+#else
+    uint8_t* m; uint32_t* gp; Cart cart; uint8_t* gray; const uint8_t* lut; uint32_t np; bool render;
+#endif
+};
+
+// The machine with its registers as variables, for the length of one function.
+struct Core {
     // ---- memory views
-    // Addresses are a wave-uniform base and a 32-bit per-lane byte offset (the MEM array is below 4 GiB:
-    // MAX_ENVS), so a load or store is one address add into the offset and the base stays in scalar registers.
-    uint8_t* mbase;          // MEM: row r of env e at byte r * np + e
-    uint32_t eo;             // e
-    uint32_t vo;             // byte offset of this env's VRAM word 0 (word w at vo + 4 w np)
-    uint32_t np;
-    Cart cart;
-    uint8_t* gray;           // GRAY slot + 4 e: pixels 4i..4i+3 in the 32-bit word at gray + 4 i np
-    const uint8_t* lut;      // palette value -> gray (LDS, 256 entries)
+    MH_LDS uint8_t* m;       // the console's memory in LDS: byte r is row r (ROW_*)
+    MH_LDS uint32_t* gp;     // the renderer's words in LDS (GP_*)
+    uint32_t np;             // envs of the memory block, padded: the host build's interleaved frame buffers
+    const MH_LDS uint8_t* prg_;              // 0x8000 bytes (16 KB images mirrored)
+    const MH_LDS uint8_t* chr;               // 0x2000 bytes
+    const MH_LDS uint8_t* lut;               // palette value -> gray (256 entries)
+    const uint32_t* dec;                     // decode words
+    uint32_t nt_bits;
+    uint8_t* gray;           // the env's frame buffer: pixels 4i..4i+3 in the 32-bit word at gray + 4 i gray_step()
     bool render;
-    uint8_t part;            // which of the env's LANES_PER_ENV lanes this is (all run the console; the
-                             // renderer and the sprite evaluation split their work between them)
-    // Small fields share 32-bit words as bitfields (8 or 16 bits wide, so they wrap as the byte and
-    // half-word types they stand for): the compiler keeps a word in one register instead of one per
-    // field. Fewer live registers mean fewer spills, and fewer register copies where the paths of
-    // the frame loop join.
+    uint32_t lane;           // this lane of the wave: the only field that differs between the lanes
     // ---- CPU
-    uint16_t pc;
-    uint32_t a : 8, x : 8, y : 8, sp : 8;
-    uint8_t p;
+    uint32_t pc, a, x, y, sp, p;
     int32_t exec_at, ppu_calls, nmi_thresh;  // relative to the current frame start
     uint32_t iter_lo;                        // low word of the iteration count at the frame start
-    uint32_t iter_hi;
     int32_t cur, skip;
+    uint32_t zero_skip;
     // ---- joypads
     // both ports in one word (buttons 0 | buttons 1 << 8 | shift register 0 << 16 | shift register 1 << 24);
-    // their strobes are bits 0 and 1 of joy_strobe (below)
-    uint32_t joy;
+    // their strobes are bits 0 and 1 of joy_strobe
+    uint32_t joy, joy_strobe;
     // ---- PPU
-    uint32_t pstate : 8, even : 8, vblank : 8, s0hit : 8;
-    uint32_t first_write : 8, joy_strobe : 8, zero_skip : 8, pal_dirty : 8;   // zero_skip: CPU, pal_dirty: derived
-    uint32_t fine_x : 8, oam_addr : 8, data_buffer : 8, nsl : 8;
-    // ppu_flags: the PPUCTRL / PPUMASK settings as PF_* bits; bg_key: name table and coarse y (v bits 5-11)
-    // of the tile row held in LDS (-1: none)
-    uint32_t ppu_flags : 16;
-    int32_t bg_key : 16;
+    uint32_t pstate, even, vblank, s0hit, first_write, fine_x, oam_addr, data_buffer, nsl;
+    uint32_t ppu_flags;                      // the PPUCTRL / PPUMASK settings as PF_* bits
     uint32_t sl_lo, sl_hi;                   // sprite list: 8 indices packed in two words
     int32_t pcyc, scanline;
-    uint32_t v : 16, t : 16;
-    // ---- counters
+    uint32_t v, t;
+    int32_t nmi_call;                        // the PPU call that raised an NMI in this catch-up (0: none)
+    // ---- counters of this frame
     uint32_t bad_ops, instructions;          // instructions: retired, poll-loop fast-forwards included
     uint32_t ff_instructions;                // of those, the ones poll_skip fast-forwarded without executing
-    uint32_t nframe;                         // frame() calls since load(): the wave's issue priority in frame()
     // ---- derived state (not part of the machine state)
-    // pend_line: scanline of a sprite evaluation not yet materialized (-1: the list is current);
-    // sp_line: scanline the LDS sprite line buffer holds (-1: invalid); pal_dirty (above): the LDS gray
-    // palette must be rebuilt
-    int32_t pend_line : 16, sp_line : 16;
-    uint32_t* lds_sp;        // per-lane sprite line buffer: word (x / 4) of this lane at lds_sp[(x / 4) * LDS_LANES]
-    uint32_t* lds_gp;        // per-lane gray palette: word (i / 4) at lds_gp[(i / 4) * LDS_LANES]
-    uint32_t* lds_bg;        // per-lane background tile row (same word stride), valid for v's bits 5-11 == bg_key
-    uint32_t* lds_oam;       // per-lane OAM (same word stride): the live copy between load()/power_on() and store()
+    int32_t pend_line;                       // scanline of a sprite evaluation not yet materialized (-1: the list is current)
+    uint32_t pal_dirty;                      // the gray palette in LDS must be rebuilt
 
-    // ------------------------------------------------------------ interleaved memory
-    __device__ __forceinline__ uint8_t ld(uint32_t row) const { return mbase[(uint32_t)__umul24(row, np) + eo]; }
-    __device__ __forceinline__ void st(uint32_t row, uint8_t val) { mbase[(uint32_t)__umul24(row, np) + eo] = val; }
-    __device__ __forceinline__ uint8_t ram(uint32_t a) const { return ld(ROW_RAM + (a & 0x7ff)); }
-    __device__ __forceinline__ uint8_t oam(uint32_t i) const {
-        i &= 0xff;
-        return ((const uint8_t*)lds_oam)[(i >> 2) * LDS_LANES * 4 + (i & 3)];
+    // ------------------------------------------------------------ in and out of the register file
+    __device__ __forceinline__ void attach(const Ctx& c) {
+#if defined(__AMDGCN__)
+        auto ptr = [&](int k) { return (uint64_t)c.w.get(k) | (uint64_t)c.w.get(k + 1) << 32; };
+        m = (MH_LDS uint8_t*)(uintptr_t)c.w.get(Ctx::M); gp = (MH_LDS uint32_t*)(uintptr_t)c.w.get(Ctx::GP);
+        prg_ = (const MH_LDS uint8_t*)(uintptr_t)c.w.get(Ctx::PRG); chr = (const MH_LDS uint8_t*)(uintptr_t)c.w.get(Ctx::CHR);
+        lut = (const MH_LDS uint8_t*)(uintptr_t)c.w.get(Ctx::LUT); dec = (const uint32_t*)ptr(Ctx::DEC_LO);
+        gray = (uint8_t*)ptr(Ctx::GRAY_LO); nt_bits = c.w.get(Ctx::NT_BITS); np = c.w.get(Ctx::NP);
+        render = c.w.get(Ctx::RENDER) != 0; lane = __lane_id();
+#else
+        m = c.m; gp = c.gp; prg_ = c.cart.prg; chr = c.cart.chr; lut = c.lut; dec = c.cart.dec; gray = c.gray;
+        nt_bits = c.cart.nt_bits; np = c.np; render = c.render; lane = 0;
+#endif
     }
-    __device__ __forceinline__ void set_oam(uint32_t i, uint8_t val) {
-        i &= 0xff;
-        ((uint8_t*)lds_oam)[(i >> 2) * LDS_LANES * 4 + (i & 3)] = val;
+    __device__ __forceinline__ void open_ppu(const File& f) {
+        pstate = f.get(S_PSTATE); even = f.get(S_EVEN); vblank = f.get(S_VBLANK); s0hit = f.get(S_S0HIT);
+        fine_x = f.get(S_FINE_X); oam_addr = f.get(S_OAM_ADDR); nsl = f.get(S_NSL); ppu_flags = f.get(F_PPU_FLAGS);
+        sl_lo = f.get(S_SL_LO); sl_hi = f.get(S_SL_HI); pcyc = (int32_t)f.get(S_PCYC); scanline = (int32_t)f.get(S_SCANLINE);
+        v = f.get(S_V); t = f.get(S_T); ppu_calls = (int32_t)f.get(F_PPU_CALLS); nmi_thresh = (int32_t)f.get(F_NMI_THRESH);
+        pend_line = (int32_t)f.get(F_PEND_LINE); pal_dirty = f.get(F_PAL_DIRTY);
     }
-    // sprite k's four OAM bytes: y | tile << 8 | attr << 16 | x << 24
-    __device__ __forceinline__ uint32_t oam_sprite(int k) const { return lds_oam[k * LDS_LANES]; }
-    __device__ __forceinline__ uint8_t pal(uint32_t i) const { return ld(ROW_PAL + (i & 0x1f)); }
-    // VRAM is word-interleaved: byte i of this env is byte i % 4 of 32-bit word i / 4, and word w sits at
-    // byte vo + 4 w np of MEM, so a name-table row is 8 word loads
-    __device__ __forceinline__ uint8_t vram(uint32_t i) const {
-        i &= 0x7ff;
-        return mbase[vo + (uint32_t)__umul24(i >> 2, 4 * np) + (i & 3)];
+    __device__ __forceinline__ void close_ppu(File& f) const {   // what a catch-up changes
+        f.set(S_PSTATE, pstate); f.set(S_EVEN, even); f.set(S_VBLANK, vblank); f.set(S_S0HIT, s0hit);
+        f.set(S_PCYC, (uint32_t)pcyc); f.set(S_SCANLINE, (uint32_t)scanline); f.set(S_V, v);
+        f.set(F_PPU_CALLS, (uint32_t)ppu_calls); f.set(F_NMI_THRESH, (uint32_t)nmi_thresh); f.set(F_NMI_CALL, (uint32_t)nmi_call);
+        f.set(F_PEND_LINE, (uint32_t)pend_line); f.set(F_PAL_DIRTY, pal_dirty);
     }
-    __device__ __forceinline__ void set_vram(uint32_t i, uint8_t d) {
-        i &= 0x7ff;
-        mbase[vo + (uint32_t)__umul24(i >> 2, 4 * np) + (i & 3)] = d;
+    __device__ __forceinline__ void open_io(const File& f) {     // the registers behind the CPU's bus
+        open_ppu(f);
+        first_write = f.get(S_FIRST_WRITE); data_buffer = f.get(S_DATA_BUFFER); joy = f.get(F_JOY);
+        joy_strobe = f.get(F_JOY_STROBE); iter_lo = f.get(S_ITER_LO);
     }
-    __device__ __forceinline__ uint32_t vram_word(uint32_t w) const {
-        return *(const uint32_t*)(mbase + (vo + (uint32_t)__umul24(w & 0x1ff, 4 * np)));
+    __device__ __forceinline__ void close_io(File& f) const {    // what a register access changes
+        f.set(S_VBLANK, vblank); f.set(S_FIRST_WRITE, first_write); f.set(S_DATA_BUFFER, data_buffer); f.set(F_JOY, joy);
+        f.set(F_JOY_STROBE, joy_strobe); f.set(S_OAM_ADDR, oam_addr); f.set(S_FINE_X, fine_x); f.set(F_PPU_FLAGS, ppu_flags);
+        f.set(S_V, v); f.set(S_T, t); close_sprites(f); f.set(F_PAL_DIRTY, pal_dirty);
     }
-    __device__ __forceinline__ uint8_t sl(int k) const {
-        return (uint8_t)((k < 4 ? sl_lo >> (8 * k) : sl_hi >> (8 * (k - 4))) & 0xff);
+    __device__ __forceinline__ void close_sprites(File& f) const {
+        f.set(S_NSL, nsl); f.set(S_SL_LO, sl_lo); f.set(S_SL_HI, sl_hi); f.set(F_PEND_LINE, (uint32_t)pend_line);
     }
-    __device__ __forceinline__ void set_sl(int k, uint8_t i) {
-        if (k < 4) sl_lo = (sl_lo & ~(0xffu << (8 * k))) | ((uint32_t)i << (8 * k));
-        else sl_hi = (sl_hi & ~(0xffu << (8 * (k - 4)))) | ((uint32_t)i << (8 * (k - 4)));
+    __device__ __forceinline__ void open_cpu(const File& f) {
+        pc = f.get(S_PC); a = f.get(S_A); x = f.get(S_X); y = f.get(S_Y); sp = f.get(S_SP); p = f.get(S_P);
+        exec_at = (int32_t)f.get(S_EXEC_REL); zero_skip = f.get(S_ZERO_SKIP);
+        bad_ops = f.get(F_BAD); instructions = f.get(F_INSTR); ff_instructions = f.get(F_FF);
     }
-    __device__ __forceinline__ uint8_t prg(uint16_t a) const { return cart.prg[a & 0x7fff]; }
+    __device__ __forceinline__ void close_cpu(File& f) const {
+        f.set(S_PC, pc); f.set(S_A, a); f.set(S_X, x); f.set(S_Y, y); f.set(S_SP, sp); f.set(S_P, p);
+        f.set(S_EXEC_REL, (uint32_t)exec_at); f.set(S_ZERO_SKIP, zero_skip);
+        f.set(F_BAD, bad_ops); f.set(F_INSTR, instructions); f.set(F_FF, ff_instructions);
+    }
+
+    // ------------------------------------------------------------ memory
+    // The wave has stored to LDS (or to its own memory block) what its lanes read next: a wave's LDS accesses complete
+    // in order, so only the compiler has to keep them so; memory accesses are waited for.
+    __device__ __forceinline__ static void lds_sync() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    __device__ __forceinline__ static void mem_sync() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    }
+    __device__ __forceinline__ uint32_t ram(uint32_t ad) const { return uni(m[ROW_RAM + (ad & 0x7ff)]); }
+    __device__ __forceinline__ void set_ram(uint32_t ad, uint32_t val) { m[ROW_RAM + (ad & 0x7ff)] = (uint8_t)val; }
+    __device__ __forceinline__ uint32_t oam(uint32_t i) const { return uni(m[ROW_OAM + (i & 0xff)]); }
+    __device__ __forceinline__ void set_oam(uint32_t i, uint32_t val) { m[ROW_OAM + (i & 0xff)] = (uint8_t)val; }
+    // sprite k's four OAM bytes: y | tile << 8 | attr << 16 | x << 24 (oam_word: of a lane's own sprite)
+    __device__ __forceinline__ uint32_t oam_word(uint32_t k) const { return ((const MH_LDS uint32_t*)(m + ROW_OAM))[k]; }
+    __device__ __forceinline__ uint32_t oam_sprite(uint32_t k) const { return uni(oam_word(k)); }
+    __device__ __forceinline__ uint32_t sl(int k) const { return ((k < 4 ? sl_lo >> (8 * k) : sl_hi >> (8 * (k - 4))) & 0xffu); }
+    __device__ __forceinline__ void set_sl(int k, uint32_t i) {
+        if (k < 4) sl_lo = (sl_lo & ~(0xffu << (8 * k))) | (i << (8 * k));
+        else sl_hi = (sl_hi & ~(0xffu << (8 * (k - 4)))) | (i << (8 * (k - 4)));
+    }
+    // words between a frame buffer's words: frames are whole on the GPU (a lane's 16 pixels are one 16-byte store),
+    // interleaved by env on the host build
+    __device__ __forceinline__ uint32_t gray_step() const { return ON_GPU ? 1u : np; }
+    __device__ __forceinline__ uint32_t prg(uint32_t ad) const { return uni(prg_[ad & 0x7fff]); }
     // PPUCTRL / PPUMASK settings (0 or 1; inc(): the VRAM address increment, 1 or 32)
     __device__ __forceinline__ uint32_t show_bg() const { return ppu_flags & 1u; }
     __device__ __forceinline__ uint32_t show_spr() const { return (ppu_flags >> 1) & 1u; }
@@ -601,116 +396,42 @@ struct Console {
     __device__ __forceinline__ uint32_t nmi_en() const { return (ppu_flags >> 5) & 1u; }
     __device__ __forceinline__ uint32_t bg_page() const { return (ppu_flags >> 6) & 1u; }
     __device__ __forceinline__ uint32_t spr_page() const { return (ppu_flags >> 7) & 1u; }
-    __device__ __forceinline__ uint16_t inc() const { return (ppu_flags & PF_INC32) ? 32 : 1; }
-    // joypad port 0's buttons for the next frames (the env layer's action)
-    __device__ __forceinline__ void set_buttons0(uint8_t b) { joy = (joy & ~0xffu) | b; }
-
-    // ------------------------------------------------------------ state in / out
-    __device__ void load(const uint32_t* sc, uint32_t e) {
-        auto w = [&](int k) { return sc[(size_t)k * np + e]; };
-        iter_lo = w(S_ITER_LO); iter_hi = w(S_ITER_HI);
-        exec_at = (int32_t)w(S_EXEC_REL);
-        ppu_calls = 0;
-        pc = (uint16_t)w(S_PC); sp = (uint8_t)w(S_SP); a = (uint8_t)w(S_A); x = (uint8_t)w(S_X);
-        y = (uint8_t)w(S_Y); p = (uint8_t)w(S_P); zero_skip = (uint8_t)w(S_ZERO_SKIP);
-        joy_strobe = (uint8_t)((w(S_JOY_STROBE0) & 1u) | (w(S_JOY_STROBE1) & 1u) << 1);
-        joy = (w(S_JOY_BUTTONS0) & 0xffu) | (w(S_JOY_BUTTONS1) & 0xffu) << 8 | (w(S_JOY_BITS0) & 0xffu) << 16 |
-              (w(S_JOY_BITS1) & 0xffu) << 24;
-        pstate = (uint8_t)w(S_PSTATE); even = (uint8_t)w(S_EVEN); vblank = (uint8_t)w(S_VBLANK);
-        s0hit = (uint8_t)w(S_S0HIT); first_write = (uint8_t)w(S_FIRST_WRITE);
-        data_buffer = (uint8_t)w(S_DATA_BUFFER); oam_addr = (uint8_t)w(S_OAM_ADDR); fine_x = (uint8_t)w(S_FINE_X);
-        ppu_flags = (w(S_SHOW_BG) ? PF_SHOW_BG : 0u) | (w(S_SHOW_SPR) ? PF_SHOW_SPR : 0u) |
-                    (w(S_HIDE_EDGE_BG) ? PF_HIDE_EDGE_BG : 0u) | (w(S_HIDE_EDGE_SPR) ? PF_HIDE_EDGE_SPR : 0u) |
-                    (w(S_LONG_SPR) ? PF_LONG_SPR : 0u) | (w(S_NMI_EN) ? PF_NMI_EN : 0u) |
-                    (w(S_BG_PAGE) ? PF_BG_PAGE : 0u) | (w(S_SPR_PAGE) ? PF_SPR_PAGE : 0u) |
-                    (w(S_INC) == 32 ? PF_INC32 : 0u);
-        nsl = (uint8_t)w(S_NSL); sl_lo = w(S_SL_LO); sl_hi = w(S_SL_HI);
-        pcyc = (int32_t)w(S_PCYC); scanline = (int32_t)w(S_SCANLINE);
-        v = (uint16_t)w(S_V); t = (uint16_t)w(S_T);
-        pend_line = -1; sp_line = -1; pal_dirty = true; bg_key = -1;
-        for (int k = 0; k < LDS_OAM_WORDS; k++) {
-            const uint32_t r = ROW_OAM + 4 * k;
-            lds_oam[k * LDS_LANES] = (uint32_t)ld(r) | (uint32_t)ld(r + 1) << 8 | (uint32_t)ld(r + 2) << 16 |
-                                     (uint32_t)ld(r + 3) << 24;
-        }
-        nmi_threshold();
-        nframe = 0;
-    }
-    __device__ void store(uint32_t* sc, uint32_t e) {
-        materialize_sprites();
-        for (int k = 0; k < LDS_OAM_WORDS; k++) {
-            const uint32_t w = oam_sprite(k), r = ROW_OAM + 4 * k;
-            st(r, (uint8_t)w); st(r + 1, (uint8_t)(w >> 8)); st(r + 2, (uint8_t)(w >> 16)); st(r + 3, (uint8_t)(w >> 24));
-        }
-        auto w = [&](int k, uint32_t val) { sc[(size_t)k * np + e] = val; };
-        w(S_ITER_LO, iter_lo); w(S_ITER_HI, iter_hi); w(S_EXEC_REL, (uint32_t)exec_at);
-        w(S_PC, pc); w(S_SP, sp); w(S_A, a); w(S_X, x); w(S_Y, y); w(S_P, p); w(S_ZERO_SKIP, zero_skip);
-        w(S_JOY_STROBE0, joy_strobe & 1u); w(S_JOY_STROBE1, (joy_strobe >> 1) & 1u);
-        w(S_JOY_BUTTONS0, joy & 0xffu); w(S_JOY_BUTTONS1, (joy >> 8) & 0xffu);
-        w(S_JOY_BITS0, (joy >> 16) & 0xffu); w(S_JOY_BITS1, joy >> 24);
-        w(S_PSTATE, pstate); w(S_EVEN, even); w(S_VBLANK, vblank); w(S_S0HIT, s0hit);
-        w(S_FIRST_WRITE, first_write); w(S_DATA_BUFFER, data_buffer); w(S_OAM_ADDR, oam_addr);
-        w(S_FINE_X, fine_x); w(S_SHOW_BG, show_bg()); w(S_SHOW_SPR, show_spr());
-        w(S_HIDE_EDGE_BG, hide_edge_bg()); w(S_HIDE_EDGE_SPR, hide_edge_spr()); w(S_LONG_SPR, long_spr());
-        w(S_NMI_EN, nmi_en()); w(S_BG_PAGE, bg_page()); w(S_SPR_PAGE, spr_page());
-        w(S_NSL, nsl); w(S_SL_LO, sl_lo); w(S_SL_HI, sl_hi); w(S_PCYC, (uint32_t)pcyc);
-        w(S_SCANLINE, (uint32_t)scanline); w(S_V, v); w(S_T, t); w(S_INC, inc());
-    }
-
-    // power-on: zeroed machine, then CPU and PPU reset (nes_core.hpp:123-147)
-    __device__ void power_on() {
-        for (uint32_t r = 0; r < MEM_ROWS; r++)
-            if (r < ROW_VRAM || r >= ROW_VRAM + 2048) st(r, 0);
-        for (uint32_t w = 0; w < 512; w++) *(uint32_t*)(mbase + (vo + (uint32_t)__umul24(w, 4 * np))) = 0;
-        iter_lo = iter_hi = 0; exec_at = 0; ppu_calls = 0;
-        joy_strobe = 3; joy = 0;
-        zero_skip = 0; a = x = y = 0; p = 0x34;
-        pc = (uint16_t)(prg(0xfffc) | prg(0xfffd) << 8);
-        sp = 0xfd;
-        s0hit = 0; data_buffer = 0; vblank = 0; even = 1; ppu_flags = PF_SHOW_BG | PF_SHOW_SPR;
-        first_write = 1; v = 0; pcyc = 0; scanline = 0;
-        oam_addr = 0; fine_x = 0; t = 0; pstate = ST_PRE; nsl = 0; sl_lo = sl_hi = 0;
-        pend_line = -1; sp_line = -1; pal_dirty = true; bg_key = -1;
-        for (int k = 0; k < LDS_OAM_WORDS; k++) lds_oam[k * LDS_LANES] = 0;
-        nmi_threshold();
-    }
-
+    __device__ __forceinline__ uint32_t inc() const { return (ppu_flags & PF_INC32) ? 32 : 1; }
     // ------------------------------------------------------------ CPU bus (nes_core.hpp:150-208)
     // Accesses for which needs_sync() holds see the PPU caught up to 3 * (cur + 1): frame() syncs
     // before it issues them (the reference catches up inside the access; the target is the same).
-    __device__ __forceinline__ static bool needs_sync(uint16_t ad, bool wr) {
-        const bool ppu = (ad & 0xe000) == 0x2000, r2 = (ad & 7) == 2, r7 = (ad & 7) == 7;
-        return (ppu & (wr | r2 | r7)) | (wr & (ad == 0x4014));
+    __device__ __forceinline__ static bool needs_sync(uint32_t ad, bool wr) {
+        if ((ad & 0xe000) == 0x2000) return wr || (ad & 7) == 2 || (ad & 7) == 7;
+        return wr && ad == 0x4014;
     }
-    __device__ __forceinline__ uint8_t read(uint16_t ad) {
+    __device__ __forceinline__ uint32_t read(uint32_t ad) {
         if (ad >= 0x8000) return prg(ad);
         if (ad < 0x2000) return ram(ad);
         if (ad < 0x4000) {
-            const uint16_t r = ad & 0x2007;
-            if (r == 0x2002) return status_read();
-            if (r == 0x2007) return data_read();
-            if (r == 0x2004) return oam(oam_addr);
+            const uint32_t r = ad & 7;
+            if (r == 2) return status_read();
+            if (r == 7) return data_read();
+            if (r == 4) return oam(oam_addr);
             return 0;
         }
         if (ad == 0x4016) return pad_read(0);
         if (ad == 0x4017) return pad_read(1);
         return 0;
     }
-    __device__ __forceinline__ void write(uint16_t ad, uint8_t val) {
-        if (ad < 0x2000) { st(ROW_RAM + (ad & 0x7ff), val); return; }
+    __device__ __forceinline__ void write(uint32_t ad, uint32_t val) {
+        if (ad < 0x2000) { set_ram(ad, val); return; }
         if (ad < 0x4000) {
-            // a pending sprite evaluation is materialized before its inputs (OAM, oam_addr, sprite
-            // size) change; the sprite line buffer is rebuilt after any write that can change it
-            const uint16_t r = ad & 0x2007;
-            if (r == 0x2000 || r == 0x2003 || r == 0x2004) materialize_sprites();
+            // a pending sprite evaluation is materialized before its inputs (OAM, oam_addr, sprite size) change
+            const uint32_t r = ad & 7;
+            if (r == 0 || r == 3 || r == 4) materialize_sprites();
             switch (r) {
-                case 0x2000: ctrl_write(val); sp_line = -1; break;
-                case 0x2001: mask_write(val); break;
-                case 0x2003: oam_addr = val; break;
-                case 0x2004: set_oam(oam_addr, val); oam_addr++; sp_line = -1; break;
-                case 0x2005: scroll_write(val); break;
-                case 0x2006: addr_write(val); break;
-                case 0x2007: data_write(val); sp_line = -1; break;
+                case 0: ctrl_write(val); break;
+                case 1: mask_write(val); break;
+                case 3: oam_addr = val; break;
+                case 4: set_oam(oam_addr, val); oam_addr = (oam_addr + 1) & 0xffu; break;
+                case 5: scroll_write(val); break;
+                case 6: addr_write(val); break;
+                case 7: data_write(val); break;
                 default: break;
             }
             return;
@@ -718,21 +439,11 @@ struct Console {
         if (ad == 0x4014) {  // OAM DMA: 513 cycles, +1 on an odd absolute cycle; copies from RAM pages only
             materialize_sprites();
             skip += 513 + (int)((iter_lo + (uint32_t)cur + 1u) & 1u);
-            const uint16_t src = (uint16_t)(val << 8);
+            const uint32_t src = val << 8;
             if (src < 0x2000) {
-                if (!(oam_addr & 3)) {
-                    // word-aligned: sprite words straight from four RAM bytes each
-                    for (int k = 0; k < LDS_OAM_WORDS; k++) {
-                        const uint32_t a0 = src + 4 * k;
-                        lds_oam[((k + (oam_addr >> 2)) & 63) * LDS_LANES] =
-                            (uint32_t)ram(a0) | (uint32_t)ram(a0 + 1) << 8 | (uint32_t)ram(a0 + 2) << 16 |
-                            (uint32_t)ram(a0 + 3) << 24;
-                    }
-                } else {
-                    for (int i = 0; i < 256; i++) set_oam(oam_addr + i, ram(src + i));
-                }
+                for (uint32_t i = lane; i < 256; i += LANES) m[ROW_OAM + ((oam_addr + i) & 0xff)] = m[ROW_RAM + ((src + i) & 0x7ff)];
+                lds_sync();
             }
-            sp_line = -1;
             return;
         }
         if (ad == 0x4016) {   // strobe both ports; its falling edge latches the buttons into the shift registers
@@ -741,145 +452,120 @@ struct Console {
         }
     }
     // port i: while strobed, button A; else the next bit of its shift register, which then shifts
-    __device__ __forceinline__ uint8_t pad_read(int i) {
+    __device__ __forceinline__ uint32_t pad_read(int i) {
         const uint32_t sh = 16 + 8 * i;
-        const uint8_t bit = (joy_strobe >> i) & 1 ? (uint8_t)((joy >> (8 * i)) & 1u) : (uint8_t)((joy >> sh) & 1u);
-        if (!((joy_strobe >> i) & 1)) joy = (joy & ~(0xffu << sh)) | ((((joy >> sh) & 0xffu) >> 1) << sh);
-        return bit | 0x40;
+        if ((joy_strobe >> i) & 1) return ((joy >> (8 * i)) & 1u) | 0x40u;
+        const uint32_t bit = (joy >> sh) & 1u;
+        joy = (joy & ~(0xffu << sh)) | ((((joy >> sh) & 0xffu) >> 1) << sh);
+        return bit | 0x40u;
     }
 
     // ------------------------------------------------------------ PPU registers (nes_core.hpp:211-260)
-    __device__ void ctrl_write(uint8_t c) {
+    __device__ __forceinline__ void ctrl_write(uint32_t c) {
         ppu_flags = (ppu_flags & (PF_SHOW_BG | PF_SHOW_SPR | PF_HIDE_EDGE_BG | PF_HIDE_EDGE_SPR)) |
                     ((c >> 7) & 1 ? PF_NMI_EN : 0u) | ((c >> 5) & 1 ? PF_LONG_SPR : 0u) |
                     ((c >> 4) & 1 ? PF_BG_PAGE : 0u) | ((c >> 3) & 1 ? PF_SPR_PAGE : 0u) | ((c & 4) ? PF_INC32 : 0u);
-        t = (uint16_t)((t & 0xf3ff) | ((c & 3) << 10));
+        t = (t & 0xf3ff) | ((c & 3) << 10);
     }
-    __device__ void mask_write(uint8_t k) {
+    __device__ __forceinline__ void mask_write(uint32_t k) {
         ppu_flags = (ppu_flags & ~(PF_SHOW_BG | PF_SHOW_SPR | PF_HIDE_EDGE_BG | PF_HIDE_EDGE_SPR)) |
                     (!(k & 2) ? PF_HIDE_EDGE_BG : 0u) | (!(k & 4) ? PF_HIDE_EDGE_SPR : 0u) |
                     ((k >> 3) & 1 ? PF_SHOW_BG : 0u) | ((k >> 4) & 1 ? PF_SHOW_SPR : 0u);
     }
-    __device__ uint8_t status_read() {
-        uint8_t r = (uint8_t)((s0hit << 6) | (vblank << 7));
+    __device__ __forceinline__ uint32_t status_read() {
+        const uint32_t r = (s0hit << 6) | (vblank << 7);
         vblank = 0; first_write = 1;
         return r;
     }
-    __device__ void addr_write(uint8_t d) {
-        if (first_write) { t = (uint16_t)((t & 0x00ff) | ((d & 0x3f) << 8)); first_write = 0; }
-        else { t = (uint16_t)((t & 0xff00) | d); v = t; first_write = 1; }
+    __device__ __forceinline__ void addr_write(uint32_t d) {
+        if (first_write) { t = (t & 0x00ff) | ((d & 0x3f) << 8); first_write = 0; }
+        else { t = (t & 0xff00) | d; v = t; first_write = 1; }
     }
-    __device__ uint8_t data_read() {
-        uint8_t d = vbus_read(v);
-        v = (uint16_t)(v + inc());
-        if (v < 0x3f00) { uint8_t b = data_buffer; data_buffer = d; d = b; }
+    __device__ __forceinline__ uint32_t data_read() {
+        uint32_t d = uni(vbus_read(v));
+        v = (v + inc()) & 0xffffu;
+        if (v < 0x3f00) { const uint32_t b = data_buffer; data_buffer = d; d = b; }
         return d;
     }
-    __device__ void data_write(uint8_t d) { vbus_write(v, d); v = (uint16_t)(v + inc()); }
-    __device__ void scroll_write(uint8_t d) {
-        if (first_write) { t = (uint16_t)((t & ~0x1f) | (d >> 3)); fine_x = d & 7; first_write = 0; }
-        else { t = (uint16_t)((t & ~0x73e0) | ((d & 7) << 12) | ((d & 0xf8) << 2)); first_write = 1; }
+    __device__ __forceinline__ void data_write(uint32_t d) { vbus_write(v, d); v = (v + inc()) & 0xffffu; }
+    __device__ __forceinline__ void scroll_write(uint32_t d) {
+        if (first_write) { t = (t & ~0x1fu) | (d >> 3); fine_x = d & 7; first_write = 0; }
+        else { t = (t & ~0x73e0u) | ((d & 7) << 12) | ((d & 0xf8) << 2); first_write = 1; }
     }
 
     // ------------------------------------------------------------ picture bus (nes_core.hpp:263-285)
-    __device__ __forceinline__ uint32_t nt_row(uint16_t ad) const {
+    // (vbus_read and nametable take a lane's own address too)
+    __device__ __forceinline__ uint32_t nt_row(uint32_t ad) const {
         const uint32_t k = ad < 0x2400 ? 0 : ad < 0x2800 ? 1 : ad < 0x2c00 ? 2 : 3;
-        return (((cart.nt_bits >> k) & 1u) << 10) | (ad & 0x3ffu);
+        return (((nt_bits >> k) & 1u) << 10) | (ad & 0x3ffu);
     }
-    __device__ uint8_t vbus_read(uint16_t ad) const {
-        if (ad < 0x2000) return cart.chr[ad];
-        if (ad < 0x3eff) return vram(nt_row(ad));
-        if (ad < 0x3fff) return pal(ad);
+    __device__ __forceinline__ uint32_t vbus_read(uint32_t ad) const {
+        if (ad < 0x2000) return chr[ad];
+        if (ad < 0x3eff) return m[ROW_VRAM + nt_row(ad)];
+        if (ad < 0x3fff) return m[ROW_PAL + (ad & 0x1f)];
         return 0;
     }
-    __device__ void vbus_write(uint16_t ad, uint8_t d) {
+    __device__ __forceinline__ void vbus_write(uint32_t ad, uint32_t d) {
         if (ad < 0x2000) return;
-        if (ad < 0x3eff) { set_vram(nt_row(ad), d); bg_key = -1; }
-        else if (ad < 0x3fff) { st(ROW_PAL + (ad == 0x3f10 ? 0 : (ad & 0x1f)), d); pal_dirty = true; }
+        if (ad < 0x3eff) m[ROW_VRAM + nt_row(ad)] = (uint8_t)d;
+        else if (ad < 0x3fff) { m[ROW_PAL + (ad == 0x3f10 ? 0 : (ad & 0x1f))] = (uint8_t)d; pal_dirty = 1; }
     }
-    __device__ __forceinline__ uint8_t nametable(uint16_t ad) const {
-        return vram((((cart.nt_bits >> ((ad >> 10) & 3u)) & 1u) << 10) | (ad & 0x3ffu));
+    __device__ __forceinline__ uint32_t nametable(uint32_t ad) const {
+        return m[ROW_VRAM + ((((nt_bits >> ((ad >> 10) & 3u)) & 1u) << 10) | (ad & 0x3ffu))];
     }
 
     // ------------------------------------------------------------ PPU timing (nes_core.hpp:289-308)
-    __device__ void nmi_threshold() {
-        int line = pstate == ST_PRE ? -1 : pstate == ST_POST ? 240 : scanline;
-        int32_t pos = (line + 1) * 341 + (pcyc - 1);
+    __device__ __forceinline__ void nmi_threshold() {
+        const int line = pstate == ST_PRE ? -1 : pstate == ST_POST ? 240 : scanline;
+        const int32_t pos = (line + 1) * 341 + (pcyc - 1);
         const int32_t vbl = 242 * 341;
-        int32_t d = pos <= vbl ? vbl - pos + 1 : (262 * 341 - pos) + vbl + 1;
+        const int32_t d = pos <= vbl ? vbl - pos + 1 : (262 * 341 - pos) + vbl + 1;
         nmi_thresh = ppu_calls + d - 8;
     }
-    __device__ void advance_to(int32_t target) {
-        if (target > ppu_calls) { ppu_run(target - ppu_calls); nmi_threshold(); }
-    }
 
-    __device__ void coarse_x_add(int n) {
-        int tot = (v & 0x1f) + n;
-        v = (uint16_t)((v & ~0x1f) | (tot & 31));
-        if ((tot >> 5) & 1) v ^= 0x400;
+    __device__ __forceinline__ static uint32_t coarse_x_added(uint32_t v, uint32_t n) {
+        const uint32_t tot = (v & 0x1f) + n;
+        return ((v & ~0x1fu) | (tot & 31)) ^ ((tot & 32) << 5);
     }
-    __device__ void fine_y_step() {
-        if ((v & 0x7000) != 0x7000) { v += 0x1000; return; }
-        v &= ~0x7000;
-        int yy = (v >> 5) & 31;
+    __device__ __forceinline__ void coarse_x_add(int n) { v = coarse_x_added(v, (uint32_t)n); }
+    __device__ __forceinline__ void fine_y_step() {
+        if ((v & 0x7000) != 0x7000) { v = (v + 0x1000) & 0xffffu; return; }
+        v &= ~0x7000u;
+        uint32_t yy = (v >> 5) & 31;
         if (yy == 29) { yy = 0; v ^= 0x800; }
         else if (yy == 31) yy = 0;
         else yy++;
-        v = (uint16_t)((v & ~0x3e0) | (yy << 5));
+        v = (v & ~0x3e0u) | (yy << 5);
     }
-    __device__ void copy_h() { v = (uint16_t)((v & ~0x41f) | (t & 0x41f)); }
-    __device__ void copy_v() { v = (uint16_t)((v & ~0x7be0) | (t & 0x7be0)); }
+    __device__ __forceinline__ void copy_h() { v = (v & ~0x41fu) | (t & 0x41f); }
+    __device__ __forceinline__ void copy_v() { v = (v & ~0x7be0u) | (t & 0x7be0); }
 
     // Per-line sprite list from oam_addr/4 (nes_core.hpp:336-349). The PPU only records the scanline
-    // of an evaluation; the list is computed from OAM when something needs it (rendering, a change
-    // of OAM / oam_addr / sprite size, or the end of the kernel). Until then its inputs are unchanged,
-    // so the late evaluation gives the same list.
-    __device__ void materialize_sprites() {
-        if (pend_line < 0) return;
-        // in-range sprites as a 64-bit mask (bit i: pend_line - y_i in [0, h)), from index oam_addr / 4 on;
-        // the list is its first (at most 8) set bits, entries past the count keep their old values
-        const uint32_t h = long_spr() ? 16u : 8u;
-        // The env's parts each test 64 / LANES_PER_ENV sprites (part q: sprites NS q .. NS q + NS - 1) into
-        // exchange word q of the env, then every part reads every word. The wave barrier is a convergence
-        // point: every lane active here has stored its word before any lane loads (a wave's LDS accesses
-        // complete in order). All parts must be here together, or a part would read a stale word: a part
-        // missing from the wave's active lanes sets ERR_TWIN.
-        constexpr int NS = 64 / LANES_PER_ENV;
-        const uint32_t in_wave = __lane_id() & (ENVS_PER_WAVE - 1);
-        if (((__ballot(1) >> in_wave) & PART_LANES) != PART_LANES) bad_ops |= ERR_TWIN;
-        auto in_range = [&](int i) { return ((uint32_t)(pend_line - (int)(oam_sprite(i) & 0xffu)) < h ? 1u : 0u); };
-        uint32_t mlo = 0, mhi = 0;
-        if constexpr (LANES_PER_ENV == 1) {
-#pragma unroll
-            for (int i = 0; i < 32; i++) { mlo |= in_range(i) << i; mhi |= in_range(32 + i) << i; }
+    // of an evaluation; the list is computed from OAM when something needs it (a change of OAM / oam_addr / sprite
+    // size, or the end of the kernel). Until then its inputs are unchanged, so the late evaluation gives the same
+    // list; a line drawn meanwhile evaluates its own (draw_lines).
+    // The sprites in range of an evaluation at scanline `line`, as a 64-bit mask (bit i: line - y_i in [0, h)), from
+    // index oam_addr / 4 on: the list is its first (at most 8) set bits. Lane i tests sprite i.
+    // `more`: lines before it, too.
+    __device__ __forceinline__ uint64_t in_range(int line, uint32_t more = 0) const {
+        const uint32_t h = (long_spr() ? 16u : 8u) + more;
+        uint64_t b = 0;
+        if constexpr (ON_GPU) {
+            b = __ballot((uint32_t)(line - (int)(oam_word(lane) & 0xffu)) < h);
         } else {
-            uint32_t piece = 0;
-#pragma unroll
-            for (int i = 0; i < NS; i++) piece |= in_range(NS * part + i) << i;
-            uint32_t* const xw = lds_oam + LDS_OAM_WORDS * LDS_LANES;
-            xw[part * LDS_LANES] = piece;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if (LANES_PER_ENV == 2) {
-                mlo = xw[0]; mhi = xw[LDS_LANES];
-            } else {
-                mlo = xw[0] | xw[LDS_LANES] << 16; mhi = xw[2 * LDS_LANES] | xw[3 * LDS_LANES] << 16;
-            }
+            for (uint32_t i = 0; i < 64; i++) b |= (uint64_t)((uint32_t)(line - (int)(oam_word(i) & 0xffu)) < h) << i;
         }
-        const int i0 = oam_addr >> 2;
-        if (i0 < 32) mlo &= ~0u << i0;
-        else { mlo = 0; mhi &= ~0u << (i0 - 32); }
+        return b & (~0ull << (oam_addr >> 2));
+    }
+    __device__ __forceinline__ void materialize_sprites() {
+        if (pend_line < 0) return;
+        uint64_t b = in_range(pend_line);   // entries past the count keep their old values
         int n = 0;
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const bool has = (mlo | mhi) != 0;
-            const uint32_t i = mlo ? (uint32_t)__builtin_ctz(mlo) : 32u + (uint32_t)__builtin_ctz(mhi | 0x80000000u);
-            if (has) set_sl(k, (uint8_t)i);
-            n += has;
-            if (mlo) mlo &= mlo - 1; else mhi &= mhi - 1;
+        while (b && n < 8) {
+            set_sl(n++, (uint32_t)__builtin_ctzll(b));
+            b &= b - 1;
         }
-        nsl = (uint8_t)n;
+        nsl = (uint32_t)n;
         pend_line = -1;
     }
     // "nsl > 0 && sl[0] == 0" without materializing: sprite 0 heads the list exactly when the
@@ -887,351 +573,318 @@ struct Console {
     __device__ __forceinline__ bool sprite0_first() const {
         if (pend_line < 0) return nsl > 0 && sl(0) == 0;
         if (oam_addr >= 4) return false;
-        int d = pend_line - (int)(oam_sprite(0) & 0xffu);
+        const int d = pend_line - (int)(oam_sprite(0) & 0xffu);
         return d >= 0 && d < (long_spr() ? 16 : 8);
     }
-    __device__ uint8_t bg_colour(int px, uint8_t* pattern) const {
-        int xf = (fine_x + px) % 8;
-        uint8_t tile = nametable((uint16_t)(0x2000 | (v & 0x0fff)));
-        uint16_t pa = (uint16_t)(((tile * 16) + ((v >> 12) & 7)) | (bg_page() << 12));
-        uint8_t c = (uint8_t)(((cart.chr[pa] >> (7 ^ xf)) & 1) | (((cart.chr[pa + 8] >> (7 ^ xf)) & 1) << 1));
-        *pattern = c;
-        uint16_t aa = (uint16_t)(0x23c0 | (v & 0x0c00) | ((v >> 4) & 0x38) | ((v >> 2) & 7));
-        int sh = ((v >> 4) & 4) | (v & 2);
-        return (uint8_t)(c | (((nametable(aa) >> sh) & 3) << 2));
+    // the background pattern at pixel px, with v at its tile (a lane's own px and v)
+    __device__ __forceinline__ uint32_t bg_pattern(int px, uint32_t v) const {
+        const uint32_t xf = (fine_x + (uint32_t)px) & 7u;
+        const uint32_t pa = ((nametable(0x2000 | (v & 0x0fff)) * 16) + ((v >> 12) & 7)) | (bg_page() << 12);
+        return ((chr[pa] >> (7 ^ xf)) & 1u) | (((chr[pa + 8] >> (7 ^ xf)) & 1u) << 1);
     }
-    // sprite i's 2-bit pattern at (px, py), with C++ int semantics for stale lists (nes_core.hpp:369-391)
-    __device__ uint8_t sprite_pattern(int i, int px, int py) const {
-        const uint32_t ow = oam_sprite(i);
-        uint8_t sx = (uint8_t)(ow >> 24);
-        uint8_t sy = (uint8_t)((ow & 0xffu) + 1), tile = (uint8_t)(ow >> 8), attr = (uint8_t)(ow >> 16);
-        int h = long_spr() ? 16 : 8;
-        int xs = (px - sx) % 8, yo = (py - sy) % h;
-        if (!(attr & 0x40)) xs ^= 7;
-        if (attr & 0x80) yo ^= (h - 1);
-        uint16_t ad;
-        if (!long_spr()) {
-            ad = (uint16_t)(tile * 16 + yo);
-            if (spr_page()) ad += 0x1000;
-        } else {
-            yo = (yo & 7) | ((yo & 8) << 1);
-            ad = (uint16_t)((tile >> 1) * 32 + yo);
-            ad |= (tile & 1) << 12;
-        }
-        return (uint8_t)(((vbus_read(ad) >> xs) & 1) | (((vbus_read((uint16_t)(ad + 8)) >> xs) & 1) << 1));
+    // the picture-bus address of row py of the sprite with OAM word ow, with C++ int semantics for stale lists
+    // (nes_core.hpp:369-391)
+    __device__ __forceinline__ uint32_t sprite_row(uint32_t ow, int py) const {
+        const int sy = (int)((ow + 1u) & 0xffu), h = long_spr() ? 16 : 8;
+        const uint32_t tile = (ow >> 8) & 0xffu;
+        int yo = (py - sy) % h;
+        if (ow & 0x800000u) yo ^= (h - 1);
+        if (!long_spr()) return (uint32_t)((int)tile * 16 + yo + (spr_page() ? 0x1000 : 0)) & 0xffffu;
+        yo = (yo & 7) | ((yo & 8) << 1);
+        return ((uint32_t)((int)(tile >> 1) * 32 + yo) & 0xffffu) | ((tile & 1) << 12);
+    }
+    // sprite 0's 2-bit pattern at (px, py)
+    __device__ __forceinline__ uint32_t sprite0_pattern(uint32_t ow, int px, int py) const {
+        int xs = (px - (int)(ow >> 24)) % 8;
+        if (!(ow & 0x400000u)) xs ^= 7;
+        const uint32_t ad = sprite_row(ow, py);
+        return ((vbus_read(ad) >> xs) & 1u) | (((vbus_read((ad + 8) & 0xffffu) >> xs) & 1u) << 1);
     }
 
-    // Visible dots [x0, x1): sprite-0 hit and the coarse-x increments of v (nes_core.hpp:394-413).
-    // Rendered and unrendered frames both take the hit from here; dots_drawn only adds pixels.
+    // Visible dots [x0, x1): sprite-0 hit and the coarse-x increments of v (nes_core.hpp:394-413). The lanes test the
+    // (at most 8) pixels under sprite 0 at once.
     __device__ __forceinline__ void dots_hit_scroll(int x0, int x1) {
         if (!show_bg()) return;
         if (!s0hit && show_spr() && sprite0_first()) {
-            int sx = (int)(oam_sprite(0) >> 24);
+            const uint32_t ow = oam_sprite(0);
+            const int sx = (int)(ow >> 24);
             int lo = x0 > sx ? x0 : sx;
-            int hi = x1 < sx + 8 ? x1 : sx + 8;
+            const int hi = x1 < sx + 8 ? x1 : sx + 8;
             if (hide_edge_spr() && lo < 8) lo = 8;
-            if (lo < hi) {
-                coarse_x_add(inc_count(x0, lo));
-                for (int px = lo; px < hi; px++) {
-                    if (!s0hit && (!hide_edge_bg() || px >= 8)) {
-                        uint8_t pat;
-                        bg_colour(px, &pat);
-                        if (pat && sprite_pattern(0, px, scanline)) s0hit = 1;
-                    }
-                    if ((fine_x + px) % 8 == 7) coarse_x_add(1);
-                }
-                coarse_x_add(inc_count(hi, x1));
-                return;
+            if (hide_edge_bg() && lo < 8) lo = 8;
+            bool hit = false;
+            for (int px = lo + (int)lane; px < hi; px += LANES) {
+                const uint32_t vp = coarse_x_added(v, (uint32_t)inc_count(x0, px));
+                hit |= bg_pattern(px, vp) && sprite0_pattern(ow, px, scanline);
             }
+            if (__any(hit)) s0hit = 1;
         }
         coarse_x_add(inc_count(x0, x1));
     }
     __device__ __forceinline__ int inc_count(int lo, int hi) const {   // x in [lo, hi) with (fine_x + x) % 8 == 7
-        int r = (7 - fine_x) & 7;
+        const int r = (7 - (int)fine_x) & 7;
         return (hi - r + 7) / 8 - (lo - r + 7) / 8;
     }
 
-    // an optimization barrier: the value is materialized in a register here
-    __device__ __forceinline__ static void in_register(uint32_t& x) { MH_REG_BARRIER(x); }
     // bytes of the 8-byte value hi:lo picked by the selector bytes of sel (each 0..7)
     __device__ __forceinline__ static uint32_t byte_perm(uint32_t hi, uint32_t lo, uint32_t sel) {
         return __builtin_amdgcn_perm(hi, lo, sel);
     }
 
-    // ---- per-lane LDS buffers of the renderer
-    __device__ __forceinline__ uint8_t lds_byte(const uint32_t* base, int i) const {
-        return (uint8_t)(base[(i >> 2) * LDS_LANES] >> (8 * (i & 3)));
-    }
+    // ---- the renderer
     // gray value of every palette address, lut[pal[i]]; rebuilt after palette writes
-    __device__ void build_gray_palette() {
-        for (int w = 0; w < LDS_GP_WORDS; w++) {
-            uint32_t word = 0;
-            for (int b = 0; b < 4; b++) word |= (uint32_t)lut[pal(4 * w + b)] << (8 * b);
-            lds_gp[w * LDS_LANES] = word;
-        }
-        pal_dirty = false;
+    __device__ __forceinline__ void build_gray_palette() {
+        for (uint32_t i = lane; i < 32; i += LANES) ((MH_LDS uint8_t*)(gp + GP_PALETTE))[i] = lut[m[ROW_PAL + i]];
+        lds_sync();
+        pal_dirty = 0;
     }
-    // First opaque listed sprite per x of line py (nes_core.hpp:427-441), one byte per x: bits 0-3 the
-    // sprite palette entry (attr << 2 | pattern, palette address 0x10 + it), bit 6 in front of the
-    // background, bit 7 set (a sprite pixel is here; 0: none). The pattern row of each listed sprite is
-    // fetched once, with the addressing of sprite_pattern().
-    __device__ void build_sprite_line(int py) {
-        for (int w = 0; w < LDS_SP_WORDS; w++) lds_sp[w * LDS_LANES] = 0;
-        const int h = long_spr() ? 16 : 8;
-        for (int k = 0; k < nsl; k++) {
-            const int i = sl(k);
-            const uint32_t ow = oam_sprite(i);
-            const uint8_t sx = (uint8_t)(ow >> 24), sy = (uint8_t)((ow & 0xffu) + 1), tile = (uint8_t)(ow >> 8),
-                          attr = (uint8_t)(ow >> 16);
-            int yo = (py - sy) % h;
-            if (attr & 0x80) yo ^= (h - 1);
-            uint16_t ad;
-            if (!long_spr()) {
-                ad = (uint16_t)(tile * 16 + yo);
-                if (spr_page()) ad += 0x1000;
-            } else {
-                yo = (yo & 7) | ((yo & 8) << 1);
-                ad = (uint16_t)((tile >> 1) * 32 + yo);
-                ad |= (tile & 1) << 12;
-            }
-            const uint8_t lo = vbus_read(ad), hi = vbus_read((uint16_t)(ad + 8));
-            const uint32_t tag = 0x80u | ((attr & 3u) << 2) | (attr & 0x20 ? 0u : 0x40u);
-            // The sprite's 8 pixels as 8 bytes (pixel sx + j in byte j: pattern | tag, or 0 where transparent),
-            // merged into the (at most 3) line words they cover: a byte takes the sprite only where no
-            // earlier listed sprite is opaque (a written byte always has bit 7 set). Pixels past x = 255 fall
-            // in words past the line and are dropped.
-            const uint32_t rlo = (attr & 0x40) ? (uint32_t)lo : __builtin_bitreverse32((uint32_t)lo) >> 24;
-            const uint32_t rhi = (attr & 0x40) ? (uint32_t)hi : __builtin_bitreverse32((uint32_t)hi) >> 24;
-            uint32_t cw[2];
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                const uint32_t pat = (__umul24((rlo >> (4 * q)) & 0xfu, 0x204081u) & 0x01010101u) |
-                                     ((__umul24((rhi >> (4 * q)) & 0xfu, 0x204081u) & 0x01010101u) << 1);
-                const uint32_t nz = (pat + 0x7f7f7f7fu) & 0x80808080u;
-                cw[q] = (pat | tag * 0x01010101u) & (nz | (nz - (nz >> 7)));
-            }
-            const uint64_t span = ((uint64_t)cw[1] << 32 | cw[0]) ;
-            const int w0 = sx >> 2, sh = 8 * (sx & 3);
-            const uint64_t lo64 = span << sh;
-            const uint32_t cv[3] = {(uint32_t)lo64, (uint32_t)(lo64 >> 32), sh ? (uint32_t)(span >> (64 - sh)) : 0u};
-#pragma unroll
-            for (int i = 0; i < 3; i++) {
-                if (w0 + i < LDS_SP_WORDS) {
-                    uint32_t* wp = &lds_sp[(w0 + i) * LDS_LANES];
-                    const uint32_t old = *wp, occ = old & 0x80808080u;
-                    *wp = old | (cv[i] & ~(occ | (occ - (occ >> 7))));
-                }
-            }
+    // v at the start of the i-th line after this one (i > 0), both layers on: fine_y_step i times, and copy_h. (Coarse y
+    // 30 and 31 wrap to 0 without the mirror switch that 29 makes.)
+    __device__ __forceinline__ uint32_t v_lines_on(uint32_t i) const {
+        uint32_t yy = ((v >> 5) & 31u) * 8u + ((v >> 12) & 7u), mirror = 0;   // i <= 240
+        if (yy >= 240u) yy = (yy + i) & 255u;
+        else {
+            yy += i;
+            if (yy >= 240u) { yy -= 240u; mirror = 0x800u; }
         }
-        sp_line = py;
+        return (v & 0x8000u) | ((v ^ mirror) & 0x800u) | (t & 0x41fu) | (yy >> 3) << 5 | (yy & 7u) << 12;
+    }
+    // A sprite's row on line py as one word: x | the row's two planes, bit j pixel x + j, << 8 and << 16 | palette
+    // (bits 24-25), behind the background (bit 29), bit 31 set.
+    __device__ __forceinline__ uint32_t sprite_entry(uint32_t ow, int py) const {
+        const uint32_t ad = sprite_row(ow, py);
+        uint32_t lo = vbus_read(ad), hi = vbus_read((ad + 8) & 0xffffu);
+        if (!(ow & 0x400000u)) {
+            lo = __builtin_bitreverse32(lo) >> 24;
+            hi = __builtin_bitreverse32(hi) >> 24;
+        }
+        return (ow >> 24) | lo << 8 | hi << 16 | ((ow >> 16) & 0x23u) << 24 | 0x80000000u;
     }
 
-    // Background tiles of a line into the per-lane LDS cache: the 32-tile name-table row at coarse y of
-    // v0's name table A (words 0-7) and of its horizontal neighbour B (words 8-15, where coarse x wraps
-    // to; nes_core.hpp:394-413), and the two attribute rows (words 16-19: bytes 0-7 A, 8-15 B). The row
-    // depends on v0's bits 5-11 only: lines of one coarse y share it whatever their scroll. 20 word
-    // loads, independent of each other.
-    __device__ __forceinline__ void fill_bg_row(uint16_t v0) {
-        const uint32_t na = (v0 >> 10) & 3u, cy = (v0 >> 5) & 31u;
-        const uint32_t pa = ((cart.nt_bits >> na) & 1u) << 8, pb = ((cart.nt_bits >> (na ^ 1u)) & 1u) << 8;  // words
-        uint32_t w[LDS_BG_WORDS];
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            w[i] = vram_word(pa + cy * 8 + i);
-            w[8 + i] = vram_word(pb + cy * 8 + i);
-        }
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            w[16 + i] = vram_word(pa + 0xf0 + (cy >> 2) * 2 + i);
-            w[18 + i] = vram_word(pb + 0xf0 + (cy >> 2) * 2 + i);
-        }
-#pragma unroll
-        for (int i = 0; i < LDS_BG_WORDS; i++) lds_bg[i * LDS_LANES] = w[i];
-    }
-    // Tile k (0..32) of the line whose row is cached (c0: the line's starting coarse x, cy: its coarse
-    // y): index | attribute byte << 8 | the attribute's shift in it << 16, unpacked by bg_planes (the
-    // loads are not waited for here). Column c0 + k is in name table A below 32, else in B.
-    __device__ __forceinline__ uint32_t bg_tile_of(int k, uint32_t c0, uint32_t cy) const {
-        const uint8_t* row = (const uint8_t*)lds_bg;
-        const uint32_t col = c0 + (uint32_t)k;                                   // 0 .. 63
-        const uint32_t tile = row[(col >> 2) * LDS_LANES * 4 + (col & 3)];
-        const uint32_t ab = LDS_BG_ATTR + (col >> 5) * 8 + ((col & 31) >> 2);   // attribute byte
-        const uint32_t at = row[(ab >> 2) * LDS_LANES * 4 + (ab & 3)];
-        const uint32_t sh = ((cy & 2u) << 1) | (col & 2u);
-        return tile | at << 8 | sh << 16;
-    }
-    // Pattern planes of row fy of tile ta (bg_tile_of) and its gray table: byte p is the gray value of
-    // background pattern p (p = 0: the universal background, palette address 0; else palette address
-    // 4 at + p). pal[w]: gray values of palette addresses 4w .. 4w+3.
-    __device__ __forceinline__ void bg_planes(uint32_t ta, int fy, const uint32_t (&pal)[4], uint32_t& lo, uint32_t& hi,
-                                              uint32_t& gt) const {
-        const uint16_t pa = (uint16_t)((((ta & 0xffu) * 16) + fy) | (bg_page() << 12));
-        lo = cart.chr[pa];
-        hi = cart.chr[pa + 8];
-        const uint32_t at = (ta >> (8 + (ta >> 16))) & 3u;
-        const uint32_t w01 = (at & 1u) ? pal[1] : pal[0], w23 = (at & 1u) ? pal[3] : pal[2];
-        gt = (((at & 2u) ? w23 : w01) & 0xffffff00u) | (pal[0] & 0xffu);
-    }
-
-    // Pixels of visible dots [x0, x1): gray values into the frame buffer (nes_core.hpp:467-513), with
-    // v as it is at x0 (dots_hit_scroll advances it afterwards). Pixels go in screen-aligned groups
-    // of 8, so every lane of a wave runs the same code whatever its fine scroll: a group spans two
-    // background tiles, kept as a 16-bit window per pattern plane (a PPU's shift registers), and the
-    // tile after them is fetched one group ahead from the LDS tile row. Sprites come from the LDS line
-    // buffer, where the first opaque listed sprite of each x sits.
+    // Pixels [x0, x1) of `count` lines from this one on: gray values into the frame buffer (nes_core.hpp:427-513), with v
+    // as it is at x0 of this line, and at the later lines' starts as the scroll leaves it (v_lines_on; with the
+    // background off v stays and does not matter). Whole lines (x0 = 0, x1 = 256) go four at a time, 16 lanes a line
+    // and 16 pixels (two screen-aligned groups of 8, from three background tiles) a lane; a line that a catch-up cuts
+    // goes alone.
+    //
+    // First the lines' sprites: lane i tests sprite i against each line (in_range's ballot); a sprite in range is the
+    // line's entry number "sprites before it in the ballot" if that is below 8, and the lanes that hold one fetch
+    // its pattern row at once and leave it as a word in LDS. Each lane then merges the line's entries that reach
+    // its pixels, in list order: a byte takes the sprite only where no earlier one is opaque. Line i > 0 takes its
+    // sprites from the evaluation at the line before it, this line from the pending one or the list.
     //
     // Four pixels are one 32-bit word, a byte each, and are computed together without branches: the
     // pattern bits of the four pixels are spread to the four bytes by a multiply, the background gray
     // value is a byte permute of the two tiles' gray tables, a sprite pixel's gray value is a byte
     // permute of the sprite palette's 16 gray values, and priority is a per-byte mask.
-    __device__ __forceinline__ void dots_drawn(int x0, int x1) {
-        const int py = scanline;
-        materialize_sprites();
+    __device__ __forceinline__ void draw_lines(uint32_t count, int x0, int x1) {
         if (pal_dirty) build_gray_palette();
-        const bool spr = show_spr() && nsl;
-        if (spr && sp_line != py) build_sprite_line(py);
-        const int f = fine_x, fy = (v >> 12) & 7;
-        const int g0 = x0 >> 3, g1 = (x1 + 7) >> 3;
-        uint32_t bc0 = 0, bcy = 0;             // line-start coarse x and coarse y
-        if (show_bg()) {
-            // line-start address: v addresses the tile of pixel x0, (f + x0) / 8 tiles into the line
-            const int kb = (f + x0) >> 3;
-            int c0 = (v & 0x1f) - kb;
-            uint16_t v0 = v;
-            if (c0 < 0) { c0 += 32; v0 ^= 0x400; }
-            v0 = (uint16_t)((v0 & ~0x1f) | c0);
-            if ((int32_t)((v0 >> 5) & 0x7f) != bg_key) { fill_bg_row(v0); bg_key = (v0 >> 5) & 0x7f; }
-            bc0 = v0 & 31u; bcy = (v0 >> 5) & 31u;
+        MH_LDS uint32_t* const ent = gp + GP_SPRITES;
+        // any sprite on any of the lines?
+        bool some = false;
+        if (show_spr()) {
+            if (pend_line >= 0 && count > 1) some = in_range(scanline + (int)count - 2, count) != 0;
+            else some = true;
         }
-        // gray values of the background palettes (addresses 0..15) and the sprite palettes (0x10 + 0..15)
-        uint32_t bp0 = lds_gp[0], bp1 = lds_gp[LDS_LANES], bp2 = lds_gp[2 * LDS_LANES], bp3 = lds_gp[3 * LDS_LANES];
-        // keep them in registers: a select of these loads must not become a load from a selected address
-        in_register(bp0); in_register(bp1); in_register(bp2); in_register(bp3);
-        uint32_t sp0 = 0, sp1 = 0, sp2 = 0, sp3 = 0;
-        if (spr) {
-            sp0 = lds_gp[4 * LDS_LANES]; sp1 = lds_gp[5 * LDS_LANES];
-            sp2 = lds_gp[6 * LDS_LANES]; sp3 = lds_gp[7 * LDS_LANES];
+        for (uint32_t base = 0; base < count; base += DRAW_LINES) draw_batch(base, count, x0, x1, some, ent);
+    }
+    __device__ __forceinline__ void draw_batch(uint32_t base, uint32_t count, int x0, int x1, bool some, MH_LDS uint32_t* ent) {
+        const uint32_t cnt = count - base < (uint32_t)DRAW_LINES ? count - base : (uint32_t)DRAW_LINES;
+        uint32_t most = 0;                      // sprites of the line that has most
+        if (some) {
+            for (uint32_t i = lane; i < 8 * DRAW_LINES; i += LANES) ent[i] = 0;
+            lds_sync();
+            for (uint32_t li = 0; li < cnt; li++) {
+                const int py = scanline + (int)(base + li);
+                uint64_t b = 0;
+                if (base + li > 0) b = in_range(py - 1);
+                else if (pend_line >= 0) b = in_range(pend_line);
+                else for (uint32_t k = 0; k < nsl; k++) b |= 1ull << sl((int)k);
+                if (!b) continue;
+#if defined(__AMDGCN__)
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0));
+                if (((b >> lane) & 1u) && rank < 8u) ent[8 * li + rank] = sprite_entry(oam_word(lane), py);
+#else
+                for (uint32_t i = 0, rank = 0; i < 64 && rank < 8; i++)
+                    if ((b >> i) & 1u) ent[8 * li + rank++] = sprite_entry(oam_word(i), py);
+#endif
+                const uint32_t n = (uint32_t)__popcll(b) < 8u ? (uint32_t)__popcll(b) : 8u;
+                most = n > most ? n : most;
+            }
+            lds_sync();
         }
-        const bool any_spr = __any(spr);
-        const uint32_t bgpal[4] = {bp0, bp1, bp2, bp3};
-        // pixel bb of a group takes the second tile's attribute when f + bb >= 8: bytes bb >= 8 - f
+        const MH_LDS uint32_t* const pal = gp + GP_PALETTE;
+        const uint32_t f = fine_x;
+        // pixel bb of a group takes the second tile's gray table when f + bb >= 8: bytes bb >= 8 - f
         const uint64_t second = f ? (~0ull << (8 * (8 - f))) : 0ull;
         const uint32_t tsel0 = (uint32_t)second & 0x04040404u, tsel1 = (uint32_t)(second >> 32) & 0x04040404u;
-        // The env's parts split the groups in pairs: part q draws groups S m + 2 q and S m + 2 q + 1, S = 2 x
-        // LANES_PER_ENV (a fixed owner per group, so a group cut by a catch-up boundary is finished by the
-        // lane that started it). One iteration draws one pair (p, p + 1) from tiles p, p + 1 and p + 2, and
-        // fetches the planes of the next pair's three tiles, the indices of the pair after it and the next
-        // pair's sprite bytes, which are used one iteration later, so no LDS round trip sits between two
-        // pairs. The fetches are unconditional (indices clamped to the buffers; a layer that is off masks
-        // its values afterwards), so every iteration issues the same LDS operations. A group of a pair that
-        // lies outside [x0, x1) gets an empty pixel mask and is not written.
-        constexpr int S = 2 * LANES_PER_ENV;   // groups between two pairs of one part
-        auto tile_of = [&](int k) { return bg_tile_of(k < 32 ? k : 32, bc0, bcy); };
-        int pg = (g0 & ~(S - 1)) + 2 * (int)part;
-        if (pg + 1 < g0) pg += S;
-        uint32_t alo, ahi, agt, blo, bhi, bgt, clo, chi, cgt;
-        bg_planes(tile_of(pg), fy, bgpal, alo, ahi, agt);
-        bg_planes(tile_of(pg + 1), fy, bgpal, blo, bhi, bgt);
-        bg_planes(tile_of(pg + 2), fy, bgpal, clo, chi, cgt);
-        uint32_t nxa = tile_of(pg + S), nxb = tile_of(pg + S + 1), nxc = tile_of(pg + S + 2);
-        const int ws0 = 2 * pg < 60 ? 2 * pg : 60;
-        uint32_t s0 = lds_sp[ws0 * LDS_LANES], s1 = lds_sp[(ws0 + 1) * LDS_LANES];   // the pair's sprite bytes
-        uint32_t s2 = lds_sp[(ws0 + 2) * LDS_LANES], s3 = lds_sp[(ws0 + 3) * LDS_LANES];
-        // A layer that is off is masked out of every pixel rather than zeroed at its fetch: with the background
-        // pattern masked to 0 a pixel takes byte 0 of its tile's gray table, the universal background, as it
-        // does with the background off; with the sprite bytes masked no sprite pixel is taken.
-        const uint32_t keep_bg = show_bg() ? ~0u : 0u, keep_sp = spr ? ~0u : 0u;
-        uint32_t* wp = (uint32_t*)gray + ((size_t)py * 64 + 2 * pg) * np;   // word of pixels 8pg .. 8pg+3
-        // the two words of the group drawn from tiles (lo0, hi0, gt0) and (lo1, hi1, gt1) with sprite bytes ca, cb
-        auto group_words = [&](uint32_t lo0, uint32_t hi0, uint32_t gt0, uint32_t lo1, uint32_t hi1, uint32_t gt1,
-                               uint32_t ca, uint32_t cb, uint32_t keep_bg, uint32_t keep_sp, uint32_t (&out)[2]) {
-            // pixel 8g + bb is bit 15 - bb of the window after the fine-scroll shift; reversed: bit 16 + bb
-            const uint32_t rlo = __builtin_bitreverse32(((lo0 << 8) | lo1) << f);
-            const uint32_t rhi = __builtin_bitreverse32(((hi0 << 8) | hi1) << f);
+        const uint32_t bg_on = show_bg() ? ~0u : 0u, gs = gray_step();
+        for (uint32_t unit = lane; unit < 16 * cnt; unit += LANES) {
+            const uint32_t li = unit >> 4, q = unit & 15u, i = base + li, py = (uint32_t)scanline + i;
+            const uint32_t vl = i && show_bg() ? v_lines_on(i) : v, fy = (vl >> 12) & 7u, cy = (vl >> 5) & 31u;
+            // the line's first tile: v addresses the tile of pixel x0, (f + x0) / 8 tiles into the line
+            int c0 = (int)(vl & 31u) - (int)((f + (uint32_t)x0) >> 3);
+            uint32_t nt = (vl >> 10) & 3u;
+            if (c0 < 0) { c0 += 32; nt ^= 1u; }
+            const uint32_t bp0 = pal[0], bp1 = pal[1], bp2 = pal[2], bp3 = pal[3];
+            uint32_t lo[3], hi[3], gt[3];       // the three tiles' pattern rows and gray tables
 #pragma unroll
-            for (int q = 0; q < 2; q++) {
-                // background pattern of the four pixels, one per byte (0..3)
-                const uint32_t nlo = (rlo >> (16 + 4 * q)) & 0xfu, nhi = (rhi >> (16 + 4 * q)) & 0xfu;
-                const uint32_t bgp = (((__umul24(nlo, 0x204081u) & 0x01010101u) |
-                                       ((__umul24(nhi, 0x204081u) & 0x01010101u) << 1))) & keep_bg;
-                uint32_t word = byte_perm(gt1, gt0, bgp | (q ? tsel1 : tsel0));
-                if (any_spr) {
-                    const uint32_t c = q ? cb : ca;
-                    const uint32_t opaque = (bgp + 0x7f7f7f7fu) & 0x80808080u;       // background pattern != 0
-                    const uint32_t take = c & (~opaque | (c << 1)) & 0x80808080u & keep_sp;
-                    const uint32_t tmask = take | (take - (take >> 7));
-                    const uint32_t sel = c & 0x07070707u;
-                    const uint32_t hi8 = (c << 4) & 0x80808080u;                    // entry 8..15
-                    const uint32_t hmask = hi8 | (hi8 - (hi8 >> 7));
-                    const uint32_t sg = (byte_perm(sp3, sp2, sel) & hmask) | (byte_perm(sp1, sp0, sel) & ~hmask);
-                    word = (sg & tmask) | (word & ~tmask);
-                }
-                out[q] = word;
+            for (int k = 0; k < 3; k++) {
+                const uint32_t col = (uint32_t)c0 + 2 * q + (uint32_t)k, n2 = nt ^ ((col >> 5) & 1u), cx = col & 31u;
+                const MH_LDS uint8_t* const row = m + ROW_VRAM + (((nt_bits >> n2) & 1u) << 10);
+                const uint32_t tile = row[cy * 32 + cx], at8 = row[0x3c0 + (cy >> 2) * 8 + (cx >> 2)];
+                const uint32_t at = (at8 >> (((cy & 2u) << 1) | (cx & 2u))) & 3u;
+                const uint32_t pa = (tile * 16 + fy) | (bg_page() << 12);
+                lo[k] = chr[pa] & bg_on;   // the background off: pattern 0, the universal background
+                hi[k] = chr[pa + 8] & bg_on;
+                // byte p: the gray value of background pattern p (0: palette address 0; else palette address 4 at + p)
+                const uint32_t w01 = (at & 1u) ? bp1 : bp0, w23 = (at & 1u) ? bp3 : bp2;
+                gt[k] = (((at & 2u) ? w23 : w01) & 0xffffff00u) | (bp0 & 0xffu);
             }
-        };
-        // the group's two words at w (pixels xg .. xg + 7): streaming stores when all 8 pixels are in [x0, x1)
-        // (the frame buffers are read by the next kernel only, so they should not evict the console state from
-        // the L2), else a read-modify-write of the pixels in [x0, x1)
-        auto store_group = [&](int xg, uint32_t* w, const uint32_t (&out)[2]) {
-            if (xg >= x0 && xg + 8 <= x1) { __builtin_nontemporal_store(out[0], w); __builtin_nontemporal_store(out[1], w + np); }
-            else {
+            // the line's sprites over these 16 pixels: a byte a pixel, the sprite palette entry (bits 0-3), in front
+            // of the background (bit 6), bit 7 set (0: none)
+            uint32_t sb[4] = {0, 0, 0, 0};
+            for (uint32_t k = 0; k < most; k++) {
+                const uint32_t en = ent[8 * li + k];
+                const int off = (int)(en & 0xffu) - (int)(16 * q);
+                if (!en || off <= -8 || off >= 16) continue;
+                const uint32_t tag = 0x80u | ((en >> 22) & 0xcu) | ((en & 0x20000000u) ? 0u : 0x40u);
+                uint32_t cw[2];
 #pragma unroll
-                for (int q = 0; q < 2; q++) {
-                    const int xq = xg + 4 * q;
-                    const int lo = x0 > xq ? x0 - xq : 0, hi = x1 < xq + 4 ? x1 - xq : 4;
-                    if (lo < hi) {
-                        const uint32_t in = (uint32_t)((((1ull << (8 * hi)) - 1) >> (8 * lo)) << (8 * lo));
-                        uint32_t* wq = w + q * np;
-                        *wq = (*wq & ~in) | (out[q] & in);
+                for (int h = 0; h < 2; h++) {
+                    const uint32_t pat = (__umul24((en >> (8 + 4 * h)) & 0xfu, 0x204081u) & 0x01010101u) |
+                                         ((__umul24((en >> (16 + 4 * h)) & 0xfu, 0x204081u) & 0x01010101u) << 1);
+                    const uint32_t nz = (pat + 0x7f7f7f7fu) & 0x80808080u;
+                    cw[h] = (pat | tag * 0x01010101u) & (nz | (nz - (nz >> 7)));
+                }
+                const uint64_t span = (uint64_t)cw[1] << 32 | cw[0];
+                const uint32_t so = 8u * (uint32_t)(off < 0 ? -off : off & 7);
+                const uint64_t s0 = off < 0 ? span >> so : span << so;                    // at byte 0 (or 8)
+                const uint64_t s1 = off > 0 && (off & 7) ? span >> (64u - so) : 0ull;     // what it pushes out
+                const uint64_t w0 = off < 8 ? s0 : 0ull, w1 = off < 8 ? (off < 0 ? 0ull : s1) : s0;
+                const uint32_t c[4] = {(uint32_t)w0, (uint32_t)(w0 >> 32), (uint32_t)w1, (uint32_t)(w1 >> 32)};
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    const uint32_t occ = sb[b] & 0x80808080u;
+                    sb[b] |= c[b] & ~(occ | (occ - (occ >> 7)));
+                }
+            }
+            uint32_t out[4];
+#pragma unroll
+            for (int g = 0; g < 2; g++) {
+                // pixel 8g + bb is bit 15 - bb of the window after the fine-scroll shift; reversed: bit 16 + bb
+                const uint32_t rlo = __builtin_bitreverse32(((lo[g] << 8) | lo[g + 1]) << f);
+                const uint32_t rhi = __builtin_bitreverse32(((hi[g] << 8) | hi[g + 1]) << f);
+                const bool edge = q == 0 && g == 0;   // pixels 0-7 may hide either layer
+                const uint32_t keep_bg = edge && hide_edge_bg() ? 0u : ~0u, keep_sp = edge && hide_edge_spr() ? 0u : ~0u;
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    // background pattern of the four pixels, one per byte (0..3)
+                    const uint32_t nlo = (rlo >> (16 + 4 * h)) & 0xfu, nhi = (rhi >> (16 + 4 * h)) & 0xfu;
+                    const uint32_t bgp = (((__umul24(nlo, 0x204081u) & 0x01010101u) |
+                                           ((__umul24(nhi, 0x204081u) & 0x01010101u) << 1))) & keep_bg;
+                    uint32_t word = byte_perm(gt[g + 1], gt[g], bgp | (h ? tsel1 : tsel0));
+                    if (most) {
+                        const uint32_t c = sb[2 * g + h];
+                        const uint32_t opaque = (bgp + 0x7f7f7f7fu) & 0x80808080u;       // background pattern != 0
+                        const uint32_t take = c & (~opaque | (c << 1)) & 0x80808080u & keep_sp;
+                        const uint32_t tmask = take | (take - (take >> 7));
+                        const uint32_t sel = c & 0x07070707u;
+                        const uint32_t hi8 = (c << 4) & 0x80808080u;                    // entry 8..15
+                        const uint32_t hmask = hi8 | (hi8 - (hi8 >> 7));
+                        const uint32_t sg = (byte_perm(pal[7], pal[6], sel) & hmask) | (byte_perm(pal[5], pal[4], sel) & ~hmask);
+                        word = (sg & tmask) | (word & ~tmask);
                     }
+                    out[2 * g + h] = word;
                 }
             }
-        };
-        for (; pg < g1; pg += S) {
-            uint32_t dlo, dhi, dgt, elo, ehi, egt, flo, fhi, fgt;
-            bg_planes(nxa, fy, bgpal, dlo, dhi, dgt);
-            bg_planes(nxb, fy, bgpal, elo, ehi, egt);
-            bg_planes(nxc, fy, bgpal, flo, fhi, fgt);
-            const uint32_t na = tile_of(pg + 2 * S), nb = tile_of(pg + 2 * S + 1), nc = tile_of(pg + 2 * S + 2);
-            const int ws = 2 * pg + 2 * S < 60 ? 2 * pg + 2 * S : 60;
-            const uint32_t t0 = lds_sp[ws * LDS_LANES], t1 = lds_sp[(ws + 1) * LDS_LANES];
-            const uint32_t t2 = lds_sp[(ws + 2) * LDS_LANES], t3 = lds_sp[(ws + 3) * LDS_LANES];
-            uint32_t out0[2], out1[2];
-            // pixels 0-7 may hide either layer
-            group_words(alo, ahi, agt, blo, bhi, bgt, s0, s1, (pg == 0 && hide_edge_bg()) ? 0u : keep_bg,
-                        (pg == 0 && hide_edge_spr()) ? 0u : keep_sp, out0);
-            group_words(blo, bhi, bgt, clo, chi, cgt, s2, s3, keep_bg, keep_sp, out1);
-            store_group(8 * pg, wp, out0);
-            store_group(8 * pg + 8, wp + 2 * np, out1);
-            wp += 2 * S * np;
-            alo = dlo; ahi = dhi; agt = dgt;
-            blo = elo; bhi = ehi; bgt = egt;
-            clo = flo; chi = fhi; cgt = fgt;
-            nxa = na; nxb = nb; nxc = nc;
-            s0 = t0; s1 = t1; s2 = t2; s3 = t3;
+            uint32_t* const w = (uint32_t*)gray + ((size_t)py * 64 + 4 * q) * gs;   // word of pixels 16q .. 16q+3
+            const int xg = 16 * (int)q;
+            if (xg >= x0 && xg + 16 <= x1) {
+                // streaming stores: the frames are read once, after the frame loop
+                if constexpr (ON_GPU) __builtin_nontemporal_store(mh_u32x4{out[0], out[1], out[2], out[3]}, (mh_u32x4*)w);
+                else for (int b = 0; b < 4; b++) w[b * gs] = out[b];
+            } else if (xg < x1 && xg + 16 > x0) {
+                for (int b = 0; b < 16; b++)
+                    if (xg + b >= x0 && xg + b < x1) ((uint8_t*)(w + (b >> 2) * gs))[b & 3] = (uint8_t)(out[b >> 2] >> (8 * (b & 3)));
+            }
         }
     }
 
-    // NMI raised by PPU call `call` (1-based, frame-relative); nes_core.hpp:520-531
-    __device__ void nmi(int32_t call) {
-        int32_t it = (call - 1) / 3;
-        push((uint8_t)(pc >> 8)); push((uint8_t)pc); push((uint8_t)(p | 0x20));
-        p |= FI;
-        pc = (uint16_t)(prg(0xfffa) | prg(0xfffb) << 8);
-        int32_t d = (zero_skip && it == exec_at) ? 0 : (exec_at - it + 1);
-        exec_at = it + d + 6;
-        zero_skip = 0;
+    // Of the n whole render lines from this one's start on, how many can go by at once: none that could raise the
+    // sprite-0 hit (0: the first one could, or the scroll goes line by line because copy_h is off).
+    __device__ __forceinline__ int plain_lines(int n) const {
+        if (!show_bg()) return n;
+        if (!show_spr()) return 0;
+        if (s0hit) return n;
+        if (sprite0_first()) return 0;
+        if (oam_addr >= 4) return n;
+        // the lists still to come: evaluated at the end of line s - 1 for line s, sprite 0 in range from y0 on
+        const int y0 = (int)(oam_sprite(0) & 0xffu), h = long_spr() ? 16 : 8;
+        const int first = y0 + 1 > scanline + 1 ? y0 + 1 : scanline + 1;
+        if (first - 1 >= y0 + h) return n;
+        const int k = first - scanline;
+        return k < n ? k : n;
     }
 
     // advance the PPU by n calls (nes_core.hpp:539-616)
-    __device__ void ppu_run(int32_t n) {
+    __device__ __forceinline__ void ppu_run(int32_t n) {
         while (n > 0) {
             int c = pcyc;
-            if (pstate == ST_PRE) {
-                bool on = show_bg() && show_spr();
-                int end = LINE_END - (!even && on);
-                int k = c >= end ? 1 : (n < end - c ? n : end - c);
-                int lo = c, hi = c + k;
+            if (pstate == ST_RENDER) {
+                if (c >= 1 && c <= 256) {
+                    // whole lines, or a piece of one
+                    const bool whole = c == 1 && n >= LINE_END;
+                    int k = 0;
+                    if (whole) {
+                        const int left = 240 - scanline, due = n / LINE_END;
+                        k = plain_lines(due < left ? due : left);
+                    }
+                    const int len = whole ? 256 : n < 257 - c ? n : 257 - c;
+                    if (render) draw_lines(k > 0 ? (uint32_t)k : 1u, c - 1, c - 1 + len);
+                    if (k == 0) {
+                        dots_hit_scroll(c - 1, c - 1 + len);
+                        if (whole) {
+                            if (show_bg()) { fine_y_step(); if (show_spr()) copy_h(); }
+                            k = 1;
+                        }
+                    } else if (show_bg()) {
+                        v = v_lines_on((uint32_t)k);
+                    }
+                    if (k > 0) {
+                        scanline += k;
+                        ppu_calls += k * LINE_END; n -= k * LINE_END;
+                        pend_line = scanline - 1;   // sprite evaluation for the next line (materialized lazily)
+                        if (scanline >= 240) pstate = ST_POST;
+                        continue;
+                    }
+                    pcyc += len; ppu_calls += len; n -= len;
+                    c = pcyc;
+                }
+                if (n <= 0) {
+                    // the calls ran out inside the visible dots
+                } else if (c == 257) {
+                    if (show_bg()) fine_y_step();
+                    pcyc++; ppu_calls++; n--;
+                } else if (c == 258) {
+                    if (show_bg() && show_spr()) copy_h();
+                    pcyc++; ppu_calls++; n--;
+                } else if (c > 258 && c < LINE_END) {
+                    const int k = n < LINE_END - c ? n : LINE_END - c;
+                    pcyc += k; ppu_calls += k; n -= k;
+                } else if (c >= LINE_END) {
+                    pend_line = scanline;   // sprite evaluation for the next line (materialized lazily)
+                    scanline++;
+                    pcyc = 1; ppu_calls++; n--;
+                    if (scanline >= 240) pstate = ST_POST;
+                } else {
+                    pcyc++; ppu_calls++; n--;
+                }
+            } else if (pstate == ST_PRE) {
+                const bool on = show_bg() && show_spr();
+                const int end = LINE_END - (!even && on);
+                const int k = c >= end ? 1 : (n < end - c ? n : end - c);
+                const int lo = c, hi = c + k;
                 if (lo <= 1 && 1 < hi) vblank = s0hit = 0;
                 if (on) {
                     if (lo <= 258 && 258 < hi) copy_h();
@@ -1240,59 +893,26 @@ struct Console {
                 ppu_calls += k; n -= k;
                 if (hi - 1 >= end) { pstate = ST_RENDER; scanline = 0; pcyc = 1; }
                 else pcyc = hi;
-            } else if (pstate == ST_RENDER) {
-                if (c >= 1 && c <= 256) {
-                    int k = n < 257 - c ? n : 257 - c;
-                    if (render) dots_drawn(c - 1, c - 1 + k);
-                    dots_hit_scroll(c - 1, c - 1 + k);
-                    pcyc += k; ppu_calls += k; n -= k;
-                    c = pcyc;
-                }
-                if (n <= 0) {
-                    // the calls ran out inside the visible dots
-                } else if (c == 257 && n >= LINE_END - 256) {
-                    // the rest of the line in one step when all of it is due: dot 257 (fine y), dot 258
-                    // (copy_h), dots 259..340, and the line end (85 calls), as the cases below would
-                    if (show_bg()) fine_y_step();
-                    if (show_bg() && show_spr()) copy_h();
-                    pend_line = scanline;   // sprite evaluation for the next line (materialized lazily)
-                    sp_line = -1;
-                    scanline++;
-                    pcyc = 1; ppu_calls += LINE_END - 256; n -= LINE_END - 256;
-                    if (scanline >= 240) pstate = ST_POST;
-                } else if (c == 257) {
-                    if (show_bg()) fine_y_step();
-                    pcyc++; ppu_calls++; n--;
-                } else if (c == 258) {
-                    if (show_bg() && show_spr()) copy_h();
-                    pcyc++; ppu_calls++; n--;
-                } else if (c > 258 && c < LINE_END) {
-                    int k = n < LINE_END - c ? n : LINE_END - c;
-                    pcyc += k; ppu_calls += k; n -= k;
-                } else if (c >= LINE_END) {
-                    pend_line = scanline;   // sprite evaluation for the next line (materialized lazily)
-                    sp_line = -1;
-                    scanline++;
-                    pcyc = 1; ppu_calls++; n--;
-                    if (scanline >= 240) pstate = ST_POST;
-                } else {
-                    pcyc++; ppu_calls++; n--;
-                }
             } else if (pstate == ST_POST) {
                 if (c >= LINE_END) { scanline++; pcyc = 1; pstate = ST_VBLANK; ppu_calls++; n--; }
-                else { int k = n < LINE_END - c ? n : LINE_END - c; pcyc += k; ppu_calls += k; n -= k; }
+                else { const int k = n < LINE_END - c ? n : LINE_END - c; pcyc += k; ppu_calls += k; n -= k; }
             } else {
-                if (c >= LINE_END) {
+                if (n >= LINE_END && scanline >= 241 && scanline < 260 && !(scanline == 241 && c <= 1) && c <= LINE_END) {
+                    // whole lines of the vertical blank past its start, up to its last one, at the same dot
+                    int k = n / LINE_END;
+                    if (k > 260 - scanline) k = 260 - scanline;
+                    scanline += k; ppu_calls += k * LINE_END; n -= k * LINE_END;
+                } else if (c >= LINE_END) {
                     scanline++; pcyc = 1;
                     if (scanline >= 261) { pstate = ST_PRE; scanline = 0; even = !even; }
                     ppu_calls++; n--;
                 } else if (c == 1 && scanline == 241) {
                     vblank = 1; ppu_calls++; n--; pcyc = 2;
-                    if (nmi_en()) nmi(ppu_calls);
+                    if (nmi_en()) { nmi_call = ppu_calls; n = 0; }   // the caller raises it and goes on
                 } else {
                     int lim = LINE_END - c;
                     if (scanline == 241 && c < 1) lim = 1 - c;
-                    int k = n < lim ? n : lim;
+                    const int k = n < lim ? n : lim;
                     pcyc += k; ppu_calls += k; n -= k;
                 }
             }
@@ -1300,25 +920,42 @@ struct Console {
     }
 
     // ------------------------------------------------------------ CPU (nes_core.hpp:619-899)
-    __device__ __forceinline__ void set_nz(uint8_t r) { p = (uint8_t)((p & ~(FZ | FN)) | (r ? 0 : FZ) | (r & 0x80 ? FN : 0)); }
-    __device__ __forceinline__ void flag(uint8_t f, bool on) { p = on ? (uint8_t)(p | f) : (uint8_t)(p & ~f); }
-    __device__ __forceinline__ bool has(uint8_t f) const { return (p & f) != 0; }
-    __device__ __forceinline__ void push(uint8_t d) { st(ROW_RAM + ((0x100 | sp) & 0x7ff), d); sp--; }
-    __device__ __forceinline__ uint8_t pull() { sp++; return ram(0x100 | sp); }
-    __device__ __forceinline__ void cross_penalty(uint16_t u, uint16_t w, int k) { if ((u & 0xff00) != (w & 0xff00)) skip += k; }
-
-    // End of the next frame slice: the PPU call after which dots 1..256 of the last line of the next
-    // group of SLICE_LINES render lines are done (the current group's if its last line is still ahead),
-    // capped at the frame end `cap`.
-    __device__ __forceinline__ int32_t next_slice(int32_t cap) const {
-        int line = 0;
-        if (pstate == ST_RENDER) line = pcyc < 257 ? scanline : scanline + 1;
-        const int last = (line | (SLICE_LINES - 1)) < 239 ? (line | (SLICE_LINES - 1)) : 239;
-        int32_t d = line <= 239 ? calls_until(last, 257) : calls_until(SLICE_LINES - 1, 257);
-        if (d < 1) d = 1;
-        const int32_t s = ppu_calls + d;
-        return s < cap ? s : cap;
+    __device__ __forceinline__ void set_nz(uint32_t r) { p = (p & ~(uint32_t)(FZ | FN)) | (r ? 0u : (uint32_t)FZ) | (r & 0x80 ? (uint32_t)FN : 0u); }
+    __device__ __forceinline__ void push(uint32_t d) { set_ram(0x100 | sp, d); sp = (sp - 1) & 0xffu; }
+    // NMI raised by PPU call `call` (1-based, frame-relative); nes_core.hpp:520-531
+    __device__ __forceinline__ void nmi(int32_t call) {
+        const int32_t it = (call - 1) / 3;
+        push(pc >> 8); push(pc & 0xffu); push(p | 0x20);
+        p |= FI;
+        pc = prg(0xfffa) | prg(0xfffb) << 8;
+        const int32_t d = (zero_skip && it == exec_at) ? 0 : (exec_at - it + 1);
+        exec_at = it + d + 6;
+        zero_skip = 0;
     }
+#if defined(__AMDGCN__)
+    // The CPU on the scalar unit from instruction j on, up to frame()'s stopping rules as one limit on the catch-up
+    // point 3 (j + 1): at most 3 end (j < end), and no NMI check that needs a catch-up first (below nmi_thresh, or
+    // already caught up to it). False if it ran nothing.
+    __device__ __forceinline__ bool cpu_run(int32_t j, int32_t end, const uint32_t* recs) {
+        int32_t lim = nmi_thresh - 1 > ppu_calls ? nmi_thresh - 1 : ppu_calls;
+        lim = lim < 3 * end ? lim : 3 * end;
+        const int32_t exlim = lim / 3 - 1;      // lim >= 3 (j + 1) > 0
+        ScalarRegs r{a, x, y, sp, ((p & FN) ? 0x100u : 0u) | ((p & FZ) ? 0u : 1u), (p & FC) ? 1u : 0u, (p & FV) ? 0x80u : 0u,
+                     p & ~(uint32_t)(FN | FV | FZ | FC), (uint32_t)(exlim - j) << 16, pc << 2};
+        scalar_run(r, recs, (uint32_t)(uintptr_t)(m + ROW_RAM), (uint32_t)(uintptr_t)prg_);
+        const uint32_t n = r.left & 0xffffu;
+        if (!n) return false;
+        a = r.a; x = r.x; y = r.y; sp = r.sp;
+        p = r.p_rest | ((r.nz & 0x180u) ? (uint32_t)FN : 0u) | ((r.nz & 0xffu) ? 0u : (uint32_t)FZ) |
+            (r.c ? (uint32_t)FC : 0u) | ((r.v & 0x80u) ? (uint32_t)FV : 0u);
+        pc = (r.pc4 >> 2) & 0xffffu;
+        exec_at = exlim - ((int32_t)r.left >> 16);
+        zero_skip = 0;
+        instructions += n;
+        return true;
+    }
+#endif
+    __device__ __forceinline__ void cross_penalty(uint32_t u, uint32_t w, int k) { if ((u ^ w) & 0xff00) skip += k; }
 
     // The data operation of decode word D: the result byte and the new flags, from the packed registers regs
     // (a | x << 8 | y << 16 | sp << 24), the data operand m (the first operand byte when nothing was read), the
@@ -1368,105 +1005,94 @@ struct Console {
     // One whole instruction from its decode word: addressing, at most one data read and one data
     // write through the bus, the ALU as register selects, and one small switch for the stack /
     // control-flow operations, in the reference's bus order (operand bytes, pointer, data read, data
-    // write; JSR pushes before reading its operand, a branch reads its offset only when taken).
-    // `pf`: the opcode and both following bytes are in PRG (pc <= 0xfffd) and were read as op, q1, q2,
-    // which has no side effects; otherwise they are fetched through the bus, with the PPU caught up
-    // first because a fetch may hit a PPU register. Returns false, with no effect, when the PPU must be
-    // caught up to `tgt` first; the caller does that and starts the instruction again.
-    __device__ __forceinline__ bool instruction(int32_t j, int32_t tgt, bool pf, uint8_t op, uint8_t q1, uint8_t q2) {
+    // write; JSR pushes before reading its operand; a branch reads its offset only when taken). It runs what
+    // scalar_run leaves: invalid opcodes, code outside PRG, computed addresses of registers, BRK.
+    // `pf`: the opcode and both following bytes are in PRG (pc <= 0xfffd); otherwise they are fetched through the bus,
+    // with the PPU caught up first because a fetch may hit a PPU register. Returns false, with no effect, when the
+    // PPU must be caught up to `tgt` first; the caller does that and starts the instruction again.
+    __device__ __forceinline__ bool instruction(int32_t j, int32_t tgt) {
         using namespace dec;
+        const bool pf = pc >= 0x8000u && pc <= 0xfffdu;
         if (!pf && ppu_calls < tgt) return false;
-        uint8_t b1 = q1, b2 = q2;
-        uint32_t D;
+        uint32_t op, b1 = 0, b2 = 0, D;
         if (!pf) {
-            // Opcode and operand bytes through the bus. Their loads are waited for inside this branch: a wait
-            // where the paths join would also wait for every store still in flight from earlier instructions.
-            uint32_t o = read(pc);
-            in_register(o);
-            op = (uint8_t)o;
-            D = cart.dec[op];
+            op = read(pc);
+            D = dec[op];
             const uint32_t xop0 = (D >> X_SH) & 15u;
             if (xop0 != X_JSR && xop0 != X_BRANCH) {   // JSR and branches fetch below, in their order
                 const uint32_t am0 = D & 15u;
-                uint32_t t1 = b1, t2 = b2;
-                if (am0 != M_NONE) t1 = read((uint16_t)(pc + 1));
-                if (am0 == M_ABS || am0 == M_ABSX || am0 == M_ABSY) t2 = read((uint16_t)(pc + 2));
-                in_register(t1); in_register(t2);
-                b1 = (uint8_t)t1; b2 = (uint8_t)t2;
+                if (am0 != M_NONE) b1 = read((pc + 1) & 0xffffu);
+                if (am0 == M_ABS || am0 == M_ABSX || am0 == M_ABSY) b2 = read((pc + 2) & 0xffffu);
             }
         } else {
-            D = cart.dec[op];
+            op = prg(pc); b1 = prg(pc + 1); b2 = prg(pc + 2);
+            D = dec[op];
         }
         const uint32_t am = D & 15u, xop = (D >> X_SH) & 15u, dst = (D >> DST_SH) & 7u;
         const bool rd = (D & RD) != 0, wr = dst == D_MEM;
-        // addressing as selects on mode-set bits (no branch except for the zero-page pointer loads)
         const uint32_t mb = 1u << am;
         constexpr uint32_t X_IDX = 1u << M_ZPX | 1u << M_ABSX, Y_IDX = 1u << M_ZPY | 1u << M_ABSY | 1u << M_INDY;
         constexpr uint32_t ZP_EA = 1u << M_ZP | 1u << M_ZPX | 1u << M_ZPY, IND = 1u << M_INDX | 1u << M_INDY;
-        const uint16_t absv = (uint16_t)(b1 | b2 << 8);
-        uint16_t base = absv;
+        const uint32_t absv = b1 | b2 << 8;
+        uint32_t base = absv;
         if (mb & IND) {   // pointer from the zero page
-            const uint8_t z = am == M_INDX ? (uint8_t)(b1 + x) : b1;
-            base = (uint16_t)(ram(z) | ram((uint8_t)(z + 1)) << 8);
+            const uint32_t z = am == M_INDX ? (b1 + x) & 0xffu : b1;
+            base = ram(z) | ram((z + 1) & 0xffu) << 8;
         }
-        const uint32_t idx = (mb & X_IDX) ? (uint32_t)x : (mb & Y_IDX) ? (uint32_t)y : 0u;
-        const uint16_t ea = (mb & ZP_EA) ? (uint16_t)((b1 + idx) & 0xffu)
-                          : am == M_IMM ? (uint16_t)(pc + 1) : (uint16_t)(base + idx);
-        const uint16_t p2 = (uint16_t)((absv & 0xff00) | ((absv + 1) & 0xff));   // JMP (ind): high byte, page wrap
-        const bool sync = xop == X_JMPI ? (needs_sync(absv, false) | needs_sync(p2, false))
-                                        : ((rd & needs_sync(ea, false)) | (wr & needs_sync(ea, true)));
+        const uint32_t idx = (mb & X_IDX) ? x : (mb & Y_IDX) ? y : 0u;
+        const uint32_t ea = (mb & ZP_EA) ? (b1 + idx) & 0xffu : am == M_IMM ? (pc + 1) & 0xffffu : (base + idx) & 0xffffu;
+        const uint32_t p2 = (absv & 0xff00) | ((absv + 1) & 0xff);   // JMP (ind): high byte, page wrap
+        const bool sync = xop == X_JMPI ? (needs_sync(absv, false) || needs_sync(p2, false))
+                                        : ((rd && needs_sync(ea, false)) || (wr && needs_sync(ea, true)));
         if (sync && ppu_calls < tgt) return false;   // only when pf: no bus access has happened yet
         cur = j;
         skip = 0;
         instructions++;
-        if (D & PEN) cross_penalty(base, (uint16_t)(base + idx), 1);
+        if (D & PEN) cross_penalty(base, base + idx, 1);
         // data operand and ALU
-        const uint8_t m = rd && am != M_IMM ? read(ea) : b1;
-        const uint32_t regs = (uint32_t)a | (uint32_t)x << 8 | (uint32_t)y << 16 | (uint32_t)sp << 24;
-        const AluOut ao = alu_op(D, regs, m, p, rd);
-        p = (uint8_t)ao.p;
-        const uint8_t r8 = (uint8_t)ao.r8;
-        // the destination register as a byte insert into the packed a | x << 8 | y << 16 | sp << 24 (D_A .. D_SP
-        // are 1 .. 4): the four fields share one word, so writing all four from it is one register write
-        const uint32_t dsh = (8u * (dst - D_A)) & 31u, dmask = 0xffu << dsh;   // masked: no register for D_NONE / D_MEM
-        const uint32_t nregs = (dst - D_A) < 4u ? (regs & ~dmask) | ((uint32_t)r8 << dsh) : regs;
-        a = nregs; x = nregs >> 8; y = nregs >> 16; sp = nregs >> 24;
+        const uint32_t mv = rd && am != M_IMM ? read(ea) : b1;
+        const AluOut ao = alu_op(D, a | x << 8 | y << 16 | sp << 24, mv, p, rd);
+        p = ao.p;
+        const uint32_t r8 = ao.r8;
+        if (dst == D_A) a = r8;
+        if (dst == D_X) x = r8;
+        if (dst == D_Y) y = r8;
+        if (dst == D_SP) sp = r8;
         if (wr) write(ea, r8);
-        // control flow: the next pc by instruction length, branches and JMP as selects
+        // control flow: the next pc by instruction length, branches and JMP
         constexpr uint32_t ABS3 = 1u << M_ABS | 1u << M_ABSX | 1u << M_ABSY;
-        uint16_t npc = (uint16_t)(pc + (am == M_NONE ? 1 : (mb & ABS3) ? 3 : 2));
-        const uint16_t ret = (uint16_t)(pc + 2);
-        {   // branch on N, V, C, Z (op bits 6-7) equal to op bit 5; 2 bytes; the offset is read only when taken
-            const uint32_t fbit = (0x40800201u >> (8 * (op >> 6))) & 0xffu;   // FN FV FC FZ
-            const bool taken = (xop == X_BRANCH) & (((p & fbit) != 0) == ((op & 0x20) != 0));
-            uint8_t off = b1;
-            if (taken && !pf) off = read((uint16_t)(pc + 1));
-            const uint16_t to = (uint16_t)(ret + (int8_t)off);
-            npc = xop == X_BRANCH ? (taken ? to : ret) : xop == X_JMP ? absv : npc;
-            skip += taken ? (((ret ^ to) & 0xff00) ? 3 : 1) : 0;
+        const uint32_t ret = (pc + 2) & 0xffffu;
+        uint32_t npc = (pc + (am == M_NONE ? 1 : (mb & ABS3) ? 3 : 2)) & 0xffffu;
+        switch (xop) {
+            case X_BRANCH: {   // on N, V, C, Z (op bits 6-7) equal to op bit 5; 2 bytes; the offset is read only when taken
+                const uint32_t fbit = (0x40800201u >> (8 * (op >> 6))) & 0xffu;   // FN FV FC FZ
+                npc = ret;
+                if (((p & fbit) != 0) == ((op & 0x20) != 0)) {
+                    const uint32_t off = pf ? b1 : read((pc + 1) & 0xffffu);
+                    npc = (ret + (uint32_t)(int32_t)(int8_t)off) & 0xffffu;
+                    skip += ((ret ^ npc) & 0xff00) ? 3 : 1;
+                }
+                break;
+            }
+            case X_JMP: npc = absv; break;
+            case X_BRK:
+                push(ret >> 8); push(ret & 0xffu); push(p | 0x30);
+                p |= FI; npc = prg(0xfffe) | prg(0xffff) << 8; skip += 7;
+                break;
+            case X_JSR:
+                push(ret >> 8); push(ret & 0xffu);
+                npc = absv;
+                if (!pf) { const uint32_t lo = read((pc + 1) & 0xffffu); npc = lo | read((pc + 2) & 0xffffu) << 8; }
+                break;
+            case X_PHA: push(a); break;
+            case X_PHP: push(p); break;
+            case X_RTS: { const uint32_t lo = pull(); npc = ((lo | pull() << 8) + 1) & 0xffffu; break; }
+            case X_RTI: { p = pull(); const uint32_t lo = pull(); npc = lo | pull() << 8; break; }
+            case X_PLA: a = pull(); set_nz(a); break;
+            case X_PLP: p = pull(); break;
+            case X_JMPI: { const uint32_t lo = read(absv); npc = lo | read(p2) << 8; break; }
+            default: break;
         }
-        // Stack operations as at most three pushes or three pulls with predicated accesses (the pulls are
-        // in flight together), then their results as selects: BRK, JSR, PHA, PHP push; RTI, RTS, PLA, PLP pull.
-        if (xop >= X_BRK && xop <= X_PLP) {
-            const uint32_t npush = xop == X_BRK ? 3u : xop == X_JSR ? 2u : (xop == X_PHA || xop == X_PHP) ? 1u : 0u;
-            const uint32_t npull = xop == X_RTI ? 3u : xop == X_RTS ? 2u : (xop == X_PLA || xop == X_PLP) ? 1u : 0u;
-            const uint8_t v0 = (xop == X_BRK || xop == X_JSR) ? (uint8_t)(ret >> 8) : xop == X_PHA ? a : p;
-            if (npush > 0) st(ROW_RAM + (0x100 | sp), v0);
-            if (npush > 1) st(ROW_RAM + (0x100 | (uint8_t)(sp - 1)), (uint8_t)ret);
-            if (npush > 2) st(ROW_RAM + (0x100 | (uint8_t)(sp - 2)), (uint8_t)(p | 0x30));
-            uint8_t u0 = 0, u1 = 0, u2 = 0;
-            if (npull > 0) u0 = ram(0x100 | (uint8_t)(sp + 1));
-            if (npull > 1) u1 = ram(0x100 | (uint8_t)(sp + 2));
-            if (npull > 2) u2 = ram(0x100 | (uint8_t)(sp + 3));
-            sp = (uint8_t)(sp - npush + npull);
-            if (xop == X_BRK) { p |= FI; npc = (uint16_t)(prg(0xfffe) | prg(0xffff) << 8); skip += 7; }
-            if (xop == X_JSR) npc = pf ? absv : (uint16_t)(read((uint16_t)(pc + 1)) | read((uint16_t)(pc + 2)) << 8);
-            if (xop == X_RTS) npc = (uint16_t)((u0 | u1 << 8) + 1);
-            if (xop == X_RTI) { p = u0; npc = (uint16_t)(u1 | u2 << 8); }
-            if (xop == X_PLA) { a = u0; set_nz(a); }
-            if (xop == X_PLP) p = u0;
-        }
-        if (xop == X_JMPI) { const uint8_t lo = read(absv); const uint8_t hi = read(p2); npc = (uint16_t)(lo | hi << 8); }
         pc = npc;
         if (D & OK) skip += (int)((D >> CYC_SH) & 7u);
         else bad_ops++;
@@ -1474,51 +1100,7 @@ struct Console {
         zero_skip = skip <= 0;
         return true;
     }
-
-    // ------------------------------------------------------------ a lone console's instruction run
-    // While a console is one of the last few of its wave with an instruction to run (at most LONE_MAX_ENVS; the
-    // others parked at their slice end, or out of the frame loop), an iteration of frame()'s loop costs about
-    // what it costs a full wave: every opcode's work as selects, the wave votes and the catch-up checks.
-    // lone_run() runs that console's instructions back to back instead (the frame loop calls it for those
-    // consoles one after the other, each under its own lanes' exec mask), in lone_long(), with its registers
-    // wave-uniform and one body per opcode.
-    // It runs the instructions whose opcode and operands are in PRG and whose bus accesses touch only RAM, PRG,
-    // or addresses that read as 0 or ignore writes ($4000-$7FFF but the joypads and OAM DMA), as instruction()
-    // would; it stops before any other instruction (PPU register, joypad or DMA access, invalid opcode), before
-    // the idle loop `JMP *` (fast-forwarded by frame()), before an instruction at the NMI check, and at the
-    // slice or frame end, leaving that instruction to frame()'s own iteration. Returns the number of instructions
-    // run. Called by this console's lanes only (its parts, with identical values), while no lane of the wave
-    // waits for a catch-up.
-    __device__ __forceinline__ static uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
-    __device__ __forceinline__ uint32_t lone_run(int32_t end, int32_t slice) {
-        // frame()'s stopping rules as one limit on the catch-up point 3 (j + 1) of instruction j: at most the slice
-        // end, at most 3 end (j < end), and no NMI check that needs a catch-up first (below nmi_thresh, or
-        // already caught up to it)
-        const int32_t calls = (int32_t)uniform((uint32_t)ppu_calls), nmi = (int32_t)uniform((uint32_t)nmi_thresh);
-        const int32_t last = (int32_t)uniform((uint32_t)slice);
-        int32_t lim = nmi - 1 > calls ? nmi - 1 : calls;
-        lim = lim < last ? lim : last;
-        lim = lim < 3 * end ? lim : 3 * end;
-        const uint32_t pflags = ((ppu_flags & (PF_SHOW_BG | PF_SHOW_SPR)) ? 0u : LP_WRITES) |
-                                ((ppu_flags & PF_INC32) ? LP_INC32 : 0u) | cart.nt_bits << LP_NT_SHIFT;
-        const LoneRegs o = lone_long(LoneRegs{pc, a, x, y, sp, p, exec_at, zero_skip, (uint32_t)v | (uint32_t)t << 16,
-                                              (uint32_t)fine_x | (uint32_t)first_write << 8, 0u},
-                                     lim, mbase + eo, mbase + vo, np, pflags, cart.gprg);
-        if (o.n) {
-            pc = (uint16_t)o.pc;
-            a = o.a; x = o.x; y = o.y; sp = o.sp;
-            p = (uint8_t)o.p;
-            exec_at = o.ex;
-            zero_skip = o.zs;
-            if (o.px >> 17) {   // the run wrote a PPU register
-                v = o.vt & 0xffffu; t = o.vt >> 16;
-                fine_x = o.px & 0xffu; first_write = (o.px >> 8) & 1u;
-                if (o.px & 0x10000u) { bg_key = -1; sp_line = -1; }   // name tables written: the tile-row and sprite-line caches
-            }
-            instructions += o.n;
-        }
-        return o.n;
-    }
+    __device__ __forceinline__ uint32_t pull() { sp = (sp + 1) & 0xffu; return ram(0x100 | sp); }
 
     // PPU calls from the current PPU position to (line, dot) on the frame timeline of
     // nmi_threshold() (pre-render line = -1, 262 x 341 calls); the one-dot-shorter odd pre-render
@@ -1580,126 +1162,302 @@ struct Console {
         ff_instructions += 3 * (uint32_t)k;
         return true;
     }
+};
 
-    // One nes-py Emulator::step (nes_core.hpp:1166-1204) with the exact `JMP *` idle fast-forward.
-    //
-    // Every lane runs the same loop body: one whole instruction per iteration, and one PPU catch-up
-    // site (`want`) for the NMI point, PPU-register accesses, the poll fast-forward and the frame
-    // slices. Branching per opcode is confined to register arithmetic, so a wave whose lanes run
-    // different instructions stays converged on the memory accesses.
-    //
-    // The frame is cut into slices that end right after the visible dots of every SLICE_LINES-th render
-    // line (and at the frame end). A lane only starts an instruction j whose catch-up point 3 (j + 1) is
-    // at most its slice end; once every lane of the wave is parked at its slice end, all of them catch
-    // their PPU up to it together, so the slice's lines are rendered with the whole wave active. This is the
-    // reference's catch-up PPU cut at more points (the PPU result does not depend on where it is
-    // caught up), and never past a parked lane's next catch-up point 3 (j + 1), so an NMI raised
-    // inside the slice catch-up sees exactly the CPU state of the reference's catch-up at the start
-    // of j.
-    __device__ __forceinline__ void frame() {
-        // The kernel ends with its slowest wave (at steady state ~1.35x the mean wave), and the two waves of a
-        // SIMD compete for its issue slots: a wave at an earlier frame of its agent step issues first (frames
-        // 0 and 1 of the step at priority 3, frame 2 at 2, later frames, hack frames and re-emulations at 1; the
-        // observation tails after the frame loop run at 0), so a wave that falls behind takes the slots of a
-        // SIMD-mate that is ahead. Measured on 32,768 envs of 1-1: k_step 17.27 -> 16.57 ms (frame-index
-        // mappings 3/2/1/1 16.86, 3/2/2/1 16.76, 3/3/3/2 16.69, 3/3/2/2 16.93 ms; priorities from a global count
-        // of the frames the waves have started 17.17 ms).
-        {
-            const uint32_t f = __builtin_amdgcn_readfirstlane(nframe);
-            nframe++;
-            if (f < 2) __builtin_amdgcn_s_setprio(3);
-            else if (f < 3) __builtin_amdgcn_s_setprio(2);
-            else __builtin_amdgcn_s_setprio(1);
+// The functions of a console: registers in, registers out. Each is inlined at one place of run_frame(): only the file
+// and the CPU's registers live across them. (As calls, every entry and return waited for the frame stores in flight.)
+#if defined(__AMDGCN__)
+#define MH_FN __device__ __attribute__((noinline))
+#else
+#define MH_FN inline
+#endif
+// The PPU caught up to `target` calls, or to the call that raises an NMI (F_NMI_CALL) if that comes before.
+__device__ __forceinline__ File ppu_advance(File f, Ctx c, int32_t target) {
+    Core k;
+    k.attach(c);
+    k.open_ppu(f);
+    target = (int32_t)uni((uint32_t)target);
+    k.nmi_call = 0;
+    if (target > k.ppu_calls) {
+        k.ppu_run(target - k.ppu_calls);
+        k.nmi_threshold();
+    }
+    k.close_ppu(f);
+    return f;
+}
+// An absolute access of instruction j to a register (record `rec`, REC_STORE of `val` or REC_LOAD). data: what was read;
+// skip: the instruction's cycles.
+struct IoResult { File f; uint32_t data; int32_t skip; };
+__device__ __forceinline__ IoResult io_access(File f, Ctx c, uint32_t rec, uint32_t val, int32_t j) {
+    Core k;
+    k.attach(c);
+    k.open_io(f);
+    rec = uni(rec);
+    k.cur = (int32_t)uni((uint32_t)j);
+    k.skip = 4;
+    uint32_t d = 0;
+    if ((rec & 0xf0u) == REC_STORE) k.write(rec >> 16, uni(val));
+    else d = k.read(rec >> 16);
+    k.close_io(f);
+    return IoResult{f, d, k.skip};
+}
+// poll_skip at instruction j; f's CPU words hold pc (in) and a, p, exec_at, zero_skip (out). F_NMI_CALL: 1 if it advanced.
+__device__ __forceinline__ File poll_wait(File f, Ctx c, int32_t j, int32_t end, uint32_t wait_hit) {
+    Core k;
+    k.attach(c);
+    k.open_ppu(f);
+    k.open_cpu(f);
+    k.first_write = f.get(S_FIRST_WRITE);
+    const bool on = k.poll_skip((int32_t)uni((uint32_t)j), (int32_t)uni((uint32_t)end), uni(wait_hit) != 0);
+    k.close_cpu(f);
+    f.set(S_VBLANK, k.vblank);
+    f.set(S_FIRST_WRITE, k.first_write);
+    f.set(F_NMI_CALL, on ? 1u : 0u);
+    return f;
+}
+// One whole instruction j, CPU words in f. F_NMI_CALL: 1 if the PPU must be caught up to `tgt` first (nothing done).
+__device__ __forceinline__ File whole_instruction(File f, Ctx c, int32_t j, int32_t tgt) {
+    Core k;
+    k.attach(c);
+    k.open_io(f);
+    k.open_cpu(f);
+    const bool done = k.instruction((int32_t)uni((uint32_t)j), (int32_t)uni((uint32_t)tgt));
+    k.close_io(f);
+    k.close_cpu(f);
+    f.set(F_NMI_CALL, done ? 0u : 1u);
+    return f;
+}
+// The sprite list of a pending evaluation, before the registers leave the kernel or its inputs change
+MH_FN File sprites_listed(File f, Ctx c) {
+    Core k;
+    k.attach(c);
+    k.open_ppu(f);
+    k.materialize_sprites();
+    k.close_sprites(f);
+    return f;
+}
+
+// One nes-py Emulator::step (nes_core.hpp:1166-1204) with the exact `JMP *` idle fast-forward.
+//
+// The CPU runs ahead (scalar_run) until something needs the PPU or a rule of its own: the NMI point, an access to a
+// PPU register (the catch-up point of instruction j is 3 (j + 1)), the frame end. The records say what an
+// instruction that stops a run is; the common ones (the registers' absolute loads and stores, the idle loop, the
+// sprite-0 wait) are handled here, the rest by instruction().
+// While rendering is off (both PPUMASK show bits clear), the catch-up PPU neither moves v nor draws anything but
+// the universal background colour, so the scroll and address writes and the $2007 writes to the pattern or name
+// tables do not depend on where the PPU has been caught up to, and are made without a catch-up. ($2007 writes
+// to the palette, $3EFF-$3FFE, change that colour.)
+MH_FN File run_frame(File f, Ctx c) {
+    constexpr int32_t end = FRAME_ITERS, last_call = 3 * FRAME_ITERS;
+    Core k;                                     // its CPU registers, memory and PPU position only
+    k.attach(c);
+    k.open_cpu(f);
+    k.ppu_calls = (int32_t)f.get(F_PPU_CALLS); k.nmi_thresh = (int32_t)f.get(F_NMI_THRESH);
+#if defined(__AMDGCN__)
+    const MH_SCALAR_CONST uint32_t* const recs =
+        (const MH_SCALAR_CONST uint32_t*)((uint64_t)c.w.get(Ctx::RECS_LO) | (uint64_t)c.w.get(Ctx::RECS_HI) << 32);
+    auto record = [&](uint32_t ad) { return recs[ad]; };
+#else
+    // (the host build runs every instruction in C++)
+    auto record = [&](uint32_t ad) { return decode_record(c.cart.prg, ad, c.cart.dec) & 0xffff00ffu; };
+#endif
+    int32_t want = -1;                          // catch the PPU up to here first
+    bool over = false;                          // the CPU is at the frame end
+    for (;;) {
+        if (want >= 0) {
+            f = ppu_advance(f, c, want);
+            k.ppu_calls = (int32_t)f.get(F_PPU_CALLS); k.nmi_thresh = (int32_t)f.get(F_NMI_THRESH);
+            const int32_t call = (int32_t)f.get(F_NMI_CALL);
+            if (call) { k.nmi(call); if (k.ppu_calls < want) continue; }
+            if (over) break;
+            want = -1;
         }
-        const int32_t end = FRAME_ITERS, last_call = 3 * FRAME_ITERS;
-        int32_t want = -1;
-        int32_t slice = next_slice(last_call);   // end of this lane's current slice, in PPU calls
-        bool parked = false, synced = false;
-        for (;;) {
-            if (__any(want >= 0)) {
-                // Every lane catches up with the one that must, each to its own next catch-up point
-                // 3 (j + 1) (the reference's point before its instruction j; an NMI due by then is raised
-                // exactly as in the lane's own catch-up), at most its slice end: the lines pending in
-                // the wave are rendered together instead of by one lane at a time.
-                int32_t t = want;
-                if (t < 0) { const int32_t nx = 3 * (exec_at + 1); t = nx < slice ? nx : slice; }
-                advance_to(t);
-                want = -1;
+        if (k.exec_at >= end) { want = last_call; over = true; continue; }
+        const int32_t j = k.exec_at, tgt = 3 * (j + 1);
+        if (tgt >= k.nmi_thresh && k.ppu_calls < tgt) { want = tgt; continue; }
+        const uint32_t rec = record(k.pc), kind = rec & 0xf0u;
+        if (rec & 0xff00u) {
+#if defined(__AMDGCN__)
+            if (k.cpu_run(j, end, (const uint32_t*)recs)) continue;
+#endif
+        } else if (kind == REC_IDLE) {
+            const int32_t lim_end = end - j, lim_nmi = k.nmi_thresh - tgt;
+            const int32_t k1 = lim_end > 0 ? (lim_end + 2) / 3 : 0;
+            const int32_t k2 = lim_nmi > 0 ? (lim_nmi + 8) / 9 : 0;
+            const int32_t kk = k1 < k2 ? k1 : k2;
+            if (kk > 1) { k.exec_at = j + 3 * (kk - 1); k.zero_skip = 0; continue; }
+        } else if (kind >= REC_STORE) {
+            const uint32_t ad = rec >> 16, reg = rec & 3u;
+            const bool st = kind == REC_STORE;
+            bool lazy = false;
+            if (st && ad < 0x4000u && (ad & 7u) >= 5u && !(f.get(F_PPU_FLAGS) & (PF_SHOW_BG | PF_SHOW_SPR)))
+                lazy = (ad & 7u) != 7u || f.get(S_V) - 0x3effu >= 0x100u;
+            if (!lazy && k.ppu_calls < tgt && Core::needs_sync(ad, st)) { want = tgt; continue; }
+            if (kind == REC_POLL) {
+                k.close_cpu(f);
+                f = poll_wait(f, c, j, end, rec & 4u);
+                k.open_cpu(f);
+                if (f.get(F_NMI_CALL)) continue;
             }
-            if (__all(parked)) {
-                // The whole wave is at the slice boundary: catch up together (next iteration), then
-                // open the next slice. `slice` and `synced` are wave-uniform, so every lane takes
-                // the same path here. (No early `continue`: after the catch-up request every lane is still
-                // parked, so the rest of this iteration does nothing; after a new slice opens, this
-                // iteration's actions are those the next one would take.)
-                if (!synced) {
-                    synced = true;
-                    want = ppu_calls < slice ? slice : -1;
+            const IoResult o = io_access(f, c, rec, reg == 0 ? k.a : reg == 1 ? k.x : k.y, j);
+            f = o.f;
+            if (!st) {
+                const uint32_t d = uni(o.data);
+                if (reg == 3u) {   // BIT
+                    k.p = (k.p & ~(uint32_t)(FZ | FV | FN)) | ((k.a & d) ? 0u : (uint32_t)FZ) | ((d & 0x40u) ? (uint32_t)FV : 0u) | (d >> 7);
                 } else {
-                    if (__all(slice >= last_call)) break;
-                    if (slice < last_call) { slice = next_slice(last_call); parked = false; }
-                    synced = false;
+                    if (reg == 0) k.a = d; else if (reg == 1) k.x = d; else k.y = d;
+                    k.set_nz(d);
                 }
             }
-            // One action per lane and iteration, chosen through `act` rather than early exits from the
-            // loop body (each exit is a path whose state the next iteration must merge): park at the
-            // slice end, ask for a catch-up, fast-forward, or run one instruction.
-            const int32_t j = exec_at;
-            const int32_t tgt = 3 * (j + 1);
-            bool act = !parked;
-            if (act && (j >= end || tgt > slice)) { parked = true; act = false; }
-            if (act && tgt >= nmi_thresh && ppu_calls < tgt) { want = tgt; act = false; }
-            {   // at most LONE_MAX_ENVS consoles left to run instructions and no catch-up asked for: each one's
-                // run of lone instructions, one console after the other (its own lanes only)
-                const uint64_t go = __ballot(act);
-                // (a run of at least one instruction is this iteration's action: no early `continue`, whose
-                // extra path into the loop top would make the compiler merge the console state there)
-                if (go && __popcll(go) <= LONE_MAX_ENVS * LANES_PER_ENV && !__any(want >= 0)) {
-                    uint64_t rest = go;
-                    do {   // wave-uniform: rest is a ballot
-                        const uint64_t env = PART_LANES << (__builtin_ctzll(rest) & (ENVS_PER_WAVE - 1));
-                        if ((env >> __lane_id()) & 1u)
-                            if (act && lone_run(end, slice) != 0) act = false;
-                        rest &= ~env;
-                    } while (rest);
-                }
-            }
-            // PRG bytes pc .. pc + 6 for the fast paths, from three aligned LDS words and two byte-aligns (the
-            // words past the last PRG word are the staged CHR bank's first ones: in bounds, and the bytes taken
-            // from them are not used); the idle check reads 0xff past 0xffff
-            const bool in_prg = pc >= 0x8000;
-            const uint32_t pa = pc & 0x7fffu;
-            const uint32_t* pw = (const uint32_t*)cart.prg + (pa >> 2);
-            const uint32_t w0 = pw[0], w1 = pw[1], w2 = pw[2];
-            const uint32_t b0 = __builtin_amdgcn_alignbyte(w1, w0, pa & 3u);   // bytes pc .. pc + 3
-            const uint32_t b4 = __builtin_amdgcn_alignbyte(w2, w1, pa & 3u);   // bytes pc + 4 .. pc + 7
-            const uint8_t op0 = in_prg ? (uint8_t)b0 : (uint8_t)0;
-            const uint8_t q1 = in_prg && pc != 0xffff ? (uint8_t)(b0 >> 8) : (uint8_t)0xff;
-            const uint8_t q2 = in_prg && pc < 0xfffe ? (uint8_t)(b0 >> 16) : (uint8_t)0xff;
-            if (act && in_prg && op0 == 0x4c && (uint16_t)(q1 | q2 << 8) == pc) {
-                const int32_t lim_end = end - j, lim_nmi = nmi_thresh - tgt;
-                const int32_t k1 = lim_end > 0 ? (lim_end + 2) / 3 : 0;
-                const int32_t k2 = lim_nmi > 0 ? (lim_nmi + 8) / 9 : 0;
-                const int32_t k = k1 < k2 ? k1 : k2;
-                if (k > 1) { exec_at = j + 3 * (k - 1); zero_skip = 0; act = false; }
-            }
-            // LDA $2002 / AND #$40 / BEQ|BNE back to the LDA: bytes AD 02 20 29 40 (F0|D0) F9
-            if (act && in_prg && pc <= 0xfff8 && b0 == 0x292002adu && (b4 & 0x00ff00ffu) == 0x00f90040u) {
-                const uint8_t br = (uint8_t)(b4 >> 8);
-                if (br == 0xf0 || br == 0xd0) {
-                    if (ppu_calls < tgt) { want = tgt; act = false; }   // the sync of the LDA $2002 at j
-                    else if (poll_skip(j, end, br == 0xf0)) act = false;
-                }
-            }
-            if (act && !instruction(j, tgt, in_prg && pc <= 0xfffd, op0, q1, q2)) want = tgt;
+            k.instructions++;
+            k.pc = (k.pc + 3) & 0xffffu;
+            k.exec_at = j + (int32_t)uni((uint32_t)o.skip);
+            k.zero_skip = 0;
+            continue;
         }
-        // rebase the frame-relative counters on the new frame start
-        exec_at -= FRAME_ITERS;
-        ppu_calls -= 3 * FRAME_ITERS;
-        nmi_thresh -= 3 * FRAME_ITERS;
-        const uint32_t lo = iter_lo + FRAME_ITERS;
-        iter_hi += lo < iter_lo;
-        iter_lo = lo;
+        k.close_cpu(f);
+        f = whole_instruction(f, c, j, tgt);
+        k.open_cpu(f);
+        if (f.get(F_NMI_CALL)) want = tgt;
+    }
+    // rebase the frame-relative counters on the new frame start
+    k.exec_at -= FRAME_ITERS;
+    k.close_cpu(f);
+    f.set(F_PPU_CALLS, (uint32_t)(k.ppu_calls - 3 * FRAME_ITERS));
+    f.set(F_NMI_THRESH, (uint32_t)(k.nmi_thresh - 3 * FRAME_ITERS));
+    const uint32_t lo0 = f.get(S_ITER_LO), lo = lo0 + FRAME_ITERS;
+    f.set(S_ITER_HI, f.get(S_ITER_HI) + (lo < lo0 ? 1u : 0u));
+    f.set(S_ITER_LO, lo);
+    return f;
+}
+
+// A console of the env layer and the kernels.
+struct Console {
+    MH_LDS uint8_t* m;       // its memory in LDS, between load() / power_on() and store()
+    MH_LDS uint32_t* gp;
+    Cart cart;
+    const MH_LDS uint8_t* lut;
+    uint32_t np;             // envs of the memory block, padded
+    uint32_t lane;
+    uint8_t* gray;           // the frame buffer frame() draws into, if `render`
+    bool render;
+    File f;
+    uint32_t bad_ops, instructions, ff_instructions;
+    uint32_t nframe;         // frame() calls since load(): the wave's issue priority in frame()
+
+    __device__ __forceinline__ Ctx ctx() const {
+        Ctx c;
+#if defined(__AMDGCN__)
+        c.w.r = 0;
+        auto ptr = [&](int k, uint64_t p) { c.w.set(k, (uint32_t)p); c.w.set(k + 1, (uint32_t)(p >> 32)); };
+        c.w.set(Ctx::M, (uint32_t)(uintptr_t)m); c.w.set(Ctx::GP, (uint32_t)(uintptr_t)gp);
+        c.w.set(Ctx::PRG, (uint32_t)(uintptr_t)cart.prg); c.w.set(Ctx::CHR, (uint32_t)(uintptr_t)cart.chr);
+        c.w.set(Ctx::LUT, (uint32_t)(uintptr_t)lut); ptr(Ctx::DEC_LO, (uint64_t)cart.dec); ptr(Ctx::RECS_LO, (uint64_t)cart.recs);
+        ptr(Ctx::GRAY_LO, (uint64_t)gray); c.w.set(Ctx::NT_BITS, cart.nt_bits); c.w.set(Ctx::NP, np); c.w.set(Ctx::RENDER, render);
+#else
+        c.m = m; c.gp = gp; c.cart = cart; c.gray = gray; c.lut = lut; c.np = np; c.render = render;
+#endif
+        return c;
+    }
+    __device__ __forceinline__ uint32_t ram(uint32_t ad) const { return uni(m[ROW_RAM + (ad & 0x7ff)]); }
+    __device__ __forceinline__ void set_ram(uint32_t ad, uint32_t val) { m[ROW_RAM + (ad & 0x7ff)] = (uint8_t)val; }
+    // joypad port 0's buttons for the next frames (the env layer's action)
+    __device__ __forceinline__ void set_buttons0(uint32_t b) { f.set(F_JOY, (f.get(F_JOY) & ~0xffu) | b); }
+    __device__ __forceinline__ static void mem_sync() { Core::mem_sync(); }
+
+    // ---- the register words of a block: lane k loads and stores word k
+    __device__ __forceinline__ void load_regs(const uint32_t* sc, uint32_t e) {
+#if defined(__AMDGCN__)
+        f.r = sc[(size_t)(lane < S_COUNT ? lane : 0u) * np + e];
+#else
+        for (int k = 0; k < S_COUNT; k++) f.r[k] = sc[(size_t)k * np + e];
+#endif
+        auto w = [&](int k) { return f.get(k); };
+        f.set(F_PPU_FLAGS, (w(S_SHOW_BG) ? PF_SHOW_BG : 0u) | (w(S_SHOW_SPR) ? PF_SHOW_SPR : 0u) |
+                           (w(S_HIDE_EDGE_BG) ? PF_HIDE_EDGE_BG : 0u) | (w(S_HIDE_EDGE_SPR) ? PF_HIDE_EDGE_SPR : 0u) |
+                           (w(S_LONG_SPR) ? PF_LONG_SPR : 0u) | (w(S_NMI_EN) ? PF_NMI_EN : 0u) |
+                           (w(S_BG_PAGE) ? PF_BG_PAGE : 0u) | (w(S_SPR_PAGE) ? PF_SPR_PAGE : 0u) |
+                           (w(S_INC) == 32 ? PF_INC32 : 0u));
+        f.set(F_JOY, (w(S_JOY_BUTTONS0) & 0xffu) | (w(S_JOY_BUTTONS1) & 0xffu) << 8 | (w(S_JOY_BITS0) & 0xffu) << 16 |
+                     (w(S_JOY_BITS1) & 0xffu) << 24);
+        f.set(F_JOY_STROBE, (w(S_JOY_STROBE0) & 1u) | (w(S_JOY_STROBE1) & 1u) << 1);
+        started();
+    }
+    __device__ __forceinline__ void started() {
+        f.set(F_PEND_LINE, 0xffffffffu); f.set(F_PAL_DIRTY, 1); f.set(F_PPU_CALLS, 0); f.set(F_NMI_CALL, 0);
+        f.set(F_BAD, 0); f.set(F_INSTR, 0); f.set(F_FF, 0);
+        Core k;
+        k.pstate = f.get(S_PSTATE); k.scanline = (int32_t)f.get(S_SCANLINE); k.pcyc = (int32_t)f.get(S_PCYC); k.ppu_calls = 0;
+        k.nmi_threshold();
+        f.set(F_NMI_THRESH, (uint32_t)k.nmi_thresh);
+        nframe = 0;
+    }
+    __device__ __forceinline__ void store_regs(uint32_t* sc, uint32_t e) {
+        f = sprites_listed(f, ctx());
+        const uint32_t fl = f.get(F_PPU_FLAGS), joy = f.get(F_JOY), js = f.get(F_JOY_STROBE);
+        auto w = [&](int k, uint32_t val) { f.set(k, val); };
+        w(S_JOY_STROBE0, js & 1u); w(S_JOY_STROBE1, (js >> 1) & 1u);
+        w(S_JOY_BUTTONS0, joy & 0xffu); w(S_JOY_BUTTONS1, (joy >> 8) & 0xffu);
+        w(S_JOY_BITS0, (joy >> 16) & 0xffu); w(S_JOY_BITS1, joy >> 24);
+        w(S_SHOW_BG, fl & PF_SHOW_BG ? 1u : 0u); w(S_SHOW_SPR, fl & PF_SHOW_SPR ? 1u : 0u);
+        w(S_HIDE_EDGE_BG, fl & PF_HIDE_EDGE_BG ? 1u : 0u); w(S_HIDE_EDGE_SPR, fl & PF_HIDE_EDGE_SPR ? 1u : 0u);
+        w(S_LONG_SPR, fl & PF_LONG_SPR ? 1u : 0u); w(S_NMI_EN, fl & PF_NMI_EN ? 1u : 0u);
+        w(S_BG_PAGE, fl & PF_BG_PAGE ? 1u : 0u); w(S_SPR_PAGE, fl & PF_SPR_PAGE ? 1u : 0u);
+        w(S_INC, fl & PF_INC32 ? 32u : 1u);
+#if defined(__AMDGCN__)
+        if (lane < S_COUNT) sc[(size_t)lane * np + e] = f.r;
+#else
+        for (int k = 0; k < S_COUNT; k++) sc[(size_t)k * np + e] = f.r[k];
+#endif
+    }
+    // ---- the memory of console e of a block: to LDS, and back
+    __device__ __forceinline__ void load_rows(const uint8_t* mem, uint32_t e) {
+        if constexpr (ON_GPU) {
+            const mh_u32x4* src = (const mh_u32x4*)(mem + mem_offset(np, e, 0));
+#pragma unroll
+            for (uint32_t i = lane; i < MEM_ROWS / 16; i += 64) ((MH_LDS mh_u32x4*)m)[i] = src[i];
+            Core::lds_sync();
+        } else {
+            for (uint32_t r = 0; r < MEM_ROWS; r++) m[r] = mem[mem_offset(np, e, r)];
+        }
+    }
+    __device__ __forceinline__ void store_rows(uint8_t* mem, uint32_t e) const {
+        if constexpr (ON_GPU) {
+            mh_u32x4* dst = (mh_u32x4*)(mem + mem_offset(np, e, 0));
+#pragma unroll
+            for (uint32_t i = lane; i < MEM_ROWS / 16; i += 64) dst[i] = ((const MH_LDS mh_u32x4*)m)[i];
+        } else {
+            for (uint32_t r = 0; r < MEM_ROWS; r++) mem[mem_offset(np, e, r)] = m[r];
+        }
+    }
+    // the whole console e of a memory block and its register words
+    __device__ __forceinline__ void load(const uint8_t* mem, const uint32_t* sc, uint32_t e) { load_regs(sc, e); load_rows(mem, e); }
+    __device__ __forceinline__ void store(uint8_t* mem, uint32_t* sc, uint32_t e) { store_regs(sc, e); store_rows(mem, e); }
+
+    // power-on: zeroed machine, then CPU and PPU reset (nes_core.hpp:123-147)
+    __device__ __forceinline__ void power_on() {
+        for (uint32_t i = lane; i < MEM_ROWS / 4; i += LANES) ((MH_LDS uint32_t*)m)[i] = 0;
+        Core::lds_sync();
+        auto prg = [&](uint32_t ad) { return uni(cart.prg[ad & 0x7fff]); };
+        for (int k = 0; k < F_COUNT; k++) f.set(k, 0);
+        f.set(S_P, 0x34); f.set(S_PC, prg(0xfffc) | prg(0xfffd) << 8); f.set(S_SP, 0xfd);
+        f.set(F_JOY_STROBE, 3); f.set(S_EVEN, 1); f.set(F_PPU_FLAGS, PF_SHOW_BG | PF_SHOW_SPR); f.set(S_FIRST_WRITE, 1);
+        f.set(S_PSTATE, ST_PRE);
+        started();
+    }
+    __device__ __forceinline__ void frame() {
+        // The kernel ends with its slowest wave, and the waves of a SIMD compete for its issue slots: a wave at an
+        // earlier frame of its agent step issues first (frames 0 and 1 of the step at priority 3, frame 2 at 2, later
+        // frames, hack frames and re-emulations at 1; the observations after the frame loop at 0), so a wave that
+        // falls behind takes the slots of a SIMD-mate that is ahead.
+        const uint32_t n = nframe++;
+        if (n < 2) __builtin_amdgcn_s_setprio(3);
+        else if (n < 3) __builtin_amdgcn_s_setprio(2);
+        else __builtin_amdgcn_s_setprio(1);
+        f = run_frame(f, ctx());
+        instructions += f.get(F_INSTR); ff_instructions += f.get(F_FF); bad_ops += f.get(F_BAD);
+        f.set(F_INSTR, 0); f.set(F_FF, 0); f.set(F_BAD, 0);
     }
 };
 

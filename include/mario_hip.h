@@ -41,7 +41,7 @@ const char* mh_last_error(void);
  *   lut           256 bytes, palette value -> gray, host memory
  *   rng           6*n u64 per env: numpy PCG64 (state_hi, state_lo, inc_hi, inc_lo, has_uint32, uinteger)
  *   skip 1..16, frame_stack 1..16, maxpool 0/1, sticky in [0, 1], noop_max >= 0, max_steps >= 1,
- *   1 <= n <= 979648 (the console memory is addressed with 32-bit offsets).
+ *   1 <= n <= 979648.
  * Blocks until construction is finished. */
 MhEnv* mh_create(const uint8_t* rom, int64_t rom_len, int n, const int* levels, const uint8_t* lut,
                  int skip, int max_steps, double sticky, int noop_max, int maxpool, int frame_stack,
@@ -81,8 +81,8 @@ void mh_destroy(MhEnv* h);
 
 /* Per-stage timing of mh_step_async with HIP events recorded on the step's own stream (no counterpart
  * in the reference; used by the benchmark). Stages: 0 k_step (emulation, render, and the max-pool +
- * INTER_AREA observation of most envs), 1 k_obs_late (the observation of the envs of the waves that finish
- * k_step last), 2 k_reset, 3 k_stack. mh_timing(h, 1) clears and starts
+ * INTER_AREA observation), 1 empty (k_obs_late, the observations once left to a kernel of their own), 2 k_reset,
+ * 3 k_stack. mh_timing(h, 1) clears and starts
  * recording; mh_timing_read synchronizes and returns the summed milliseconds per stage and the number
  * of timed steps. */
 #define MH_STAGES 4
@@ -122,9 +122,9 @@ int64_t mh_state_bytes(void);
 int64_t mh_env_bytes(MhEnv* h);
 
 /* ---- raw consoles: frame stepping without the env layer (replaces fm_raw_*, fastmario.cpp:651-673) */
-/* 1 <= n <= 979648 consoles (32-bit offsets into the console memory). The consoles run 1 to 16 per wave (the
-   most that still give every SIMD two waves); MH_RAW_CONSOLES_PER_WAVE=1|2|4|8|16 in the environment at this
-   call sets it instead (any other value: NULL, with mh_last_error()). Results do not depend on it. */
+/* 1 <= n <= 979648 consoles, a wave each. MH_RAW_CONSOLES_PER_WAVE in the environment at this call, once the number
+   of consoles a wave runs, has no effect; a value other than 1, 2, 4, 8 or 16 is still refused (NULL, with
+   mh_last_error()). */
 MhRaw*  mh_raw_create(const uint8_t* rom, int64_t rom_len, int n, int device);
 /* one frame of every console; d_buttons: n u8 device pointer; render != 0 draws the screen */
 int     mh_raw_frame(MhRaw* h, const uint8_t* d_buttons, int render, void* stream);
