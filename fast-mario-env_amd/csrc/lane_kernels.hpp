@@ -472,9 +472,19 @@ __device__ inline void cache_lane(const CacheArgs& A, const LaneCtx& x, int ci) 
     A.cframes[ci] = ev.frames; A.cinstr[ci] = c.instructions; A.cff[ci] = c.ff_instructions; A.cbad[ci] = c.bad_ops;
 }
 
+// Half-octaves of a step's executed instructions, for the order of the next step: 0 up to 3,071 (a step of a still
+// picture is about 2,000), 15 from 2^18 * 1.5.
+constexpr int WORK_BUCKETS = 16;
+__device__ inline uint32_t work_bucket(uint32_t executed) {
+    const uint32_t v = executed | 2048u;   // at least 2^11
+    const uint32_t lg = 31u - (uint32_t)__builtin_clz(v);
+    const uint32_t b = 2 * (lg - 11) + (v >> (lg - 1) & 1u);
+    return b < WORK_BUCKETS ? b : WORK_BUCKETS - 1;
+}
+
 // One agent step of the env in console slot e (fastmario.cpp:403-411 + 336-374).
 // Returns what the env's new observation needs: bit 0 pool, bit 1 the last frame is in frame buffer 1, bit 2
-// the boot observation, bits 8.. the level.
+// the boot observation, bits 4-7 the work bucket, bits 8.. the level.
 __device__ inline uint32_t step_lane(const StepArgs& A, const LaneCtx& x, uint32_t e) {
     const uint32_t o = (uint32_t)A.slot_env[e];   // the env's index in the action and output arrays
     Console c;
@@ -511,7 +521,8 @@ __device__ inline uint32_t step_lane(const StepArgs& A, const LaneCtx& x, uint32
     for (int k = 0; k < 3; k++)
         if ((ev.reemu >> k) & 1u) A.ev[(size_t)(E_REEMU_ONE + k) * A.np + e] += 1;
     A.ev[(size_t)E_HACK_REDRAWS * A.np + e] += ev.hack_redraws;
-    return (ev.pooled ? 1u : 0u) | (ev.slot_swap ? 2u : 0u) | (ev.shows_boot ? 4u : 0u) | level << 8;
+    return (ev.pooled ? 1u : 0u) | (ev.slot_swap ? 2u : 0u) | (ev.shows_boot ? 4u : 0u) |
+           work_bucket(c.instructions - c.ff_instructions) << 4 | level << 8;
 }
 
 // Auto-reset (fastmario.cpp:389-401): k = integers(noop_max + 1) from the env's stream, the draws of

@@ -136,65 +136,21 @@ __global__ void EMU_BOUNDS k_cache(CacheArgs A) {
     if (ci < A.nc) cache_lane(A, lane_ctx(A.R, s_rom, s_lut, s_env), ci);
 }
 
-// k_step's launch order for the next step. When k_step has more blocks than the GPU has CUs (past 32,768 envs on
-// 256 CUs), a block that starts late and runs long holds the kernel's end, and a block holds its CU until its slowest
-// env is done. A group's busy run (an area transition, a death, a level load) lasts several steps, so the last step's
-// work predicts the next one's: the groups run in order of their slowest env's executed 6502 instructions in the
-// last step, most first, and the cheap ones fill the CUs they free (longest-first list scheduling).
-// k_work: each group's slowest env's executed instructions since the last call, from the env counters.
-constexpr int ORDER_GROUP = WAVES_PER_BLOCK;   // envs of a full block
-static_assert(64 % ORDER_GROUP == 0, "k_work: whole groups per wave");
-__global__ __launch_bounds__(64) void k_work(const uint32_t* ev, uint32_t np, int n, uint64_t* prev,
-                                                    uint32_t* work) {
-    const uint32_t e = blockIdx.x * 64 + threadIdx.x;
-    uint32_t w = 0;
-    if (e < (uint32_t)n) {
-        auto counter = [&](int lo) {
-            return (uint64_t)ev[(size_t)lo * np + e] | (uint64_t)ev[(size_t)(lo + 1) * np + e] << 32;
-        };
-        const uint64_t c = counter(E_INSTR_LO) - counter(E_FF_LO);
-        const uint64_t d = c - prev[e];
-        w = d > 0xffffffffull ? 0xffffffffu : (uint32_t)d;
-        prev[e] = c;
-    }
-    for (int off = ORDER_GROUP / 2; off >= 1; off >>= 1) {
-        const uint32_t o = (uint32_t)__shfl_xor((int)w, off);
-        w = o > w ? o : w;
-    }
-    if (threadIdx.x % ORDER_GROUP == 0 && e < (uint32_t)n) work[e / ORDER_GROUP] = w;
-}
-// k_order: one block; a bitonic sort of (work, ~index) keys in LDS (ties: the lower index first).
-constexpr int ORDER_MAX = 8192;   // groups; past 131,072 envs the launch keeps its own order
-__global__ __launch_bounds__(1024) void k_order(const uint32_t* work, uint32_t* perm, int ng) {
-    __shared__ uint64_t key[ORDER_MAX];
-    int P = 1;
-    while (P < ng) P <<= 1;
-    for (int i = threadIdx.x; i < P; i += blockDim.x)
-        key[i] = i < ng ? ((uint64_t)work[i] << 32 | (uint32_t)~(uint32_t)i) : 0ull;   // padding sorts last
-    __syncthreads();
-    for (int k = 2; k <= P; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = threadIdx.x; i < P; i += blockDim.x) {
-                const int l = i ^ j;
-                if (l > i) {
-                    const uint64_t a = key[i], b = key[l];
-                    if ((i & k) == 0 ? a < b : a > b) { key[i] = b; key[l] = a; }   // descending overall
-                }
-            }
-            __syncthreads();
-        }
-    for (int i = threadIdx.x; i < ng; i += blockDim.x) perm[i] = ~(uint32_t)key[i];
-}
-
-__device__ __forceinline__ void step_block(const StepArgs& A, uint32_t block) {
-    ROM_LDS
-    stage_rom(A.R, s_rom, s_lut);
-    const uint32_t e = wave_console(block);
-    if (e >= (uint32_t)A.n) return;
-    const uint32_t bits = step_lane(A, lane_ctx(A.R, s_rom, s_lut, s_env), e);
-    __builtin_amdgcn_s_setprio(0);   // the frame loops of the other waves issue first
-    obs_tail(A.gray, A.np, A.fresh, A.boot_obs, e, threadIdx.x & 63u, bits);
-}
+// k_step's order when it has more envs than the GPU holds waves at once (past 4,096 on 256 CUs). The grid is then one
+// block per CU, and a wave that is done with an env takes the next one from a counter, so that no wave waits for the
+// slowest env of its block and the cartridge is staged once per CU. What is left is the end, when the last waves run
+// alone: the envs start in order of the last step's executed 6502 instructions, most first, in half-octave buckets
+// (longest-first list scheduling; a busy run, an area transition or a death, lasts several steps). k_step appends each
+// env to the next step's buckets itself, and k_reset, which follows it on the stream, turns the two lists over: no
+// launch and no pass of its own. The order within a bucket is that of the appends; no result depends on it.
+// Measured at 32,768 / 65,536 envs: k_step 9.0 / 18.8 ms, against 10.6 (unsorted) / 22.9 ms with blocks of 16 envs in
+// the order of each block's slowest env (8.4 / 16.1 ms of it are the waves' mean busy time).
+struct StepQueue {
+    uint32_t side;                          // the lists this step reads; it appends to the others
+    uint32_t next;                          // position of the next env to take, past the grid's first ones
+    uint32_t count[2][WORK_BUCKETS];
+};
+// the envs of bucket b, side s: list[(s * WORK_BUCKETS + b) * np ..]
 
 // What bounds it: scalar issue. A SIMD issues one scalar instruction per 4 cycles whichever of its waves it is from; the
 // headline step (32,768 envs of 1-1) is 126,000 scalar, 78,000 vector and 19,000 branch instructions per env, of which
@@ -202,10 +158,43 @@ __device__ __forceinline__ void step_block(const StepArgs& A, uint32_t block) {
 // lockstep (4 lanes each, every opcode's work as selects, 15 to 12 of 16 consoles active): a lockstep iteration issues
 // ~470 instructions for ~12 6502 instructions but each env waits for all of them; here a 6502 instruction is ~17
 // instructions and nothing waits for another console. Measured (k_step, the same envs): 256 envs 11.6 -> 1.03 ms,
-// 4,096 envs 19.9 -> 2.99 ms, 32,768 envs 14.57 -> 10.64 ms, 65,536 envs of 32 levels 40.9 -> 22.9 ms.
-__global__ void EMU_BOUNDS k_step(StepArgs A) { step_block(A, blockIdx.x); }
-// k_step in the launch order of k_order: block b runs group perm[b]
-__global__ void EMU_BOUNDS k_step_ordered(StepArgs A, const uint32_t* perm) { step_block(A, uni(perm[blockIdx.x])); }
+// 4,096 envs 19.9 -> 2.99 ms, 32,768 envs 14.57 -> 10.64 ms, 65,536 envs of 32 levels 40.9 -> 22.9 ms (9.0 and 18.8 with
+// the queue).
+// q null: every env has its wave.
+__global__ void EMU_BOUNDS k_step(StepArgs A, StepQueue* q, uint32_t* list) {
+    ROM_LDS
+    stage_rom(A.R, s_rom, s_lut);
+    const uint32_t lane = threadIdx.x & 63u, n = (uint32_t)A.n;
+    uint32_t i = q ? wave_slot() * gridDim.x + blockIdx.x : wave_console(blockIdx.x);   // the heaviest, one per CU
+    uint32_t side = 0, count = 0, upto = 0;   // lane k: bucket WORK_BUCKETS - 1 - k, and the envs up to its end
+    if (q) {
+        side = uni(q->side);
+        if (lane < WORK_BUCKETS) count = q->count[side][WORK_BUCKETS - 1 - lane];
+        upto = count;
+        for (int d = 1; d < WORK_BUCKETS; d <<= 1) {
+            const uint32_t o = (uint32_t)__shfl_up((int)upto, d);
+            if ((int)lane >= d) upto += o;
+        }
+    }
+    while (i < n) {
+        uint32_t e = i;
+        if (q) {
+            const uint32_t k = (uint32_t)__builtin_popcountll(__ballot(lane < WORK_BUCKETS - 1 && upto <= i));
+            const uint32_t first = uni((uint32_t)__shfl((int)(upto - count), (int)k));
+            e = uni(list[(size_t)(side * WORK_BUCKETS + WORK_BUCKETS - 1 - k) * A.np + (i - first)]);
+        }
+        const uint32_t bits = step_lane(A, lane_ctx(A.R, s_rom, s_lut, s_env), e);
+        __builtin_amdgcn_s_setprio(0);   // the frame loops of the other waves issue first
+        obs_tail(A.gray, A.np, A.fresh, A.boot_obs, e, lane, bits);
+        if (!q) return;
+        if (lane == 0) {
+            const uint32_t b = bits >> 4 & (WORK_BUCKETS - 1), o = side ^ 1u;
+            list[(size_t)(o * WORK_BUCKETS + b) * A.np + atomicAdd(&q->count[o][b], 1u)] = e;
+            i = atomicAdd(&q->next, 1u);   // grows past n by one per wave at most: every wave ends
+        }
+        i = uni(i);
+    }
+}
 
 __global__ void EMU_BOUNDS k_raw(RawArgs A) {
     ROM_LDS
@@ -216,7 +205,12 @@ __global__ void EMU_BOUNDS k_raw(RawArgs A) {
 
 // One wave of 64 envs per block: each lane draws its env's reset, then the wave copies the chosen cache
 // consoles one env at a time with all 64 lanes.
-__global__ void __launch_bounds__(64) k_reset(ResetArgs A) {
+__global__ void __launch_bounds__(64) k_reset(ResetArgs A, StepQueue* q, uint32_t first) {
+    if (q && blockIdx.x == 0) {   // after a step: its lists are done, the next step reads the others
+        const uint32_t s = q->side;
+        if (threadIdx.x < WORK_BUCKETS) q->count[s][threadIdx.x] = 0;
+        if (threadIdx.x == 0) { q->side = s ^ 1u; q->next = first; }
+    }
     const uint32_t e = blockIdx.x * 64 + threadIdx.x;
     const int ci = e < (uint32_t)A.n ? reset_lane(A, e) : -1;
     uint64_t m = __ballot(ci >= 0);
@@ -627,10 +621,9 @@ struct MhEnv {
     AreaTables* T = nullptr;
     uint8_t *mem = nullptr, *gray = nullptr, *fresh = nullptr;
     EmuLaunch ls{};                    // k_step's launch shape
-    // k_step's launch order (k_work, k_order), when it has more blocks than the GPU has CUs: null otherwise
-    uint32_t *grp_work = nullptr, *grp_perm = nullptr;
-    uint64_t* grp_prev = nullptr;      // each env's executed-instruction count at the last k_work
-    int n_groups = 0;
+    StepQueue* queue = nullptr;        // k_step's order, when it has more envs than the GPU holds waves: null otherwise
+    uint32_t* queue_list = nullptr;
+    uint32_t queue_first = 0;          // waves of k_step's grid
     uint32_t *sc = nullptr, *ev = nullptr;
     uint8_t* snap_mem = nullptr;     // 2 snapshot slots of the live consoles (early-termination re-emulation)
     uint32_t* snap_sc = nullptr;
@@ -780,14 +773,11 @@ MhEnv* mh_create_roms(const uint8_t* roms, const int64_t* rom_lens, int n_roms, 
     h->snap_sc = B.alloc<uint32_t>((size_t)2 * S_COUNT * h->np, good);
     h->fresh = B.alloc<uint8_t>((size_t)OBS_PIX * h->np, good);
     h->ls = emu_launch(h->n, h->cus);
-    {
-        const EmuLaunch& ls = h->ls;
-        if ((int)ls.grid.x > h->cus && (int)ls.grid.x <= ORDER_MAX) {   // more than one block per CU: the launch order decides what runs last
-            h->n_groups = (int)ls.grid.x;
-            h->grp_work = B.alloc<uint32_t>(h->n_groups, good);
-            h->grp_perm = B.alloc<uint32_t>(h->n_groups, good);
-            h->grp_prev = B.alloc<uint64_t>(h->np, good);
-        }
+    if ((int)h->ls.grid.x > h->cus && h->cus > 0) {
+        h->ls.grid = dim3((unsigned)h->cus);
+        h->queue_first = (uint32_t)h->cus * WAVES_PER_BLOCK;
+        h->queue = B.alloc<StepQueue>(1, good);
+        h->queue_list = B.alloc<uint32_t>((size_t)2 * WORK_BUCKETS * h->np, good);
     }
     h->boot_mem = B.alloc<uint8_t>((size_t)MEM_ROWS * h->nlp, good);
     h->boot_sc = B.alloc<uint32_t>((size_t)S_COUNT * h->nlp, good);
@@ -833,6 +823,16 @@ MhEnv* mh_create_roms(const uint8_t* roms, const int64_t* rom_lens, int n_roms, 
         !ok(hipMemcpy(d_levels, lv.data(), lv.size() * sizeof(int), hipMemcpyHostToDevice), "upload levels") ||
         !ok(hipMemcpy(h->ev, ev.data(), ev.size() * 4, hipMemcpyHostToDevice), "upload env words"))
         return fail();
+    if (h->queue) {   // the first step: every env in one bucket, in slot order
+        std::vector<uint32_t> all(n);
+        for (int i = 0; i < n; i++) all[i] = (uint32_t)i;
+        StepQueue q{};
+        q.next = h->queue_first;
+        q.count[0][0] = (uint32_t)n;
+        if (!ok(hipMemcpy(h->queue_list, all.data(), all.size() * 4, hipMemcpyHostToDevice), "upload step order") ||
+            !ok(hipMemcpy(h->queue, &q, sizeof(q), hipMemcpyHostToDevice), "upload step queue"))
+            return fail();
+    }
     h->R.rom = d_rom; h->R.lut = d_lut; h->R.recs = d_recs; h->R.n_chr = n_roms;
     h->R.nt_bits = 0;
     for (int i = 0; i < 4; i++) h->R.nt_bits |= (nt[i] ? 1u : 0u) << i;
@@ -894,7 +894,7 @@ int mh_reset(MhEnv* h, void* stream) {
     if (!h || !h->obs) { g_err = "buffers not set"; return -1; }
     CK(hipSetDevice(h->device));
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_reset, dim3(h->np / 64), dim3(64), 0, s, h->reset_args(1));
+    hipLaunchKernelGGL(k_reset, dim3(h->np / 64), dim3(64), 0, s, h->reset_args(1), (StepQueue*)nullptr, 0u);
     CK(hipGetLastError());
     launch_stack(h, s, 1);
     CK(hipGetLastError());
@@ -923,18 +923,11 @@ int mh_step_async(MhEnv* h, const int64_t* d_actions, void* stream) {
                 h->rew, h->term, h->trunc, h->info, h->ep_ret, h->ep_len, h->key_bank, h->slot_env, h->fresh,
                 h->boot_obs};
     const EmuLaunch& ls = h->ls;
-    if (h->grp_perm) {   // this step's launch order, from the last step's work
-        hipLaunchKernelGGL(k_work, dim3((unsigned)(h->np / 64)), dim3(64), 0, s, h->ev, h->np, h->n,
-                           h->grp_prev, h->grp_work);
-        hipLaunchKernelGGL(k_order, dim3(1), dim3(1024), 0, s, h->grp_work, h->grp_perm, h->n_groups);
-        hipLaunchKernelGGL(k_step_ordered, ls.grid, ls.block, 0, s, sa, (const uint32_t*)h->grp_perm);
-    } else {
-        hipLaunchKernelGGL(k_step, ls.grid, ls.block, 0, s, sa);
-    }
+    hipLaunchKernelGGL(k_step, ls.grid, ls.block, 0, s, sa, h->queue, h->queue_list);
     CK(hipGetLastError());
     if (mark(h, s, 1)) return -1;
     if (mark(h, s, 2)) return -1;   // (a stage of its own until the observations moved into k_step: empty)
-    hipLaunchKernelGGL(k_reset, dim3(h->np / 64), dim3(64), 0, s, h->reset_args(0));
+    hipLaunchKernelGGL(k_reset, dim3(h->np / 64), dim3(64), 0, s, h->reset_args(0), h->queue, h->queue_first);
     CK(hipGetLastError());
     if (mark(h, s, 3)) return -1;
     launch_stack(h, s, 0);
