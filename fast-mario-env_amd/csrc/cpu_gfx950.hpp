@@ -13,7 +13,8 @@
 //   bits 31-16  operand: the immediate or zero-page byte, the absolute RAM address (& $7FF) or index base, or the
 //               target of a branch, JMP or JSR
 //   bits 15-8   slot (the opcode, or a variant of it): the byte offset of the slot's code is bits 15-0 & $FF00
-//   bits 7-0    for slot 0 only: what the instruction is (REC_*), with its address as the operand, else 0
+//   bits 7-0    for slot 0 only: what the instruction is (REC_*, a multiple of 4: slot 0 is a table of branches to
+//               the end, so that it needs no mask), with its address as the operand, else 0
 // Slot 0 ends the run before the instruction: what is not an official opcode, whose operands are not in PRG, whose
 // static address is a register of the PPU, joypad or DMA, the idle loop `JMP *`, the sprite-0 wait, BRK. Addresses
 // below $8000 have record 0, so a run ends when the program leaves PRG.
@@ -26,10 +27,10 @@ namespace mh {
 
 constexpr uint32_t REC_COUNT = 0x10000 + 16;     // a run that walks off $FFFF reads records 0 there
 constexpr uint32_t REC_IDLE = 0x10u;             // JMP *
-constexpr uint32_t REC_STORE = 0x20u;            // | source (0 A, 1 X, 2 Y): an absolute store to a register
-constexpr uint32_t REC_LOAD = 0x30u;             // | destination (0 A, 1 X, 2 Y, 3 BIT): an absolute load from one
-// the sprite-0 wait: LDA $2002 / AND #$40 / BEQ|BNE back to the LDA (a REC_LOAD to A); | 4: BEQ, waiting for the hit
-constexpr uint32_t REC_POLL = 0x40u;
+constexpr uint32_t REC_STORE = 0x20u;            // | 4 * source (0 A, 1 X, 2 Y): an absolute store to a register
+constexpr uint32_t REC_LOAD = 0x30u;             // | 4 * destination (0 A, 1 X, 2 Y, 3 BIT): an absolute load from one
+// the sprite-0 wait: LDA $2002 / AND #$40 / BEQ|BNE back to the LDA (a REC_LOAD to A); REC_POLL_HIT: BEQ, waiting for the hit
+constexpr uint32_t REC_POLL = 0x40u, REC_POLL_HIT = 0x50u;
 // slots of opcode variants, at opcodes the 6502 does not have
 constexpr uint32_t SLOT_BR_CROSS[8] = {0x12, 0x32, 0x52, 0x72, 0x92, 0xb2, 0xd2, 0xf2};   // branches that cross a page
 constexpr uint32_t SLOT_STORE_IGNORED = 0x0b;    // a 4-cycle store to an address that ignores writes
@@ -82,13 +83,13 @@ inline uint32_t decode_record(const uint8_t* prg, uint32_t pc, const uint32_t* d
         if (op == 0xad && absv == 0x2002u && pc <= 0xfff8u) {
             const uint8_t* q = prg + (pc - 0x8000u);
             if (q[3] == 0x29 && q[4] == 0x40 && (q[5] == 0xf0 || q[5] == 0xd0) && q[6] == 0xf9)
-                return absv << 16 | REC_POLL | (q[5] == 0xf0 ? 4u : 0u);
+                return absv << 16 | (q[5] == 0xf0 ? REC_POLL_HIT : REC_POLL);
         }
-        return absv << 16 | REC_LOAD | dst;
+        return absv << 16 | REC_LOAD | 4u * dst;
     }
     if (!wr) return 0;
     if (absv >= 0x4000u && (absv & ~2u) != 0x4014u) return rec(SLOT_STORE_IGNORED, 0);
-    return absv << 16 | REC_STORE | (op == 0x8d ? 0u : op == 0x8e ? 1u : 2u);
+    return absv << 16 | REC_STORE | (op == 0x8d ? 0u : op == 0x8e ? 4u : 8u);
 }
 inline void decode_prg(const uint8_t* prg, const uint32_t* dec_words, uint32_t* out) {
     for (uint32_t pc = 0; pc < REC_COUNT; pc++) out[pc] = decode_record(prg, pc, dec_words);
@@ -110,40 +111,55 @@ struct ScalarRegs {
 #if defined(__AMDGCN__)
 // The code, once in the device library; scalar_run calls it.
 // Registers: s0 A, s1 X, s2 Y, s3 SP, s4 nz, s5 c, s6 v, s7 p_rest, s8 left, s9 pc4, s10 record, s11 operand,
-// s12 s13 scratch, s[14:15] target, s[16:17] slot 0, s[18:19] records, s20 $10000, s21 $FF00, s22 $FF, s23 $7FF,
-// s24 address, s25 $2000, s26 ram, s27 prg - $8000 (LDS byte offsets), s[28:29] the exec mask, s[30:31] the return;
-// v5 ram, v6 prg - $8000, v7 ram + $100.
+// s12 s13 scratch, s[14:15] target, s16 slot 0 (low half), s[18:19] records, s20 $10000, s22 $FF,
+// s24 address, s25 $800, s26 ram, s27 prg - $8000 (LDS byte offsets), s28 s29 the words of 4 and 5 cycles, s[30:31] the
+// return; v5 ram, v6 prg - $8000, v7 ram + $100.
 // Hazards seen to: a VALU instruction never reads a scalar register that v_readfirstlane wrote last (scalar
-// instructions stand between), and every load is waited for before its register is used, at the end too.
+// instructions stand between) and v_readfirstlane never a vector register that the VALU wrote last; every load is
+// waited for before its register is used, at the end too.
+// What bounds it with the chip full is scalar issue, so a body does its addresses on the vector unit (HDV takes the
+// operand out of the record and adds the base in one v_mad_u32_u16), and dispatch is three scalar instructions and
+// the jump: with the code 64 KB aligned, a slot's address is the record's low half under the code's high half. An
+// LDA from the zero page is 5 scalar instructions and the jump; it was 10 with a mask, an add and a carry for the
+// target. k_step of 256 / 32,768 envs by that: 0.89 -> 0.87 / 8.2 -> 7.75 ms, 121,000 -> 103,000 scalar
+// instructions an env.
+// Indexed addresses past $7FF are not RAM's first image: PRG has its own tail (FAR), a mirror is left to frame().
 // (Device code has no file-scope assembly: the code stands in a function that nothing calls.)
 __device__ __attribute__((used, noinline)) void cpu_code() {
     asm volatile(R"ASM(
 .macro NX cyc                    // the next instruction, after one of cyc cycles
  s_sub_u32 s8, s8, ((\cyc)<<16)-1
- s_cselect_b32 s12, 0, s21
- s_waitcnt lgkmcnt(0)
- s_and_b32 s12, s10, s12
- s_add_u32 s14, s16, s12
- s_addc_u32 s15, s17, 0
- s_setpc_b64 s[14:15]
+ GO
 .endm
 .macro NXK                       // the same with the cycles' word in s13 (PEN)
  s_sub_u32 s8, s8, s13
- s_cselect_b32 s12, 0, s21
+ GO
+.endm
+.macro GO                        // to the record's slot, or the end if scc: the code is 64 KB aligned, slot 0 first
  s_waitcnt lgkmcnt(0)
- s_and_b32 s12, s10, s12
- s_add_u32 s14, s16, s12
- s_addc_u32 s15, s17, 0
+ s_cselect_b32 s12, 0, s10
+ s_pack_lh_b32_b16 s14, s12, s16
  s_setpc_b64 s[14:15]
 .endm
-.macro PEN cyc                   // s13: cyc cycles, one more if s24 (address) is not in s11's (base) page
+.macro PEN cyc                   // s13: the cycles' word, one cycle more if s24 (address) is not in s11's (base) page
  s_xor_b32 s12, s11, s24
  s_bitcmp1_b32 s12, 8
+.if \cyc == 4
+ s_cselect_b32 s13, s29, s28
+.elseif \cyc == 5
+ s_cselect_b32 s13, (6<<16)-1, s29
+.else
  s_cselect_b32 s13, s20, 0
  s_add_u32 s13, s13, ((\cyc)<<16)-1
+.endif
 .endm
 .macro HD len                    // operand to s11; on to the next record
  s_lshr_b32 s11, s10, 16
+ s_add_u32 s9, s9, 4*(\len)
+ s_load_dword s10, s[18:19], s9
+.endm
+.macro HDV len                   // operand + RAM to v0; on to the next record
+ v_mad_u32_u16 v0, s10, 1, v5 op_sel:[1,0,0,0]
  s_add_u32 s9, s9, 4*(\len)
  s_load_dword s10, s[18:19], s9
 .endm
@@ -163,15 +179,14 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
  s_add_u32 s11, s11, \r
  s_and_b32 s11, s11, s22
 .endm
-.macro PTRY                      // (zp),Y: base to s11, address to s24
- v_add_u32 v0, s11, v5
+.macro PTRY len                  // (zp),Y: base to s11, address to s24
+ HDV \len
  ds_read_u8 v1, v0
  ds_read_u8 v2, v0 offset:1
  s_waitcnt lgkmcnt(0)
- v_readfirstlane_b32 s12, v1
- v_readfirstlane_b32 s13, v2
- s_lshl_b32 s13, s13, 8
- s_or_b32 s11, s12, s13
+ v_lshl_or_b32 v1, v2, 8, v1
+ s_nop 0
+ v_readfirstlane_b32 s11, v1
  s_add_u32 s24, s11, s2
 .endm
 .macro PTRX                      // (zp,X): address to s24
@@ -229,9 +244,8 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
  A_ADC
 .endm
 .macro CMPR r
- s_cmp_ge_u32 \r, s11
- s_cselect_b32 s5, 1, 0
  s_sub_u32 s4, \r, s11
+ s_cselect_b32 s5, 0, 1
  s_and_b32 s4, s4, s22
 .endm
 .macro A_CMP
@@ -284,6 +298,88 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
  s_and_b32 \r, \r, s22
  s_mov_b32 s4, \r
 .endm
+// ---- the same on the byte that is being read into v1
+.macro L_LDA
+ s_waitcnt lgkmcnt(0)
+ v_readfirstlane_b32 s0, v1
+ s_mov_b32 s4, s0
+.endm
+.macro L_LDX
+ s_waitcnt lgkmcnt(0)
+ v_readfirstlane_b32 s1, v1
+ s_mov_b32 s4, s1
+.endm
+.macro L_LDY
+ s_waitcnt lgkmcnt(0)
+ v_readfirstlane_b32 s2, v1
+ s_mov_b32 s4, s2
+.endm
+.macro L_ORA
+ GETM
+ A_ORA
+.endm
+.macro L_AND
+ GETM
+ A_AND
+.endm
+.macro L_EOR
+ GETM
+ A_EOR
+.endm
+.macro L_ADC
+ GETM
+ A_ADC
+.endm
+.macro L_SBC
+ GETM
+ A_SBC
+.endm
+.macro L_CMP
+ GETM
+ A_CMP
+.endm
+.macro L_CPX
+ GETM
+ A_CPX
+.endm
+.macro L_CPY
+ GETM
+ A_CPY
+.endm
+.macro L_BIT
+ GETM
+ A_BIT
+.endm
+// ---- read-modify-write of the byte in s11, result to s4
+.macro W_ASL
+ s_lshr_b32 s5, s11, 7
+ s_lshl_b32 s11, s11, 1
+ s_and_b32 s4, s11, s22
+.endm
+.macro W_ROL
+ s_lshl_b32 s12, s11, 1
+ s_or_b32 s12, s12, s5
+ s_lshr_b32 s5, s11, 7
+ s_and_b32 s4, s12, s22
+.endm
+.macro W_LSR
+ s_and_b32 s5, s11, 1
+ s_lshr_b32 s4, s11, 1
+.endm
+.macro W_ROR
+ s_lshl_b32 s12, s5, 7
+ s_and_b32 s5, s11, 1
+ s_lshr_b32 s11, s11, 1
+ s_or_b32 s4, s11, s12
+.endm
+.macro W_INC
+ s_add_u32 s11, s11, 1
+ s_and_b32 s4, s11, s22
+.endm
+.macro W_DEC
+ s_sub_u32 s11, s11, 1
+ s_and_b32 s4, s11, s22
+.endm
 // ---- slots (SLOT n: the code at byte offset 256 n; an overlong one fails to assemble)
 .macro SLOT n
  .org .Lmh_slots + 256*(\n), 0
@@ -298,12 +394,19 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
  A_\op
  NX 2
 .endm
+.macro LDI n, r                  // LDA, LDX, LDY immediate
+ SLOT \n
+ s_lshr_b32 \r, s10, 16
+ s_add_u32 s9, s9, 8
+ s_load_dword s10, s[18:19], s9
+ s_mov_b32 s4, \r
+ NX 2
+.endm
 .macro ZP n, op
  SLOT \n
- HD 2
- LDB
- GETM
- A_\op
+ HDV 2
+ ds_read_u8 v1, v0
+ L_\op
  NX 3
 .endm
 .macro ZPI n, op, r
@@ -311,16 +414,14 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
  HD 2
  IDXZ \r
  LDB
- GETM
- A_\op
+ L_\op
  NX 4
 .endm
 .macro ABS n, op
  SLOT \n
- HD 3
- LDB
- GETM
- A_\op
+ HDV 3
+ ds_read_u8 v1, v0
+ L_\op
  NX 4
 .endm
 .macro ABSI n, op, r             // not RAM: .Lmh_far_n
@@ -329,26 +430,21 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
  s_add_u32 s24, s11, \r
  s_cmp_ge_u32 s24, s25
  s_cbranch_scc1 .Lmh_far_\n
- s_and_b32 s12, s24, s23
- v_add_u32 v0, s12, v5
+ v_add_u32 v0, s24, v5
  ds_read_u8 v1, v0
  PEN 4
- GETM
- A_\op
+ L_\op
  NXK
 .endm
 .macro INDY n, op
  SLOT \n
- HD 2
- PTRY
+ PTRY 2
  s_cmp_ge_u32 s24, s25
  s_cbranch_scc1 .Lmh_far_\n
- s_and_b32 s12, s24, s23
- v_add_u32 v0, s12, v5
+ v_add_u32 v0, s24, v5
  ds_read_u8 v1, v0
  PEN 5
- GETM
- A_\op
+ L_\op
  NXK
 .endm
 .macro INDX n, op
@@ -357,11 +453,9 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
  PTRX
  s_cmp_ge_u32 s24, s25
  s_cbranch_scc1 .Lmh_far_\n
- s_and_b32 s12, s24, s23
- v_add_u32 v0, s12, v5
+ v_add_u32 v0, s24, v5
  ds_read_u8 v1, v0
- GETM
- A_\op
+ L_\op
  NX 6
 .endm
 .macro FAR n, op, cyc, len       // the rest of ABSI / INDY for PRG
@@ -371,8 +465,7 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
  v_add_u32 v0, s24, v6
  ds_read_u8 v1, v0
  PEN \cyc
- GETM
- A_\op
+ L_\op
  NXK
 .endm
 .macro FARX n, op                // of INDX
@@ -381,19 +474,21 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
  s_cbranch_scc0 .Lmh_ref_2
  v_add_u32 v0, s24, v6
  ds_read_u8 v1, v0
- GETM
- A_\op
+ L_\op
  NX 6
 .endm
-.macro PUT r                     // RAM byte s11 = r
- v_add_u32 v0, s11, v5
+.macro PUTV r                    // the byte at v0 = r
  v_mov_b32 v1, \r
  ds_write_b8 v0, v1
 .endm
+.macro PUT r                     // RAM byte s11 = r
+ v_add_u32 v0, s11, v5
+ PUTV \r
+.endm
 .macro STZP n, r
  SLOT \n
- HD 2
- PUT \r
+ HDV 2
+ PUTV \r
  NX 3
 .endm
 .macro STZPI n, r, i
@@ -405,15 +500,15 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
 .endm
 .macro STABS n, r
  SLOT \n
- HD 3
- PUT \r
+ HDV 3
+ PUTV \r
  NX 4
 .endm
 .macro STORE_AT n, cyc           // A to the computed address s24
  s_cmp_ge_u32 s24, s25
  s_cbranch_scc1 .Lmh_far_\n
- s_and_b32 s11, s24, s23
- PUT s0
+ v_add_u32 v0, s24, v5
+ PUTV s0
  NX \cyc
 .endm
 .macro STABSI n, i
@@ -435,15 +530,14 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
 .endm
 .macro RMW_TAIL op, cyc
  GETM
- M_\op s11
- v_mov_b32 v1, s11
- ds_write_b8 v0, v1
+ W_\op
+ PUTV s4
  NX \cyc
 .endm
 .macro RMZP n, op
  SLOT \n
- HD 2
- LDB
+ HDV 2
+ ds_read_u8 v1, v0
  RMW_TAIL \op, 5
 .endm
 .macro RMZPX n, op
@@ -455,8 +549,8 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
 .endm
 .macro RMABS n, op
  SLOT \n
- HD 3
- LDB
+ HDV 3
+ ds_read_u8 v1, v0
  RMW_TAIL \op, 6
 .endm
 .macro RMABSX n, op
@@ -465,14 +559,12 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
  s_add_u32 s24, s11, s1
  s_cmp_ge_u32 s24, s25
  s_cbranch_scc1 .Lmh_ref_3
- s_and_b32 s12, s24, s23
- v_add_u32 v0, s12, v5
+ v_add_u32 v0, s24, v5
  ds_read_u8 v1, v0
  PEN 7
  GETM
- M_\op s11
- v_mov_b32 v1, s11
- ds_write_b8 v0, v1
+ W_\op
+ PUTV s4
  NXK
 .endm
 .macro ACC n, op
@@ -541,12 +633,15 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
  s_and_b32 s12, s4, s22
  BR_TAIL \n, \nt, \cyc
 .endm
+.macro SPDN
+ s_sub_u32 s3, s3, 1
+ s_and_b32 s3, s3, s22
+.endm
 .macro PUSH r                    // RAM byte $100 + SP = r
  v_add_u32 v0, s3, v7
  v_mov_b32 v1, \r
  ds_write_b8 v0, v1
- s_sub_u32 s3, s3, 1
- s_and_b32 s3, s3, s22
+ SPDN
 .endm
 .macro SPUP
  s_add_u32 s3, s3, 1
@@ -563,31 +658,11 @@ __device__ __attribute__((used, noinline)) void cpu_code() {
  s_or_b32 s4, s4, s12
 .endm
 
- .p2align 8
-mh_cpu_run:
- s_mov_b64 s[28:29], exec          // one lane is enough
- s_mov_b64 exec, 1
- s_mov_b32 s20, 0x10000
- s_mov_b32 s21, 0xff00
- s_movk_i32 s22, 0xff
- s_movk_i32 s23, 0x7ff
- s_movk_i32 s25, 0x2000
- s_load_dword s10, s[18:19], s9
- v_mov_b32 v5, s26
- v_mov_b32 v6, s27
- v_add_u32 v7, 0x100, v5
- s_getpc_b64 s[16:17]
-.Lmh_here:
- s_add_u32 s16, s16, .Lmh_slots-.Lmh_here
- s_addc_u32 s17, s17, 0
- s_waitcnt lgkmcnt(0)
- s_and_b32 s12, s10, s21
- s_add_u32 s14, s16, s12
- s_addc_u32 s15, s17, 0
- s_setpc_b64 s[14:15]
- .p2align 8
+ .p2align 16
 .Lmh_slots:
- STOP  0x00
+ .rept 64
+ s_branch .Lmh_exit
+ .endr
  INDX  0x01, ORA
  STOP  0x02
  STOP  0x03
@@ -641,9 +716,14 @@ mh_cpu_run:
  s_lshr_b32 s12, s9, 2
  s_add_u32 s12, s12, 2
  GOTO
- s_lshr_b32 s11, s12, 8
- PUSH s11
- PUSH s12
+ v_mov_b32 v1, s12
+ v_lshrrev_b32 v2, 8, v1
+ v_add_u32 v0, s3, v7
+ ds_write_b8 v0, v2
+ SPDN
+ v_add_u32 v0, s3, v7
+ ds_write_b8 v0, v1
+ SPDN
  NX 6
  INDX  0x21, AND
  STOP  0x22
@@ -754,13 +834,11 @@ mh_cpu_run:
  v_add_u32 v2, s3, v7
  ds_read_u8 v1, v0
  ds_read_u8 v2, v2
- GETM
- v_readfirstlane_b32 s12, v2
- s_lshl_b32 s12, s12, 8
- s_or_b32 s11, s11, s12
- s_add_u32 s11, s11, 1
- s_and_b32 s11, s11, 0xffff
- s_lshl_b32 s9, s11, 2
+ s_waitcnt lgkmcnt(0)
+ v_lshl_or_b32 v1, v2, 8, v1
+ s_nop 0
+ v_readfirstlane_b32 s11, v1
+ s_lshl2_add_u32 s9, s11, 4      // ($FFFF + 1: record 0 there, and its pc is 0)
  s_load_dword s10, s[18:19], s9
  NX 6
  INDX  0x61, ADC
@@ -775,8 +853,7 @@ mh_cpu_run:
  SPUP
  v_add_u32 v0, s3, v7
  ds_read_u8 v1, v0
- GETM
- A_LDA
+ L_LDA
  NX 4
  IMM   0x69, ADC
  ACC   0x6a, ROR
@@ -786,10 +863,10 @@ mh_cpu_run:
  v_add_u32 v0, s11, v5
  ds_read_u8 v1, v0
  ds_read_u8 v2, v0 offset:1
- GETM
- v_readfirstlane_b32 s12, v2
- s_lshl_b32 s12, s12, 8
- s_or_b32 s11, s11, s12
+ s_waitcnt lgkmcnt(0)
+ v_lshl_or_b32 v1, v2, 8, v1
+ s_nop 0
+ v_readfirstlane_b32 s11, v1
  s_lshl_b32 s9, s11, 2
  s_load_dword s10, s[18:19], s9
  NX 5
@@ -833,8 +910,7 @@ mh_cpu_run:
  STOP  0x8f
  BR_C  0x90, 1, 3
  SLOT  0x91                      // STA (zp),Y
- HD 2
- PTRY
+ PTRY 2
  STORE_AT 0x91, 6
  BR_C  0x92, 1, 5
  STOP  0x93
@@ -853,16 +929,16 @@ mh_cpu_run:
  STABSI 0x9d, s1
  STOP  0x9e
  STOP  0x9f
- IMM   0xa0, LDY
+ LDI   0xa0, s2
  INDX  0xa1, LDA
- IMM   0xa2, LDX
+ LDI   0xa2, s1
  STOP  0xa3
  ZP    0xa4, LDY
  ZP    0xa5, LDA
  ZP    0xa6, LDX
  STOP  0xa7
  XFER  0xa8, s2, s0              // TAY
- IMM   0xa9, LDA
+ LDI   0xa9, s0
  XFER  0xaa, s1, s0              // TAX
  STOP  0xab
  ABS   0xac, LDY
@@ -987,6 +1063,24 @@ mh_cpu_run:
  FARST 0x91, 6, 2
  FARST 0x99, 5, 3
  FARST 0x9d, 5, 3
+mh_cpu_run:
+ s_mov_b64 exec, 1                 // one lane is enough
+ s_mov_b32 s20, 0x10000
+ s_movk_i32 s22, 0xff
+ s_movk_i32 s25, 0x800
+ s_mov_b32 s28, (4<<16)-1
+ s_mov_b32 s29, (5<<16)-1
+ s_load_dword s10, s[18:19], s9
+ v_mov_b32 v5, s26
+ v_mov_b32 v6, s27
+ v_add_u32 v7, 0x100, v5
+ s_getpc_b64 s[16:17]
+.Lmh_here:
+ s_sub_u32 s16, s16, .Lmh_here-.Lmh_slots
+ s_subb_u32 s15, s17, 0
+ s_and_b32 s12, s16, 0xffff        // (loaded out of line: nothing runs here, and frame() runs everything itself)
+ s_cbranch_scc1 .Lmh_exit
+ GO
 .Lmh_ref_2:                          // left to frame(): back to the instruction
  s_sub_u32 s9, s9, 8
  s_branch .Lmh_exit
@@ -994,7 +1088,7 @@ mh_cpu_run:
  s_sub_u32 s9, s9, 12
 .Lmh_exit:
  s_waitcnt lgkmcnt(0)
- s_mov_b64 exec, s[28:29]
+ s_mov_b64 exec, -1
  s_setpc_b64 s[30:31]
 )ASM");
 }
@@ -1012,7 +1106,7 @@ __device__ __forceinline__ void scalar_run(ScalarRegs& r, const uint32_t* record
                  : "+{s0}"(r.a), "+{s1}"(r.x), "+{s2}"(r.y), "+{s3}"(r.sp), "+{s4}"(r.nz), "+{s5}"(r.c), "+{s6}"(r.v),
                    "+{s7}"(r.p_rest), "+{s8}"(r.left), "+{s9}"(r.pc4)
                  : "{s[18:19]}"(records), "{s26}"(ram), "{s27}"(prg - 0x8000u)
-                 : "s10", "s11", "s12", "s13", "s14", "s15", "s16", "s17", "s20", "s21", "s22", "s23", "s24", "s25", "s28", "s29", "s30", "s31",
+                 : "s10", "s11", "s12", "s13", "s14", "s15", "s16", "s17", "s20", "s22", "s24", "s25", "s28", "s29", "s30", "s31",
                    "v0", "v1", "v2", "v3", "v5", "v6", "v7", "scc", "memory");
 }
 #endif

@@ -153,8 +153,8 @@ struct StepQueue {
 // the envs of bucket b, side s: list[(s * WORK_BUCKETS + b) * np ..]
 
 // What bounds it: scalar issue. A SIMD issues one scalar instruction per 4 cycles whichever of its waves it is from; the
-// headline step (32,768 envs of 1-1) is 126,000 scalar, 78,000 vector and 19,000 branch instructions per env, of which
-// the 5,217 6502 instructions are about 70,000 scalar ones. Why one console per wave, against 16 per wave in
+// headline step (32,768 envs of 1-1) is 103,000 scalar, 69,000 vector and 16,000 branch instructions per env, of which
+// the 5,217 6502 instructions are about 45,000 scalar ones (scalar issue 77% busy, vector 51%). Why one console per wave, against 16 per wave in
 // lockstep (4 lanes each, every opcode's work as selects, 15 to 12 of 16 consoles active): a lockstep iteration issues
 // ~470 instructions for ~12 6502 instructions but each env waits for all of them; here a 6502 instruction is ~17
 // instructions and nothing waits for another console. Measured (k_step, the same envs): 256 envs 11.6 -> 1.03 ms,

@@ -1333,15 +1333,15 @@ MH_FN File run_frame(File f, Ctx c) {
             const int32_t kk = k1 < k2 ? k1 : k2;
             if (kk > 1) { k.exec_at = j + 3 * (kk - 1); k.zero_skip = 0; continue; }
         } else if (kind >= REC_STORE) {
-            const uint32_t ad = rec >> 16, reg = rec & 3u;
+            const uint32_t ad = rec >> 16, reg = rec >> 2 & 3u;
             const bool st = kind == REC_STORE;
             bool lazy = tgt <= quiet;
             if (!lazy && st && ad < 0x4000u && (ad & 7u) >= 5u && !(f.get(F_PPU_FLAGS) & (PF_SHOW_BG | PF_SHOW_SPR)))
                 lazy = (ad & 7u) != 7u || f.get(S_V) - 0x3effu >= 0x100u;
             if (!lazy && k.ppu_calls < tgt && Core::needs_sync(ad, st)) { want = tgt; continue; }
-            if (kind == REC_POLL) {
+            if (kind >= REC_POLL) {
                 k.close_cpu(f);
-                f = poll_wait(f, c, j, end, rec & 4u);
+                f = poll_wait(f, c, j, end, kind == REC_POLL_HIT);
                 k.open_cpu(f);
                 if (f.get(F_NMI_CALL)) continue;
             }
