@@ -1122,12 +1122,42 @@ struct Core {
         return pstate == ST_VBLANK && !(scanline == 241 && pcyc <= 1) ? ppu_calls + calls_until(-1, 1) : -1;
     }
 
+    // While sprite 0 heads the list of the line being drawn: PPU calls from now up to the one that raises the hit on
+    // the rest of this line or the 7 lines after it (nothing writes to the PPU meanwhile), or else to the first dot past
+    // them. Lane 8 i + k tests pixel k of the sprite on the i-th line. A wait loop read $2002 every 27 dots of these lines
+    // before, with a catch-up, a piece of a line to draw and a status read each: k_step of 256 / 32,768 envs 0.87 -> 0.85 /
+    // 7.75 -> 7.40 ms.
+    __device__ __forceinline__ int32_t calls_to_hit() const {
+        if (show_bg() && show_spr()) {
+            const uint32_t ow = oam_sprite(0);
+            const int sx = (int)(ow >> 24), y0 = (int)(ow & 0xffu), h = long_spr() ? 16 : 8;
+            const int edge = hide_edge_spr() || hide_edge_bg() ? 8 : 0;
+            auto hits = [&](int l) {
+                const int i = l >> 3, px = sx + (l & 7), py = scanline + i, x0 = i ? 0 : pcyc - 1;
+                // its later lists: evaluated at the end of the line before, from sprite 0 on
+                const bool listed = i == 0 || (oam_addr < 4 && (uint32_t)(py - 1 - y0) < (uint32_t)h);
+                if (!listed || py > 239 || px > 255 || px < x0 || px < edge) return false;
+                const uint32_t vp = coarse_x_added(i ? v_lines_on((uint32_t)i) : v, (uint32_t)inc_count(x0, px));
+                return bg_pattern(px, vp) && sprite0_pattern(ow, px, py);
+            };
+            uint64_t b = 0;
+            if constexpr (ON_GPU) b = __ballot(hits((int)lane));
+            else for (int l = 63; l >= 0; l--) b = b << 1 | (uint64_t)hits(l);
+            if (b) {
+                const int l = __builtin_ctzll(b);
+                return calls_until(scanline + (l >> 3), sx + (l & 7) + 1) + 1;
+            }
+        }
+        return calls_until(scanline + 8 < 240 ? scanline + 8 : 240, 1);
+    }
+
     // Exact fast-forward of the sprite-0 wait loops `LDA $2002 / AND #$40 / BEQ|BNE *-5` at pc (BEQ:
     // wait for the hit, BNE: wait for the clear at the pre-render line), with the PPU caught up to the
     // read of the first iteration (at j). Iterations whose $2002 reads provably return the same value
     // are not executed: they would only re-read an unchanged s0hit, clear an already clear vblank flag
     // and set first_write, and the PPU is caught up lazily anyway. The span ends before the first dot
-    // where s0hit could change (sprite 0's first line, or the pre-render clear), before the NMI sync
+    // where s0hit could change (the hit itself on a line that sprite 0 is on, its first line before that, or the
+    // pre-render clear), before the NMI sync
     // point and inside the frame. Returns true if it advanced.
     __device__ __forceinline__ bool poll_skip(int32_t j, int32_t end, bool wait_hit) {
         if (wait_hit == (s0hit != 0)) return false;   // this read ends the loop: run it normally
@@ -1139,10 +1169,10 @@ struct Core {
             // onwards in RENDER, 0 onwards elsewhere) and serve line m + 1 (240: line 0 of the next
             // frame); with OAM, oam_addr and sprite size fixed (the loop writes nothing) sprite 0 can
             // head one only for y0 <= m < y0 + h.
-            if (sprite0_first() && pstate == ST_RENDER) return false;
             const int y0 = (int)(oam_sprite(0) & 0xffu), h = long_spr() ? 16 : 8;
             const int m = pstate == ST_RENDER && scanline > y0 ? scanline : y0;
-            if (m <= 239 && m < y0 + h) limit = ppu_calls + calls_until(m + 1, 1) - 2;
+            if (pstate == ST_RENDER && sprite0_first()) limit = ppu_calls + calls_to_hit();   // on the line being drawn
+            else if (m <= 239 && m < y0 + h) limit = ppu_calls + calls_until(m + 1, 1) - 2;
             else if (y0 <= 238) limit = ppu_calls + calls_until(y0 + 1, 1) - 2;   // next frame
             else limit = 0x7fffffff;
             if (pstate != ST_RENDER && sprite0_first()) {
