@@ -604,6 +604,55 @@ __global__ void __launch_bounds__(256) k_policy_conv(const uint16_t* x, const ui
     }
 }
 
+// ---- generalized advantage estimation (fast_mario_env_amd.rollout.gae): a lane per env, backwards over the T steps.
+// Bound by memory: 17 bytes in and 8 out an env-step, every row read and written once, whole rows of 256 bytes a wave.
+// Few waves run (an env is a serial chain: 512 waves for 32,768 envs), so each keeps GAE_AHEAD steps of loads in flight
+// behind the chain. The float operations and their order are those of the row-by-row form
+//   keep = 1 - s[t+1];  delta = (r[t] + (gamma v[t+1]) keep) - v[t];  a = delta + ((gamma lam) keep) a
+// T 128, 32,768 envs: 20 us (3.6 TB/s of the 4.9 that a large copy reaches); the row-by-row form, 8 launches a row, took 5,700.
+constexpr int GAE_AHEAD = 16;
+__global__ void __launch_bounds__(64) k_gae(const float* __restrict__ rew, const float* __restrict__ val,
+                                            const uint8_t* __restrict__ start, const float* __restrict__ next_val,
+                                            const uint8_t* __restrict__ next_start, int64_t T, int64_t n, float gamma,
+                                            float gamma_lam, float* __restrict__ adv, float* __restrict__ ret) {
+    const int64_t e = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    if (e >= n) return;
+    float nv = next_val[e], ns = next_start[e] ? 1.f : 0.f, last = 0.f;
+    float r[2][GAE_AHEAD], v[2][GAE_AHEAD];
+    uint8_t s[2][GAE_AHEAD];
+    auto load = [&](int64_t t, int b) {         // steps t, t - 1, .. (past the start: step 0, not used)
+#pragma unroll
+        for (int i = 0; i < GAE_AHEAD; i++) {
+            const int64_t at = (t > i ? t - i : 0) * n + e;
+            r[b][i] = rew[at]; v[b][i] = val[at]; s[b][i] = start[at];
+        }
+    };
+    auto run = [&](int64_t t, int b) {
+#pragma unroll
+        for (int i = 0; i < GAE_AHEAD; i++) {
+            if (t < i) return;
+            const float keep = 1.f - ns;
+            const float delta = r[b][i] + gamma * nv * keep - v[b][i];
+            last = delta + gamma_lam * keep * last;
+            adv[(t - i) * n + e] = last;
+            ret[(t - i) * n + e] = last + v[b][i];
+            nv = v[b][i];
+            ns = s[b][i] ? 1.f : 0.f;
+        }
+    };
+    int64_t t = T - 1;
+    load(t, 0);
+    while (t >= 0) {
+        load(t - GAE_AHEAD, 1);
+        run(t, 0);
+        t -= GAE_AHEAD;
+        if (t < 0) break;
+        load(t - GAE_AHEAD, 0);
+        run(t, 1);
+        t -= GAE_AHEAD;
+    }
+}
+
 }  // namespace
 
 // compute units of a device (the emulator kernels' launch shape depends on it)
@@ -1224,6 +1273,23 @@ int mh_policy_conv(const void* d_x, const void* d_w, const void* d_b, void* d_ou
     uint16_t* y = (uint16_t*)d_out;
     if (layer == 2) hipLaunchKernelGGL((k_policy_conv<32, 64, 4, 2, 20, 9>), dim3((unsigned)blocks), dim3(256), 0, s, x, w, b, y, n);
     else hipLaunchKernelGGL((k_policy_conv<64, 64, 3, 1, 9, 7>), dim3((unsigned)blocks), dim3(256), 0, s, x, w, b, y, n);
+    CK(hipGetLastError());
+    return 0;
+}
+
+int mh_gae(const float* rew, const float* val, const uint8_t* start, const float* next_val, const uint8_t* next_start,
+           int64_t T, int64_t n, float gamma, float gamma_lam, float* adv, float* ret, void* stream) {
+    if (!rew || !val || !start || !next_val || !next_start || !adv || !ret || T < 1 || n < 1 || n > ((int64_t)1 << 36)) {
+        g_err = "invalid arguments (T >= 1, 1 <= n <= 2^36)";
+        return -1;
+    }
+    for (const void* p : {(const void*)rew, (const void*)val, (const void*)next_val, (const void*)adv, (const void*)ret})
+        if (((uintptr_t)p) & 3) { g_err = "the float rows must be 4-byte aligned"; return -1; }
+    if (!on_gpu(rew, "rew") || !on_gpu(val, "val") || !on_gpu(start, "start") || !on_gpu(next_val, "next_val") ||
+        !on_gpu(next_start, "next_start") || !on_gpu(adv, "adv") || !on_gpu(ret, "ret"))
+        return -1;
+    hipLaunchKernelGGL(k_gae, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, (hipStream_t)stream, rew, val, start, next_val,
+                       next_start, T, n, gamma, gamma_lam, adv, ret);
     CK(hipGetLastError());
     return 0;
 }

@@ -68,6 +68,7 @@ def lib() -> ctypes.CDLL:
     L.mh_raw_destroy.argtypes = [_P]
     L.mh_resize.argtypes = [_P, _P, _i32, _P]
     L.mh_resize_noalloc.argtypes = [_P, _P, _i32, _P]
+    L.mh_gae.argtypes = [_P, _P, _P, _P, _P, _i64, _i64, ctypes.c_float, ctypes.c_float, _P, _P, _P]
     L.mh_policy_input.argtypes = [_P, _P, _i64, _i32, _P]
     L.mh_policy_conv1.argtypes = [_P, _P, _P, _P, _i64, _P]
     L.mh_policy_conv.argtypes = [_P, _P, _P, _P, _i64, _i32, _P]

@@ -185,12 +185,45 @@ def make_net(n_actions: int = N_ACTIONS, in_ch: int = 4, seed: int = 0, device="
     return net
 
 
+def _gae_kernel_takes(rew, val, start, next_val, next_start, gamma, lam):
+    """Whether mh_gae computes `gae` of these: float32 rows and bool flags on one GPU, (T, N) and (N,), contiguous, plain
+    tensors that nothing records or transforms (autograd, forward-mode tangents, vmap and the like, tracing). The rest
+    takes the row-by-row form, as do empty rollouts."""
+    torch = _torch()
+    ts = (rew, val, start, next_val, next_start)
+    if not all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.layout == torch.strided for t in ts):
+        return False
+    if not rew.is_cuda or rew.dim() != 2 or not all(isinstance(g, (int, float)) for g in (gamma, lam)):
+        return False
+    if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
+        return False
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack():
+        return False
+    if any(torch._C._functorch.is_functorch_wrapped_tensor(t) for t in ts):
+        return False
+    if any(torch.autograd.forward_ad.unpack_dual(t).tangent is not None for t in (rew, val, next_val)):
+        return False
+    T, n = rew.shape
+    return (T > 0 and n > 0 and val.shape == rew.shape == start.shape and next_val.shape == next_start.shape == (n,)
+            and all(t.dtype == torch.float32 for t in (rew, val, next_val))
+            and all(t.dtype == torch.bool for t in (start, next_start))
+            and all(t.device == rew.device and t.is_contiguous() and not t.is_neg() for t in ts))
+
+
 def gae(rew, val, start, next_val, next_start, gamma: float = 0.99, lam: float = 0.95):
     """Advantages and returns (T, N) from rewards, values and episode starts (T, N) plus the bootstrap value and
     start flag of the step after the last: delta_t = r_t + gamma v_{t+1} (1 - s_{t+1}) - v_t,
     A_t = delta_t + gamma lam (1 - s_{t+1}) A_{t+1}."""
     torch = _torch()
     T = rew.shape[0]
+    if _gae_kernel_takes(rew, val, start, next_val, next_start, gamma, lam):
+        from ._native import check, lib
+        with torch.cuda.device(rew.device):
+            adv, ret = torch.empty_like(rew), torch.empty_like(rew)
+            check(lib().mh_gae(rew.data_ptr(), val.data_ptr(), start.data_ptr(), next_val.data_ptr(), next_start.data_ptr(),
+                               T, rew.shape[1], gamma, gamma * lam, adv.data_ptr(), ret.data_ptr(),
+                               torch.cuda.current_stream(rew.device).cuda_stream), "mh_gae")
+        return adv, ret
     adv = torch.zeros_like(rew)
     last = torch.zeros_like(next_val)
     for t in reversed(range(T)):

@@ -182,6 +182,14 @@ int mh_policy_conv1(const uint8_t* d_obs, const void* d_w, const void* d_b, void
  * (channels last), d_b the bf16 bias (64). d_x and d_w 16-byte aligned. */
 int mh_policy_conv(const void* d_x, const void* d_w, const void* d_b, void* d_out, int64_t n, int layer, void* stream);
 
+/* Generalized advantage estimation over T steps of n envs, backwards (ppo/train.py:140-150): rew, val, adv, ret (T, n)
+ * float32 and start (T, n) bytes (0, else the step starts an episode), all contiguous; next_val (n) and next_start (n)
+ * the step after the last. adv[t] = delta + gamma_lam keep adv[t + 1] with keep = 1 - start[t + 1] and
+ * delta = rew[t] + gamma val[t + 1] keep - val[t]; ret = adv + val. adv and ret overlap none of the inputs. Float rows
+ * 4-byte aligned, all memory of the current GPU (device, or pinned host memory); -1 otherwise. */
+int mh_gae(const float* rew, const float* val, const uint8_t* start, const float* next_val, const uint8_t* next_start,
+           int64_t T, int64_t n, float gamma, float gamma_lam, float* adv, float* ret, void* stream);
+
 /* ---- frame-deduplicating replay ring (device storage owned by the caller)
  * The ring of FrameReplay (src/fast_mario_env/replay.py:43-60) for n_envs envs and `capacity` slots each,
  * all device memory, slot s of env e at index e * capacity + s:

@@ -36,3 +36,61 @@ def test_step_queue_edges(extra):
     assert torch.equal(big.canon()[n - m:], parts[1][1].canon())
     for e in (big, parts[0][1], parts[1][1]):
         e.close()
+
+
+def _rollout(T, n, seed):
+    g = torch.Generator().manual_seed(seed)
+    rew, val = torch.randn(T, n, generator=g), torch.randn(T, n, generator=g) * 10
+    start, cut = torch.rand(T, n, generator=g) < 0.1, torch.rand(n, generator=g) < 0.5
+    val[-1, 0] = float("inf")             # a product of the recurrence, as in its row-by-row form: inf * 0 is NaN
+    return rew, val, start, torch.randn(n, generator=g), cut
+
+
+@pytest.mark.parametrize("T,n", [(1, 1), (15, 63), (16, 64), (17, 65), (33, 1000), (128, 257)])
+def test_gae_kernel_is_the_row_by_row_form(T, n):
+    """The kernel at the edges of its blocks of steps and envs, bit for bit the row-by-row form on the CPU (the same
+    float32 operations in the same order); twice from a captured graph."""
+    from fast_mario_env_amd.rollout import gae
+    host = _rollout(T, n, T)
+    dev = [x.cuda() for x in host]
+    want = gae(*host)
+    for a, b in zip(gae(*dev), want):
+        assert torch.equal(a.cpu().nan_to_num(7e30), b.nan_to_num(7e30))
+        assert torch.equal(a.cpu().isnan(), b.isnan())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = gae(*dev)
+    for k in range(3):
+        dev[0].add_(1.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(out, gae(*[x.cpu() for x in dev])):
+            assert torch.equal(a.cpu().nan_to_num(7e30), b.nan_to_num(7e30)), k
+
+
+def test_gae_calls_the_kernel_does_not_take():
+    """Other strides, types, gradients, vmap and empty rollouts keep the row-by-row form and its results."""
+    from fast_mario_env_amd import rollout
+    host = _rollout(5, 40, 3)
+    host[1][-1, 0] = 1.0
+    dev = [x.cuda() for x in host]
+    want = rollout.gae(*host)
+    def same(got, rel=1e-6):
+        for a, b in zip(got, want):
+            assert torch.allclose(a.detach().cpu().float(), b, rtol=rel, atol=rel * 40)
+    assert rollout._gae_kernel_takes(*dev, 0.99, 0.95)
+    strided = [x.t().contiguous().t() if x.dim() == 2 else x for x in dev]
+    wide = [x.double() if x.is_floating_point() else x for x in dev]
+    flags = [x.float() if x.dtype == torch.bool else x for x in dev]
+    for other in (strided, wide, flags):
+        assert not rollout._gae_kernel_takes(*other, 0.99, 0.95)
+        same(rollout.gae(*other))
+    g = [x.clone().requires_grad_() if x.is_floating_point() else x for x in dev]
+    out = rollout.gae(*g)
+    same(out)
+    out[0].sum().backward()
+    assert g[0].grad is not None and g[3].grad is not None
+    adv, ret = torch.vmap(rollout.gae, in_dims=(0, None, None, None, None), out_dims=0)(torch.stack([dev[0]] * 2), *dev[1:])
+    same((adv[1], ret[1]))
+    e = rollout.gae(*[x[:0] if x.dim() == 2 else x for x in dev])
+    assert e[0].shape == (0, 40)
