@@ -456,153 +456,151 @@ __global__ void __launch_bounds__(256) k_policy_input_k1(const uint8_t* obs, uin
     out[2 * t + 1] = bf16_rne((float)((v >> 16) & 0xffu) * s) | bf16_rne((float)(v >> 24) * s) << 16;
 }
 
-// ---- the PPO policy's first convolution (Nature CNN: 4 -> 32 channels, 8x8 kernel, stride 4, 84x84 -> 20x20)
-// fused with the input scaling, the bias and the ReLU, on the matrix cores: relu(conv(bf16(obs / 255), W) + b)
-// as an implicit GEMM, M = output pixels, N = 32 channels, K = 4 x 8 x 8 = 256 in the weight's own (ci, kh, kw)
-// order, one v_mfma_f32_32x32x16_bf16 per 16 of K with float32 accumulation.
-// A wave holds the whole weight matrix in registers (lane l: output channel l % 32, k = 16 s + 8 (l / 32) ..
-// + 7 of step s) and walks tiles of 32 output pixels: lane l's A operand of step s is input row 4 oy + kh of
-// channel ci, columns 4 ox .. 4 ox + 7 (two aligned u32 loads of 4 pixels) for pixel l % 32 of the tile,
-// scaled to bf16 as mh_policy_input scales it. Output: the (n, 32, 20, 20) bf16 tensor in channels-last memory
-// (pixel m's 32 channels at m * 32 ..), written as bf16(relu(acc + b)).
+// ---- the PPO policy's convolutions on the matrix cores (Nature CNN: 4 -> 32 channels 8x8 stride 4, 84x84 -> 20x20;
+// 32 -> 64 4x4 stride 2, 20x20 -> 9x9; 64 -> 64 3x3 stride 1, 9x9 -> 7x7), each an implicit GEMM with float32
+// accumulation, its bias and its ReLU; activations bf16 in channels-last memory (pixel m's channels at m * C ..).
+// A block stages whole images in LDS and a wave's tiles of 32 output pixels read their patches from there: a patch
+// read from global memory touches a cache line per pixel (64 lines for the 1 KB of one MFMA step), and every input
+// pixel is in 4 (9 in the third layer) patches of two waves, which is what bounded the kernels without staging. The
+// weights stay in registers (lane l: output channel l % 32, K = 16 s + 8 (l / 32) .. + 7 of step s of
+// v_mfma_f32_32x32x16_bf16); they are the first operand, so that a lane ends up with its pixel's channels
+// 8 q + 4 (l / 32) .. + 3, q = 0 .. 3, and stores them 8 bytes at a time. The next images' loads are in flight while
+// these compute. 32,768 images, before -> now (reading and writing the activations alone at a copy's 4.9 TB/s): first layer
+// 600 -> 430 us (360), second 600 -> 260 (240), third 430 -> 148 (110).
 typedef __bf16 mh_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float mh_f32x16 __attribute__((ext_vector_type(16)));
-constexpr int CONV1_OUT = 20 * 20;   // output pixels per image
-__global__ void __launch_bounds__(256) k_policy_conv1(const uint8_t* obs, const uint16_t* w, const uint16_t* bias,
-                                                      uint16_t* out, int64_t n) {
-    const int l = threadIdx.x & 63;
-    const int j = l & 31, kg = l >> 5;
-    // B operand of the 16 steps: W[j][16 s + 8 kg .. + 7] (OIHW, K = ci * 64 + kh * 8 + kw)
-    mh_bf16x8 wb[16];
+__device__ __forceinline__ mh_bf16x8 as_bf16x8(mh_u32x4 q) { return __builtin_bit_cast(mh_bf16x8, q); }
+// a lane's 16 sums (its pixel's channels) + bias, ReLU, bf16, to out (the pixel's first channel of these 32, + 4 kg);
+// wide: out is 8-byte aligned
+__device__ __forceinline__ void conv_out(const mh_f32x16& acc, const float (&bias)[16], uint16_t* out, bool wide) {
 #pragma unroll
-    for (int s = 0; s < 16; s++) {
-        const uint4 q = *(const uint4*)(w + (size_t)j * 256 + 16 * s + 8 * kg);
-        const uint32_t q4[4] = {q.x, q.y, q.z, q.w};
+    for (int q = 0; q < 4; q++) {
+        uint32_t h[4];
 #pragma unroll
-        for (int e = 0; e < 8; e++) wb[s][e] = __builtin_bit_cast(__bf16, (uint16_t)(q4[e >> 1] >> (16 * (e & 1))));
-    }
-    const float bj = __uint_as_float((uint32_t)bias[j] << 16);
-    const float sc = (float)(1.0 / 255.0);
-    const int64_t M = n * CONV1_OUT, tiles = (M + 31) / 32;
-    const int64_t wave = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 6, waves = (int64_t)gridDim.x * 4;
-    for (int64_t t = wave; t < tiles; t += waves) {
-        // this lane's A pixel: row l % 32 of the tile (clamped to the last pixel past the end; not stored)
-        int64_t m = t * 32 + j;
-        if (m >= M) m = M - 1;
-        const int64_t b = m / CONV1_OUT;
-        const int p = (int)(m - b * CONV1_OUT), oy = p / 20, ox = p - oy * 20;
-        const uint8_t* img = obs + (size_t)b * 4 * OBS_PIX + (size_t)(4 * oy) * 84 + 4 * ox;
-        uint32_t raw[16][2];
-#pragma unroll
-        for (int s = 0; s < 16; s++) {
-            const int k0 = 16 * s + 8 * kg, ci = k0 >> 6, kh = (k0 >> 3) & 7;
-            const uint32_t* r = (const uint32_t*)(img + (size_t)ci * OBS_PIX + kh * 84);
-            raw[s][0] = r[0];
-            raw[s][1] = r[1];
+        for (int i = 0; i < 4; i++) {
+            const float r = acc[4 * q + i] + bias[4 * q + i];
+            h[i] = __builtin_bit_cast(uint16_t, (__bf16)(r > 0.f ? r : 0.f));   // to nearest even
         }
-        mh_f32x16 acc = {};
-#pragma unroll
-        for (int s = 0; s < 16; s++) {
-            mh_bf16x8 a;
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const uint32_t v = (raw[s][e >> 2] >> (8 * (e & 3))) & 0xffu;
-                a[e] = __builtin_bit_cast(__bf16, (uint16_t)bf16_rne((float)v * sc));
-            }
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, wb[s], acc, 0, 0, 0);
-        }
-        // D: register v holds output pixel 8 (v / 4) + 4 kg + v % 4 of the tile, channel j
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int64_t mo = t * 32 + 8 * (v >> 2) + 4 * kg + (v & 3);
-            if (mo < M) {
-                const float y = acc[v] + bj;
-                out[(size_t)mo * 32 + j] = (uint16_t)bf16_rne(y > 0.f ? y : 0.f);
-            }
-        }
+        if (wide) *(uint2*)(out + 8 * q) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+        else
+            for (int i = 0; i < 4; i++) out[8 * q + i] = (uint16_t)h[i];
     }
 }
 
-// ---- the PPO policy's second and third convolutions (Nature CNN: 32 -> 64 channels 4x4 stride 2, 20x20 -> 9x9;
-// 64 -> 64 channels 3x3 stride 1, 9x9 -> 7x7), each fused with its bias and ReLU, on the matrix cores. Input and
-// output are bf16 in channels-last memory (pixel m's channels at m * C ..), the weight is (CO, KS, KS, CI)
-// (channels last), so K = (kh, kw, ci) and lane l's A operand of a step is 8 consecutive input channels of one
-// input pixel (one 16-byte load). A wave holds one half of the output channels' weights in registers (lane l:
-// channel 32 h + l % 32, K = 16 s + 8 (l / 32) .. + 7 of step s) and walks tiles of 32 output pixels; the two
-// halves are the block's even and odd waves. Output: bf16(relu(sum + b)) with float32 accumulation.
-template <int CI, int CO, int KS, int ST, int HI, int HO>
-__global__ void __launch_bounds__(256) k_policy_conv(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
-                                                     uint16_t* y, int64_t n) {
-    static_assert(CI % 8 == 0 && CO == 64, "8-channel loads, two 32-channel halves");
-    constexpr int K = KS * KS * CI, STEPS = K / 16, PIX = HO * HO;
-    static_assert(K % 16 == 0, "whole MFMA steps");
-    const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int j = l & 31, kg = l >> 5, half = wv & 1;
-    const int ch = 32 * half + j;
-    mh_bf16x8 wb[STEPS];
+// The first layer, with the input scaled as mh_policy_input scales it: K = 4 x 8 x 8 in the weight's own (ci, kh, kw)
+// order. An image is 56,448 bytes of bf16 in LDS, scaled once (2.5 vector instructions a pixel; scaled per patch, 7 a
+// patch element, it bounded the layer). A wave has all 32 channels and every fourth tile.
+constexpr int CONV1_OUT = 20 * 20;   // output pixels per image
+__global__ void __launch_bounds__(256, 2) k_policy_conv1(const uint8_t* obs, const uint16_t* w, const uint16_t* bias,
+                                                         uint16_t* out, int64_t n, int wide) {
+    constexpr int WORDS = 4 * OBS_PIX / 4, PER = (WORDS + 255) / 256;   // 4-pixel words an image, a thread
+    __shared__ __attribute__((aligned(16))) uint16_t s_x[4 * OBS_PIX];
+    const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6, j = l & 31, kg = l >> 5;
+    mh_bf16x8 wb[16];
 #pragma unroll
-    for (int s = 0; s < STEPS; s++) {
-        const uint4 q = *(const uint4*)(w + (size_t)ch * K + 16 * s + 8 * kg);
-        const uint32_t q4[4] = {q.x, q.y, q.z, q.w};
+    for (int s = 0; s < 16; s++) wb[s] = as_bf16x8(*(const mh_u32x4*)(w + (size_t)j * 256 + 16 * s + 8 * kg));
+    float bj[16];
 #pragma unroll
-        for (int e = 0; e < 8; e++) wb[s][e] = __builtin_bit_cast(__bf16, (uint16_t)(q4[e >> 1] >> (16 * (e & 1))));
-    }
-    const float bj = __uint_as_float((uint32_t)bias[ch] << 16);
-    const int64_t M = n * PIX, tiles = (M + 31) / 32;
-    const int64_t pair = (int64_t)blockIdx.x * 2 + (wv >> 1), pairs = (int64_t)gridDim.x * 2;
-    // this lane's input pixel of tile t (past the end: a valid pixel, not stored)
-    auto pixel = [&](int64_t t) {
-        int64_t m = t * 32 + j;
-        if (m >= M) m = M - 1;
-        const int64_t b = m / PIX;
-        const int p = (int)(m - b * PIX), oy = p / HO, ox = p - oy * HO;
-        return x + ((size_t)(b * HI + ST * oy) * HI + ST * ox) * CI;
-    };
-    // the A operands of steps c .. c + CH - 1: 16-byte loads issued a chunk ahead of their MFMAs
-    constexpr int CH = STEPS % 8 == 0 ? 8 : 6, NCH = STEPS / CH;
-    static_assert(STEPS % CH == 0, "whole chunks");
-    auto load_chunk = [&](const uint16_t* px, int c, uint4 (&q)[CH]) {
+    for (int v = 0; v < 16; v++) bj[v] = __uint_as_float((uint32_t)bias[8 * (v >> 2) + 4 * kg + (v & 3)] << 16);
+    const float sc = (float)(1.0 / 255.0);
+    uint32_t raw[PER];
+    auto load = [&](int64_t b) {
+        const uint32_t* src = (const uint32_t*)(obs + (size_t)b * 4 * OBS_PIX);
 #pragma unroll
-        for (int i = 0; i < CH; i++) {
-            const int k0 = 16 * (CH * c + i) + 8 * kg, kh = k0 / (KS * CI), kw = (k0 / CI) % KS, ci = k0 % CI;
-            q[i] = *(const uint4*)(px + ((size_t)kh * HI + kw) * CI + ci);
+        for (int i = 0; i < PER; i++) {
+            const int c = tid + 256 * i;
+            raw[i] = src[c < WORDS ? c : 0];
         }
     };
-    uint4 qa[CH], qb[CH];
-    const uint16_t* px = pixel(pair);
-    if (pair < tiles) load_chunk(px, 0, qa);
-    for (int64_t t = pair; t < tiles; t += pairs) {
-        mh_f32x16 acc = {};
+    int64_t b = blockIdx.x;
+    if (b < n) load(b);
+    for (; b < n; b += gridDim.x) {
 #pragma unroll
-        for (int c = 0; c < NCH; c++) {
-            uint4 (&cur)[CH] = (c & 1) ? qb : qa;
-            uint4 (&nxt)[CH] = (c & 1) ? qa : qb;
-            if (c + 1 < NCH) load_chunk(px, c + 1, nxt);
-            else if (t + pairs < tiles) load_chunk(pixel(t + pairs), 0, nxt);   // the next tile's first chunk
+        for (int i = 0; i < PER; i++) {
+            const int c = tid + 256 * i;
+            uint32_t h[4];
 #pragma unroll
-            for (int i = 0; i < CH; i++) {
-                const uint32_t q4[4] = {cur[i].x, cur[i].y, cur[i].z, cur[i].w};
-                mh_bf16x8 a;
+            for (int e = 0; e < 4; e++) h[e] = __builtin_bit_cast(uint16_t, (__bf16)((float)((raw[i] >> (8 * e)) & 0xffu) * sc));
+            if (c < WORDS) *(uint2*)(s_x + 4 * c) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+        }
+        __syncthreads();
+        if (b + gridDim.x < n) load(b + gridDim.x);
+        for (int t = wv; t * 32 < CONV1_OUT; t += 4) {
+            const int m = t * 32 + j, p = m < CONV1_OUT ? m : CONV1_OUT - 1, oy = p / 20, ox = p - oy * 20;
+            const uint16_t* at = s_x + (4 * oy + kg) * 84 + 4 * ox;
+            mh_f32x16 acc = {};
 #pragma unroll
-                for (int e = 0; e < 8; e++) a[e] = __builtin_bit_cast(__bf16, (uint16_t)(q4[e >> 1] >> (16 * (e & 1))));
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, wb[CH * c + i], acc, 0, 0, 0);
+            for (int s = 0; s < 16; s++) {   // K = 16 s + 8 kg ..: channel s / 4, rows 2 (s % 4) + kg
+                const uint2* r = (const uint2*)(at + (s >> 2) * OBS_PIX + 2 * (s & 3) * 84);
+                const uint2 a = r[0], c = r[1];
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wb[s], as_bf16x8(mh_u32x4{a.x, a.y, c.x, c.y}), acc, 0, 0, 0);
             }
+            if (m < CONV1_OUT) conv_out(acc, bj, out + ((size_t)b * CONV1_OUT + m) * 32 + 4 * kg, wide);
         }
-        if constexpr (NCH & 1) {   // the next tile's first chunk landed in qb: move it to qa
-#pragma unroll
-            for (int i = 0; i < CH; i++) qa[i] = qb[i];
-        }
-        if (t + pairs < tiles) px = pixel(t + pairs);
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int64_t mo = t * 32 + 8 * (v >> 2) + 4 * kg + (v & 3);
-            if (mo < M) {
-                const float r = acc[v] + bj;
-                y[(size_t)mo * CO + ch] = (uint16_t)bf16_rne(r > 0.f ? r : 0.f);
-            }
-        }
+        __syncthreads();
     }
 }
+
+// The second and third layers: the weight is (64, KS, KS, CI), so K = (kh, kw, ci) and a step is 16 channels of one
+// input pixel. IMGS images at a time: their output pixels in one row of tiles, the even and odd waves the two halves of
+// the output channels, the block's two pairs of waves every second tile. A pixel takes 16 bytes more than its
+// channels in LDS, so that the 8 lanes of a 16-byte read are in different banks.
+template <int CI, int KS, int ST, int HI, int HO, int IMGS>
+__global__ void __launch_bounds__(256, 2) k_policy_conv(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
+                                                        uint16_t* y, int64_t n, int wide) {
+    constexpr int CO = 64, K = KS * KS * CI, STEPS = K / 16, PIX = HO * HO, INP = HI * HI, PXW = CI + 8;
+    constexpr int PARTS = CI / 8, CHUNKS = IMGS * INP * PARTS, PER = (CHUNKS + 255) / 256;   // 16-byte pieces
+    static_assert(CI % 16 == 0, "whole MFMA steps");
+    __shared__ __attribute__((aligned(16))) uint16_t s_x[IMGS * INP * PXW];
+    const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6, j = l & 31, kg = l >> 5, half = wv & 1;
+    mh_bf16x8 wb[STEPS];
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) wb[s] = as_bf16x8(*(const mh_u32x4*)(w + (size_t)(32 * half + j) * K + 16 * s + 8 * kg));
+    float bj[16];
+#pragma unroll
+    for (int v = 0; v < 16; v++) bj[v] = __uint_as_float((uint32_t)bias[32 * half + 8 * (v >> 2) + 4 * kg + (v & 3)] << 16);
+    const int64_t groups = (n + IMGS - 1) / IMGS;
+    auto images = [&](int64_t g) { return n - g * IMGS < IMGS ? (int)(n - g * IMGS) : IMGS; };
+    mh_u32x4 raw[PER];
+    auto load = [&](int64_t g) {
+        const mh_u32x4* src = (const mh_u32x4*)(x + (size_t)g * IMGS * INP * CI);
+        const int last = images(g) * INP * PARTS - 1;
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const int c = tid + 256 * i;
+            raw[i] = src[c < last ? c : last];
+        }
+    };
+    int64_t g = blockIdx.x;
+    if (g < groups) load(g);
+    for (; g < groups; g += gridDim.x) {
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const int c = tid + 256 * i;
+            if (c < CHUNKS) *(mh_u32x4*)(s_x + (c / PARTS) * PXW + 8 * (c % PARTS)) = raw[i];
+        }
+        __syncthreads();
+        const int pixels = images(g) * PIX;
+        if (g + gridDim.x < groups) load(g + gridDim.x);
+        for (int t = wv >> 1; t * 32 < pixels; t += 2) {
+            const int m = t * 32 + j, q = m < pixels ? m : pixels - 1;
+            const int b = q / PIX, p = q - b * PIX, oy = p / HO, ox = p - oy * HO;
+            const uint16_t* at = s_x + (b * INP + ST * oy * HI + ST * ox) * PXW + 8 * kg;
+            mh_f32x16 acc = {};
+#pragma unroll
+            for (int s = 0; s < STEPS; s++) {
+                const int k0 = 16 * s, kh = k0 / (KS * CI), kw = (k0 / CI) % KS, ci = k0 % CI;
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    wb[s], as_bf16x8(*(const mh_u32x4*)(at + (kh * HI + kw) * PXW + ci)), acc, 0, 0, 0);
+            }
+            if (m < pixels) conv_out(acc, bj, y + ((size_t)g * IMGS * PIX + m) * CO + 32 * half + 4 * kg, wide);
+        }
+        __syncthreads();
+    }
+}
+// images a block takes at a time in the second and third layers once that leaves every CU a block: 162 pixels are 6
+// tiles, 245 are 8 (one image is 81 and 49: 3 and 2)
+constexpr int CONV2_IMGS = 2, CONV3_IMGS = 5;
 
 // ---- generalized advantage estimation (fast_mario_env_amd.rollout.gae): a lane per env, backwards over the T steps.
 // Bound by memory: 17 bytes in and 8 out an env-step, every row read and written once, whole rows of 256 bytes a wave.
@@ -1245,10 +1243,9 @@ int mh_policy_conv1(const uint8_t* d_obs, const void* d_w, const void* d_b, void
     int dev = 0, cus = 0;
     CK(hipGetDevice(&dev));
     CK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const int64_t tiles = (n * CONV1_OUT + 31) / 32;
-    const int64_t blocks = std::min<int64_t>((tiles + 3) / 4, (int64_t)cus * 8);   // persistent: tiles per wave
+    const int64_t blocks = std::min<int64_t>(n, (int64_t)std::max(cus, 1) * 2);   // what a CU holds: 2
     hipLaunchKernelGGL(k_policy_conv1, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, d_obs,
-                       (const uint16_t*)d_w, (const uint16_t*)d_b, (uint16_t*)d_out, n);
+                       (const uint16_t*)d_w, (const uint16_t*)d_b, (uint16_t*)d_out, n, (((uintptr_t)d_out) & 7) == 0);
     CK(hipGetLastError());
     return 0;
 }
@@ -1266,13 +1263,19 @@ int mh_policy_conv(const void* d_x, const void* d_w, const void* d_b, void* d_ou
     int dev = 0, cus = 0;
     CK(hipGetDevice(&dev));
     CK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const int64_t pix = layer == 2 ? 81 : 49, tiles = (n * pix + 31) / 32;
-    const int64_t blocks = std::min<int64_t>((tiles + 1) / 2, (int64_t)cus * 8);   // 2 tiles in flight per block
+    cus = std::max(cus, 1);
     hipStream_t s = (hipStream_t)stream;
     const uint16_t *x = (const uint16_t*)d_x, *w = (const uint16_t*)d_w, *b = (const uint16_t*)d_b;
     uint16_t* y = (uint16_t*)d_out;
-    if (layer == 2) hipLaunchKernelGGL((k_policy_conv<32, 64, 4, 2, 20, 9>), dim3((unsigned)blocks), dim3(256), 0, s, x, w, b, y, n);
-    else hipLaunchKernelGGL((k_policy_conv<64, 64, 3, 1, 9, 7>), dim3((unsigned)blocks), dim3(256), 0, s, x, w, b, y, n);
+    const int wide = (((uintptr_t)d_out) & 7) == 0;
+    auto run = [&](auto kernel, int images) {   // 2 blocks a CU
+        const int64_t blocks = std::min<int64_t>((n + images - 1) / images, (int64_t)cus * 2);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, x, w, b, y, n, wide);
+    };
+    if (layer == 2 && n >= (int64_t)cus * CONV2_IMGS) run(k_policy_conv<32, 4, 2, 20, 9, CONV2_IMGS>, CONV2_IMGS);
+    else if (layer == 2) run(k_policy_conv<32, 4, 2, 20, 9, 1>, 1);
+    else if (n >= (int64_t)cus * CONV3_IMGS) run(k_policy_conv<64, 3, 1, 9, 7, CONV3_IMGS>, CONV3_IMGS);
+    else run(k_policy_conv<64, 3, 1, 9, 7, 1>, 1);
     CK(hipGetLastError());
     return 0;
 }

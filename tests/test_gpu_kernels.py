@@ -94,3 +94,36 @@ def test_gae_calls_the_kernel_does_not_take():
     same((adv[1], ret[1]))
     e = rollout.gae(*[x[:0] if x.dim() == 2 else x for x in dev])
     assert e[0].shape == (0, 40)
+
+
+@pytest.mark.parametrize("extra", [-1, 0, 1, 3])
+@pytest.mark.parametrize("layer", [1, 2, 3])
+def test_policy_conv_batch_edges(layer, extra):
+    """Each layer around the batch where a block starts taking several images (two or five per CU), and past what the
+    blocks take in one turn: an image's activations are the bits that it has in a batch of its own (the same sums in the
+    same order), also into an output that is aligned to 2 bytes only."""
+    from fast_mario_env_amd._native import check, lib
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    n = {1: 2, 2: 2, 3: 5}[layer] * cus + extra
+    ci, hi, co, ho, k = {1: (4, 84, 32, 20, 8), 2: (32, 20, 64, 9, 4), 3: (64, 9, 64, 7, 3)}[layer]
+    g = torch.Generator(device="cuda").manual_seed(layer)
+    w = (torch.randn(co, k * k * ci, generator=g, device="cuda") * 0.05).to(torch.bfloat16)
+    b = torch.randn(co, generator=g, device="cuda").to(torch.bfloat16)
+    if layer == 1:
+        x = torch.randint(0, 256, (n, ci, hi, hi), dtype=torch.uint8, device="cuda", generator=g)
+    else:
+        x = torch.randn(n, hi, hi, ci, generator=g, device="cuda").to(torch.bfloat16)
+
+    def conv(x, out):
+        args = (x.data_ptr(), w.data_ptr(), b.data_ptr(), out.data_ptr(), x.shape[0])
+        check(lib().mh_policy_conv1(*args, 0) if layer == 1 else lib().mh_policy_conv(*args, layer, 0), "conv")
+        torch.cuda.synchronize()
+        return out
+
+    size = ho * ho * co
+    y = conv(x, torch.zeros(n, size, dtype=torch.bfloat16, device="cuda"))
+    for i in (0, 1, n // 2, n - 2, n - 1):
+        one = conv(x[i:i + 1].clone(), torch.zeros(size, dtype=torch.bfloat16, device="cuda"))
+        assert torch.equal(one, y[i]), i
+    odd = torch.zeros(n * size + 2, dtype=torch.bfloat16, device="cuda")
+    assert torch.equal(conv(x, odd[1:-1]).view(n, size), y) and odd[0] == 0 and odd[-1] == 0
