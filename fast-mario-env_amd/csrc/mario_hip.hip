@@ -602,6 +602,103 @@ __global__ void __launch_bounds__(256, 2) k_policy_conv(const uint16_t* x, const
 // tiles, 245 are 8 (one image is 81 and 49: 3 and 2)
 constexpr int CONV2_IMGS = 2, CONV3_IMGS = 5;
 
+// ---- the network's float32 parameters as the bf16 operands of a forward pass, in one launch: the first layer's weight
+// as (co, ci, kh, kw), the others' as (co, kh, kw, ci), the fully connected one's columns from (c, h, w) to (h, w, c)
+// order, and the biases. Bound by memory (6.7 MB in, 3.4 out); what it saves is launches: a small batch's pass spends
+// its time on them, and these were 12 of 21 (casts and permutes): with it and k_policy_heads a pass is 6, and a pass over
+// 300 observations takes 101 us instead of 197 (of it 8 for this). A row of the fully connected weight goes through LDS,
+// so that it is read and written whole.
+struct PackArgs {
+    const float* w[3]; int64_t st[3][4];   // convolution weights and their strides (co, ci, kh, kw)
+    const float* b[4];                     // biases
+    const float* fc;                       // (512, 3136) contiguous
+    uint16_t* out;
+};
+constexpr int PACK_W[4] = {0, 8192, 40960, 77824};          // the convolutions' weights in out; then the biases,
+constexpr int PACK_B[5] = {77824, 77856, 77920, 77984, 78496}, PACK_FC = 78496, FC_IN = 64 * 49, FC_OUT = 512;
+static_assert(PACK_FC + FC_OUT * FC_IN == MH_POLICY_PACKED, "the header's size");
+constexpr int PACK_SMALL = (PACK_FC + 255) / 256;           // blocks of the small ones, after a block per row of fc
+__global__ void __launch_bounds__(256) k_policy_pack(PackArgs A) {
+    __shared__ float row[FC_IN];
+    const int tid = threadIdx.x;
+    auto half = [](float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); };   // to nearest even
+    if (blockIdx.x < FC_OUT) {
+        const float* src = A.fc + (size_t)blockIdx.x * FC_IN;
+        for (int i = tid; i < FC_IN; i += 256) row[i] = src[i];
+        __syncthreads();
+        uint32_t* dst = (uint32_t*)(A.out + PACK_FC + (size_t)blockIdx.x * FC_IN);
+        for (int i = tid; i < FC_IN / 2; i += 256) {   // channels c, c + 1 of pixel p
+            const int p = i >> 5, c = 2 * (i & 31);
+            dst[i] = half(row[c * 49 + p]) | (uint32_t)half(row[(c + 1) * 49 + p]) << 16;
+        }
+        return;
+    }
+    const int i = (int)(blockIdx.x - FC_OUT) * 256 + tid;
+    if (i >= PACK_FC) return;
+    float f;
+    if (i >= PACK_B[0]) {
+        int k = 0;
+        while (i >= PACK_B[k + 1]) k++;
+        f = A.b[k][i - PACK_B[k]];
+    } else {
+        const int k = i < PACK_W[1] ? 0 : i < PACK_W[2] ? 1 : 2, e = i - PACK_W[k];
+        int co, ci, kh, kw;
+        if (k == 0) { co = e >> 8; ci = e >> 6 & 3; kh = e >> 3 & 7; kw = e & 7; }
+        else if (k == 1) { co = e >> 9; kh = e >> 7 & 3; kw = e >> 5 & 3; ci = e & 31; }
+        else { co = e / 576; const int r = e - co * 576; kh = r / 192; kw = r / 64 - 3 * kh; ci = r & 63; }
+        f = A.w[k][co * A.st[k][0] + ci * A.st[k][1] + kh * A.st[k][2] + kw * A.st[k][3]];
+    }
+    A.out[i] = half(f);
+}
+
+// ---- the two heads: logits and value of relu(h), h the bf16 (n, 512) output of the fully connected layer, in float32
+// (products fused into the sums). A wave per row: a lane has 8 of the row's 512 features and of each of 8 outputs' weights
+// (blockIdx.y: which 8 of the A + 1), then the lanes' 8 sums are added by halves (4 + 2 + 1 exchanges, then 3). Bound by
+// launches for a small batch, by reading h for a large one. 300 / 32,768 rows: 4 / 23 us; as a ReLU, a conversion and two
+// matrix products 30 / 70.
+constexpr int HEAD_IN = 512;
+__global__ void __launch_bounds__(256) k_policy_heads(const uint16_t* h, const float* w_pi, const float* b_pi, const float* w_vf,
+                                                      const float* b_vf, float* logits, float* value, int64_t n, int A) {
+    const int l = threadIdx.x & 63, first = 8 * (int)blockIdx.y;
+    float w[8][8];
+#pragma unroll
+    for (int o = 0; o < 8; o++) {
+        const int k = first + o;
+        const float* src = k < A ? w_pi + (size_t)k * HEAD_IN : w_vf;
+#pragma unroll
+        for (int i = 0; i < 8; i++) w[o][i] = src[8 * l + i];
+    }
+    // this lane's output after the reduction: bits 5, 4, 3 of the lane choose the halves
+    const int mine = first + (l >> 3 & 4) + (l >> 3 & 2) + (l >> 3 & 1);
+    const float bias = mine < A ? b_pi[mine] : b_vf[0];
+    const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), waves = (int64_t)gridDim.x * 4;
+    for (int64_t r = wave; r < n; r += waves) {
+        const mh_u32x4 q = *(const mh_u32x4*)(h + r * HEAD_IN + 8 * l);
+        float s[8] = {};
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float f = __uint_as_float(i & 1 ? q[i >> 1] & 0xffff0000u : q[i >> 1] << 16), x = f < 0.f ? 0.f : f;
+#pragma unroll
+            for (int o = 0; o < 8; o++) s[o] = __builtin_fmaf(x, w[o][i], s[o]);
+        }
+#pragma unroll
+        for (int half = 4, bit = 32; half >= 1; half >>= 1, bit >>= 1) {
+            const bool upper = l & bit;
+#pragma unroll
+            for (int o = 0; o < half; o++) {
+                const float give = upper ? s[o] : s[o + half], keep = upper ? s[o + half] : s[o];
+                s[o] = keep + __shfl_xor(give, bit);
+            }
+        }
+#pragma unroll
+        for (int bit = 4; bit >= 1; bit >>= 1) s[0] += __shfl_xor(s[0], bit);
+        if ((l & 7) == 0) {
+            if (mine < A) logits[r * A + mine] = s[0] + bias;
+            else if (mine == A) value[r] = s[0] + bias;
+        }
+    }
+}
+
 // ---- generalized advantage estimation (fast_mario_env_amd.rollout.gae): a lane per env, backwards over the T steps.
 // Bound by memory: 17 bytes in and 8 out an env-step, every row read and written once, whole rows of 256 bytes a wave.
 // Few waves run (an env is a serial chain: 512 waves for 32,768 envs), so each keeps GAE_AHEAD steps of loads in flight
@@ -1276,6 +1373,49 @@ int mh_policy_conv(const void* d_x, const void* d_w, const void* d_b, void* d_ou
     else if (layer == 2) run(k_policy_conv<32, 4, 2, 20, 9, 1>, 1);
     else if (n >= (int64_t)cus * CONV3_IMGS) run(k_policy_conv<64, 3, 1, 9, 7, CONV3_IMGS>, CONV3_IMGS);
     else run(k_policy_conv<64, 3, 1, 9, 7, 1>, 1);
+    CK(hipGetLastError());
+    return 0;
+}
+
+int mh_policy_pack(const float* const* params, const int64_t* strides, void* d_out, void* stream) {
+    if (!params || !strides || !d_out) { g_err = "invalid arguments"; return -1; }
+    if (((uintptr_t)d_out) & 15) { g_err = "out must be 16-byte aligned"; return -1; }
+    PackArgs a{};
+    for (int i = 0; i < 8; i++) {
+        if (!params[i] || (((uintptr_t)params[i]) & 3)) { g_err = "a parameter is null or not 4-byte aligned"; return -1; }
+        if (!on_gpu(params[i], "parameter")) return -1;
+    }
+    if (!on_gpu(d_out, "out")) return -1;
+    for (int k = 0; k < 3; k++) {
+        a.w[k] = params[2 * k];
+        for (int d = 0; d < 4; d++) a.st[k][d] = strides[4 * k + d];
+    }
+    for (int k = 0; k < 4; k++) a.b[k] = params[2 * k + 1];
+    a.fc = params[6];
+    a.out = (uint16_t*)d_out;
+    hipLaunchKernelGGL(k_policy_pack, dim3(FC_OUT + PACK_SMALL), dim3(256), 0, (hipStream_t)stream, a);
+    CK(hipGetLastError());
+    return 0;
+}
+
+int mh_policy_heads(const void* d_h, const float* w_pi, const float* b_pi, const float* w_vf, const float* b_vf, float* logits,
+                    float* value, int64_t n, int actions, void* stream) {
+    if (!d_h || !w_pi || !b_pi || !w_vf || !b_vf || !logits || !value || n < 1 || actions < 1 || actions > 1024) {
+        g_err = "invalid arguments (n >= 1, 1 <= actions <= 1024)";
+        return -1;
+    }
+    if (((uintptr_t)d_h) & 15) { g_err = "h must be 16-byte aligned"; return -1; }
+    for (const void* p : {(const void*)w_pi, (const void*)b_pi, (const void*)w_vf, (const void*)b_vf, (const void*)logits, (const void*)value}) {
+        if (((uintptr_t)p) & 3) { g_err = "parameters and outputs must be 4-byte aligned"; return -1; }
+        if (!on_gpu(p, "parameter or output")) return -1;
+    }
+    if (!on_gpu(d_h, "h")) return -1;
+    int dev = 0, cus = 0;
+    CK(hipGetDevice(&dev));
+    CK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    const int64_t blocks = std::min<int64_t>((n + 3) / 4, (int64_t)std::max(cus, 1) * 8);
+    hipLaunchKernelGGL(k_policy_heads, dim3((unsigned)blocks, (unsigned)(actions / 8 + 1)), dim3(256), 0, (hipStream_t)stream,
+                       (const uint16_t*)d_h, w_pi, b_pi, w_vf, b_vf, logits, value, n, actions);
     CK(hipGetLastError());
     return 0;
 }

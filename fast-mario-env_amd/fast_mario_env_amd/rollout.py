@@ -20,6 +20,7 @@ The env-kernel share of a rollout is timed with events on the stream both run on
 """
 from __future__ import annotations
 
+import ctypes
 import math
 
 import numpy as np
@@ -97,6 +98,73 @@ def policy_conv(x, weight, bias, layer, out=None):
     return out
 
 
+_PACKED = 1684128   # MH_POLICY_PACKED
+
+
+def _packed_params(convs, fc, obs):
+    """The parameters of the convolutions and the fully connected layer as one bf16 tensor (mh_policy_pack), made anew
+    for this call: None unless they are the standard network's float32 tensors on the GPU of obs."""
+    torch = _torch()
+    from ._native import check, lib
+    if obs.dtype != torch.uint8 or tuple(obs.shape[1:]) != (4, 84, 84):
+        return None
+    ps = [p for m in (*convs, fc) for p in (m.weight, m.bias)]
+    shapes = ((32, 4, 8, 8), (32,), (64, 32, 4, 4), (64,), (64, 64, 3, 3), (64,), (512, 3136), (512,))
+    if not all(type(p) in (torch.Tensor, torch.nn.Parameter) and p.dtype == torch.float32 and p.device == obs.device
+               and p.shape == s and (p.dim() == 4 or p.is_contiguous()) for p, s in zip(ps, shapes)):
+        return None
+    out = torch.empty(_PACKED, dtype=torch.bfloat16, device=obs.device)
+    check(lib().mh_policy_pack((ctypes.c_void_p * 8)(*[p.data_ptr() for p in ps]),
+                               (ctypes.c_int64 * 12)(*[s for p in ps[0:6:2] for s in p.stride()]), out.data_ptr(),
+                               torch.cuda.current_stream(obs.device).cuda_stream), "mh_policy_pack")
+    return out
+
+
+def _packed_convs(packed, obs, buffer):
+    """The three convolutions of obs with the packed parameters: their output as (B, 3136) in (h, w, c) order, and the
+    fully connected layer's weight and bias."""
+    torch = _torch()
+    from ._native import check, lib
+    L, B, at = lib(), obs.shape[0], packed.data_ptr()
+    stream = torch.cuda.current_stream(obs.device).cuda_stream
+    y = [buffer((B,) + s, obs.device) for s in ((32, 20, 20), (64, 9, 9), (64, 7, 7))]
+    w = lambda i: at + 2 * i   # noqa: E731
+    check(L.mh_policy_conv1(obs.data_ptr(), w(0), w(77824), y[0].data_ptr(), B, stream), "mh_policy_conv1")
+    check(L.mh_policy_conv(y[0].data_ptr(), w(8192), w(77856), y[1].data_ptr(), B, 2, stream), "mh_policy_conv")
+    check(L.mh_policy_conv(y[1].data_ptr(), w(40960), w(77920), y[2].data_ptr(), B, 3, stream), "mh_policy_conv")
+    return y[2].permute(0, 2, 3, 1).reshape(B, 3136), packed[78496:].view(512, 3136), packed[77984:78496]
+
+
+def _plain_heads(pi, vf, h):
+    """Whether mh_policy_heads is what calling the two modules on relu(h) in float32 does: plain linear layers without
+    hooks, float32 parameters on the GPU of h, no autocast around the network."""
+    torch = _torch()
+    for m, rows in ((pi, None), (vf, 1)):
+        if type(m) is not torch.nn.Linear or m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+            return False
+        w, b = m.weight, m.bias
+        if not all(type(p) in (torch.Tensor, torch.nn.Parameter) and p.dtype == torch.float32 and p.device == h.device
+                   and p.is_contiguous() for p in (w, b)):
+            return False
+        if w.shape[1:] != (512,) or b.shape != w.shape[:1] or (rows and w.shape[0] != rows):
+            return False
+    hooks = torch.nn.modules.module
+    return (1 <= pi.weight.shape[0] <= 1024 and h.dtype == torch.bfloat16 and h.is_contiguous()
+            and not torch.is_autocast_enabled("cuda") and not hooks._global_forward_hooks
+            and not hooks._global_forward_pre_hooks)
+
+
+def _packed_heads(pi, vf, h):
+    torch = _torch()
+    from ._native import check, lib
+    B, A = h.shape[0], pi.weight.shape[0]
+    logits, value = (torch.empty(s, dtype=torch.float32, device=h.device) for s in ((B, A), (B,)))
+    check(lib().mh_policy_heads(h.data_ptr(), pi.weight.data_ptr(), pi.bias.data_ptr(), vf.weight.data_ptr(),
+                                vf.bias.data_ptr(), logits.data_ptr(), value.data_ptr(), B, A,
+                                torch.cuda.current_stream(h.device).cuda_stream), "mh_policy_heads")
+    return logits, value
+
+
 def make_net(n_actions: int = N_ACTIONS, in_ch: int = 4, seed: int = 0, device="cuda"):
     """The Nature-CNN actor-critic with the reference's architecture and initialisation, random weights."""
     torch = _torch()
@@ -148,6 +216,15 @@ def make_net(n_actions: int = N_ACTIONS, in_ch: int = 4, seed: int = 0, device="
                 # (mh_policy_conv1, mh_policy_conv); the fully connected layer takes the last one's
                 # channels-last output as it lies, with its weight's columns permuted to (h, w, c) order
                 B, dev = obs_u8.shape[0], obs_u8.device
+                packed = _packed_params(convs, self.fc, obs_u8)
+                if packed is not None and B:
+                    x, wfc, bfc = _packed_convs(packed, obs_u8, self._input)
+                    with torch.autocast("cuda", dtype=torch.bfloat16):
+                        h = F.linear(x, wfc, bfc)
+                    if _plain_heads(self.pi, self.vf, h):
+                        return _packed_heads(self.pi, self.vf, h)
+                    h = F.relu(h).float()
+                    return self.pi(h), self.vf(h).squeeze(-1)
                 x = policy_conv1(obs_u8, convs[0].weight, convs[0].bias, self._input((B, 32, 20, 20), dev))
                 x = policy_conv(x, convs[1].weight, convs[1].bias, 2, self._input((B, 64, 9, 9), dev))
                 x = policy_conv(x, convs[2].weight, convs[2].bias, 3, self._input((B, 64, 7, 7), dev))

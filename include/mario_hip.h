@@ -182,6 +182,21 @@ int mh_policy_conv1(const uint8_t* d_obs, const void* d_w, const void* d_b, void
  * (channels last), d_b the bf16 bias (64). d_x and d_w 16-byte aligned. */
 int mh_policy_conv(const void* d_x, const void* d_w, const void* d_b, void* d_out, int64_t n, int layer, void* stream);
 
+/* The network's float32 parameters as the bf16 operands of a forward pass (rounded to nearest even), in one launch.
+ * params: 8 device pointers in host memory: the weights and biases of the convolutions (32, 4, 8, 8), (64, 32, 4, 4),
+ * (64, 64, 3, 3) and of the fully connected layer (512, 3136); strides: the three convolution weights' (co, ci, kh, kw)
+ * strides in elements; the others are contiguous. d_out (16-byte aligned): MH_POLICY_PACKED halfs, at 0 the first weight
+ * as mh_policy_conv1 takes it, at 8192 and 40960 the next two as mh_policy_conv takes them, at 77824, 77856, 77920
+ * and 77984 the biases, at 78496 the fully connected weight with its columns in (h, w, c) order. Pointers as above. */
+#define MH_POLICY_PACKED 1684128
+int mh_policy_pack(const float* const* params, const int64_t* strides, void* d_out, void* stream);
+
+/* The policy's two heads in float32: logits (n, actions) = relu(h) w_pi^T + b_pi and value (n) = relu(h) w_vf^T + b_vf
+ * of the bf16 (n, 512) output h of the fully connected layer (16-byte aligned); w_pi (actions, 512), b_pi (actions),
+ * w_vf (512), b_vf (1), all contiguous. 1 <= actions <= 1024. Pointers as above. */
+int mh_policy_heads(const void* d_h, const float* w_pi, const float* b_pi, const float* w_vf, const float* b_vf, float* logits,
+                    float* value, int64_t n, int actions, void* stream);
+
 /* Generalized advantage estimation over T steps of n envs, backwards (ppo/train.py:140-150): rew, val, adv, ret (T, n)
  * float32 and start (T, n) bytes (0, else the step starts an episode), all contiguous; next_val (n) and next_start (n)
  * the step after the last. adv[t] = delta + gamma_lam keep adv[t + 1] with keep = 1 - start[t + 1] and

@@ -127,3 +127,40 @@ def test_policy_conv_batch_edges(layer, extra):
         assert torch.equal(one, y[i]), i
     odd = torch.zeros(n * size + 2, dtype=torch.bfloat16, device="cuda")
     assert torch.equal(conv(x, odd[1:-1]).view(n, size), y) and odd[0] == 0 and odd[-1] == 0
+
+
+@pytest.mark.parametrize("channels_last", [False, True])
+def test_policy_pack_is_the_cast_and_permuted_parameters(channels_last):
+    from fast_mario_env_amd.rollout import _packed_params, make_net
+    net = make_net(seed=3)
+    for p in net.parameters():
+        p.data += 0.01 * torch.randn_like(p)
+    net = net.to(memory_format=torch.channels_last if channels_last else torch.contiguous_format)
+    obs = torch.zeros(2, 4, 84, 84, dtype=torch.uint8, device="cuda")
+    got = _packed_params(list(net.convs), net.fc, obs)
+    parts = [net.convs[0].weight] + [c.weight.permute(0, 2, 3, 1) for c in net.convs[1:]] + [c.bias for c in net.convs]
+    parts += [net.fc.bias, net.fc.weight.view(512, 64, 49).permute(0, 2, 1)]
+    assert torch.equal(got, torch.cat([p.detach().reshape(-1) for p in parts]).to(torch.bfloat16))
+    assert _packed_params(list(net.convs), net.fc.double(), obs) is None
+
+
+@pytest.mark.parametrize("n,actions", [(1, 7), (3, 1), (300, 7), (8197, 7), (5, 8), (6, 12), (4, 15), (4, 16)])
+def test_policy_heads_against_64_bits(n, actions):
+    """512 products summed in float32: the error is below 512 units in the last place of the sum of their sizes, and not
+    above that of torch's float32 layers."""
+    from fast_mario_env_amd.rollout import _packed_heads, _plain_heads
+    torch.manual_seed(n + actions)
+    pi, vf = torch.nn.Linear(512, actions).cuda(), torch.nn.Linear(512, 1).cuda()
+    h = torch.randn(n, 512, device="cuda").to(torch.bfloat16)
+    assert _plain_heads(pi, vf, h)
+    with torch.no_grad():
+        x = h.float().relu()
+        for got, m, plain in zip(_packed_heads(pi, vf, h), (pi, vf), (pi(x), vf(x).squeeze(-1))):
+            want = (x.double() @ m.weight.double().T + m.bias.double()).reshape(got.shape)
+            size = (x.double() @ m.weight.double().abs().T + m.bias.double().abs()).reshape(got.shape)
+            assert ((got.double() - want).abs() <= 512 * 2.0 ** -24 * size).all()
+            assert (got.double() - want).abs().max() <= 2 * (plain.double() - want).abs().max() + 2.0 ** -24 * size.max()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not _plain_heads(pi, vf, h)
+    pi.register_forward_hook(lambda *a: None)
+    assert not _plain_heads(pi, vf, h)
