@@ -1529,6 +1529,29 @@ int mh_replay_add(uint8_t* frames, uint8_t* age, int16_t* act, float* rew, uint8
     return 0;
 }
 
+int mh_replay_candidates(const int64_t* ptr, int n_envs, int capacity, int k, int64_t n_step, int64_t* cand, int64_t* count,
+                         void* stream) {
+    if (!ptr || !cand || !count || n_envs < 1 || capacity < 2 || k < 1) { g_err = "invalid arguments"; return -1; }
+    hipLaunchKernelGGL(k_replay_candidates, dim3(1), dim3(DRAW_THREADS), 0, (hipStream_t)stream, ptr, n_envs, capacity, k,
+                       n_step, cand, count);
+    CK(hipGetLastError());
+    return 0;
+}
+
+int mh_replay_draw(const int64_t* ptr, const uint8_t* flags, int n_envs, int capacity, int k, int64_t n_step, const int64_t* cand,
+                   const int64_t* pick, const double* u, const int64_t* rows, int64_t n, int64_t* env, int64_t* pos,
+                   uint8_t* open, int64_t* rows_out, int64_t* count, void* stream) {
+    if (!ptr || !flags || !cand || !pick || !u || !env || !pos || !open || !rows_out || !count || rows_out == rows ||
+        n_envs < 1 || capacity < 2 || k < 1 || n < 1 || n > ((int64_t)1 << 38)) {
+        g_err = "invalid arguments"; return -1;
+    }
+    DrawArgs A{ptr, flags, n_envs, capacity, k, n_step, cand, pick, u, rows, n, env, pos, open, rows_out, count};
+    hipLaunchKernelGGL(k_replay_draw, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, A);
+    hipLaunchKernelGGL(k_replay_open, dim3(1), dim3(DRAW_THREADS), 0, (hipStream_t)stream, A);
+    CK(hipGetLastError());
+    return 0;
+}
+
 int mh_replay_gather(const uint8_t* frames, const uint8_t* age, const int16_t* act, const float* rew,
                      const uint8_t* flags, int n_envs, int capacity, int frame_bytes, int k, const int64_t* env,
                      const int64_t* pos, int batch, int n_step, const float* gamma_pow, uint8_t* obs,

@@ -128,25 +128,29 @@ class FrameReplay:
     def draw(self, batch: int, n_step: int = 1):
         """(env, pos) of `batch` transitions: env uniform among the envs with a sampleable window, pos uniform
         in [max(ptr - C + k - 1, 0), ptr - 1 - n_step], redrawn while the slot does not start a transition."""
-        torch, C, d = self.torch, self.C, self.dev
-        lo = torch.clamp(self._ptr - C + self.k - 1, min=0)      # the k-1 frames behind pos are still in the ring
-        hi = self._ptr - 1 - n_step                               # the frame after pos + n_step - 1 is written
-        cand = torch.nonzero(hi >= lo).flatten()
-        if len(cand) == 0:
+        torch, d, st = self.torch, self.dev, _stream(self.torch, self.dev)
+        ring = (self.E, self.C, self.k, int(n_step))
+        cand = torch.empty(self.E, dtype=torch.long, device=d)
+        count = torch.empty(1, dtype=torch.long, device=d)
+        _check(lib().mh_replay_candidates(_ptr(self._ptr), *ring, _ptr(cand), _ptr(count), st), "mh_replay_candidates")
+        n_cand = int(count)
+        if n_cand == 0:
             raise ValueError("not enough data in buffer")
         env = torch.empty(batch, dtype=torch.long, device=d)
         pos = torch.empty(batch, dtype=torch.long, device=d)
-        open_rows = torch.arange(batch, device=d)
+        n, rows, spare = batch, None, None
+        opened = torch.empty(batch, dtype=torch.uint8, device=d)
         for _ in range(64):
-            n = len(open_rows)
-            ee = cand[torch.randint(len(cand), (n,), device=d, generator=self.g)]
-            width = (hi[ee] - lo[ee] + 1).double()
-            pp = lo[ee] + (torch.rand(n, device=d, generator=self.g, dtype=torch.float64) * width).long()
-            ok = (self.flags[ee, pp % C] & 1).bool()
-            env[open_rows[ok]] = ee[ok]
-            pos[open_rows[ok]] = pp[ok]
-            open_rows = open_rows[~ok]
-            if len(open_rows) == 0:
+            pick = torch.randint(n_cand, (n,), device=d, generator=self.g)
+            u = torch.rand(n, device=d, generator=self.g, dtype=torch.float64)
+            if n == 0:
+                return env, pos
+            rows_out = torch.empty(n, dtype=torch.long, device=d) if spare is None else spare
+            _check(lib().mh_replay_draw(_ptr(self._ptr), _ptr(self.flags), *ring, _ptr(cand), _ptr(pick), _ptr(u),
+                                        None if rows is None else _ptr(rows), n, _ptr(env), _ptr(pos), _ptr(opened),
+                                        _ptr(rows_out), _ptr(count), st), "mh_replay_draw")
+            n, rows, spare = int(count), rows_out, rows
+            if n == 0:
                 return env, pos
         raise RuntimeError("sampling failed")
 

@@ -224,6 +224,16 @@ int mh_replay_add(uint8_t* frames, uint8_t* age, int16_t* act, float* rew, uint8
                   const uint8_t* next_obs, const int64_t* action, const float* reward, const uint8_t* done,
                   const uint8_t* truncated, void* stream);
 
+/* The draw of a batch for mh_replay_gather: env uniform among those whose window [max(ptr - capacity + k - 1, 0),
+ * ptr - 1 - n_step] is not empty, pos uniform in it. mh_replay_candidates lists those envs in order in cand (n_envs) and
+ * their number in count[0]. mh_replay_draw takes n rows (rows, or null: 0 .. n - 1) with their candidate pick (0 <= pick <
+ * the number) and their u in [0, 1): a row whose slot lo + (int64)(u * width) starts a transition gets its env and pos, the
+ * others are listed in order in rows_out (not rows), their number in count[0]; open: n bytes of scratch. Device memory. */
+int mh_replay_candidates(const int64_t* ptr, int n_envs, int capacity, int k, int64_t n_step, int64_t* cand, int64_t* count,
+                         void* stream);
+int mh_replay_draw(const int64_t* ptr, const uint8_t* flags, int n_envs, int capacity, int k, int64_t n_step, const int64_t* cand,
+                   const int64_t* pick, const double* u, const int64_t* rows, int64_t n, int64_t* env, int64_t* pos,
+                   uint8_t* open, int64_t* rows_out, int64_t* count, void* stream);
 /* Batch assembly of FrameReplay.sample (replay.py:99-106, 131-145) for `batch` sampled (env, pos): the
  * n-step return (gamma_pow[i] = float32(gamma ** i), i = 0..n_step), steps m, terminal, discount
  * gamma_pow[m] * (1 - terminal), the action at pos, and the zero-padded (k, frame_bytes) stacks ending at

@@ -164,3 +164,44 @@ def test_policy_heads_against_64_bits(n, actions):
         assert not _plain_heads(pi, vf, h)
     pi.register_forward_hook(lambda *a: None)
     assert not _plain_heads(pi, vf, h)
+
+
+def _draw_by_tensor_operations(rb, batch, n_step):
+    C, d = rb.C, rb.dev
+    lo = torch.clamp(rb._ptr - C + rb.k - 1, min=0)
+    hi = rb._ptr - 1 - n_step
+    cand = torch.nonzero(hi >= lo).flatten()
+    env, pos = (torch.empty(batch, dtype=torch.long, device=d) for _ in range(2))
+    rows = torch.arange(batch, device=d)
+    while True:
+        ee = cand[torch.randint(len(cand), (len(rows),), device=d, generator=rb.g)]
+        width = (hi[ee] - lo[ee] + 1).double()
+        pp = lo[ee] + (torch.rand(len(rows), device=d, generator=rb.g, dtype=torch.float64) * width).long()
+        ok = (rb.flags[ee, pp % C] & 1).bool()
+        env[rows[ok]], pos[rows[ok]] = ee[ok], pp[ok]
+        rows = rows[~ok]
+        if len(rows) == 0:
+            return env, pos
+
+
+@pytest.mark.parametrize("n_envs,batch,n_step", [(1, 1, 1), (70, 1023, 3), (1025, 1025, 1), (2600, 70001, 2), (5, 0, 1)])
+def test_replay_draw_is_the_tensor_operations(n_envs, batch, n_step):
+    """The same (env, pos) from the same generator as drawing with tensor operations, over rings at every stage of
+    filling (some envs without a window), about a third of the slots no start, several rounds."""
+    from fast_mario_env_amd.replay import FrameReplay
+    rb = FrameReplay(9, n_envs, 4, hw=(4, 4), seed=7)
+    g = torch.Generator(device="cuda").manual_seed(n_envs)
+    rb._ptr.copy_(torch.randint(0, 40, (n_envs,), device="cuda", generator=g))
+    rb._ptr[-1] = 30
+    rb.flags.copy_(torch.randint(0, 3, (n_envs, 9), device="cuda", generator=g) > 0)
+    rb.flags[-1] = 1
+    state = rb.g.get_state()
+    env, pos = rb.draw(batch, n_step)
+    after = rb.g.get_state()
+    rb.g.set_state(state)
+    e2, p2 = _draw_by_tensor_operations(rb, batch, n_step)
+    assert torch.equal(env, e2) and torch.equal(pos, p2) and torch.equal(after, rb.g.get_state())
+    assert batch == 0 or bool((rb.flags[env, pos % 9] == 1).all())
+    rb._ptr.zero_()
+    with pytest.raises(ValueError):
+        rb.draw(4, n_step)
