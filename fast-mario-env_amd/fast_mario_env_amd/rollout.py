@@ -101,6 +101,15 @@ def policy_conv(x, weight, bias, layer, out=None):
 _PACKED = 1684128   # MH_POLICY_PACKED
 
 
+def _transformed(*ts):
+    """Whether something follows the operations on these tensors, which a kernel called by address would pass by:
+    forward-mode tangents, vmap and the like, a dispatch mode (a FLOP counter, fake tensors), tracing or compiling."""
+    torch = _torch()
+    return (torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0
+            or torch.jit.is_tracing() or torch.compiler.is_compiling()
+            or any(torch._C._functorch.is_functorch_wrapped_tensor(t) for t in ts))
+
+
 def _packed_params(convs, fc, obs):
     """The parameters of the convolutions and the fully connected layer as one bf16 tensor (mh_policy_pack), made anew
     for this call: None unless they are the standard network's float32 tensors on the GPU of obs."""
@@ -111,7 +120,7 @@ def _packed_params(convs, fc, obs):
     ps = [p for m in (*convs, fc) for p in (m.weight, m.bias)]
     shapes = ((32, 4, 8, 8), (32,), (64, 32, 4, 4), (64,), (64, 64, 3, 3), (64,), (512, 3136), (512,))
     if not all(type(p) in (torch.Tensor, torch.nn.Parameter) and p.dtype == torch.float32 and p.device == obs.device
-               and p.shape == s and (p.dim() == 4 or p.is_contiguous()) for p, s in zip(ps, shapes)):
+               and p.shape == s and (p.dim() == 4 or p.is_contiguous()) for p, s in zip(ps, shapes)) or _transformed(*ps):
         return None
     out = torch.empty(_PACKED, dtype=torch.bfloat16, device=obs.device)
     check(lib().mh_policy_pack((ctypes.c_void_p * 8)(*[p.data_ptr() for p in ps]),
@@ -137,7 +146,7 @@ def _packed_convs(packed, obs, buffer):
 
 def _plain_heads(pi, vf, h):
     """Whether mh_policy_heads is what calling the two modules on relu(h) in float32 does: plain linear layers without
-    hooks, float32 parameters on the GPU of h, no autocast around the network."""
+    hooks, float32 parameters on the GPU of h that nothing transforms, no autocast around the network."""
     torch = _torch()
     for m, rows in ((pi, None), (vf, 1)):
         if type(m) is not torch.nn.Linear or m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
@@ -148,6 +157,8 @@ def _plain_heads(pi, vf, h):
             return False
         if w.shape[1:] != (512,) or b.shape != w.shape[:1] or (rows and w.shape[0] != rows):
             return False
+    if _transformed(pi.weight, pi.bias, vf.weight, vf.bias, h):
+        return False
     hooks = torch.nn.modules.module
     return (1 <= pi.weight.shape[0] <= 1024 and h.dtype == torch.bfloat16 and h.is_contiguous()
             and not torch.is_autocast_enabled("cuda") and not hooks._global_forward_hooks
@@ -274,11 +285,7 @@ def _gae_kernel_takes(rew, val, start, next_val, next_start, gamma, lam):
         return False
     if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
         return False
-    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack():
-        return False
-    if any(torch._C._functorch.is_functorch_wrapped_tensor(t) for t in ts):
-        return False
-    if any(torch.autograd.forward_ad.unpack_dual(t).tangent is not None for t in (rew, val, next_val)):
+    if _transformed(*ts):
         return False
     T, n = rew.shape
     return (T > 0 and n > 0 and val.shape == rew.shape == start.shape and next_val.shape == next_start.shape == (n,)

@@ -166,6 +166,30 @@ def test_policy_heads_against_64_bits(n, actions):
     assert not _plain_heads(pi, vf, h)
 
 
+def test_policy_transforms_take_the_layers():
+    """What follows the tensor operations (tangents, vmap over head weights, a dispatch mode) sees them without autograd too."""
+    from torch.autograd import forward_ad
+    from torch.utils.flop_counter import FlopCounterMode
+    from fast_mario_env_amd.rollout import make_net
+    net = make_net(seed=4)
+    obs = torch.randint(0, 256, (3, 4, 84, 84), dtype=torch.uint8, device="cuda")
+    w, b = net.pi.weight.detach().clone(), net.pi.bias.detach()
+    def logits(weight):
+        return torch.func.functional_call(net, {"pi.weight": weight}, (obs,))[0]
+    with torch.no_grad():
+        want = logits(w)
+        both = torch.vmap(logits)(torch.stack([w, 2 * w]))
+        # float32 sums of 512 products in another order
+        assert torch.allclose(both[0], want, rtol=1e-4, atol=1e-5)
+        assert torch.allclose(both[1] - b, 2 * (want - b), rtol=1e-4, atol=1e-5)
+        with forward_ad.dual_level():
+            out = logits(forward_ad.make_dual(w, torch.ones_like(w)))
+            assert forward_ad.unpack_dual(out).tangent is not None
+        with FlopCounterMode(display=False) as count:
+            net(obs)
+    assert count.get_total_flops() >= 2 * 3 * 512 * (3136 + 8)
+
+
 def _draw_by_tensor_operations(rb, batch, n_step):
     C, d = rb.C, rb.dev
     lo = torch.clamp(rb._ptr - C + rb.k - 1, min=0)
