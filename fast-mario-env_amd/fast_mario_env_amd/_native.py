@@ -71,6 +71,7 @@ def lib() -> ctypes.CDLL:
     L.mh_gae.argtypes = [_P, _P, _P, _P, _P, _i64, _i64, ctypes.c_float, ctypes.c_float, _P, _P, _P]
     L.mh_policy_input.argtypes = [_P, _P, _i64, _i32, _P]
     L.mh_policy_conv1.argtypes = [_P, _P, _P, _P, _i64, _P]
+    L.mh_policy_conv12.argtypes = [_P, _P, _P, _P, _P, _P, _i64, _P]
     L.mh_policy_pack.argtypes = [_P, _P, _P, _P]
     L.mh_policy_heads.argtypes = [_P, _P, _P, _P, _P, _P, _P, _i64, _i32, _P]
     L.mh_policy_conv.argtypes = [_P, _P, _P, _P, _i64, _i32, _P]

@@ -136,12 +136,11 @@ def _packed_convs(packed, obs, buffer):
     from ._native import check, lib
     L, B, at = lib(), obs.shape[0], packed.data_ptr()
     stream = torch.cuda.current_stream(obs.device).cuda_stream
-    y = [buffer((B,) + s, obs.device) for s in ((32, 20, 20), (64, 9, 9), (64, 7, 7))]
+    y = [buffer((B,) + s, obs.device) for s in ((64, 9, 9), (64, 7, 7))]
     w = lambda i: at + 2 * i   # noqa: E731
-    check(L.mh_policy_conv1(obs.data_ptr(), w(0), w(77824), y[0].data_ptr(), B, stream), "mh_policy_conv1")
-    check(L.mh_policy_conv(y[0].data_ptr(), w(8192), w(77856), y[1].data_ptr(), B, 2, stream), "mh_policy_conv")
-    check(L.mh_policy_conv(y[1].data_ptr(), w(40960), w(77920), y[2].data_ptr(), B, 3, stream), "mh_policy_conv")
-    return y[2].permute(0, 2, 3, 1).reshape(B, 3136), packed[78496:].view(512, 3136), packed[77984:78496]
+    check(L.mh_policy_conv12(obs.data_ptr(), w(0), w(77824), w(8192), w(77856), y[0].data_ptr(), B, stream), "mh_policy_conv12")
+    check(L.mh_policy_conv(y[0].data_ptr(), w(40960), w(77920), y[1].data_ptr(), B, 3, stream), "mh_policy_conv")
+    return y[1].permute(0, 2, 3, 1).reshape(B, 3136), packed[78496:].view(512, 3136), packed[77984:78496]
 
 
 def _plain_heads(pi, vf, h):

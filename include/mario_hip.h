@@ -182,6 +182,11 @@ int mh_policy_conv1(const uint8_t* d_obs, const void* d_w, const void* d_b, void
  * (channels last), d_b the bf16 bias (64). d_x and d_w 16-byte aligned. */
 int mh_policy_conv(const void* d_x, const void* d_w, const void* d_b, void* d_out, int64_t n, int layer, void* stream);
 
+/* mh_policy_conv1 and mh_policy_conv's layer 2 in one pass, with the same results: d_out the bf16 (n, 9, 9, 64) output,
+ * 8-byte aligned; the first layer's (n, 20, 20, 32) output stays on chip. The others as above. */
+int mh_policy_conv12(const uint8_t* d_obs, const void* d_w1, const void* d_b1, const void* d_w2, const void* d_b2, void* d_out,
+                     int64_t n, void* stream);
+
 /* The network's float32 parameters as the bf16 operands of a forward pass (rounded to nearest even), in one launch.
  * params: 8 device pointers in host memory: the weights and biases of the convolutions (32, 4, 8, 8), (64, 32, 4, 4),
  * (64, 64, 3, 3) and of the fully connected layer (512, 3136); strides: the three convolution weights' (co, ci, kh, kw)

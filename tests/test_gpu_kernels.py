@@ -129,6 +129,25 @@ def test_policy_conv_batch_edges(layer, extra):
     assert torch.equal(conv(x, odd[1:-1]).view(n, size), y) and odd[0] == 0 and odd[-1] == 0
 
 
+@pytest.mark.parametrize("turns,extra", [(0, 1), (0, 2), (1, -1), (1, 0), (1, 1), (2, 1), (3, 0)])
+def test_policy_first_two_layers_in_one_pass(turns, extra):
+    """Around whole turns of one image per CU: the bits of the two layers' own kernels, and nothing past the output."""
+    from fast_mario_env_amd._native import check, lib
+    n = turns * torch.cuda.get_device_properties(0).multi_processor_count + extra
+    g = torch.Generator(device="cuda").manual_seed(n)
+    w1, w2 = ((torch.randn(s, generator=g, device="cuda") * 0.05).to(torch.bfloat16) for s in ((32, 256), (64, 512)))
+    b1, b2 = (torch.randn(s, generator=g, device="cuda").to(torch.bfloat16) for s in (32, 64))
+    x = torch.randint(0, 256, (n, 4, 84, 84), dtype=torch.uint8, device="cuda", generator=g)
+    y1 = torch.empty(n, 20, 20, 32, dtype=torch.bfloat16, device="cuda")
+    want = torch.empty(n * 5184, dtype=torch.bfloat16, device="cuda")
+    got = torch.zeros(n * 5184 + 4, dtype=torch.bfloat16, device="cuda")
+    check(lib().mh_policy_conv1(x.data_ptr(), w1.data_ptr(), b1.data_ptr(), y1.data_ptr(), n, 0), "conv1")
+    check(lib().mh_policy_conv(y1.data_ptr(), w2.data_ptr(), b2.data_ptr(), want.data_ptr(), n, 2, 0), "conv")
+    check(lib().mh_policy_conv12(x.data_ptr(), w1.data_ptr(), b1.data_ptr(), w2.data_ptr(), b2.data_ptr(), got.data_ptr(), n, 0),
+          "conv12")
+    assert torch.equal(got[:-4], want) and not got[-4:].any()
+
+
 @pytest.mark.parametrize("channels_last", [False, True])
 def test_policy_pack_is_the_cast_and_permuted_parameters(channels_last):
     from fast_mario_env_amd.rollout import _packed_params, make_net
