@@ -466,26 +466,67 @@ __global__ void __launch_bounds__(256) k_policy_input_k1(const uint8_t* obs, uin
 // v_mfma_f32_32x32x16_bf16); they are the first operand, so that a lane ends up with its pixel's channels
 // 8 q + 4 (l / 32) .. + 3, q = 0 .. 3, and stores them 8 bytes at a time. The next images' loads are in flight while
 // these compute. 32,768 images, before -> now (reading and writing the activations alone at a copy's 4.9 TB/s): first layer
-// 600 -> 430 us (360), second 600 -> 260 (240), third 430 -> 148 (110).
+// 600 -> 412 us (360), second 600 -> 257 (240), third 430 -> 150 (110).
 typedef __bf16 mh_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float mh_f32x16 __attribute__((ext_vector_type(16)));
 __device__ __forceinline__ mh_bf16x8 as_bf16x8(mh_u32x4 q) { return __builtin_bit_cast(mh_bf16x8, q); }
+typedef __bf16 mh_bf16x2 __attribute__((ext_vector_type(2)));
+typedef float mh_f32x2 __attribute__((ext_vector_type(2)));
+// lo | hi << 16 as bf16, rounded to nearest even: one instruction for the two, which an element at a time takes four
+__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(mh_f32x2{lo, hi}, mh_bf16x2));
+}
+// four pixels, a byte each, as bf16(float(v) * sc)
+__device__ __forceinline__ uint2 scaled_pixels(uint32_t v, float sc) {
+    return make_uint2(bf16_pair((float)(v & 0xffu) * sc, (float)(v >> 8 & 0xffu) * sc),
+                      bf16_pair((float)(v >> 16 & 0xffu) * sc, (float)(v >> 24) * sc));
+}
 // a lane's 16 sums (its pixel's channels) + bias, ReLU, bf16, to out (the pixel's first channel of these 32, + 4 kg);
 // wide: out is 8-byte aligned
 __device__ __forceinline__ void conv_out(const mh_f32x16& acc, const float (&bias)[16], uint16_t* out, bool wide) {
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        uint32_t h[4];
+        float r[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const float r = acc[4 * q + i] + bias[4 * q + i];
-            h[i] = __builtin_bit_cast(uint16_t, (__bf16)(r > 0.f ? r : 0.f));   // to nearest even
+            r[i] = acc[4 * q + i] + bias[4 * q + i];
+            r[i] = r[i] > 0.f ? r[i] : 0.f;
         }
-        if (wide) *(uint2*)(out + 8 * q) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+        const uint2 h = make_uint2(bf16_pair(r[0], r[1]), bf16_pair(r[2], r[3]));
+        if (wide) *(uint2*)(out + 8 * q) = h;
         else
-            for (int i = 0; i < 4; i++) out[8 * q + i] = (uint16_t)h[i];
+            for (int i = 0; i < 4; i++) out[8 * q + i] = (uint16_t)((i < 2 ? h.x : h.y) >> (16 * (i & 1)));
     }
 }
+
+// The products of a tile's STEPS steps, operand(s) of step s read from LDS a group of 4 ahead of the products that use it.
+// (Left to itself the compiler reads one step ahead, and a read takes as long as 4 products: k_policy_conv12 606 us of
+// 32,768 images against 535. The layers' own kernels have no registers left for it.)
+template <int STEPS, class F>
+__device__ __forceinline__ mh_f32x16 tile_products(const mh_bf16x8 (&w)[STEPS], F&& operand) {
+    static_assert(STEPS % 4 == 0, "groups of 4 steps");
+    mh_f32x16 acc = {};
+    mh_u32x4 a[4], ahead[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) ahead[i] = operand(i);
+#pragma unroll
+    for (int s = 0; s < STEPS; s += 4) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) a[i] = ahead[i];
+        if (s + 4 < STEPS) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) ahead[i] = operand(s + 4 + i);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[s + i], as_bf16x8(a[i]), acc, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    return acc;
+}
+// The weights have arrived. Before a loop that keeps loads in flight: else the compiler waits in it for the weights, and
+// so for all that is in flight, ahead of every first product.
+__device__ __forceinline__ void weights_arrived() { __builtin_amdgcn_s_waitcnt(0); }
 
 // The first layer, with the input scaled as mh_policy_input scales it: K = 4 x 8 x 8 in the weight's own (ci, kh, kw)
 // order. An image is 56,448 bytes of bf16 in LDS, scaled once (2.5 vector instructions a pixel; scaled per patch, 7 a
@@ -512,16 +553,14 @@ __global__ void __launch_bounds__(256, 2) k_policy_conv1(const uint8_t* obs, con
             raw[i] = src[c < WORDS ? c : 0];
         }
     };
+    weights_arrived();
     int64_t b = blockIdx.x;
     if (b < n) load(b);
     for (; b < n; b += gridDim.x) {
 #pragma unroll
         for (int i = 0; i < PER; i++) {
             const int c = tid + 256 * i;
-            uint32_t h[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) h[e] = __builtin_bit_cast(uint16_t, (__bf16)((float)((raw[i] >> (8 * e)) & 0xffu) * sc));
-            if (c < WORDS) *(uint2*)(s_x + 4 * c) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+            if (c < WORDS) *(uint2*)(s_x + 4 * c) = scaled_pixels(raw[i], sc);
         }
         __syncthreads();
         if (b + gridDim.x < n) load(b + gridDim.x);
@@ -571,6 +610,7 @@ __global__ void __launch_bounds__(256, 2) k_policy_conv(const uint16_t* x, const
             raw[i] = src[c < last ? c : last];
         }
     };
+    weights_arrived();
     int64_t g = blockIdx.x;
     if (g < groups) load(g);
     for (; g < groups; g += gridDim.x) {
@@ -603,99 +643,101 @@ __global__ void __launch_bounds__(256, 2) k_policy_conv(const uint16_t* x, const
 constexpr int CONV2_IMGS = 2, CONV3_IMGS = 5;
 
 // The first two layers in one pass, the first one's output in LDS alone (32,768 images: 1.7 GB less of memory traffic).
-// A block of 8 waves a CU: waves 0 .. 3 are the first layer's, of image i, while waves 4 .. 7 do the second layer of
-// image i - 1 from the other of two LDS buffers, so that a SIMD has a wave of each and its matrix core one or the
-// other's step. Operands, sums and their order are those of the two kernels above, and so are the results.
-// 300 / 32,768 images: 22 / 693 us as two kernels, 16 / 578 here.
+// A block of 8 waves a CU, in phases of half an image (10 of the first layer's 20 output rows): waves 0 .. 3 are the first
+// layer's, of image i, while waves 4 .. 7 do the second layer of image i - 1 from the other of two LDS buffers; both
+// stage the next half image, the first ones after their products and the second ones before, so that a SIMD, which has
+// a wave of each, scales with one while it multiplies with the other. A row of s_y is padded so that pixel p of the second
+// layer's 81 reads at p times a pixel's words, modulo the banks, across its rows too. Operands, sums and their order are
+// those of the two kernels above, and so are the results. 300 / 32,768 images: 22 / 669 us as two kernels, 16.5 /
+// 535 here (whole images at a time, all waves staging before the products: 16 / 578; operands read one step ahead: 606).
 __global__ void __launch_bounds__(512, 2) k_policy_conv12(const uint8_t* obs, const uint16_t* w1, const uint16_t* bias1,
                                                           const uint16_t* w2, const uint16_t* bias2, uint16_t* y, int64_t n) {
-    constexpr int WORDS = 4 * OBS_PIX / 4, PER = (WORDS + 511) / 512;   // 4-pixel words an image, a thread
-    constexpr int PXW = 40, HI = 20, HO = 9, PIX = HO * HO;             // halfs of a first-layer pixel in LDS: 32 + padding
-    __shared__ __attribute__((aligned(16))) uint16_t s_x[4 * OBS_PIX];
-    __shared__ __attribute__((aligned(16))) uint16_t s_y[2][CONV1_OUT * PXW];
+    constexpr int ROWS = 44, CH = ROWS * 84 / 4, WORDS = 4 * CH, PER = (WORDS + 511) / 512;   // 4-pixel words of a half
+    constexpr int PXW = 40, ROWW = 20 * PXW + 8, HALF_PIX = CONV1_OUT / 2, HO = 9, PIX = HO * HO;   // s_y's, in halfs
+    __shared__ __attribute__((aligned(16))) uint16_t s_x[2][4 * WORDS];
+    __shared__ __attribute__((aligned(16))) uint16_t s_y[2][20 * ROWW];
     const int tid = threadIdx.x, l = tid & 63, wv = (int)uni((uint32_t)tid >> 6), j = l & 31, kg = l >> 5;
     const float sc = (float)(1.0 / 255.0);
+    const int64_t step = gridDim.x, phases = 2 * ((n - blockIdx.x + step - 1) / step);   // blockIdx.x < n
     uint32_t raw[PER];
-    auto load = [&](int64_t b) {
-        const uint32_t* src = (const uint32_t*)(obs + (size_t)b * 4 * OBS_PIX);
+    auto load = [&](int64_t q) {   // the half image of phase q
+        if (q >= phases) return;
+        const uint32_t* src = (const uint32_t*)(obs + (size_t)(blockIdx.x + (q >> 1) * step) * 4 * OBS_PIX) + (q & 1) * (40 * 21);
 #pragma unroll
         for (int i = 0; i < PER; i++) {
-            const int c = tid + 512 * i;
-            raw[i] = src[c < WORDS ? c : 0];
+            const int c = tid + 512 * i, d = c < WORDS ? c : 0;
+            raw[i] = src[d / CH * (OBS_PIX / 4) + d % CH];
         }
     };
-    auto stage = [&]() {
+    auto stage = [&](int64_t q) {
+        if (q >= phases) return;
 #pragma unroll
         for (int i = 0; i < PER; i++) {
             const int c = tid + 512 * i;
-            uint32_t h[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) h[e] = __builtin_bit_cast(uint16_t, (__bf16)((float)((raw[i] >> (8 * e)) & 0xffu) * sc));
-            if (c < WORDS) *(uint2*)(s_x + 4 * c) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+            if (c < WORDS) *(uint2*)(s_x[q & 1] + 4 * c) = scaled_pixels(raw[i], sc);
         }
     };
     auto biases = [&](const uint16_t* bias, float (&bj)[16]) {
 #pragma unroll
         for (int v = 0; v < 16; v++) bj[v] = __uint_as_float((uint32_t)bias[8 * (v >> 2) + 4 * kg + (v & 3)] << 16);
     };
-    // both roles pass the same barriers, two an image
-    const int64_t step = gridDim.x;
-    int64_t b = blockIdx.x;   // below n
-    load(b);
+    // both roles pass the same barriers: one before the first phase and one after each. Phase q reads s_x[q & 1], which
+    // was staged in phase q - 1, and stages the other; an image's s_y is written in its two phases and read in the two after.
+    load(0);
+    stage(0);
+    load(1);
     if (wv < 4) {
         mh_bf16x8 wb[16];
 #pragma unroll
         for (int s = 0; s < 16; s++) wb[s] = as_bf16x8(*(const mh_u32x4*)(w1 + (size_t)j * 256 + 16 * s + 8 * kg));
         float bj[16];
         biases(bias1, bj);
-        for (int turn = 0; b < n; b += step, turn ^= 1) {
-            stage();
-            __syncthreads();
-            if (b + step < n) load(b + step);
-            for (int t = wv; t * 32 < CONV1_OUT; t += 4) {
-                const int m = t * 32 + j, p = m < CONV1_OUT ? m : CONV1_OUT - 1, oy = p / 20, ox = p - oy * 20;
-                const uint16_t* at = s_x + (4 * oy + kg) * 84 + 4 * ox;
-                mh_f32x16 acc = {};
-#pragma unroll
-                for (int s = 0; s < 16; s++) {
-                    const uint2* r = (const uint2*)(at + (s >> 2) * OBS_PIX + 2 * (s & 3) * 84);
-                    const uint2 a = r[0], c = r[1];
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wb[s], as_bf16x8(mh_u32x4{a.x, a.y, c.x, c.y}), acc, 0, 0, 0);
-                }
-                if (m < CONV1_OUT) conv_out(acc, bj, s_y[turn] + m * PXW + 4 * kg, true);
+        weights_arrived();
+        __syncthreads();
+        for (int64_t q = 0; q < phases; q++) {
+            const int part = (int)(q & 1), turn = (int)(q >> 1 & 1);
+            // of the half's 7 tiles two, two, two and one; one, one, three and two beside the second layer's third tile
+            for (int t = wv, by = part ? (wv < 2 ? 8 : 2) : 4; t * 32 < HALF_PIX; t += by) {
+                const int m = t * 32 + j, p = m < HALF_PIX ? m : HALF_PIX - 1, oy = p / 20, ox = p - oy * 20;
+                const uint16_t* at = s_x[part] + (4 * oy + kg) * 84 + 4 * ox;
+                const mh_f32x16 acc = tile_products<16>(wb, [&](int s) {
+                    const uint2* r = (const uint2*)(at + (s >> 2) * (4 * CH) + 2 * (s & 3) * 84);
+                    return mh_u32x4{r[0].x, r[0].y, r[1].x, r[1].y};
+                });
+                if (m < HALF_PIX) conv_out(acc, bj, s_y[turn] + (10 * part + oy) * ROWW + ox * PXW + 4 * kg, true);
             }
+            stage(q + 1);
+            load(q + 2);
             __syncthreads();
         }
     } else {
-        const int half = wv & 1, first = wv < 6 ? 1 : 0;   // tile 1, or 0 and 2: SIMD 0 has one first-layer tile more
+        const int half = wv & 1, first = (wv - 4) >> 1;
         mh_bf16x8 wb[32];
 #pragma unroll
         for (int s = 0; s < 32; s++) wb[s] = as_bf16x8(*(const mh_u32x4*)(w2 + (size_t)(32 * half + j) * 512 + 16 * s + 8 * kg));
         float bj[16];
         biases(bias2 + 32 * half, bj);
-        auto second = [&](int64_t image, int turn) {
-            for (int t = first; t * 32 < PIX; t += 2) {
-                const int m = t * 32 + j, p = m < PIX ? m : PIX - 1, oy = p / HO, ox = p - oy * HO;
-                const uint16_t* at = s_y[turn] + (2 * oy * HI + 2 * ox) * PXW + 8 * kg;
-                mh_f32x16 acc = {};
-#pragma unroll
-                for (int s = 0; s < 32; s++) {   // K = 16 s + 8 kg ..: row s / 8, column s / 2 % 4, half a pixel's channels
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        wb[s], as_bf16x8(*(const mh_u32x4*)(at + ((s >> 3) * HI + ((s >> 1) & 3)) * PXW + 16 * (s & 1))), acc, 0, 0, 0);
-                }
-                if (m < PIX) conv_out(acc, bj, y + ((size_t)image * PIX + m) * 64 + 32 * half + 4 * kg, true);
-            }
+        auto tile = [&](int64_t i, int t) {   // of the block's i-th image
+            const int m = t * 32 + j, p = m < PIX ? m : PIX - 1, oy = p / HO, ox = p - oy * HO;
+            const uint16_t* at = s_y[i & 1] + 2 * oy * ROWW + 2 * ox * PXW + 8 * kg;
+            // K = 16 s + 8 kg ..: row s / 8, column s / 2 % 4, half a pixel's channels
+            const mh_f32x16 acc = tile_products<32>(wb, [&](int s) {
+                return *(const mh_u32x4*)(at + (s >> 3) * ROWW + ((s >> 1) & 3) * PXW + 16 * (s & 1));
+            });
+            if (m < PIX) conv_out(acc, bj, y + ((size_t)(blockIdx.x + i * step) * PIX + m) * 64 + 32 * half + 4 * kg, true);
         };
-        int turn = 0;
-        const int64_t start = b;
-        for (; b < n; b += step, turn ^= 1) {
-            stage();
-            __syncthreads();
-            if (b + step < n) load(b + step);
-            if (b != start) second(b - step, turn ^ 1);
-            __syncthreads();
+        weights_arrived();
+        __syncthreads();
+        // tiles 0 and 1 in an image's first phase, 2 in its second; in the end the last image's
+        for (int64_t q = 0; q < phases + 2; q++) {
+            if (q < phases) {
+                stage(q + 1);
+                load(q + 2);
+            }
+            if (q >= 2 && !(q & 1)) tile((q >> 1) - 1, first);
+            else if (q >= 2 && first == 0) tile((q >> 1) - 1, 2);
+            if (q < phases) __syncthreads();
         }
-        second(b - step, turn ^ 1);
     }
 }
 
