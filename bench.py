@@ -16,7 +16,7 @@ ppo / replay: the PPO rollout feeding a Nature CNN, and the GPU FrameReplay.
 
 The ROM is the real one when the reference's lookup finds it, else this repository's synthetic NROM stand-in
 (tests/golden/roms/mini_smb_*.nes); the JSON line names which. One step is one mh_step_async (k_step,
-k_obs_late, k_reset, k_stack) or, for raw, one frame and its outputs, on torch's current stream with inputs resident in
+k_reset, k_stack) or, for raw, one frame and its outputs, on torch's current stream with inputs resident in
 HBM. Before the W warm-up steps, --preroll untimed steps carry the envs past their first episodes so that the
 timed window has episode ends, resets and early-termination re-emulations in it (the first steps after a
 reset are the cheapest ones). K steps are timed between two device synchronizations; per-kernel times come
@@ -89,42 +89,43 @@ def traffic_from_profiles(profile, workload_key):
         return None
 
 
-# Peak wave64 VALU issue of the chip: 256 CUs x 4 SIMDs, one wave64 VALU instruction per SIMD every 4 cycles
-# (16 lanes wide), at the 2.4 GHz peak engine clock: 614.4 G wave-instructions/s.
-VALU_PEAK_G = 1024 * 2.4 / 4
+# Peak issue of the chip, of wave64 VALU instructions as of scalar ones: 256 CUs x 4 SIMDs, one per SIMD every 4
+# cycles at the 2.4 GHz peak engine clock: 614.4 G wave-instructions/s.
+ISSUE_PEAK_G = 1024 * 2.4 / 4
 
 
-def valu_profile(profile, workload_key):
-    """The committed rocprofv3 SQ-counter summary of a kernel on this workload (profiles/<profile>): VALU
-    instructions per launch, its counter-based issue fraction, the window and the kernel build it measured.
+def issue_profile(profile, workload_key):
+    """The committed rocprofv3 SQ-counter summary of a kernel on this workload (profiles/<profile>): scalar and VALU
+    instructions per launch, the counter-based issue fractions, the window and the kernel build it measured.
     Counters cannot be read inside this run; the summary names its command."""
     v = profile_values(profile, workload_key)
     try:
-        valu = float(v["valu_per_launch"])
-        frac = float(v["valu_issue_fraction"])
+        for k in ("salu_per_launch", "salu_issue_fraction", "valu_per_launch", "valu_issue_fraction"):
+            v[k] = float(v[k])
     except (KeyError, ValueError):
         return None
-    v["_valu"], v["_frac"] = valu, frac
     return v
 
 
-def valu_roofline(kernel, profile, workload_key, kernel_ms, executed_per_launch, traffic, hbm):
-    """The binding roofline of an interpreter kernel: VALU issue. achieved = the VALU wave-instructions of one
-    launch (the committed SQ profile of this workload, same window) / this run's average launch time from HIP
-    events on the launch stream, against VALU_PEAK_G. Falls back to the HBM figure when no profile exists."""
-    v = valu_profile(profile, workload_key)
+def issue_roofline(kernel, profile, workload_key, kernel_ms, executed_per_launch, traffic, hbm):
+    """The binding roofline of an interpreter kernel with a console per wave: scalar issue. achieved = the scalar
+    instructions of one launch (the committed SQ profile of this workload, same window) / this run's average launch
+    time from HIP events on the launch stream, against ISSUE_PEAK_G. Falls back to the HBM figure when no profile exists."""
+    v = issue_profile(profile, workload_key)
     if v is None:
         return dict(hbm, note=f"no SQ-counter profile for this workload in profiles/{profile}: HBM figure only")
-    achieved = v["_valu"] / (kernel_ms * 1e-3) / 1e9
+    achieved = v["salu_per_launch"] / (kernel_ms * 1e-3) / 1e9
     sha = v.get("kernel_source_sha1", "").split(" ")[0]
-    out = {"bound": "valu_issue", "kernel": kernel, "achieved": round(achieved, 2), "peak": VALU_PEAK_G,
-           "unit": "G VALU wave-instructions/s (wave64; 1024 SIMDs x 2.4 GHz / 4 cycles)",
-           "frac": round(achieved / VALU_PEAK_G, 4), "traffic": traffic,
-           "valu_per_launch": v["_valu"],
-           "valu_per_executed_instruction": round(v["_valu"] / max(1.0, executed_per_launch), 2),
-           "frac_counters": v["_frac"], "source": f"profiles/{profile}",
+    out = {"bound": "scalar_issue", "kernel": kernel, "achieved": round(achieved, 2), "peak": ISSUE_PEAK_G,
+           "unit": "G scalar instructions/s (1024 SIMDs x 2.4 GHz / 4 cycles)",
+           "frac": round(achieved / ISSUE_PEAK_G, 4), "traffic": traffic,
+           "salu_per_launch": v["salu_per_launch"], "valu_per_launch": v["valu_per_launch"],
+           "salu_per_executed_instruction": round(v["salu_per_launch"] / max(1.0, executed_per_launch), 2),
+           "valu_per_executed_instruction": round(v["valu_per_launch"] / max(1.0, executed_per_launch), 2),
+           "frac_counters": v["salu_issue_fraction"], "valu_frac_counters": v["valu_issue_fraction"],
+           "source": f"profiles/{profile}",
            "profile_kernel_source_sha1": sha, "profile_matches_build": sha == kernel_source_sha1()}
-    for k in ("window", "active_lane_fraction", "occupancy_waves_per_simd", "lds_bank_conflict_per_lds_instr"):
+    for k in ("window", "occupancy_waves_per_simd", "lds_bank_conflict_per_lds_instr"):
         if k in v:
             out[k] = v[k]
     return out
@@ -474,7 +475,7 @@ def env_line(args, metric, n, m, workload_key, config, sq_profile, dtype="u8"):
         "metric": metric, "value": round(value, 1), "unit": "agent-steps/s", "n_gpus": 1, "steps": args.steps,
         "warmup": args.warmup, "ms_per_step": round(m["dt"] * 1e3 / args.steps, 3), "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": dtype, "data": "synthetic", "config": config,
-        "roofline": valu_roofline("k_step", sq_profile, workload_key, k_step_ms, executed, traffic, hbm),
+        "roofline": issue_roofline("k_step", sq_profile, workload_key, k_step_ms, executed, traffic, hbm),
         "hbm_roofline": hbm,
         "stages_ms_per_step": {k: round(v, 3) for k, v in m["stages"].items()},
         "p_done": round(m["p_done"], 5),
@@ -658,7 +659,7 @@ def run_raw(args):
         "config": {"workload": f"raw: {n} consoles, 1-1 via a {prologue}-frame Start/none prologue, then SIMPLE_MOVEMENT "
                                f"buttons from default_rng(1) per console and frame", "envs": n, "rom": rom_name,
                    "rom_sha1": rom_sha, "outputs_per_frame": "RGB24 screen (184,320 B) + RAM (2,048 B) per console"},
-        "roofline": valu_roofline("k_raw", "k_raw_sq_counters_raw.md", workload_key, k_raw_ms, (instr - ff) / frames,
+        "roofline": issue_roofline("k_raw", "k_raw_sq_counters_raw.md", workload_key, k_raw_ms, (instr - ff) / frames,
                                   None, hbm),
         "hbm_roofline": hbm,
         "k_raw_ms": round(k_raw_ms, 4),
