@@ -642,7 +642,7 @@ struct Core {
         lds_sync();
         pal_dirty = 0;
     }
-    // v at the start of the i-th line after this one (i > 0), both layers on: fine_y_step i times, and copy_h. (Coarse y
+    // v at the start of the i-th line after this one, both layers on: fine_y_step i times, and copy_h. (Coarse y
     // 30 and 31 wrap to 0 without the mirror switch that 29 makes.)
     __device__ __forceinline__ uint32_t v_lines_on(uint32_t i) const {
         uint32_t yy = ((v >> 5) & 31u) * 8u + ((v >> 12) & 7u), mirror = 0;   // i <= 240
@@ -1137,7 +1137,9 @@ struct Core {
                 // its later lists: evaluated at the end of the line before, from sprite 0 on
                 const bool listed = i == 0 || (oam_addr < 4 && (uint32_t)(py - 1 - y0) < (uint32_t)h);
                 if (!listed || py > 239 || px > 255 || px < x0 || px < edge) return false;
-                const uint32_t vp = coarse_x_added(i ? v_lines_on((uint32_t)i) : v, (uint32_t)inc_count(x0, px));
+                // (past dot 257 v has stepped to the next line already)
+                const uint32_t vl = i ? v_lines_on((uint32_t)(i - (pcyc > 257 ? 1 : 0))) : v;
+                const uint32_t vp = coarse_x_added(vl, (uint32_t)inc_count(x0, px));
                 return bg_pattern(px, vp) && sprite0_pattern(ow, px, py);
             };
             uint64_t b = 0;

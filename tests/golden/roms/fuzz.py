@@ -15,15 +15,19 @@ Two families, both fully determined by a seed:
   VRAM, scroll and address writes in that state (some with +32 increments, one a bulk $2007 loop) and
   turns rendering back on at its end, so the next frame draws with the fine x, v and name tables written
   while the screen was off.
+* ``wait_rom(seed)``: a sprite-0 wait (`LDA $2002 / AND #$40 / BEQ`) entered anywhere on the lines of sprite 0, over
+  a background with one or two opaque rows per tile, so that the hit is on a certain line; the main program counts
+  the time that is left. OAM DMA in few frames or none, and sprites at the bottom (y 232-239), whose list is
+  evaluated on the last line and drawn on line 0 of the next frame.
 """
 from __future__ import annotations
 
 import numpy as np
 
 try:
-    from .asm6502 import _OPS, _SIZE, ines
+    from .asm6502 import _OPS, _SIZE, assemble, ines
 except ImportError:  # loaded as a plain module
-    from asm6502 import _OPS, _SIZE, ines
+    from asm6502 import _OPS, _SIZE, assemble, ines
 
 _MNEMONICS = sorted(_OPS)
 _UNSAFE = {"JMP", "JSR", "RTS", "RTI", "BRK", "PHA", "PLA", "PHP", "PLP", "TXS", "SEI", "CLI",
@@ -222,3 +226,146 @@ def program_rom(seed: int, length: int = 400, screen_off: bool = False) -> bytes
     assert g.pc < 0xFFF0, "program too long"
     g.img[0x7FFA:0x8000] = bytes([nmi & 0xFF, nmi >> 8, reset & 0xFF, reset >> 8, irq & 0xFF, irq >> 8])
     return ines(bytes(g.img), bytes(chr_), int(rng.integers(0, 2)))
+
+
+# PPU set up from the reset routine: palette, name tables of tile 1, OAM by DMA from page 2
+_SETUP = """
+.org $8000
+reset:
+    SEI
+    CLD
+    LDX #$FF
+    TXS
+    LDA #0
+    STA $2000
+    STA $2001
+    LDA #$3F
+    STA $2006
+    LDA #0
+    STA $2006
+    LDX #0
+pal:
+    LDA palette,X
+    STA $2007
+    INX
+    CPX #32
+    BNE pal
+    LDA #$20
+    STA $2006
+    LDA #0
+    STA $2006
+    LDA #1
+    LDY #15
+    LDX #0
+fill:
+    STA $2007
+    DEX
+    BNE fill
+    DEY
+    BPL fill
+    LDX #0
+copy:
+    LDA sprites,X
+    STA $0200,X
+    INX
+    BNE copy
+    STX $2003
+    LDA #2
+    STA $4014
+"""
+
+
+def _tile(rows):
+    """A tile of pattern 1 in the given rows."""
+    return bytes(0xFF if r in rows else 0 for r in range(8)) + bytes(8)
+
+
+def _image(src, sprites, palette, chr_tiles, mirroring):
+    def data(label, bs):
+        return f"{label}:\n" + "".join(f"    .byte {', '.join(map(str, bs[i:i + 16]))}\n" for i in range(0, len(bs), 16))
+    prg = assemble(_SETUP + src + data("palette", list(palette)) + data("sprites", list(sprites)) +
+                   ".org $FFFA\n    .word nmi, reset, reset\n")
+    chr_ = bytearray(0x2000)
+    for page in (0, 0x1000):
+        for k, t in enumerate(chr_tiles):
+            chr_[page + 16 * k:page + 16 * k + 16] = t
+    return ines(prg, bytes(chr_), mirroring)
+
+
+def wait_rom(seed: int) -> bytes:
+    rng = np.random.default_rng(seed)
+    tall = int(rng.integers(0, 2))
+    y0, x0 = int(rng.integers(24, 200)), int(rng.integers(0, 250))
+    rows = set(rng.choice(8, int(rng.integers(1, 3)), replace=False).tolist())
+    oam = np.full((64, 4), 0xF8, np.uint8)
+    oam[0] = (y0, 2, 0, x0)
+    for k in range(int(rng.integers(0, 10))):                  # at the bottom, and a few elsewhere
+        y = int(rng.integers(232, 240)) if rng.random() < 0.8 else int(rng.integers(60, 232))
+        oam[1 + k] = (y, 2 + int(rng.integers(0, 2)), int(rng.integers(0, 4)), int(rng.integers(0, 256)))
+    # cycles from the NMI to a dot on the sprite's lines: the vertical blank and pre-render lines, then 113.67 a line
+    to = int(341 * (21 + y0 + rng.random() * (16 if tall else 8)) / 3)
+    dma = rng.random() < 0.3
+    spent = 80 + (514 if dma else 0)
+    outer, inner = divmod(max(to - spent, 20), 1287)           # LDX #0: 256 DEX / BNE, and the outer loop's own 9
+    src = f"""
+    LDA #${0x90 | tall << 5:02X}
+    STA $2000
+    LDA #$1E
+    STA $2001
+main:
+    INC $11
+    BNE main
+    INC $12
+    JMP main
+nmi:
+    PHA
+    TXA
+    PHA
+    TYA
+    PHA
+"""
+    if dma:
+        src += "    LDA $13\n    AND #7\n    BNE nodma\n    LDA #2\n    STA $4014\nnodma:\n"
+    src += f"""
+    LDA $2002
+    LDA #{int(rng.integers(0, 256))}
+    STA $2005
+    LDA #{int(rng.integers(0, 240))}
+    STA $2005
+    INC $13
+    LDY #{outer}
+    BEQ rest
+slow:
+    LDX #0
+spin:
+    DEX
+    BNE spin
+    DEY
+    BNE slow
+rest:
+    LDX #{min(max(inner // 5, 1), 255)}
+last:
+    DEX
+    BNE last
+{"    NOP" + chr(10) if rng.random() < 0.5 else ""}{"    LDA $10" + chr(10) if rng.random() < 0.5 else ""}wait:
+    LDA $2002
+    AND #$40
+    BEQ wait
+    LDA #{int(rng.integers(0, 256))}
+    STA $2005
+    LDA #0
+    STA $2005
+    INC $14
+    PLA
+    TAY
+    PLA
+    TAX
+    PLA
+    RTI
+"""
+    tiles = [_tile(()), _tile(rows), _tile(range(8)), _tile({0, 3, 7})]
+    return _image(src, oam.reshape(-1), rng.integers(0, 64, 32).tolist(), tiles, int(rng.integers(0, 2)))
+
+
+# of wait_rom: waits that read $2002 in the horizontal blank of one of sprite 0's lines, ahead of the hit
+WAIT_IN_BLANK = (31, 48, 58, 79, 85)

@@ -16,6 +16,7 @@
 //                    'R' -> obs;  'T' actions:i64[n] -> obs rew:f32[n] term:u8[n] trunc:u8[n] info:i64[10n]
 //                    ram[2048 n] fin ep_ret:f64[n] ep_len:i64[n];  'Q' -> frames bad_ops instructions ff
 //                    hack_redraws:i64, exit
+//   hits <seed>:     the sprite-0 wait's prediction against single calls (see run_hits) -> states checked, exit
 //   plant <bytes>:   reads one byte past a buffer of that size (the tests check that the sanitizers catch it)
 #include <cstdio>
 #include <cstdlib>
@@ -117,6 +118,48 @@ int run_raw(const char* rom_file) {
             die("unknown raw command");
         }
     }
+}
+
+// The call that Core::calls_to_hit predicts, from every call of random pictures' lines at which sprite 0 heads the list and
+// has not hit, against the call at which running the PPU one call at a time raises the hit. Prints the states compared.
+int run_hits(uint64_t seed) {
+    auto rnd = [&]() { seed = seed * 6364136223846793005ull + 1442695040888963407ull; return (uint32_t)(seed >> 33); };
+    uint64_t states = 0, found = 0;
+    for (int trial = 0; trial < 40; trial++) {
+        std::vector<uint8_t> m(MEM_ROWS), chr(0x2000);
+        std::vector<uint32_t> gp(LDS_GP_REGION);
+        for (auto& b : chr) b = rnd() % 8 ? 0 : (uint8_t)rnd();
+        for (int i = ROW_VRAM; i < ROW_OAM; i++) m[i] = (uint8_t)rnd();
+        for (int i = ROW_OAM; i < ROW_PAL; i++) m[i] = (uint8_t)rnd();
+        const uint32_t y0 = rnd() % 220;
+        m[ROW_OAM] = (uint8_t)y0;
+        Core k{};
+        k.m = m.data(); k.gp = gp.data(); k.chr = chr.data(); k.np = 64; k.nt_bits = rnd() & 1 ? 0xau : 0xcu;
+        k.ppu_flags = PF_SHOW_BG | PF_SHOW_SPR | (rnd() & (PF_HIDE_EDGE_BG | PF_HIDE_EDGE_SPR | PF_LONG_SPR | PF_BG_PAGE | PF_SPR_PAGE));
+        k.oam_addr = rnd() % 8 ? rnd() % 4 : rnd() & 0xffu;
+        k.fine_x = rnd() & 7u; k.v = rnd() & 0x7fffu; k.t = rnd() & 0x7fffu;
+        k.pstate = ST_RENDER; k.scanline = (int)(y0 > 2 ? y0 - 2 : 0); k.pcyc = 1; k.pend_line = k.scanline - 1;
+        if (k.pend_line < 0) k.pend_line = 239;
+        std::vector<int32_t> at, said, until;   // a state's call, what is predicted, the first dot past the lines looked at
+        while (k.pstate == ST_RENDER && !k.s0hit && k.scanline <= (int)y0 + 17) {
+            if (k.sprite0_first()) {
+                at.push_back(k.ppu_calls);
+                said.push_back(k.ppu_calls + k.calls_to_hit());
+                until.push_back(k.ppu_calls + k.calls_until(k.scanline + 8 < 240 ? k.scanline + 8 : 240, 1));
+            }
+            k.ppu_run(1);
+        }
+        for (size_t i = 0; i < at.size(); i++) {
+            const int32_t want = k.s0hit && k.ppu_calls <= until[i] ? k.ppu_calls : until[i];
+            if (said[i] != want) {
+                std::fprintf(stderr, "hits: trial %d, call %d: predicted %d, was %d\n", trial, at[i], said[i], want);
+                return 1;
+            }
+        }
+        states += at.size(); found += k.s0hit;
+    }
+    std::printf("%llu %llu\n", (unsigned long long)states, (unsigned long long)found);
+    return 0;
 }
 
 // ------------------------------------------------------------------ vector env
@@ -364,10 +407,11 @@ int run_env(const char* cfg_file) {
 }  // namespace
 
 int main(int argc, char** argv) {
-    if (argc != 3) die("usage: host_driver raw <rom> | env <config>");
+    if (argc != 3) die("usage: host_driver raw <rom> | env <config> | hits <seed> | plant <bytes>");
     const std::string mode = argv[1];
     if (mode == "raw") return run_raw(argv[2]);
     if (mode == "env") return run_env(argv[2]);
+    if (mode == "hits") return run_hits(std::strtoull(argv[2], nullptr, 10));
     if (mode == "plant") {   // a deliberate out-of-bounds read: the sanitizer build must abort on it
         std::vector<uint8_t> row(std::atoi(argv[2]));
         volatile uint8_t v = row.data()[row.size()];

@@ -99,6 +99,12 @@ def test_raw_random_fuzz(seed):
     _raw_run(fuzz.random_rom(seed), 4, scaled(40), seed=seed, render_p=0.5, backup_p=0.05)
 
 
+@pytest.mark.parametrize("seed", fuzz.WAIT_IN_BLANK)
+def test_raw_sprite0_wait(seed):
+    # the wait loop reads $2002 in the horizontal blanks of sprite 0's lines
+    _raw_run(fuzz.wait_rom(seed), 2, scaled(24), seed=seed)
+
+
 CONFIGS = {
     "default": dict(),
     "sticky_noop": dict(sticky=0.25, noop_max=30),

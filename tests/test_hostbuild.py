@@ -15,8 +15,9 @@ import pytest
 from conftest import ROOT
 
 import make_golden as G
+import fuzz
 from build_roms import rom_path
-from cpu_libs import gray_lut, rng_state
+from cpu_libs import OracleRaw, gray_lut, rng_state
 
 HB = os.path.join(ROOT, "tests", "hostbuild")
 EXE = os.path.join(HB, "host_driver_san")
@@ -162,3 +163,25 @@ def test_hostbuild_env_golden(exe, tmp_path, config):
     assert not bad, f"first mismatching step {bad[0] - 1}"
     frames, bad_ops, instr, ff, redraws = venv.finish()
     assert frames == g["frames"] and bad_ops == 0 and 0 <= ff <= instr and redraws >= 0
+
+
+@pytest.mark.parametrize("seed", [1, 2])
+def test_hostbuild_sprite0_wait_prediction(exe, seed):
+    """Where a sprite-0 wait may skip to, from every dot of the sprite's lines (the horizontal blanks among them, where v
+    has stepped to the next line): the call that raises the hit when the PPU runs one call at a time."""
+    r = subprocess.run([exe, "hits", str(seed)], capture_output=True, text=True, env=SAN_ENV, timeout=60)
+    assert r.returncode == 0, r.stderr[-2000:]
+    states, hits = map(int, r.stdout.split())
+    assert states > 50000 and hits > 10
+
+
+@pytest.mark.parametrize("seed", fuzz.WAIT_IN_BLANK)
+def test_hostbuild_sprite0_wait_roms(exe, tmp_path, seed):
+    """Sprite-0 waits whose reads fall in the horizontal blanks of the sprite's lines, against the oracle."""
+    rom = fuzz.wait_rom(seed)
+    con, cpu = HostRaw(exe, rom, str(tmp_path)), OracleRaw(rom)
+    for f in range(12):
+        con.frame(0, True)
+        cpu.frame(0, True)
+        assert np.array_equal(con.ram, cpu.ram) and np.array_equal(con.screen, cpu.screen), f
+    assert con.finish()[:2] == (cpu.bad_ops(), cpu.instructions())
