@@ -684,10 +684,10 @@ struct Core {
     __device__ __forceinline__ void draw_lines(uint32_t count, int x0, int x1) {
         if (pal_dirty) build_gray_palette();
         MH_LDS uint32_t* const ent = gp + GP_SPRITES;
-        // any sprite on any of the lines?
+        // any sprite on any of the lines? (the pending evaluation may be the last frame's, of line 239)
         bool some = false;
         if (show_spr()) {
-            if (pend_line >= 0 && count > 1) some = in_range(scanline + (int)count - 2, count) != 0;
+            if (pend_line >= 0 && count > 1) some = (in_range(scanline + (int)count - 2, count) | in_range(pend_line)) != 0;
             else some = true;
         }
         for (uint32_t base = 0; base < count; base += DRAW_LINES) draw_batch(base, count, x0, x1, some, ent);

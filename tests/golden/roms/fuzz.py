@@ -19,6 +19,9 @@ Two families, both fully determined by a seed:
   a background with one or two opaque rows per tile, so that the hit is on a certain line; the main program counts
   the time that is left. OAM DMA in few frames or none, and sprites at the bottom (y 232-239), whose list is
   evaluated on the last line and drawn on line 0 of the next frame.
+
+And ``lag_rom()``: a minimal game by the RAM protocol of the env layer (boot, busy state, time, position) with OAM DMA
+every eighth frame only and sprites at y 239, for the env-level drivers.
 """
 from __future__ import annotations
 
@@ -367,5 +370,89 @@ last:
     return _image(src, oam.reshape(-1), rng.integers(0, 64, 32).tolist(), tiles, int(rng.integers(0, 2)))
 
 
+# of wait_rom: frames without DMA with sprites at the bottom and none on the first lines, up to the first catch-up
+BOTTOM_SPRITES = (1, 2, 3, 5)
 # of wait_rom: waits that read $2002 in the horizontal blank of one of sprite 0's lines, ahead of the hit
 WAIT_IN_BLANK = (31, 48, 58, 79, 85)
+
+
+def lag_rom() -> bytes:
+    """RAM protocol of the env layer: Start on the title starts the game (time $07F8-$07FA as digits, player state $0E =
+    8); the time counts down, the position $6D / $86 and the sprites move right."""
+    oam = np.full((64, 4), 0xF8, np.uint8)
+    for k in range(10):
+        oam[1 + k] = (239, 2, k & 3, 11 + 24 * k)        # on no line but 0 of the next frame
+    src = """
+    LDA #0
+    STA $0E
+    STA $07F8
+    STA $07F9
+    STA $07FA
+    LDA #$90
+    STA $2000
+    LDA #$1E
+    STA $2001
+main:
+    JMP main
+nmi:
+    LDA $2002
+    LDA $13
+    AND #7
+    BNE nodma
+    LDA #2
+    STA $4014
+nodma:
+    INC $13
+    LDA $13
+    STA $2005
+    LDA #0
+    STA $2005
+    LDA #1
+    STA $4016
+    LDA #0
+    STA $4016
+    LDX #4
+start:
+    LDA $4016
+    DEX
+    BNE start
+    AND #1
+    BEQ run
+    LDA $07F8
+    BNE run
+    LDA #4
+    STA $07F8
+run:
+    LDA $07F8
+    BEQ done
+    LDA #8
+    STA $0E
+    LDA $13
+    AND #3
+    BNE move
+    LDA $07FA
+    BNE tick
+    LDA #9
+    STA $07FA
+    DEC $07F8
+    JMP move
+tick:
+    DEC $07FA
+move:
+    INC $86
+    BNE shift
+    INC $6D
+shift:
+    LDX #36
+slide:
+    INC $0207,X
+    DEX
+    DEX
+    DEX
+    DEX
+    BPL slide
+done:
+    RTI
+"""
+    tiles = [_tile(()), _tile(()), _tile({0, 1, 2, 3, 4, 5, 6, 7})]
+    return _image(src, oam.reshape(-1), [(7 * i + 15) % 64 for i in range(32)], tiles, 1)

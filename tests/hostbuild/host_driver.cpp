@@ -9,7 +9,8 @@
 // console's rows is an access outside its buffer.
 //
 // Protocol on stdin / stdout (little-endian binary), one session per process:
-//   raw <rom file>:  'F' buttons:u8 render:u8 -> ram[2048] screen[61440]; 'B' backup; 'S' restore;
+//   raw <rom file>:  'F' buttons:u8 render:u8 -> ram[2048] screen[61440]; 'B' backup; 'S' restore; 'M' frames:u8
+//                    buttons:u8 render:u8 -> the same, after that many frames between one load and one store;
 //                    'Q' -> bad_ops:i64 instructions:i64 ff_instructions:i64, exit
 //   env <config file> (rom_len:i64 rom n:i32 levels:i32[3n] lut:u8[256] skip max_steps:i32 sticky:f64
 //                    noop_max maxpool frame_stack:i32 rng:u64[6n]):
@@ -94,10 +95,23 @@ int run_raw(const char* rom_file) {
     A.power_on = 0;
     for (;;) {
         const char c = get1<char>();
-        if (c == 'F') {
+        if (c == 'F' || c == 'M') {
+            const int frames = c == 'M' ? get1<uint8_t>() : 1;
             buttons[0] = get1<uint8_t>();
             A.render = get1<uint8_t>();
-            raw_lane(A, L.ctx(0), 0);
+            if (c == 'F') {
+                raw_lane(A, L.ctx(0), 0);
+            } else {   // as the env kernels run the frames of an agent step
+                Console con;
+                attach(con, L.ctx(0), np);
+                con.load(mem.data(), sc.data(), 0);
+                con.gray = screen.data() + gray_lane_offset(0);
+                con.render = A.render != 0;
+                con.set_buttons0(buttons[0]);
+                for (int k = 0; k < frames; k++) con.frame();
+                con.store(mem.data(), sc.data(), 0);
+                bad[0] += con.bad_ops; instr[0] += con.instructions; ff[0] += con.ff_instructions;
+            }
             uint8_t ram[2048];
             for (int i = 0; i < 2048; i++) ram[i] = mem[(size_t)(ROW_RAM + i) * np];
             std::vector<uint8_t> scr(GRAY_PIX);

@@ -177,6 +177,24 @@ def test_env_vs_oracle_two_waves():
     _env_run(names, "headline", scaled(60))
 
 
+@pytest.mark.parametrize("config", ["default", "maxpool_sticky"])
+def test_env_without_dma_every_frame(config):
+    # the sprite list of a frame's last line is pending when the next frame of the step draws line 0 with it
+    import torch
+
+    from fast_mario_env_amd import HipVecEnv
+    rom, names, kw = fuzz.lag_rom(), ["1-1", "1-2", "4-1"], CONFIGS[config]
+    cpu = OracleVec(rom, _levels(names), 3, seed=3, **kw)
+    gpu = HipVecEnv(names, 3, seed=3, rom=rom, **kw)
+    assert np.array_equal(cpu.reset(), gpu.reset().cpu().numpy())
+    rng = np.random.default_rng(0)
+    for t in range(20):
+        a = rng.integers(0, 7, 3)
+        want, got = cpu.step(a), gpu.step(torch.from_numpy(a).cuda())
+        for w, g in zip(want[:4], got[:4]):
+            assert np.array_equal(w, g.cpu().numpy()), t
+
+
 def _env_run(names, config, steps):
     import torch
 

@@ -17,7 +17,7 @@ from conftest import ROOT
 import make_golden as G
 import fuzz
 from build_roms import rom_path
-from cpu_libs import OracleRaw, gray_lut, rng_state
+from cpu_libs import OracleRaw, OracleVec, gray_lut, rng_state
 
 HB = os.path.join(ROOT, "tests", "hostbuild")
 EXE = os.path.join(HB, "host_driver_san")
@@ -74,6 +74,12 @@ class HostRaw:
 
     def frame(self, buttons, render):
         self.proc.send(b"F" + bytes([int(buttons) & 255, int(bool(render))]))
+        self.ram = np.frombuffer(self.proc.recv(2048), np.uint8)
+        self.screen = np.frombuffer(self.proc.recv(240 * 256), np.uint8).reshape(240, 256)
+
+    def frames(self, count, buttons, render):
+        """`count` frames between one load of the console and one store, as the env kernels run an agent step's."""
+        self.proc.send(b"M" + bytes([count, int(buttons) & 255, int(bool(render))]))
         self.ram = np.frombuffer(self.proc.recv(2048), np.uint8)
         self.screen = np.frombuffer(self.proc.recv(240 * 256), np.uint8).reshape(240, 256)
 
@@ -185,3 +191,33 @@ def test_hostbuild_sprite0_wait_roms(exe, tmp_path, seed):
         cpu.frame(0, True)
         assert np.array_equal(con.ram, cpu.ram) and np.array_equal(con.screen, cpu.screen), f
     assert con.finish()[:2] == (cpu.bad_ops(), cpu.instructions())
+
+
+@pytest.mark.parametrize("seed", fuzz.BOTTOM_SPRITES + fuzz.WAIT_IN_BLANK[:2])
+def test_hostbuild_frames_without_a_store(exe, tmp_path, seed):
+    """Several frames between a load and a store, most of them without DMA: the list evaluated on the last line of one
+    frame is still pending when line 0 of the next is drawn with it."""
+    rom = fuzz.wait_rom(seed)
+    con, cpu = HostRaw(exe, rom, str(tmp_path)), OracleRaw(rom)
+    for f in range(6):
+        con.frames(4, 0, True)
+        for _ in range(4):
+            cpu.frame(0, True)
+        assert np.array_equal(con.ram, cpu.ram), (f, "ram")
+        assert np.array_equal(con.screen, cpu.screen), (f, np.flatnonzero((con.screen != cpu.screen).any(1))[:4])
+    assert con.finish()[:2] == (cpu.bad_ops(), cpu.instructions())
+
+
+@pytest.mark.parametrize("maxpool", [False, True])
+def test_hostbuild_env_without_dma_every_frame(exe, tmp_path, maxpool):
+    lv = [(1, 1, 1), (1, 2, 1), (4, 1, 1)]
+    kw = dict(seed=3, sticky=0.25, noop_max=4, maxpool=maxpool, skip=4)
+    rom = fuzz.lag_rom()
+    env, cpu = HostVec(exe, rom, lv, 3, str(tmp_path), **kw), OracleVec(rom, lv, 3, **kw)
+    assert np.array_equal(env.reset(), cpu.reset())
+    rng = np.random.default_rng(0)
+    for t in range(20):
+        a = rng.integers(0, 7, 3)
+        for got, want in zip(env.step(a), cpu.step(a)):
+            assert np.array_equal(got, want), t
+    assert env.finish()[0] == cpu.frames()
