@@ -1,4 +1,4 @@
-// Bodies of the env kernels: one env / level / cache entry per wave (reset_lane, canon_lane: per lane). The __global__
+// Bodies of the env kernels: one env / level / cache entry per wave (reset_lane: per lane). The __global__
 // wrappers in mario_hip.hip stage the cartridge in LDS and call these.
 #pragma once
 #include <cmath>
@@ -573,28 +573,31 @@ __device__ inline void raw_lane(const RawArgs& A, const LaneCtx& x, uint32_t e) 
     A.ff[e] += c.ff_instructions;
 }
 
-// Canonical state dump of console e (layout in include/mario_hip.h).
-__device__ inline void canon_lane(const uint8_t* mem, const uint32_t* sc, uint32_t np, uint32_t e, uint8_t* o) {
+// Canonical state dump of console e (layout in include/mario_hip.h), by `lanes` lanes together.
+__device__ inline void canon_lane(const uint8_t* mem, const uint32_t* sc, uint32_t np, uint32_t e, uint8_t* o, uint32_t lane,
+                                  uint32_t lanes) {
     auto w = [&](int k) { return sc[(size_t)k * np + e]; };
-    auto put = [&](int off, uint64_t v, int bytes) { for (int b = 0; b < bytes; b++) o[off + b] = (uint8_t)(v >> (8 * b)); };
-    for (int i = 0; i < 80; i++) o[i] = 0;
-    const uint64_t iter = (uint64_t)w(S_ITER_LO) | ((uint64_t)w(S_ITER_HI) << 32);
-    put(0, iter, 8);
-    put(8, iter + (int64_t)(int32_t)w(S_EXEC_REL), 8);
-    put(16, 3 * iter, 8);
-    put(24, w(S_PCYC), 4); put(28, w(S_SCANLINE), 4);
-    put(32, w(S_PC), 2); put(34, w(S_V), 2); put(36, w(S_T), 2); put(38, w(S_INC), 2);
-    const int order[] = {S_SP, S_A, S_X, S_Y, S_P, S_ZERO_SKIP, S_JOY_STROBE0, S_JOY_STROBE1, S_JOY_BUTTONS0,
-                         S_JOY_BUTTONS1, S_JOY_BITS0, S_JOY_BITS1, S_PSTATE, S_EVEN, S_VBLANK, S_S0HIT,
-                         S_FIRST_WRITE, S_DATA_BUFFER, S_OAM_ADDR, S_FINE_X, S_SHOW_BG, S_SHOW_SPR,
-                         S_HIDE_EDGE_BG, S_HIDE_EDGE_SPR, S_LONG_SPR, S_NMI_EN, S_BG_PAGE, S_SPR_PAGE, S_NSL};
-    for (int i = 0; i < 29; i++) o[40 + i] = (uint8_t)w(order[i]);
-    const uint32_t nsl = w(S_NSL);
-    const uint64_t sl = (uint64_t)w(S_SL_LO) | ((uint64_t)w(S_SL_HI) << 32);
-    for (uint32_t i = 0; i < 8; i++) o[69 + i] = i < nsl ? (uint8_t)(sl >> (8 * i)) : 0;
+    if (lane == 0) {
+        auto put = [&](int off, uint64_t v, int bytes) { for (int b = 0; b < bytes; b++) o[off + b] = (uint8_t)(v >> (8 * b)); };
+        const uint64_t iter = (uint64_t)w(S_ITER_LO) | ((uint64_t)w(S_ITER_HI) << 32);
+        put(0, iter, 8);
+        put(8, iter + (int64_t)(int32_t)w(S_EXEC_REL), 8);
+        put(16, 3 * iter, 8);
+        put(24, w(S_PCYC), 4); put(28, w(S_SCANLINE), 4);
+        put(32, w(S_PC), 2); put(34, w(S_V), 2); put(36, w(S_T), 2); put(38, w(S_INC), 2);
+        const int order[] = {S_SP, S_A, S_X, S_Y, S_P, S_ZERO_SKIP, S_JOY_STROBE0, S_JOY_STROBE1, S_JOY_BUTTONS0,
+                             S_JOY_BUTTONS1, S_JOY_BITS0, S_JOY_BITS1, S_PSTATE, S_EVEN, S_VBLANK, S_S0HIT,
+                             S_FIRST_WRITE, S_DATA_BUFFER, S_OAM_ADDR, S_FINE_X, S_SHOW_BG, S_SHOW_SPR,
+                             S_HIDE_EDGE_BG, S_HIDE_EDGE_SPR, S_LONG_SPR, S_NMI_EN, S_BG_PAGE, S_SPR_PAGE, S_NSL};
+        for (int i = 0; i < 29; i++) o[40 + i] = (uint8_t)w(order[i]);
+        const uint32_t nsl = w(S_NSL);
+        const uint64_t sl = (uint64_t)w(S_SL_LO) | ((uint64_t)w(S_SL_HI) << 32);
+        for (uint32_t i = 0; i < 8; i++) o[69 + i] = i < nsl ? (uint8_t)(sl >> (8 * i)) : 0;
+        put(77, 0, 3);
+    }
     const uint32_t rows[4][3] = {{80, ROW_OAM, 256}, {336, ROW_PAL, 32}, {368, ROW_VRAM, 2048}, {2416, ROW_RAM, 2048}};
     for (int k = 0; k < 4; k++)
-        for (uint32_t i = 0; i < rows[k][2]; i++) o[rows[k][0] + i] = mem[mem_offset(np, e, rows[k][1] + i)];
+        for (uint32_t i = lane; i < rows[k][2]; i += lanes) o[rows[k][0] + i] = mem[mem_offset(np, e, rows[k][1] + i)];
 }
 
 }  // namespace mh

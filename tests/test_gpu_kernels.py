@@ -248,3 +248,35 @@ def test_replay_draw_is_the_tensor_operations(n_envs, batch, n_step):
     rb._ptr.zero_()
     with pytest.raises(ValueError):
         rb.draw(4, n_step)
+
+
+@pytest.mark.parametrize("n", [1, 3, 65])
+def test_console_outputs_at_any_alignment(n):
+    """RAM, machine state and RGB of consoles in slots other than their env's, into outputs of every alignment: what the
+    console's own dump and its palette screen hold, and nothing past the output."""
+    from fast_mario_env_amd import HipRawNES, HipVecEnv, palette_rgb
+    from fast_mario_env_amd._native import check, lib
+    names = ["4-1", "1-1", "8-4"] * (n // 3) + ["1-1"] * (n % 3)
+    env, raw = HipVecEnv(names, n, seed=1, rom=ROM, device="cuda:0", **WRAP), HipRawNES(ROM, n, device="cuda:0")
+    env.reset()
+    for t in range(3):
+        env.step(torch.arange(n, device="cuda:0") % 7)
+    for f in range(45):
+        raw.frame(torch.tensor([(8 if f % 2 == 0 else i) & 255 for i in range(n)], dtype=torch.uint8, device="cuda:0"))
+    pal = torch.from_numpy(palette_rgb().reshape(-1).copy()).to("cuda:0")
+    rgb = torch.from_numpy(palette_rgb()).to("cuda:0")[(raw.screen & 63).long()]
+
+    def out(call, size, offset):
+        buf = torch.full((size + 32,), 0xa5, dtype=torch.uint8, device="cuda:0")
+        check(call(buf.data_ptr() + offset), "out")
+        torch.cuda.synchronize()
+        assert bool((buf[:offset] == 0xa5).all()) and bool((buf[offset + size:] == 0xa5).all())
+        return buf[offset:offset + size]
+
+    for off in (0, 1, 4, 8):
+        for con, ram, canon in ((env, lib().mh_env_ram, lib().mh_env_canon), (raw, lib().mh_raw_ram, lib().mh_raw_canon)):
+            state = out(lambda p: canon(con.h, p, 0), n * 4464, off).view(n, 4464)
+            assert torch.equal(out(lambda p: ram(con.h, p, 0), n * 2048, off).view(n, 2048), state[:, 2416:])
+        got = out(lambda p: lib().mh_raw_screen_rgb(raw.h, pal.data_ptr(), p, 0), n * 61440 * 3, off)
+        assert torch.equal(got, rgb.reshape(-1))
+    env.close()
