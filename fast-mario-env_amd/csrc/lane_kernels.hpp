@@ -476,7 +476,7 @@ __device__ inline void cache_lane(const CacheArgs& A, const LaneCtx& x, int ci) 
 // picture is about 2,000), 15 from 2^18 * 1.5.
 constexpr int WORK_BUCKETS = 16;
 __device__ inline uint32_t work_bucket(uint32_t executed) {
-    const uint32_t v = executed | 2048u;   // at least 2^11
+    const uint32_t v = executed < 2048u ? 2048u : executed;
     const uint32_t lg = 31u - (uint32_t)__builtin_clz(v);
     const uint32_t b = 2 * (lg - 11) + (v >> (lg - 1) & 1u);
     return b < WORK_BUCKETS ? b : WORK_BUCKETS - 1;

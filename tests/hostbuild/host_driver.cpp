@@ -18,6 +18,7 @@
 //                    ram[2048 n] fin ep_ret:f64[n] ep_len:i64[n];  'Q' -> frames bad_ops instructions ff
 //                    hack_redraws:i64, exit
 //   hits <seed>:     the sprite-0 wait's prediction against single calls (see run_hits) -> states checked, exit
+//   bucket <n>:      the work bucket of a step of n executed instructions
 //   plant <bytes>:   reads one byte past a buffer of that size (the tests check that the sanitizers catch it)
 #include <cstdio>
 #include <cstdlib>
@@ -421,11 +422,15 @@ int run_env(const char* cfg_file) {
 }  // namespace
 
 int main(int argc, char** argv) {
-    if (argc != 3) die("usage: host_driver raw <rom> | env <config> | hits <seed> | plant <bytes>");
+    if (argc != 3) die("usage: host_driver raw <rom> | env <config> | hits <seed> | bucket <n> | plant <bytes>");
     const std::string mode = argv[1];
     if (mode == "raw") return run_raw(argv[2]);
     if (mode == "env") return run_env(argv[2]);
     if (mode == "hits") return run_hits(std::strtoull(argv[2], nullptr, 10));
+    if (mode == "bucket") {
+        std::printf("%u\n", work_bucket((uint32_t)std::strtoul(argv[2], nullptr, 10)));
+        return 0;
+    }
     if (mode == "plant") {   // a deliberate out-of-bounds read: the sanitizer build must abort on it
         std::vector<uint8_t> row(std::atoi(argv[2]));
         volatile uint8_t v = row.data()[row.size()];

@@ -221,3 +221,13 @@ def test_hostbuild_env_without_dma_every_frame(exe, tmp_path, maxpool):
         for got, want in zip(env.step(a), cpu.step(a)):
             assert np.array_equal(got, want), t
     assert env.finish()[0] == cpu.frames()
+
+
+def test_hostbuild_work_buckets(exe):
+    """Half-octaves: bucket b from 2^(11 + b / 2) instructions, half as many more for odd b; 0 below, 15 above."""
+    def bucket(n):
+        return int(subprocess.run([exe, "bucket", str(n)], capture_output=True, text=True, env=SAN_ENV, timeout=60).stdout)
+    for b in range(1, 16):
+        lo = (2048 << b // 2) * (3 if b % 2 else 2) // 2
+        assert (bucket(lo - 1), bucket(lo)) == (b - 1, b), lo
+    assert bucket(0) == 0 and bucket(2**32 - 1) == 15
