@@ -38,6 +38,16 @@ def exe():
     return EXE
 
 
+def test_hostbuild_is_rebuilt_when_a_header_changes(exe):
+    """The Makefile names every header that the host driver includes."""
+    r = subprocess.run(["/opt/rocm/llvm/bin/clang++", "-std=c++17", "-DMH_LANES_PER_ENV=1", "-I", ".", "-I",
+                        "../../fast-mario-env_amd/csrc", "-MM", "host_driver.cpp"], cwd=HB, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    used = {os.path.basename(f) for f in r.stdout.replace("\\\n", " ").split()[1:]}
+    rule = open(os.path.join(HB, "Makefile")).read().split("host_driver_san:", 1)[1].split("\n\t")[0]
+    assert used and used <= {os.path.basename(f) for f in rule.replace("\\\n", " ").split()}
+
+
 class _Proc:
     def __init__(self, exe, mode, path):
         self.p = subprocess.Popen([exe, mode, path], stdin=subprocess.PIPE, stdout=subprocess.PIPE,
