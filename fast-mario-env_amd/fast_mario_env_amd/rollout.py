@@ -103,11 +103,18 @@ _PACKED = 1684128   # MH_POLICY_PACKED
 
 def _transformed(*ts):
     """Whether something follows the operations on these tensors, which a kernel called by address would pass by:
-    forward-mode tangents, vmap and the like, a dispatch mode (a FLOP counter, fake tensors), tracing or compiling."""
+    forward-mode tangents, vmap and the like, a dispatch mode (a FLOP counter, fake tensors) or a function mode (but
+    torch's default device), tracing or compiling. torch keeps most of it under private names: without one of them
+    the answer is yes, and the layers' own operations run."""
     torch = _torch()
-    return (torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0
-            or torch.jit.is_tracing() or torch.compiler.is_compiling()
-            or any(torch._C._functorch.is_functorch_wrapped_tensor(t) for t in ts))
+    try:
+        device_mode = getattr(getattr(torch.utils, "_device", None), "DeviceContext", ())
+        return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.autograd.forward_ad._current_level >= 0
+                or torch._C._len_torch_dispatch_stack() > 0
+                or any(not isinstance(m, device_mode) for m in torch.overrides._get_current_function_mode_stack())
+                or any(torch._C._functorch.is_functorch_wrapped_tensor(t) for t in ts))
+    except AttributeError:
+        return True
 
 
 def _packed_params(convs, fc, obs):

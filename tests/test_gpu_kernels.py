@@ -186,11 +186,20 @@ def test_policy_heads_against_64_bits(n, actions):
 
 
 def test_policy_transforms_take_the_layers():
-    """What follows the tensor operations (tangents, vmap over head weights, a dispatch mode) sees them without autograd too."""
+    """What follows the tensor operations (tangents, vmap over head weights, dispatch and function modes) sees them without
+    autograd too."""
     from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
     from torch.utils.flop_counter import FlopCounterMode
-    from fast_mario_env_amd.rollout import make_net
+    from fast_mario_env_amd.rollout import gae, make_net
     net = make_net(seed=4)
+    called = []
+
+    class Names(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            called.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
     obs = torch.randint(0, 256, (3, 4, 84, 84), dtype=torch.uint8, device="cuda")
     w, b = net.pi.weight.detach().clone(), net.pi.bias.detach()
     def logits(weight):
@@ -206,7 +215,11 @@ def test_policy_transforms_take_the_layers():
             assert forward_ad.unpack_dual(out).tangent is not None
         with FlopCounterMode(display=False) as count:
             net(obs)
+        with Names():
+            net(obs)
+            gae(*[x.cuda() for x in _rollout(3, 5, 1)])
     assert count.get_total_flops() >= 2 * 3 * 512 * (3136 + 8)
+    assert called.count("linear") == 3 and "zeros_like" in called
 
 
 def _draw_by_tensor_operations(rb, batch, n_step):

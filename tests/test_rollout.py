@@ -35,6 +35,35 @@ def test_gae_matches_recurrence():
     assert np.allclose(a0.numpy(), rew + 0.9 * nxt - val, rtol=1e-5, atol=1e-5)
 
 
+def test_what_follows_tensor_operations_is_seen(monkeypatch):
+    """Kernels called by address stand back for what follows the tensor operations, and where torch has no name for it."""
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    from torch.utils.flop_counter import FlopCounterMode
+    from fast_mario_env_amd.rollout import _transformed
+    x = torch.ones(3)
+
+    class Count(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert not _transformed(x)
+    with torch.device("cpu"):
+        assert not _transformed(x)
+    for mode in (forward_ad.dual_level(), FlopCounterMode(display=False), Count()):
+        with mode:
+            assert _transformed(x)
+    seen = []
+    torch.vmap(lambda t: (seen.append(_transformed(t)), t)[1])(torch.ones(2, 3))
+    assert seen == [True]
+    for owner, name in ((torch.autograd.forward_ad, "_current_level"), (torch._C, "_len_torch_dispatch_stack"),
+                        (torch.overrides, "_get_current_function_mode_stack"), (torch._C, "_functorch")):
+        with monkeypatch.context() as m:
+            m.delattr(owner, name)
+            assert _transformed(x), name
+    assert not _transformed(x)
+
+
 class _Stacker:
     """Explicit frame stacking of k frames with resets to [0, ..., 0, frame]."""
     def __init__(self, n, k):
