@@ -213,12 +213,8 @@ struct Stepper {
     // frames count like any other. Frames that were not rendered are re-emulated here the same way. Frame
     // K-2 (max-pool) was rendered in the first pass, and running it again from the same state with the same
     // buttons repeats it exactly: its state after the first pass is saved instead, only its partner K-3 runs
-    // again, the saved state is restored, and frame K-2 is counted a second time. No lane then runs more
-    // than K frames (plus hack frames) in a step, which would hold up its whole wave.
-    // Written as a state machine around ONE console frame so that the emulator is inlined once: a lane that
-    // re-emulates does so while the other lanes of its wave still run their remaining agent frames, and it
-    // waits (skipping the frame call) until the iterations of the wave's own rendered frames, K-2 and K-1,
-    // so that its rendered re-emulation does not turn an unrendered iteration of the wave into a rendered one.
+    // again, the saved state is restored, and frame K-2 is counted a second time.
+    // Written as a state machine around ONE console frame so that the emulator is inlined once.
     __device__ __forceinline__ double agent_step(int act0, bool want_obs, bool* term) {
         const int K = cfg.skip;
         const bool mp = cfg.maxpool != 0;
@@ -229,15 +225,12 @@ struct Stepper {
         int rf = -1;                       // agent frame being re-emulated (-1: the first pass)
         uint8_t b_prev = 0, b_cur = 0;     // buttons of agent frames i-1 and i
         uint32_t n0 = 0, b0 = 0, f0 = 0;   // instruction, bad-op and fast-forward counters at the start of agent frame i
-        int it = 0, resume_at = 0;         // loop iterations so far; the iteration a re-emulation starts at
         uint8_t* slot = gray0;
         bool undrawn = false;              // the hack frame just run was not drawn; its start state is in slot 0
         bool redraw = false;               // this iteration runs that hack frame again, drawn
         uint32_t hn = 0, hb = 0, hf = 0;   // instruction, bad-op and fast-forward counters at that start state
         ev.hack_redraws = 0;
         for (;;) {
-            if (rf >= 0 && it < resume_at) { it++; continue; }   // waiting for the wave's rendered frames
-            it++;
             uint8_t buttons = 0;
             if (hack) {
                 c.set_ram(0x7a0, 0);
@@ -316,7 +309,6 @@ struct Stepper {
                 } else {
                     rf = (mp && i >= 1) ? i - 1 : i;
                 }
-                resume_at = K - (keep_last ? 1 : i - rf + 1);   // K minus the frames to run again
                 restore_console(c, snap(rf & 1));
             } else if (rf < i) {
                 // frame last-1 again, then its hack frames (it did not end the episode)

@@ -264,6 +264,8 @@ __device__ __forceinline__ void obs_period_take(int sy, const float (&rs)[21], f
 }
 
 // ------------------------------------------------------------------ arguments
+// (consoles of count np: memory of console e at mem_offset(np, e, 0), register word w at sc[w * np + e]; frames at
+// gray_lane_offset())
 constexpr int MAX_CHR_BANKS = 4;   // ROMs per env instance: one PRG, a CHR bank each (the rom_mode variants)
 
 struct RomArgs {
@@ -306,8 +308,8 @@ struct BootArgs {
     uint32_t nlp;
     const int* levels;           // 3 * nl
     const uint8_t* key_bank;     // nl: CHR bank of each (level, ROM) key
-    uint8_t* mem; uint32_t* sc;  // boot consoles [row * nlp + l]
-    uint8_t* gray;               // frame buffer of nlp lanes (4-pixel words)
+    uint8_t* mem; uint32_t* sc;  // boot consoles
+    uint8_t* gray;               // nlp frames
     int64_t* x0; int64_t* t0;
     uint32_t* err;
 };
@@ -319,8 +321,8 @@ struct CacheArgs {
     int nl, nk, nc;
     uint32_t nlp, ncp;
     const uint8_t* boot_mem; const uint32_t* boot_sc; const int64_t* x0; const int64_t* t0;
-    uint8_t* mem; uint32_t* sc;          // cache consoles [row * ncp + c]
-    uint8_t* gray;                       // 2 frame buffers of ncp lanes (4-pixel words)
+    uint8_t* mem; uint32_t* sc;          // cache consoles
+    uint8_t* gray;                       // 2 buffers of ncp frames
     uint8_t* snap_mem; uint32_t* snap_sc;  // 2 snapshot slots of the cache consoles' layout
     int64_t* cx; int64_t* ct; int32_t* clives; int32_t* cdraws; uint8_t* cboot;
     uint64_t* cframes; uint64_t* cinstr; uint64_t* cff; uint32_t* cbad;
@@ -333,7 +335,7 @@ struct StepArgs {
     uint32_t np;
     uint8_t* mem; uint32_t* sc;
     uint32_t* ev;                 // env words [w * np + e]
-    uint8_t* gray;                // 2 frame buffers of np lanes (4-pixel words)
+    uint8_t* gray;                // 2 buffers of np frames
     uint8_t* snap_mem; uint32_t* snap_sc;   // 2 snapshot slots of the live layout (re-emulation)
     const int64_t* actions;
     float* rew; uint8_t* term; uint8_t* trunc; int32_t* info; double* ep_ret_out; int32_t* ep_len_out;
@@ -358,12 +360,11 @@ struct RawArgs {
     RomArgs R;
     int n; uint32_t np;
     uint8_t* mem; uint32_t* sc;
-    uint8_t* screen;             // [pix * np + e], palette values
+    uint8_t* screen;             // np frames of palette values
     const uint8_t* buttons;      // n
     int render;
     uint32_t* bad; uint32_t* instr; uint32_t* ff;
     int power_on;
-    int cpw;                     // consoles per wave: 1
 };
 
 // ------------------------------------------------------------------ env words

@@ -143,7 +143,7 @@ __global__ void EMU_BOUNDS k_cache(CacheArgs A) {
 // (longest-first list scheduling; a busy run, an area transition or a death, lasts several steps). k_step appends each
 // env to the next step's buckets itself, and k_reset, which follows it on the stream, turns the two lists over: no
 // launch and no pass of its own. The order within a bucket is that of the appends; no result depends on it.
-// Measured at 32,768 / 65,536 envs: k_step 9.0 / 18.8 ms, against 10.6 (unsorted) / 22.9 ms with blocks of 16 envs in
+// Measured at 32,768 / 65,536 envs when it came: k_step 9.0 / 18.8 ms, against 10.6 (unsorted) / 22.9 ms with blocks of 16 envs in
 // the order of each block's slowest env (8.4 / 16.1 ms of it are the waves' mean busy time).
 struct StepQueue {
     uint32_t side;                          // the lists this step reads; it appends to the others
@@ -153,13 +153,13 @@ struct StepQueue {
 // the envs of bucket b, side s: list[(s * WORK_BUCKETS + b) * np ..]
 
 // What bounds it: scalar issue. A SIMD issues one scalar instruction per 4 cycles whichever of its waves it is from; the
-// headline step (32,768 envs of 1-1) is 103,000 scalar, 69,000 vector and 16,000 branch instructions per env, of which
-// the 5,217 6502 instructions are about 45,000 scalar ones (scalar issue 77% busy, vector 51%). Why one console per wave, against 16 per wave in
-// lockstep (4 lanes each, every opcode's work as selects, 15 to 12 of 16 consoles active): a lockstep iteration issues
-// ~470 instructions for ~12 6502 instructions but each env waits for all of them; here a 6502 instruction is ~17
-// instructions and nothing waits for another console. Measured (k_step, the same envs): 256 envs 11.6 -> 1.03 ms,
-// 4,096 envs 19.9 -> 2.99 ms, 32,768 envs 14.57 -> 10.64 ms, 65,536 envs of 32 levels 40.9 -> 22.9 ms (9.0 and 18.8 with
-// the queue).
+// headline step (32,768 envs of 1-1) is 98,000 scalar, 68,000 vector and 15,000 branch instructions per env, of which
+// the 5,150 6502 instructions are about 45,000 scalar ones (scalar issue 71% busy, vector 49%). Why one console per wave, against
+// 16 per wave in lockstep (4 lanes each, every opcode's work as selects, 15 to 12 of 16 consoles active): a lockstep
+// iteration issues ~470 instructions for ~12 6502 instructions but each env waits for all of them; here a 6502
+// instruction is ~17 instructions and nothing waits for another console. Measured when it came (k_step, the same
+// envs): 256 envs 11.6 -> 1.03 ms, 4,096 envs 19.9 -> 2.99 ms, 32,768 envs 14.57 -> 10.64 ms, 65,536 envs of 32 levels
+// 40.9 -> 22.9 ms (9.0 and 18.8 with the queue; 7.4 and 14.6 now, by what run_frame, calls_to_hit and cpu_gfx950.hpp name).
 // q null: every env has its wave.
 __global__ void EMU_BOUNDS k_step(StepArgs A, StepQueue* q, uint32_t* list) {
     ROM_LDS
@@ -1005,7 +1005,7 @@ MhEnv* mh_create_roms(const uint8_t* roms, const int64_t* rom_lens, int n_roms, 
         g_err = "invalid arguments";
         return nullptr;
     }
-    if ((uint32_t)n > MAX_ENVS) { g_err = "too many envs (at most 979,648: console memory takes 32-bit offsets)"; return nullptr; }
+    if ((uint32_t)n > MAX_ENVS) { g_err = "too many envs (at most 979,648)"; return nullptr; }
     // the cartridge image: ROM 0's PRG, then the CHR of every ROM; the ROMs must agree on PRG and mirroring
     std::vector<uint8_t> img;
     uint16_t nt[4];
@@ -1050,9 +1050,8 @@ MhEnv* mh_create_roms(const uint8_t* roms, const int64_t* rom_lens, int n_roms, 
         env_level[i] = li;
     }
     h->nl = (int)lv.size() / 3; h->nlp = pad64(h->nl);
-    // Console slots grouped by key, ordered by (world, stage, area, ROM), envs of a key in index order: a wave then
-    // holds envs of one level (one game code path) wherever the batch mixes levels, so its lanes diverge less.
-    // State lives in slot order; actions, outputs, RAM and state dumps stay in env order (slot_env).
+    // Console slots grouped by key, ordered by (world, stage, area, ROM), envs of a key in index order, so that envs
+    // of one level, which do about the same, run beside one another. State lives in slot order; actions, outputs, RAM and state dumps stay in env order (slot_env).
     std::vector<int32_t> slot_env(h->np, 0), env_slot(n);
     {
         std::vector<int> order(n);
@@ -1342,7 +1341,7 @@ int64_t mh_env_bytes(MhEnv* h) {
 MhRaw* mh_raw_create(const uint8_t* rom, int64_t rom_len, int n, int device) {
     g_err.clear();
     if (n < 1) { g_err = "invalid arguments"; return nullptr; }
-    if ((uint32_t)n > MAX_ENVS) { g_err = "too many consoles (at most 979,648: console memory takes 32-bit offsets)"; return nullptr; }
+    if ((uint32_t)n > MAX_ENVS) { g_err = "too many consoles (at most 979,648)"; return nullptr; }
     // (a wave runs one console whatever the variable says; an ill-formed value is an error, as it was)
     if (const char* f = getenv("MH_RAW_CONSOLES_PER_WAVE"); f && *f) {
         const int cpw = atoi(f);
@@ -1382,14 +1381,14 @@ MhRaw* mh_raw_create(const uint8_t* rom, int64_t rom_len, int n, int device) {
     h->R.rom = d_rom; h->R.lut = d_lut; h->R.recs = d_recs; h->R.n_chr = 1;
     h->R.nt_bits = 0;
     for (int i = 0; i < 4; i++) h->R.nt_bits |= (nt[i] ? 1u : 0u) << i;
-    RawArgs ra{h->R, h->n, h->np, h->mem, h->sc, h->screen, nullptr, 0, h->bad, h->instr, h->ff, 1, 1};
+    RawArgs ra{h->R, h->n, h->np, h->mem, h->sc, h->screen, nullptr, 0, h->bad, h->instr, h->ff, 1};
     hipLaunchKernelGGL(k_raw, h->lr.grid, h->lr.block, 0, 0, ra);
     if (!ok(hipDeviceSynchronize(), "raw power-on")) { delete h; return nullptr; }
     return h;
 }
 int mh_raw_frame(MhRaw* h, const uint8_t* d_buttons, int render, void* stream) {
     if (!h || !d_buttons) return -1;
-    RawArgs ra{h->R, h->n, h->np, h->mem, h->sc, h->screen, d_buttons, render, h->bad, h->instr, h->ff, 0, 1};
+    RawArgs ra{h->R, h->n, h->np, h->mem, h->sc, h->screen, d_buttons, render, h->bad, h->instr, h->ff, 0};
     hipLaunchKernelGGL(k_raw, h->lr.grid, h->lr.block, 0, (hipStream_t)stream, ra);
     CK(hipGetLastError());
     return 0;

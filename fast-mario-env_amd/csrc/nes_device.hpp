@@ -39,9 +39,10 @@
 namespace mh {
 
 constexpr int ROW_RAM = 0, ROW_VRAM = 2048, ROW_OAM = 4096, ROW_PAL = 4352, MEM_ROWS = 4384;
-// Most envs (consoles) of one instance: the padded count np (a multiple of 64) keeps MEM_ROWS * np below 2^32.
+// Most envs (consoles) of one instance, a limit of the interface: MEM_ROWS * np, np the padded count (a multiple of 64),
+// stays below 2^32, and so do the host build's offsets and the output kernels' indexes.
 constexpr uint32_t MAX_ENVS = (uint32_t)((0xffffffffull / MEM_ROWS) & ~63ull);
-static_assert(MAX_ENVS == 979648 && (uint64_t)MEM_ROWS * MAX_ENVS <= 0xffffffffull, "32-bit console memory offsets");
+static_assert(MAX_ENVS == 979648 && (uint64_t)MEM_ROWS * MAX_ENVS <= 0xffffffffull, "the interface's limit");
 constexpr int LANES = MH_LANES_PER_ENV;
 static_assert(LANES == 1 || LANES == 64, "a console runs on a wave's 64 lanes, or on the host's one");
 constexpr bool ON_GPU = LANES == 64;
@@ -963,9 +964,8 @@ struct Core {
 
     // The data operation of decode word D: the result byte and the new flags, from the packed registers regs
     // (a | x << 8 | y << 16 | sp << 24), the data operand m (the first operand byte when nothing was read), the
-    // flags p and whether a data operand was read. Every choice is a select on bits of the decode word: chains of
-    // equality tests on one small field would be lowered to a branch tree, i.e. exec-mask branches on every
-    // instruction of a divergent wave.
+    // flags p and whether a data operand was read. Every choice is a select on bits of the decode word (chains of equality
+    // tests on one small field would be lowered to a branch tree).
     struct AluOut { uint32_t r8, p; };
     __device__ __forceinline__ static AluOut alu_op(uint32_t D, uint32_t regs, uint32_t m, uint32_t p, bool rd) {
         using namespace dec;
@@ -1526,9 +1526,9 @@ struct Console {
     }
     __device__ __forceinline__ void frame() {
         // The kernel ends with its slowest wave, and the waves of a SIMD compete for its issue slots: a wave at an
-        // earlier frame of its agent step issues first (frames 0 and 1 of the step at priority 3, frame 2 at 2, later
-        // frames, hack frames and re-emulations at 1; the observations after the frame loop at 0), so a wave that
-        // falls behind takes the slots of a SIMD-mate that is ahead.
+        // earlier frame since its console's load issues first (frames 0 and 1 at priority 3, frame 2 at 2, later ones at 1;
+        // the observations after the frame loop at 0; a snapshot taken back is a load too), so a wave that falls behind
+        // takes the slots of a SIMD-mate that is ahead.
         const uint32_t n = nframe++;
         if (n < 2) __builtin_amdgcn_s_setprio(3);
         else if (n < 3) __builtin_amdgcn_s_setprio(2);
