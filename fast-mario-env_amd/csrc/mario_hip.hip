@@ -1335,6 +1335,7 @@ int64_t mh_state_bytes(void) { return (int64_t)MEM_ROWS + 4LL * S_COUNT; }
 int64_t mh_env_bytes(MhEnv* h) {
     if (!h) return -1;
     int64_t per = 3LL * (MEM_ROWS + 4LL * S_COUNT) + 4LL * E_COUNT + 2LL * GRAY_PIX + OBS_PIX;
+    if (h->queue) per += 2LL * WORK_BUCKETS * 4;
     return per * h->np / h->n;
 }
 
