@@ -35,7 +35,7 @@ def test_step_queue_edges(extra):
                 assert torch.equal(a[k:k + m], b), (t, k)
     assert torch.equal(big.canon()[n - m:], parts[1][1].canon())
     # a queue's two lists of 16 buckets are among an env's bytes (whole instances, padded to 64 envs, per env)
-    own = 3 * (4384 + 164) + 144 + 2 * 61440 + 7056
+    own = 3 * (4384 + 160) + 144 + 2 * 61440 + 7056
     assert big.bytes_per_env() == (own + (128 if extra else 0)) * ((n + 63) // 64 * 64) // n
     assert parts[0][1].bytes_per_env() == own * 64 // m
     for e in (big, parts[0][1], parts[1][1]):
