@@ -10,7 +10,8 @@ instances of 32 envs on their own PCG64 streams (env_offset), on a thread pool. 
 stack, reward, terminated, truncated, the ten info values and the 2 KB of RAM; at every episode end the final
 observation stack and the episode return and length; at the end the whole console state, the frame,
 instruction and bad-opcode counts and the early-termination re-emulations. One JSON line per configuration:
-episodes, flag clears, the largest x_pos, mismatches (the first ones, with step and env) and the run time.
+episodes, flag clears, the largest x_pos, mismatches (the first ones, with step and env), the hash of the kernel
+sources that ran and the run time.
 Actions: over the 7 SIMPLE_MOVEMENT actions from default_rng(2024 + configuration index), uniform except for the
 "runner" configuration (POLICY), which reaches the flagpole; the ROM is the repository's synthetic stand-in
 (tests/golden/roms), the only one this environment has.
@@ -33,6 +34,7 @@ for p in (ROOT, os.path.join(ROOT, "fast-mario-env_amd"), os.path.join(ROOT, "te
 
 import numpy as np  # noqa: E402
 
+from bench import kernel_source_sha1  # noqa: E402
 from build_roms import rom_path  # noqa: E402
 from cpu_libs import OracleVec  # noqa: E402
 
@@ -135,7 +137,7 @@ def run(config, steps, seed, log):
            "frames": int(gpu.frames), "instructions": int(gpu.instructions()),
            "ff_instructions": int(gpu.ff_instructions()), "reemulations": re_c,
            "bad_ops": int(gpu.bad_ops()), "oracle_bad_ops": int(bad_c), "mismatches": mism, "ok": not mism,
-           "rom": "synthetic stand-in (tests/golden/roms, vanilla)", "secs": round(time.perf_counter() - t0, 1)}
+           "rom": "synthetic stand-in (tests/golden/roms, vanilla)", "kernel_source_sha1": kernel_source_sha1(), "secs": round(time.perf_counter() - t0, 1)}
     pool.shutdown()
     for c in cpu:
         c.close()
