@@ -44,7 +44,7 @@ HBM_PEAK_GBS = 8000.0
 # bytes k_step must move per env and agent step: console state read + write,
 # env words read + write, action, reward / term / trunc / info out, the new 84x84 observation out;
 # ep stats on episode end.
-STATE_BYTES = 4384 + 4 * 41
+STATE_BYTES = 4384 + 4 * 40
 ENV_WORD_BYTES = 4 * 30
 OBS = 84 * 84
 K_STEP_BYTES = 2 * STATE_BYTES + 2 * ENV_WORD_BYTES + 8 + 4 + 1 + 1 + 40 + OBS

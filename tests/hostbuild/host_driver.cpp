@@ -5,7 +5,7 @@
 // the same lane bodies the GPU kernels call, one console after another, so that the device code itself runs
 // under AddressSanitizer and UndefinedBehaviorSanitizer. The orchestration around the lane bodies (boot,
 // reset cache, reset, step, observation, frame stack) follows libmario_hip.so's host side and kernels
-// (mario_hip.hip); the arrays have the GPU's lane-interleaved layouts, sized exactly, so an access outside a
+// (mario_hip.hip); the consoles' arrays are interleaved (row or word r of console e at r * np + e), sized exactly, so an access outside a
 // console's rows is an access outside its buffer.
 //
 // Protocol on stdin / stdout (little-endian binary), one session per process:

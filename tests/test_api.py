@@ -124,9 +124,8 @@ def test_create_roms_validates_before_the_gpu():
         fme.HipVecEnv("1-1", 5, rom_mode=["vanilla", "pixel", "downsample", "rectangle", "other"])
 
 
-def test_create_rejects_more_envs_than_32bit_offsets_address():
-    """The console memory (4,384 rows of np bytes) is addressed with 32-bit offsets from its base: both
-    creators refuse more than 979,648 envs, with a message, before they touch a device."""
+def test_create_rejects_more_envs_than_the_limit():
+    """Both creators refuse more than 979,648 envs, with a message, before they touch a device."""
     L = ctypes.CDLL(_native.lib_path())
     L.mh_create_roms.restype = ctypes.c_void_p
     L.mh_raw_create.restype = ctypes.c_void_p
@@ -148,8 +147,8 @@ def test_create_rejects_more_envs_than_32bit_offsets_address():
 
 @pytest.mark.parametrize("value", ["3", "32", "0", "x"])
 def test_raw_create_rejects_bad_consoles_per_wave(monkeypatch, value):
-    """MH_RAW_CONSOLES_PER_WAVE (k_raw's consoles per wave, a power of two up to 16) is checked at creation,
-    before the device is touched."""
+    """MH_RAW_CONSOLES_PER_WAVE (without effect since a wave runs one console: 1, 2, 4, 8 or 16) is still checked at
+    creation, before the device is touched."""
     L = ctypes.CDLL(_native.lib_path())
     L.mh_raw_create.restype = ctypes.c_void_p
     L.mh_last_error.restype = ctypes.c_char_p

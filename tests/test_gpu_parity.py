@@ -17,9 +17,6 @@ from cpu_libs import OracleRaw, OracleVec
 pytestmark = pytest.mark.gpu
 
 MINI = open(rom_path("vanilla"), "rb").read()
-# k_raw's consoles per wave: "auto" lets the library choose (few consoles: one per wave, every SIMD busy), 16 fills
-# every wave, so that lanes of one wave run different consoles and force catch-ups on each other
-CPW = ["auto", "16"]
 
 
 def _first_diff(a, b):
@@ -27,13 +24,11 @@ def _first_diff(a, b):
     return d[:8].tolist()
 
 
-def _raw_run(rom, n, frames, seed, render_p=0.5, backup_p=0.0, rgb=False, cpw="auto", monkeypatch=None):
+def _raw_run(rom, n, frames, seed, render_p=0.5, backup_p=0.0, rgb=False):
     import torch
 
     from fast_mario_env_amd import HipRawNES, palette_rgb
     pal = palette_rgb()
-    if cpw != "auto":
-        monkeypatch.setenv("MH_RAW_CONSOLES_PER_WAVE", cpw)
     gpu = HipRawNES(rom, n)
     cpu = [OracleRaw(rom) for _ in range(n)]
     rng = np.random.default_rng(seed)
@@ -67,9 +62,15 @@ def _raw_run(rom, n, frames, seed, render_p=0.5, backup_p=0.0, rgb=False, cpw="a
     assert gpu.instructions() == sum(c.instructions() for c in cpu)
 
 
-@pytest.mark.parametrize("cpw", CPW)
-def test_raw_mini_smb(cpw, monkeypatch):
-    _raw_run(MINI, 8, scaled(120), seed=1, rgb=True, cpw=cpw, monkeypatch=monkeypatch)
+@pytest.mark.parametrize("seed", [1, 2])
+def test_raw_mini_smb(seed):
+    _raw_run(MINI, 8, scaled(120), seed=seed, rgb=True)
+
+
+def test_raw_consoles_per_wave_variable(monkeypatch):
+    # accepted at creation, without effect
+    monkeypatch.setenv("MH_RAW_CONSOLES_PER_WAVE", "16")
+    _raw_run(MINI, 3, scaled(20), seed=3)
 
 
 @pytest.mark.parametrize("seed", [0, 1, 2])
@@ -77,21 +78,16 @@ def test_raw_program_fuzz(seed):
     _raw_run(fuzz.program_rom(seed), 4, scaled(80), seed=seed, backup_p=0.05)
 
 
-@pytest.mark.parametrize("cpw", CPW + ["4"])
-def test_raw_program_fuzz_two_waves(cpw, monkeypatch):
-    # 40 consoles; with 16 per wave two full waves and a partial one, so catch-ups that one lane forces on the
-    # others of its wave (PPU register accesses at different points) are compared across many lanes
-    _raw_run(fuzz.program_rom(3), 40, scaled(40), seed=3, backup_p=0.05, cpw=cpw, monkeypatch=monkeypatch)
+@pytest.mark.parametrize("seed", [3, 4, 5])
+def test_raw_program_fuzz_40_consoles(seed):
+    _raw_run(fuzz.program_rom(seed), 40, scaled(40), seed=seed, backup_p=0.05)
 
 
-@pytest.mark.parametrize("cpw", CPW)
-@pytest.mark.parametrize("seed", [0, 1, 3])
-def test_raw_screen_off_fuzz(seed, cpw, monkeypatch):
+@pytest.mark.parametrize("seed", [0, 1, 2, 3, 4, 5])
+def test_raw_screen_off_fuzz(seed):
     # an NMI handler that makes its VRAM, scroll and address writes with rendering off (a bulk $2007 loop among
-    # them) and turns rendering on at its end; 40 consoles: a console often runs alone in its wave (always, with
-    # one console per wave) and its lone runs make those writes themselves
-    _raw_run(fuzz.program_rom(seed, screen_off=True), 40, scaled(60), seed=seed, backup_p=0.05, cpw=cpw,
-             monkeypatch=monkeypatch)
+    # them), without a catch-up of the PPU, and turns rendering on at its end
+    _raw_run(fuzz.program_rom(seed, screen_off=True), 40, scaled(60), seed=seed, backup_p=0.05)
 
 
 @pytest.mark.parametrize("seed", [0, 1, 2])
@@ -171,8 +167,8 @@ def test_env_rom_modes_per_env():
     assert gpu.bad_ops() == 0
 
 
-def test_env_vs_oracle_two_waves():
-    # 40 envs (two full 16-env waves and a partial one) with the headline wrappers
+def test_env_vs_oracle_40_envs():
+    # 40 envs of 8 levels, in slots of another order than the envs', with the headline wrappers
     names = ["1-1", "4-1", "8-4", "2-3", "1-2", "5-2", "3-3", "7-1"] * 5
     _env_run(names, "headline", scaled(60))
 
@@ -290,11 +286,9 @@ def test_hack_frames_redrawn_vs_oracle():
 
 
 def test_env_2048_in_kernel_observations():
-    """2,048 envs (128 waves) with the headline wrappers, every env every step against the oracle. k_step's waves
-    take tickets in the order they finish their frame loops; the first 64 compute their envs' observations inside
-    k_step (obs_tail after the frame loop, behind its release / acquire fences) and only the last 64 leave them
-    to k_obs_late. With 64 waves or fewer every wave defers, so the smaller parity tests cover k_obs_late alone.
-    The oracle runs as 16 instances of 128 envs (their own PCG64 streams by env_offset) on a thread pool."""
+    """2,048 envs with the headline wrappers, every env every step against the oracle: blocks of 8 waves, several a
+    SIMD, whose waves compute their env's observation (obs_tail, behind its release / acquire fences) while others
+    still draw frames. The oracle runs as 16 instances of 128 envs (their own PCG64 streams by env_offset) on a thread pool."""
     import os
     from concurrent.futures import ThreadPoolExecutor
 
@@ -304,7 +298,6 @@ def test_env_2048_in_kernel_observations():
     kw = CONFIGS["headline"]
     names = ["1-1", "4-1", "8-4", "2-3", "1-2", "5-2", "3-3", "7-1"] * 256
     n, m = len(names), 128
-    assert n // 16 > 64      # waves of 16 envs beyond the 64 that defer
     pool = ThreadPoolExecutor(min(16, os.cpu_count() or 1))
     cpu = list(pool.map(lambda k: OracleVec(MINI, _levels(names[k:k + m]), m, seed=3, env_offset=k, **kw),
                         range(0, n, m)))

@@ -1,11 +1,11 @@
 """GPU parity at the benchmark workloads' real sizes.
 
-The small parity tests fit in one workgroup (128 env slots). These run many:
-- the headline configuration exactly as bench.py measures it: 32,768 envs of 1-1 (2,048 waves in 256 workgroups of
-  8 waves, the benchmark's launch shape), max-pool, bench.py's own action stream over its 300 preroll steps and its
-  default warm-up and timed window (405 steps);
-- 4,096 envs of mixed levels with the headline wrappers (the launch shrinks to 256 one-wave workgroups, one per CU);
-- the 65,536-env divergence-stress instance (512 workgroups of 8 waves; its second frame buffer starts 4.03e9
+The small parity tests give a CU a few envs at most. These fill the chip:
+- the headline configuration exactly as bench.py measures it: 32,768 envs of 1-1 (256 workgroups of 16 waves that
+  take envs from the queue, the benchmark's launch shape), max-pool, bench.py's own action stream over its 300 preroll
+  steps and its default warm-up and timed window (405 steps);
+- 4,096 envs of mixed levels with the headline wrappers (256 workgroups of 16 waves, an env each);
+- the 65,536-env divergence-stress instance (16 envs a wave from the queue; its second frame buffer starts 4.03e9
   bytes in and ends past 2^33);
 - 4,096 raw consoles over 800 frames, past the point where the consoles run out of phase.
 The outputs are recorded on the device; a sample of envs (a fixed stride, the last env, and envs whose episodes
@@ -158,8 +158,8 @@ def _run(names, modes, kw, seed, actions, stride, extra, two_pass=False, counter
 
 
 def test_headline_4096_envs_mixed_levels():
-    """Headline wrappers (sticky 0.25, no-op 30, skip 4, max-pool) at 4,096 envs, levels mixed: the launch shrinks to
-    256 one-wave workgroups (one per CU), and the last 64 waves leave their observations to k_obs_late."""
+    """Headline wrappers (sticky 0.25, no-op 30, skip 4, max-pool) at 4,096 envs, levels mixed: 256
+    workgroups of 16 waves, an env each."""
     from fast_mario_env_amd import ALL_LEVELS
     n, T = 4096, 50
     lv = np.random.default_rng(11).integers(0, 32, n)
@@ -175,8 +175,8 @@ def test_divergence_stress_65536_envs():
     """The divergence-stress instance at its full size: 65,536 envs, levels drawn from default_rng(7) over the 32
     world-stage pairs, rom_mode cycled over the four variants per env, sticky 0.25, no-op 30, skip 4, no
     max-pool; per env, action 2 (right + A) with p = 0.5, else uniform over 0..6. 330 steps: as far as bench.py's
-    stress line (300 preroll steps, then its warm-up and timed window), where busy runs in one env of a wave set the
-    kernel's time."""
+    stress line (300 preroll steps, then its warm-up and timed window), where busy runs set the
+    kernel's end."""
     from fast_mario_env_amd import ALL_LEVELS
     n, T = 65536, 330
     lv = np.random.default_rng(7).integers(0, 32, n)
@@ -191,9 +191,8 @@ def test_divergence_stress_65536_envs():
 
 
 def test_ordered_launch_40960_envs_every_env_vs_oracle():
-    """Past 32,768 envs on 256 CUs k_step has more blocks than CUs, and each step launches its block groups in the
-    order k_work and k_order derive from the last step's work (k_step_ordered): 40,960 envs (320 groups) of mixed
-    levels, every env's observation, reward, done flags and info against 16 oracle instances each step, so a group
+    """Past one env a wave the waves take envs from a queue in the order of their last step's work: 40,960 envs of mixed
+    levels, every env's observation, reward, done flags and info against 16 oracle instances each step, so an env
     that ran twice or not at all in a step would show."""
     from fast_mario_env_amd import ALL_LEVELS, HipVecEnv
     n, T, m = 40960, 6, 2560
@@ -225,8 +224,8 @@ def test_ordered_launch_40960_envs_every_env_vs_oracle():
 
 def test_headline_32768_envs_bench_stream():
     """The measured configuration itself: 32,768 envs of 1-1 with the headline wrappers (sticky 0.25, no-op 30,
-    skip 4, max-pool, stack 4, seed 0), launched as bench.py launches it (2,048 waves in 256 workgroups of 8 waves,
-    two waves per SIMD), driven by bench.py's own action stream for its 300 preroll steps and its default warm-up
+    skip 4, max-pool, stack 4, seed 0), launched as bench.py launches it (256 workgroups of 16 waves that take envs from
+    the queue), driven by bench.py's own action stream for its 300 preroll steps and its default warm-up
     and timed window (5 + 100 steps), so the steady state that the benchmark times is compared too. Two passes:
     the first finds the envs whose episodes ended, the second records a sample (every 1,021st env, the last one,
     24 envs with episode ends), replayed by one-env oracles."""
@@ -256,7 +255,7 @@ def _raw_frames(n, prologue, frames):
 def test_raw_4096_consoles():
     """Raw consoles at 4,096 (the raw-emulator workload's size), every frame rendered, over 800 frames: past
     frame ~200 the consoles run out of phase (deaths, level reloads and game-over screens at different points of
-    a frame), which is where long single-console instruction runs set the launch's length. Sampled consoles
+    a frame), which is where the slowest consoles set the launch's length. Sampled consoles
     against one CPU console each, every frame: RAM, palette screen and the whole machine state; the RGB24 screen
     every 10th frame."""
     from fast_mario_env_amd import HipRawNES, palette_rgb

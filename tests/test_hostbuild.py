@@ -1,6 +1,7 @@
 """The device code on the CPU under AddressSanitizer and UndefinedBehaviorSanitizer, against the golden traces.
 
-tests/hostbuild compiles the GPU kernels' device headers (nes_device.hpp, env_device.hpp, lane_kernels.hpp)
+tests/hostbuild compiles the GPU kernels' device headers (nes_device.hpp with cpu_gfx950.hpp's records, env_device.hpp,
+lane_kernels.hpp)
 as x86 C++ with one lane per env (its hip/hip_runtime.h stands in for HIP's) and drives the same lane bodies
 the kernels call (host_driver.cpp), every buffer sized exactly. Any out-of-bounds access or undefined behaviour
 in the device code aborts the run; the outputs must equal the digests the reference C++ wrote
