@@ -153,8 +153,8 @@ struct StepQueue {
 // the envs of bucket b, side s: list[(s * WORK_BUCKETS + b) * np ..]
 
 // What bounds it: scalar issue. A SIMD issues one scalar instruction per 4 cycles whichever of its waves it is from; the
-// headline step (32,768 envs of 1-1) is 98,000 scalar, 68,000 vector and 15,000 branch instructions per env, of which
-// the 5,150 6502 instructions are about 45,000 scalar ones (scalar issue 71% busy, vector 49%). Why one console per wave, against
+// headline step (32,768 envs of 1-1) is 99,000 scalar, 67,000 vector and 15,000 branch instructions per env, of which
+// the 5,150 6502 instructions are about 45,000 scalar ones (scalar issue 71% busy, vector 48%). Why one console per wave, against
 // 16 per wave in lockstep (4 lanes each, every opcode's work as selects, 15 to 12 of 16 consoles active): a lockstep
 // iteration issues ~470 instructions for ~12 6502 instructions but each env waits for all of them; here a 6502
 // instruction is ~17 instructions and nothing waits for another console. Measured when it came (k_step, the same
@@ -600,7 +600,8 @@ __global__ void __launch_bounds__(256, 2) k_policy_conv1(const uint8_t* obs, con
 // The second and third layers: the weight is (64, KS, KS, CI), so K = (kh, kw, ci) and a step is 16 channels of one
 // input pixel. IMGS images at a time: their output pixels in one row of tiles, the even and odd waves the two halves of
 // the output channels, the block's two pairs of waves every second tile. A pixel takes 16 bytes more than its
-// channels in LDS, so that the 8 lanes of a 16-byte read are in different banks.
+// channels in LDS, so that the lanes of a 16-byte read are in different banks along an output row; across its end they
+// still meet (bank conflicts on over a quarter of the third layer's cycles).
 template <int CI, int KS, int ST, int HI, int HO, int IMGS>
 __global__ void __launch_bounds__(256, 2) k_policy_conv(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
                                                         uint16_t* y, int64_t n, int wide) {
@@ -667,6 +668,8 @@ constexpr int CONV2_IMGS = 2, CONV3_IMGS = 5;
 // layer's 81 reads at p times a pixel's words, modulo the banks, across its rows too. Operands, sums and their order are
 // those of the two kernels above, and so are the results. 300 / 32,768 images: 22 / 669 us as two kernels, 16.5 /
 // 535 here (whole images at a time, all waves staging before the products: 16 / 578; operands read one step ahead: 606).
+// No unit is full: matrix cores 38% busy, LDS accesses about half of the cycles (a quarter of it bank conflicts), vector
+// issue 33%; a wave waits 40% of its time, with two a SIMD.
 __global__ void __launch_bounds__(512, 2) k_policy_conv12(const uint8_t* obs, const uint16_t* w1, const uint16_t* bias1,
                                                           const uint16_t* w2, const uint16_t* bias2, uint16_t* y, int64_t n) {
     constexpr int ROWS = 44, CH = ROWS * 84 / 4, WORDS = 4 * CH, PER = (WORDS + 511) / 512;   // 4-pixel words of a half
