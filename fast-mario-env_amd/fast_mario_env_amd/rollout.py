@@ -107,12 +107,20 @@ def _transformed(*ts):
     torch's default device), tracing or compiling. torch keeps most of it under private names: without one of them
     the answer is yes, and the layers' own operations run."""
     torch = _torch()
+    C = torch._C
     try:
-        device_mode = getattr(getattr(torch.utils, "_device", None), "DeviceContext", ())
-        return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.autograd.forward_ad._current_level >= 0
-                or torch._C._len_torch_dispatch_stack() > 0
-                or any(not isinstance(m, device_mode) for m in torch.overrides._get_current_function_mode_stack())
-                or any(torch._C._functorch.is_functorch_wrapped_tensor(t) for t in ts))
+        if (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.autograd.forward_ad._current_level >= 0
+                or C._len_torch_dispatch_stack() > 0):
+            return True
+        if C._len_torch_function_stack() > 0:
+            device_mode = getattr(getattr(torch.utils, "_device", None), "DeviceContext", ())
+            if any(not isinstance(m, device_mode) for m in torch.overrides._get_current_function_mode_stack()):
+                return True
+        wrapped = C._functorch.is_functorch_wrapped_tensor
+        for t in ts:
+            if wrapped(t):
+                return True
+        return False
     except AttributeError:
         return True
 

@@ -57,10 +57,13 @@ def test_what_follows_tensor_operations_is_seen(monkeypatch):
     torch.vmap(lambda t: (seen.append(_transformed(t)), t)[1])(torch.ones(2, 3))
     assert seen == [True]
     for owner, name in ((torch.autograd.forward_ad, "_current_level"), (torch._C, "_len_torch_dispatch_stack"),
-                        (torch.overrides, "_get_current_function_mode_stack"), (torch._C, "_functorch")):
+                        (torch._C, "_len_torch_function_stack"), (torch._C, "_functorch")):
         with monkeypatch.context() as m:
             m.delattr(owner, name)
             assert _transformed(x), name
+    with monkeypatch.context() as m, torch.device("cpu"):
+        m.delattr(torch.overrides, "_get_current_function_mode_stack")
+        assert _transformed(x)
     assert not _transformed(x)
 
 
